@@ -18,6 +18,7 @@ namespace {
 
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ uint32_t pk_max_u16(uint32_t a, uint32_t b) {
@@ -54,14 +55,22 @@ __device__ __forceinline__ float wave_max(float v) { /* v >= 0 in every lane: th
     return __uint_as_float(wave_max(__float_as_uint(v)));
 }
 
+// Sum in the order of a butterfly over lane distances 32, 16, 8, 4, 2, 1, the order that the LayerNorm's values rest on: an
+// fp32 sum in another order moves single fp16 results, and with them int4 codes.  (From the fourth step on lanes 8 apart hold
+// equal values, so a rotation by 4 within the row of 16 meets the same number as an exchange at distance 4.)
+constexpr int kDppRotate8 = 0x128, kDppRotate4 = 0x124;
 __device__ __forceinline__ float wave_sum(float v) {
-    v += __uint_as_float(dpp<kDppSwap1, 0xF, false>(0u, __float_as_uint(v)));
+#if defined(__HIP_DEVICE_COMPILE__)
+    u32x2 r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(r.x) + __uint_as_float(r.y);
+    r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(r.x) + __uint_as_float(r.y);
+#endif
+    v += __uint_as_float(dpp<kDppRotate8, 0xF, false>(0u, __float_as_uint(v)));
+    v += __uint_as_float(dpp<kDppRotate4, 0xF, false>(0u, __float_as_uint(v)));
     v += __uint_as_float(dpp<kDppSwap2, 0xF, false>(0u, __float_as_uint(v)));
-    v += __uint_as_float(dpp<kDppHalfMirror, 0xF, false>(0u, __float_as_uint(v)));
-    v += __uint_as_float(dpp<kDppMirror, 0xF, false>(0u, __float_as_uint(v)));
-    v += __uint_as_float(dpp<kDppBcast15, 0xA, false>(0u, __float_as_uint(v)));
-    v += __uint_as_float(dpp<kDppBcast31, 0xC, false>(0u, __float_as_uint(v)));
-    return __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(__float_as_uint(v)), 63)));
+    v += __uint_as_float(dpp<kDppSwap1, 0xF, false>(0u, __float_as_uint(v)));
+    return __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(__float_as_uint(v)))));
 }
 
 // fmaxf semantics of the reference's reduction: a NaN operand is ignored.
@@ -282,7 +291,6 @@ __device__ __forceinline__ void quantize_held_row(const u32x4 (&v)[NCH], int lan
 // M stay unwritten (the GEMM never stores them); K is padded to 128 with zeros.
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned int u32x6 __attribute__((ext_vector_type(6)));
-typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 constexpr int kBf6Rows = 8;          /* rows (= waves) per workgroup of the bf6 quantizers */
 constexpr int kStringsPerGroup = 64; /* 2048 k = 64 strings of 32 k per row and group */
 constexpr int kStringBytes = 24;
@@ -512,12 +520,6 @@ constexpr int ln_full_chunks(int nch) {
     return prev;
 }
 
-// sum / K with one correction step on the product with the (1 ulp) reciprocal of K
-__device__ __forceinline__ float over_k(float sum, float k, float inv_k) {
-    const float q = sum * inv_k;
-    return __builtin_fmaf(__builtin_fmaf(-k, q, sum), inv_k, q);
-}
-
 // LayerNorm over the row (fp32 statistics, no affine) followed by the block's
 // modulation, fused in front of the quantizer -- the producer of the attn1 and
 // FFN-up inputs (dit_block.py:100, :110 of the reference):
@@ -564,8 +566,7 @@ __global__ __launch_bounds__((FMT == 1 ? kBf6Rows : kRowsPerBlock) * kWaveSize) 
             sum = __builtin_fmaf(static_cast<float>(h[1]), one, sum);
         }
     }
-    const float fk = static_cast<float>(K), inv_k = __builtin_amdgcn_rcpf(fk);
-    const float mean = over_k(wave_sum(sum), fk, inv_k);
+    const float mean = wave_sum(sum) / static_cast<float>(K);
     // Each pass converts the fp16 row again: the compiler would otherwise keep the 8 * NCH converted floats of one
     // pass for the next (80 registers for a 5120-wide row, a workgroup per CU less); the empty asm makes the row
     // a new value for it.
@@ -586,9 +587,7 @@ __global__ __launch_bounds__((FMT == 1 ? kBf6Rows : kRowsPerBlock) * kWaveSize) 
             }
         }
     }
-    // 1 / sqrt(var + eps): the hardware's value (1 ulp) and one Newton step
-    const float var_eps = over_k(wave_sum(sq), fk, inv_k) + eps, r0 = __builtin_amdgcn_rsqf(var_eps);
-    const float rstd = __builtin_fmaf(r0 * 0.5f, __builtin_fmaf(-var_eps * r0, r0, 1.0f), r0);
+    const float rstd = 1.0f / __builtin_sqrtf(wave_sum(sq) / static_cast<float>(K) + eps);
 #pragma unroll
     for (int c = 0; c < NCH; ++c) asm volatile("" : "+v"(v[c]));
 

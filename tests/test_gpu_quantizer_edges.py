@@ -74,6 +74,65 @@ def test_gelu_quantizer_row_kinds(K, clip):
     assert np.array_equal(rows_of_blocks(blocks, len(x), K), want_q.astype(np.float64))
 
 
+def _round_fma(a, b, c):
+    """fl32(a * b + c) of float32 arrays: the sum in double, its last bit made odd where the addition was inexact, so that
+    the second rounding cannot tie."""
+    p, c = a.astype(np.float64) * b.astype(np.float64), c.astype(np.float64)
+    s = p + c
+    t = s - p
+    err = (p - (s - t)) + (c - t)
+    even = (s.view(np.int64) & 1) == 0
+    return np.where((err != 0) & even, np.nextafter(s, np.where(err > 0, np.inf, -np.inf)), s).astype(np.float32)
+
+
+def _wave_sum(lanes):
+    for distance in (32, 16, 8, 4, 2, 1):
+        lanes = lanes + lanes[:, np.arange(64) ^ distance]
+    assert (lanes == lanes[:, :1]).all()
+    return lanes[:, 0]
+
+
+def layer_norm_as_defined(x, a, b, eps, mode):
+    """The fused LayerNorm's fp32 arithmetic, operation by operation: lane l of a row holds elements 512 c + 8 l ... + 7 and
+    adds them in that order, lanes are added at distances 32, 16, 8, 4, 2, 1, every division and square root is rounded
+    correctly."""
+    M, K = x.shape
+    xf = x.astype(np.float32)
+    total, sq = np.zeros((M, 64), np.float32), np.zeros((M, 64), np.float32)
+    places = [(np.arange(64) * 8 + 512 * c + e) for c in range((K + 511) // 512) for e in range(8)]
+    for k in places:
+        total[:, k < K] += xf[:, k[k < K]]
+    mean = _wave_sum(total) / np.float32(K)
+    d = xf - mean[:, None]
+    for k in places:
+        sq[:, k < K] = _round_fma(d[:, k[k < K]], d[:, k[k < K]], sq[:, k < K])
+    rstd = np.float32(1) / np.sqrt(_wave_sum(sq) / np.float32(K) + np.float32(eps))
+    n = d * rstd[:, None]
+    if mode == "affine":
+        return (n * a.astype(np.float32) + b.astype(np.float32)).astype(np.float16)
+    return n.astype(np.float16) * (np.float16(1) + a) + b
+
+
+@pytest.mark.parametrize("mode", ["modulate", "affine"])
+@pytest.mark.parametrize("K", [64, 192, 512, 1088, 1536, 2048, 3072, 5120, 8192 + 64, 13824])
+def test_layer_norm_sums_in_its_defined_order(K, mode):
+    """Bit for bit, rows with and without a mean: a sum in another order moves the last bits, and int4 codes with them."""
+    from dsaquant_amd import fused_ops
+
+    rng = np.random.default_rng(K)
+    x = (rng.standard_normal((300, K)) * 3 + rng.standard_normal((300, 1))).astype(np.float16)
+    x[:, rng.permutation(K)[: max(1, K // 100)]] *= np.float16(20)
+    a, b = ((0.1 * rng.standard_normal((1, K))).astype(np.float16) for _ in range(2))
+    want = layer_norm_as_defined(x, a, b, 1e-6, mode)
+    pre = fused_ops.LnInput(t16(x), t16(a), t16(b), 1e-6, mode)
+    assert np.array_equal(pre.materialize().cpu().numpy().view(np.uint16), want.view(np.uint16))
+    want_s = O.np_row_scale(want, 0.95)
+    want_q = O.np_quantize_rows(want, want_s)
+    blocks, sc = pre.quantize(0.95, bf6=True)
+    assert np.array_equal(sc.cpu().numpy().view(np.uint16), want_s.view(np.uint16))
+    assert np.array_equal(rows_of_blocks(blocks, len(x), K), want_q.astype(np.float64))
+
+
 @pytest.mark.parametrize("N,K", [(128, 64), (128, 1088), (1152, 448), (640, 2112), (256, 5120 + 64), (128, 9216), (128, 9216 + 64), (1024 + 128, 13824)])
 def test_pack_weight_edges(N, K):
     """One-pass weight packing: row tiles beyond and within a full group of eight 128-row blocks, rows on both sides of
