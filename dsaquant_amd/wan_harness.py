@@ -78,9 +78,10 @@ class RMSNormAcrossHeads(nn.Module):
         return (xf * torch.rsqrt(xf.pow(2).mean(dim=-1, keepdim=True) + self.eps)).to(x.dtype) * self.weight
 
 
-def rope_frequencies(head_dim: int, f: int, h: int, w: int, device) -> torch.Tensor:
-    """complex64 [f*h*w, 1, head_dim/2]: frames get head_dim - 2*(head_dim//3) channels, rows and columns head_dim//3 each."""
-    if torch.device(device).type == "cuda":  # made where it is used: the host would compute and copy it in every forward
+def rope_frequencies(head_dim: int, f: int, h: int, w: int, device, kernel: bool = False) -> torch.Tensor:
+    """complex64 [f*h*w, 1, head_dim/2]: frames get head_dim - 2*(head_dim//3) channels, rows and columns head_dim//3 each.
+    ``kernel``: made on a GPU by the library, the same values; without it the host computes and copies them."""
+    if kernel and torch.device(device).type == "cuda":
         from . import fused_ops
 
         return fused_ops.rope_table(head_dim, f, h, w, device)
@@ -393,7 +394,7 @@ class WanDiT(nn.Module):
         """latent [1, C, F, H, W] fp16, timestep [1], context [1, 512, text_dim] -> noise prediction like latent."""
         a = self.args
         _, _, f, h, w = latent.shape
-        freqs = rope_frequencies(a.head_dim, f // a.patch_size[0], h // a.patch_size[1], w // a.patch_size[2], latent.device)
+        freqs = rope_frequencies(a.head_dim, f // a.patch_size[0], h // a.patch_size[1], w // a.patch_size[2], latent.device, self._kernel_mode())
         x = self.patch_embedding_mlp(self.patchify(latent))
         if self._kernel_mode() and _plain_fp16(x) and timestep.is_cuda and timestep.dim() == 1 and not _needs_grad(timestep):
             from . import fused_ops

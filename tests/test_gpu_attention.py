@@ -91,7 +91,7 @@ def test_norm_and_rope_against_the_torch_operations(B, fhw, K, H):
     wide = (3 * torch.randn((B, L, 2 * K), generator=g, device=DEV)).half()
     xs, ws = wide.split(K, dim=-1), [(1 + 0.1 * torch.randn(K, generator=g, device=DEV)).half() for _ in range(2)]
     host = W.rope_frequencies(K // H, *fhw, "cpu")
-    freqs = W.rope_frequencies(K // H, *fhw, DEV)
+    freqs = f.rope_table(K // H, *fhw, DEV)
     # double precision on both sides, rounded to float: equal but for a rounding boundary between two double results
     assert (torch.view_as_real(freqs).cpu() - torch.view_as_real(host)).abs().max().item() <= 2.0 ** -23
     assert f.rms_norm_rope_supported(xs, ws, freqs, H)
@@ -182,3 +182,27 @@ def test_harness_head_runs_on_the_layernorm_kernel():
         fused_ops.LnInput.materialize, W._plain_fp16 = materialize, plain
     # statistics in another order: isolated fp16 steps of the normalised tokens
     assert ((got.float() - want.float()).norm() / want.float().norm()).item() <= 2.0 ** -11
+
+
+def test_harness_without_quantized_linears_needs_nothing_from_the_library(monkeypatch):
+    """A model whose linears are torch's runs on the GPU without the library, and with the same table of rotations."""
+    from dataclasses import replace
+
+    from dsaquant_amd import _lib, fused_ops
+    from dsaquant_amd import wan_harness as W
+    from dsaquant_amd.kernels import vdm_w4a4 as v
+
+    for shape in ((3, 30, 52), (21, 1, 1), (1, 5, 7)):
+        assert torch.equal(fused_ops.rope_table(128, *shape, DEV), W.rope_frequencies(128, *shape, DEV))
+
+    def refuse(*args, **kwargs):
+        raise RuntimeError("the library was asked for")
+
+    monkeypatch.setattr(v, "_load_ext", refuse)
+    monkeypatch.setattr(_lib, "load", refuse)
+    args = replace(W.WAN21_1P3B, num_layers=1, num_heads=2, ffn_dim=512, text_dim=128)
+    torch.manual_seed(8)
+    model = W.WanDiT(args).half().to(DEV)
+    latent, ctx = torch.randn((1, 16, 1, 6, 10), device=DEV).half(), torch.randn((1, 9, args.text_dim), device=DEV).half()
+    with torch.no_grad():
+        assert torch.isfinite(model(latent, torch.tensor([500.0], device=DEV), ctx)).all()
