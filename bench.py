@@ -563,10 +563,11 @@ def main():
             import bench_dit
 
             with contextlib.redirect_stdout(sys.stderr):  # (the loader reports what it loaded; this program prints one line)
-                c4 = bench_dit.measure(torch, steps=5, warmup_steps=1, fuse_ln=True, fuse_gelu=True, fuse_residual=True, reuse_context=True)
+                c4 = bench_dit.measure(torch, steps=5, warmup_steps=1, fuse_ln=True, fuse_gelu=True, fuse_residual=True, reuse_context=True,
+                                       fuse_attention=True)
                 c4_plain = bench_dit.measure(torch, steps=2, warmup_steps=0)
             result["config4"] = {"workload": "Wan-2.1 1.3B DiT, 30 blocks, 32760 tokens, cond + uncond, 5 steps after 1 warm-up step; LayerNorm, GELU and "
-                                             "residual updates fused into the W4A4 kernels, context quantized once",
+                                             "residual updates fused into the W4A4 kernels, context quantized once, attention on the library's kernel",
                                  "ms_per_step": c4["ms_per_step"], "w4a4_share": c4["value"], "attention_share": c4["attention_share"],
                                  "w4a4_ms_per_forward": c4["w4a4_ms_per_forward"], "attention_ms_per_forward": c4["attention_ms_per_forward"],
                                  "w4a4_calls_per_forward": c4["w4a4_calls_per_forward"], "forwards": c4["forwards"],

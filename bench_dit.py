@@ -22,7 +22,7 @@ sys.path.insert(0, str(Path(__file__).resolve().parent))
 
 
 def measure(torch, steps=5, layers=30, frames=21, height=60, width=104, boundary_ratio=0.4, model_name="1.3B", fuse_ln=False,
-            fuse_residual=False, fuse_gelu=False, reuse_context=False, warmup_steps=0):
+            fuse_residual=False, fuse_gelu=False, reuse_context=False, fuse_attention=False, warmup_steps=0):
     """Build the harness model, run ``warmup_steps`` untimed denoise steps (and always one untimed forward), then
     time ``steps`` denoise steps; returns the result dict."""
     from dsaquant_amd import wan_harness as W
@@ -37,11 +37,13 @@ def measure(torch, steps=5, layers=30, frames=21, height=60, width=104, boundary
     t0 = time.perf_counter()
     model = W.build_quantized(wargs, dev, seed=0)
     build_s = time.perf_counter() - t0
-    saved = (W.FeedForward.fuse_gelu, W.Block.fuse_ln, W.Block.fuse_residual, W.WanDiT.reuse_context, W.Attention.cache_cross_kv)
+    saved = (W.FeedForward.fuse_gelu, W.Block.fuse_ln, W.Block.fuse_residual, W.WanDiT.reuse_context, W.Attention.cache_cross_kv,
+             W.Attention.fuse_attention, W.WanDiT.fuse_head)
     W.FeedForward.fuse_gelu = bool(fuse_gelu)
     W.Block.fuse_ln = bool(fuse_ln)
     W.Block.fuse_residual = bool(fuse_residual)
     W.WanDiT.reuse_context = W.Attention.cache_cross_kv = bool(reuse_context)
+    W.Attention.fuse_attention = W.WanDiT.fuse_head = bool(fuse_attention)
     try:
         n_quant = sum(isinstance(m, QuantLinear) for m in model.modules())
         n_fused = sum(isinstance(m, W.Attention) and m.use_fused_qkv_kernel for m in model.modules())
@@ -70,7 +72,8 @@ def measure(torch, steps=5, layers=30, frames=21, height=60, width=104, boundary
         cnt = timers.counts()
         assert torch.isfinite(out).all()
     finally:
-        W.FeedForward.fuse_gelu, W.Block.fuse_ln, W.Block.fuse_residual, W.WanDiT.reuse_context, W.Attention.cache_cross_kv = saved
+        (W.FeedForward.fuse_gelu, W.Block.fuse_ln, W.Block.fuse_residual, W.WanDiT.reuse_context, W.Attention.cache_cross_kv,
+         W.Attention.fuse_attention, W.WanDiT.fuse_head) = saved
     return {
         "metric": "share of denoise-step time in the W4A4 kernels, Wan-2.1 %s DiT, %d steps" % (model_name, steps),
         "value": round(tot.get("w4a4", 0.0) / (wall * 1e3), 4), "unit": "fraction of wall time",
@@ -80,7 +83,7 @@ def measure(torch, steps=5, layers=30, frames=21, height=60, width=104, boundary
         "w4a4_calls_per_forward": cnt.get("w4a4", 0) // forwards, "attention_calls_per_forward": cnt.get("attention", 0) // forwards,
         "tokens_per_forward": tokens, "timesteps": ts, "quant_linears": n_quant, "fused_attention_modules": n_fused,
         "layers": layers, "fuse_gelu": bool(fuse_gelu), "fuse_ln": bool(fuse_ln), "fuse_residual": bool(fuse_residual),
-        "reuse_context": bool(reuse_context), "build_s": round(build_s, 1), "data": "synthetic", "n_gpus": 1,
+        "reuse_context": bool(reuse_context), "fuse_attention": bool(fuse_attention), "build_s": round(build_s, 1), "data": "synthetic", "n_gpus": 1,
     }
 
 
@@ -99,13 +102,16 @@ def main():
     ap.add_argument("--fuse-gelu", action="store_true", help="evaluate the FFN's GELU inside the second linear's activation quantizer")
     ap.add_argument("--reuse-context", action="store_true",
                     help="embed each context once, keep the cross-attention K/V per prompt, quantize a context once per forward")
+    ap.add_argument("--fuse-attention", action="store_true",
+                    help="run q/k norms, rotary embedding, attention and the head's LayerNorm on the library's kernels")
     args = ap.parse_args()
 
     import torch
 
     print(json.dumps(measure(torch, steps=args.steps, layers=args.layers, frames=args.frames, height=args.height, width=args.width,
                              boundary_ratio=args.boundary_ratio, model_name=args.model, fuse_ln=args.fuse_ln, fuse_residual=args.fuse_residual,
-                             fuse_gelu=args.fuse_gelu, reuse_context=args.reuse_context, warmup_steps=args.warmup_steps)))
+                             fuse_gelu=args.fuse_gelu, reuse_context=args.reuse_context,
+                             fuse_attention=args.fuse_attention, warmup_steps=args.warmup_steps)))
 
 
 if __name__ == "__main__":

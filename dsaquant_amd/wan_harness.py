@@ -179,6 +179,11 @@ class Attention(nn.Module):
     # step of a prompt: keep them per context tensor (held weakly: a new tensor at a recycled address is a miss).
     cache_cross_kv = False
 
+    # Run the q/k norms, the rotary embedding and the attention on the library's kernels, where the projections run on them
+    # (on the GPU, without autograd).  As exact as the torch operations (attention 2.84e-4 from 64 bits, both), but not their
+    # bits, and int4 quantizers downstream amplify that: up to 0.015 of the output (2-norm) after one block, 0.05 after two.
+    fuse_attention = False
+
     def _context_kv(self, context):
         """K (normalised) and V of the cross-attention context, a tensor or a SharedContext."""
         from . import fused_ops
@@ -235,7 +240,7 @@ class Attention(nn.Module):
             q, k = apply_rope(q, freqs), apply_rope(k, freqs)
         if timers is not None:
             timers.start("attention")
-        if self._kernel_mode() and fused_ops.attention_supported(q, k, v):
+        if self._on_kernels() and fused_ops.attention_supported(q, k, v):
             o = fused_ops.attention(q, k, v).flatten(2, 3)
         else:
             o = F.scaled_dot_product_attention(q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2), dropout_p=0.0, is_causal=False)
@@ -244,15 +249,13 @@ class Attention(nn.Module):
             timers.stop("attention")
         return _project_and_update(self.to_out[0], o, None, residual, gate)
 
-    # Where the projections run on the W4A4 kernels -- on the GPU, without autograd -- the norms, the rotary embedding and
-    # the attention between them run on the library's kernels too; everywhere else they are torch operations.
-    def _kernel_mode(self) -> bool:
-        return all(getattr(layer, "use_vdm_kernel", False) for layer in (self.to_q, self.to_k, self.to_v))
+    def _on_kernels(self) -> bool:
+        return self.fuse_attention and all(getattr(layer, "use_vdm_kernel", False) for layer in (self.to_q, self.to_k, self.to_v))
 
     def _kernel_norm(self, tensors, norms, freqs) -> bool:
         from . import fused_ops
 
-        return (self._kernel_mode() and all(type(n) is RMSNormAcrossHeads and n.eps == norms[0].eps for n in norms)
+        return (self._on_kernels() and all(type(n) is RMSNormAcrossHeads and n.eps == norms[0].eps for n in norms)
                 and fused_ops.rms_norm_rope_supported(tensors, [n.weight for n in norms], freqs, self.heads))
 
     def _normed(self, x, norm):
@@ -371,7 +374,10 @@ class WanDiT(nn.Module):
         x = tokens.reshape(1, f // p1, h // p2, w // p3, p1, p2, p3, c)
         return x.permute(0, 7, 1, 4, 2, 5, 3, 6).reshape(1, c, f, h, w)
 
-    # The blocks run on the W4A4 kernels: what stands between them and around them may do so too.
+    # The last LayerNorm and its modulation in one kernel, the one of the blocks' ``fuse_ln`` (last bits as there).
+    fuse_head = False
+
+    # The blocks run on the W4A4 kernels: the tables in front of them may be made on the GPU by the library, the same values.
     def _kernel_mode(self) -> bool:
         return len(self.blocks) > 0 and getattr(self.blocks[0].ffn.up, "use_vdm_kernel", False)
 
@@ -407,7 +413,7 @@ class WanDiT(nn.Module):
         for blk in self.blocks:
             x = blk(x, ctx, tproj, freqs, timers)
         shift, scale = (self.scale_shift_table.to(temb.dtype) + temb[:, None, :]).unbind(dim=1)
-        if self._kernel_mode() and self.blocks[0].fuse_ln and _plain_fp16(x) and not _needs_grad(x, scale, shift):
+        if self.fuse_head and self._kernel_mode() and _plain_fp16(x) and not _needs_grad(x, scale, shift):
             # the kernel of the blocks' LayerNorms, written out instead of quantized: six passes over the tokens become one
             from .fused_ops import LnInput
 

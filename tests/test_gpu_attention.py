@@ -118,6 +118,8 @@ def test_harness_attention_runs_on_the_kernels():
 
     args = replace(W.WAN21_1P3B, num_layers=1, num_heads=2, ffn_dim=512, text_dim=128)
     model = W.build_quantized(args, DEV, seed=3)
+    for module in (model.blocks[0].attn1, model.blocks[0].attn2):
+        module.fuse_attention = True
     g = torch.Generator(device=DEV).manual_seed(4)
     latent = torch.randn((1, 16, 3, 10, 14), generator=g, device=DEV).half()
     ctx, t = torch.randn((1, 77, args.text_dim), generator=g, device=DEV).half(), torch.tensor([500.0], device=DEV)
@@ -165,6 +167,7 @@ def test_harness_head_runs_on_the_layernorm_kernel():
     model = W.build_quantized(args, DEV, seed=5)
     for block in model.blocks:
         block.fuse_ln = True
+    model.fuse_head = True
     g = torch.Generator(device=DEV).manual_seed(6)
     latent = torch.randn((1, 16, 1, 6, 10), generator=g, device=DEV).half()
     ctx, t = torch.randn((1, 77, args.text_dim), generator=g, device=DEV).half(), torch.tensor([500.0], device=DEV)
@@ -206,3 +209,34 @@ def test_harness_without_quantized_linears_needs_nothing_from_the_library(monkey
     latent, ctx = torch.randn((1, 16, 1, 6, 10), device=DEV).half(), torch.randn((1, 9, args.text_dim), device=DEV).half()
     with torch.no_grad():
         assert torch.isfinite(model(latent, torch.tensor([500.0], device=DEV), ctx)).all()
+
+
+def test_harness_keeps_the_torch_operations_between_the_linears_unless_asked(monkeypatch):
+    """Norms, rotation, attention and the head's LayerNorm on the library's kernels are as exact as the torch operations but not
+    their bits, which the quantizers after them amplify: a forward takes them only with the module's switch, whatever else
+    is fused."""
+    from dataclasses import replace
+
+    from dsaquant_amd import fused_ops
+    from dsaquant_amd import wan_harness as W
+
+    args = replace(W.WAN21_1P3B, num_layers=2, num_heads=2, ffn_dim=512, text_dim=128)
+    model = W.build_quantized(args, DEV, seed=9)
+    for block in model.blocks:
+        block.fuse_ln = block.fuse_residual = block.ffn.fuse_gelu = True
+    g = torch.Generator(device=DEV).manual_seed(10)
+    latent = torch.randn((1, 16, 2, 10, 14), generator=g, device=DEV).half()
+    ctx, t = torch.randn((1, 77, args.text_dim), generator=g, device=DEV).half(), torch.tensor([500.0], device=DEV)
+
+    calls = []
+    for owner, name in ((fused_ops, "attention"), (fused_ops, "rms_norm_rope"), (fused_ops.LnInput, "materialize")):
+        kernel = getattr(owner, name)
+        monkeypatch.setattr(owner, name, lambda *a, kernel=kernel, name=name: (calls.append(name), kernel(*a))[1])
+    with torch.no_grad():
+        model(latent, t, ctx)
+        assert calls == []
+        model.fuse_head = True
+        for block in model.blocks:
+            block.attn1.fuse_attention = block.attn2.fuse_attention = True
+        model(latent, t, ctx)
+    assert calls == ["rms_norm_rope", "attention", "rms_norm_rope", "rms_norm_rope", "attention"] * 2 + ["materialize"]
