@@ -137,6 +137,12 @@ def _plain_fp16(x: torch.Tensor) -> bool:
     return x.is_cuda and x.dtype == torch.float16
 
 
+def _is_plain_norm(module: nn.Module) -> bool:
+    # calling it is its class's forward and nothing else: a kernel given its weight may stand in for the call
+    return (type(module) is RMSNormAcrossHeads and "forward" not in module.__dict__ and not module._forward_hooks
+            and not module._forward_pre_hooks and not nn.modules.module._has_any_global_hook())
+
+
 def _version_of(tensor: torch.Tensor):
     return None if tensor.is_inference() else tensor._version
 
@@ -255,7 +261,7 @@ class Attention(nn.Module):
     def _kernel_norm(self, tensors, norms, freqs) -> bool:
         from . import fused_ops
 
-        return (self._on_kernels() and all(type(n) is RMSNormAcrossHeads and n.eps == norms[0].eps for n in norms)
+        return (self._on_kernels() and all(_is_plain_norm(n) and n.eps == norms[0].eps for n in norms)
                 and fused_ops.rms_norm_rope_supported(tensors, [n.weight for n in norms], freqs, self.heads))
 
     def _normed(self, x, norm):

@@ -240,3 +240,33 @@ def test_harness_keeps_the_torch_operations_between_the_linears_unless_asked(mon
             block.attn1.fuse_attention = block.attn2.fuse_attention = True
         model(latent, t, ctx)
     assert calls == ["rms_norm_rope", "attention", "rms_norm_rope", "rms_norm_rope", "attention"] * 2 + ["materialize"]
+
+
+@pytest.mark.parametrize("hook", ["forward", "forward_pre", "global", "replaced"])
+def test_harness_calls_norms_that_carry_hooks(hook):
+    """With the kernels switched on, a norm that more than its own forward hangs on is still called."""
+    from dataclasses import replace
+
+    from dsaquant_amd import wan_harness as W
+
+    args = replace(W.WAN21_1P3B, num_layers=1, num_heads=2, ffn_dim=512, text_dim=128)
+    model = W.build_quantized(args, DEV, seed=11)
+    attn = model.blocks[0].attn1
+    attn.fuse_attention = model.blocks[0].attn2.fuse_attention = True
+    seen, handle = [], None
+    if hook == "forward":
+        handle = attn.norm_k.register_forward_hook(lambda m, i, o: seen.append(m))
+    elif hook == "forward_pre":
+        handle = attn.norm_k.register_forward_pre_hook(lambda m, i: seen.append(m))
+    elif hook == "global":
+        handle = torch.nn.modules.module.register_module_forward_hook(lambda m, i, o: seen.append(m))
+    else:
+        plain = attn.norm_k.forward
+        attn.norm_k.forward = lambda x: (seen.append(attn.norm_k), plain(x))[1]
+    try:
+        with torch.no_grad():
+            model(torch.randn((1, 16, 1, 6, 10), device=DEV).half(), torch.tensor([500.0], device=DEV), torch.randn((1, 7, args.text_dim), device=DEV).half())
+    finally:
+        if handle is not None:
+            handle.remove()
+    assert attn.norm_k in seen
