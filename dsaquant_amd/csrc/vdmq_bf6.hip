@@ -98,7 +98,7 @@ using Bf6Small = Bf6Cfg<128, 128, 2, 2, 3, 2>;
 [[maybe_unused]] __device__ __forceinline__ bool map_tile(const Bf6TileMap &tm, int bid, int &tile_m, int &tile_n) {
     const int xcd = bid % kXcds, slot = bid / kXcds;
     const int st = bf6_tilemap_super(tm, xcd, slot >> tm.per_log2);
-    return st >= 0 && bf6_tilemap_locate(tm, st, slot & ((1 << tm.per_log2) - 1), tile_m, tile_n);
+    return st >= 0 && bf6_tilemap_locate_any(tm, st, slot & ((1 << tm.per_log2) - 1), tile_m, tile_n);
 }
 
 [[maybe_unused]] __device__ __forceinline__ v8i ld_frag(const uint8_t *p, uint32_t la, uint32_t lb) {
@@ -816,24 +816,34 @@ int launch_bf6_cfg(const uint8_t *xblocks, const __half *ascale, const uint8_t *
         }
     }
     // Problems whose tiles the chip holds at once (a tile per CU, or two of the small ones) take one round if every XCD gets
-    // its eighth.  Super-tiles of a whole XCD's places are too coarse for that: 37 x 12 small tiles are ten of them, which
-    // gave one XCD 104 tiles, two rounds, and four XCDs 32; and where each holds only a few tiles, these lie at the same
-    // places and went to the same CUs.  Super-tiles of 4 x 2 tiles, edges regrouped, dealt as contiguous runs of equal
-    // numbers of tiles (neighbours run at the same time, so K is not walked back and forth): M x N, K, us before / now:
-    // 4680 x 1536, 8960 62 / 43; 4680 x 1536, 1536 17.5 / 12; 6000 x 1280, 2048 23 / 14.5; 2560 x 2560, 2048 19.4 / 13.5;
-    // 128 x 10240, 5120 23.7 / 16.  Within 5 % of it: 4 x 4 and 8 x 2; 2 x 2 is slower on long K.  Kept as they were:
-    // problems that give no CU of the busiest XCD a second workgroup (small tiles: and every XCD one super-tile at most).
+    // its eighth and no CU two tiles before all have one.  Super-tiles of a whole XCD's places are too coarse for that: 37 x
+    // 12 small tiles are ten of them, which gave one XCD 104 tiles, two rounds, and four XCDs 32; and where each holds only a
+    // few tiles, these went to the same CUs.  So these problems take the strip order: equal runs, no empty place.  (Empty
+    // places, in super-tiles of 4 x 2 too, are workgroups that hold a CU's place until they have ended: 15 x 31 tiles in 80
+    // workgroups per XCD took 1.4 times what 64 take.)  M x N, K, us, whole-XCD super-tiles / 4 x 2 super-tiles / strips:
+    // 4680 x 1536, 8960 61 / 41 / 42; 4680 x 1536, 1536 17.4 / 12.0 / 11.9; 6000 x 1280, 2048 23.8 / 14.3 / 14.2; 1868 x
+    // 4224, 3072 21.3 / 23.8 / 19.0; 867 x 8320, 13824 69 / 85 / 63; 3800 x 4352, 5120 (255 big tiles) 58 / 55 / 38.  On 290
+    // shapes of 20 tiles up 0.87 of whole-XCD super-tiles in the geometric mean, 1.03 at most outside what follows; strips
+    // of four or six rows are up to 1.11 (an XCD's tiles far from square read more operand rows).
+    // Kept as they were: problems that give no CU of the busiest XCD a second workgroup (small tiles: and every XCD one
+    // super-tile at most), and those where any order gives some CUs a second one and this one not to more than a quarter
+    // (640 x 7808, 5120, 40 tiles on the busiest: 23.0 us, in strips 24.5).
     const int64_t all_tiles = static_cast<int64_t>(tm.tiles_m) * tm.tiles_n;
     const bool at_once = all_tiles <= kXcds * per;
-    const bool spread = at_once ? best_load > 32 || (Cfg::kOcc == 2 && tm.total_super > kXcds) : Cfg::kOcc == 2;
-    // (small tiles of more than one round are refilled as they end: 4 x 4 there, which reads fewer operand rows)
-    if (spread) bf6_tilemap_shape(tm, tiles_m, tiles_n, at_once ? 3 : 4, at_once ? 1 : 2, true);
+    const bool few_doubled = all_tiles > kXcds * 32 && best_load <= 40;
+    const bool spread = at_once ? !few_doubled && (best_load > 32 || (Cfg::kOcc == 2 && tm.total_super > kXcds)) : Cfg::kOcc == 2;
+    if (spread && at_once)
+        bf6_tilemap_strips(tm, tiles_m, tiles_n);
+    else if (spread) /* (small tiles of more than one round are refilled as they end: 4 x 4, which reads fewer operand rows) */
+        bf6_tilemap_shape(tm, tiles_m, tiles_n, 4, 2, true);
     const int places = 1 << tm.per_log2;
     const int64_t total_super = tm.total_super;
     if (best_load < 0 || total_super * per + kXcds * per > (int64_t(1) << 30))
         return fail(VDMQ_ESHAPE, "M x N = %lld x %lld needs more workgroups than one launch can hold", (long long)M, (long long)N);
-    tm.contig = 0;
-    for (int x = 0; x <= kXcds; ++x) tm.start[x] = 0;
+    if (tm.strips == 0) {
+        tm.contig = 0;
+        for (int x = 0; x <= kXcds; ++x) tm.start[x] = 0;
+    }
     int rounds = static_cast<int>(ceil_div(total_super, kXcds));
     // Long K and wide N: every XCD takes one contiguous run of the super-tile sequence (n fastest); consecutive
     // super-tiles of an XCD then share their token rows and, walking K in opposite directions, re-use what the
@@ -841,7 +851,7 @@ int launch_bf6_cfg(const uint8_t *xblocks, const __half *ascale, const uint8_t *
     // beyond L2 and 0...2 % less time for N = 13824 and 15360; with 20 tile columns or fewer (N = 5120, 3072) it
     // fetches 4 % more and is 3...5 % slower than taking turns.
     const bool contig = spread || (K >= 2048 && tm.tiles_n >= 48);
-    if (contig) rounds = bf6_tilemap_runs(tm, true);
+    if (contig && tm.strips == 0) rounds = bf6_tilemap_runs(tm, true);
     const dim3 grid(static_cast<unsigned>(rounds) * kXcds * places), block(Cfg::kWaves * 64);
     const bool stream_out = M * N * 2 > (int64_t(224) << 20);
     const bool has_tail = tail.gate != nullptr || tail.residual != nullptr;
@@ -899,7 +909,8 @@ int launch_bf6_cfg(const uint8_t *xblocks, const __half *ascale, const uint8_t *
                        static_cast<int>(M), static_cast<int>(N), static_cast<int>(bf6_kblocks(K)), ldo, tm, tail);
     const int rc = check_launch("gemm_bf6_kernel");
     if (rc == VDMQ_OK)
-        record_gemm_launch({VDMQ_KERNEL_GEMM_BF6, Cfg::BM, Cfg::BN, places >> tm.group_n_log2, 1 << tm.group_n_log2, tm.contig,
+        record_gemm_launch({VDMQ_KERNEL_GEMM_BF6, Cfg::BM, Cfg::BN, tm.strips > 0 ? static_cast<int>(ceil_div(tiles_m, tm.strips)) : places >> tm.group_n_log2,
+                            1 << tm.group_n_log2, tm.contig,
                             static_cast<int64_t>(grid.x)});
     return rc;
 }

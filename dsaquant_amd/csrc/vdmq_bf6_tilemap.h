@@ -14,6 +14,7 @@
 namespace vdmq {
 
 constexpr int kBf6Xcds = 8;
+constexpr int kBf6StripRows = 8;
 
 // The tiles_m x tiles_n grid of output tiles is cut into super-tiles of `per` = 1 << per_log2 places, one per CU of
 // an XCD, so that the XCD's CUs work on neighbouring tiles at the same time and share their operand rows in its L2:
@@ -30,6 +31,11 @@ constexpr int kBf6Xcds = 8;
 //
 // The sequence is main, right edge, bottom edge.  XCD x takes either every eighth super-tile (x, x + 8, ...) or, with
 // `contig`, the run [start[x], start[x + 1]).
+//
+// Strips (`strips` > 0) are the order for tiles that the chip holds at once, where an even share for every XCD is what
+// counts: strips of at most kBf6StripRows tile rows, as equal as they can be (the XCDs that got a lone row would share no
+// weights between its tiles), walked two columns at a time.  There a super-tile is one tile and none is empty: the runs
+// differ by one tile at most, and no workgroup is launched in vain.
 struct Bf6TileMap {
     int tiles_m, tiles_n;
     int per_log2, group_n_log2;
@@ -39,6 +45,8 @@ struct Bf6TileMap {
     int total_super;
     int contig;
     int start[kBf6Xcds + 1];
+    int strips;
+    uint32_t strip_inverse[2], pair_inverse[2]; /* [1]: of the strips with a row more */
 };
 
 // Shape part of the map (everything but contig / start) for the main shape (per >> gn_log2) x (1 << gn_log2).
@@ -60,6 +68,46 @@ VDMQ_TILEMAP_FN void bf6_tilemap_shape(Bf6TileMap &tm, int tiles_m, int tiles_n,
     tm.edge_m_cols = tm.edge_m_rows == 0 ? 1 : !regroup ? gn : (per / tm.edge_m_rows < 16 ? per / tm.edge_m_rows : 16);
     tm.n_edge_m = tm.edge_m_rows == 0 ? 0 : (tiles_n + tm.edge_m_cols - 1) / tm.edge_m_cols;
     tm.total_super = tm.n_main + tm.n_edge_n + tm.n_edge_m;
+    tm.strips = 0;
+}
+
+// n / d by the inverse 2^32 / d + 1, d >= 2: exact for n and d below 2^16.  (As divisions, the two that locate a tile are half
+// a microsecond in front of it.)
+VDMQ_TILEMAP_FN uint32_t bf6_tilemap_inverse(uint32_t d) { return static_cast<uint32_t>((uint64_t(1) << 32) / d + 1); }
+VDMQ_TILEMAP_FN int bf6_tilemap_quotient(int n, uint32_t inverse) { return static_cast<int>(static_cast<uint64_t>(static_cast<uint32_t>(n)) * inverse >> 32); }
+
+// The strip order, whole: shape, contig and start; for less than 2^15 tiles (with a single one, only 0 is divided by 1).
+// Strips with a row more come first: n_main of the tiles and n_edge_m of the tile rows are theirs, edge_m_rows are the rows
+// of each of the others.
+VDMQ_TILEMAP_FN void bf6_tilemap_strips(Bf6TileMap &tm, int tiles_m, int tiles_n) {
+    tm = Bf6TileMap{};
+    tm.tiles_m = tiles_m;
+    tm.tiles_n = tiles_n;
+    tm.group_n_log2 = 1;
+    tm.strips = (tiles_m + kBf6StripRows - 1) / kBf6StripRows;
+    const int low = tiles_m / tm.strips;
+    tm.edge_m_rows = low;
+    tm.n_edge_m = (tiles_m - low * tm.strips) * (low + 1);
+    tm.n_main = tm.n_edge_m * tiles_n;
+    for (int i = 0; i < 2; ++i) {
+        tm.strip_inverse[i] = bf6_tilemap_inverse(static_cast<uint32_t>((low + i) * tiles_n));
+        tm.pair_inverse[i] = bf6_tilemap_inverse(static_cast<uint32_t>(2 * (low + i)));
+    }
+    tm.total_super = tiles_m * tiles_n;
+    tm.contig = 1;
+    for (int x = 0; x <= kBf6Xcds; ++x) tm.start[x] = static_cast<int>(static_cast<int64_t>(tm.total_super) * x / kBf6Xcds);
+}
+
+// The tile of super-tile st in the strip order.  (A function of its own: the kernel that walks tiles never meets strips and
+// is short of scalar registers.)
+VDMQ_TILEMAP_FN void bf6_tilemap_locate_strip(const Bf6TileMap &tm, int st, int &tile_m, int &tile_n) {
+    const bool high = st < tm.n_main;
+    const int rows = tm.edge_m_rows + (high ? 1 : 0), at = high ? st : st - tm.n_main;
+    const int strip = bf6_tilemap_quotient(at, tm.strip_inverse[high]), rest = at - strip * rows * tm.tiles_n;
+    const int pair = bf6_tilemap_quotient(rest, tm.pair_inverse[high]), cell = rest - pair * 2 * rows;
+    const bool two = 2 * pair + 1 < tm.tiles_n;
+    tile_m = (high ? 0 : tm.n_edge_m) + strip * rows + (two ? cell >> 1 : cell);
+    tile_n = 2 * pair + (two ? cell & 1 : 0);
 }
 
 // The tile at `place` (0 ... per - 1) of super-tile st; false: that place is empty.
@@ -84,6 +132,13 @@ VDMQ_TILEMAP_FN bool bf6_tilemap_locate(const Bf6TileMap &tm, int st, int place,
     tile_m = rows_main + pr;
     tile_n = st * tm.edge_m_cols + place - pr * tm.edge_m_cols;
     return pr < tm.edge_m_rows && tile_n < tm.tiles_n;
+}
+
+// Of a map that may be either.
+VDMQ_TILEMAP_FN bool bf6_tilemap_locate_any(const Bf6TileMap &tm, int st, int place, int &tile_m, int &tile_n) {
+    if (tm.strips == 0) return bf6_tilemap_locate(tm, st, place, tile_m, tile_n);
+    bf6_tilemap_locate_strip(tm, st, tile_m, tile_n);
+    return place == 0;
 }
 
 // Tiles in the super-tiles [0, st) of the sequence.

@@ -252,3 +252,40 @@ def test_bf6_tiles_that_run_at_once_are_spread_evenly(M, N, K, tile, group_n, co
         assert torch.equal(out["bf6"], out["int8"])
     finally:
         v.set_matrix_path(old)
+
+
+@pytest.mark.parametrize("M,N,K,tile,group_n", [
+    (128 * 15 - 5, 128 * 33, 64, 128, 2),   # strips of eight and seven rows, an odd column
+    (128 * 7 - 100, 128 * 65, 128, 128, 2), # one strip
+    (128 * 11, 128 * 44, 192, 128, 2),
+    (70, 128 * 87, 64, 128, 2),             # one tile row
+    (128 * 26 - 1, 128 * 11, 64, 128, 2),   # four strips, two of them with a row more
+    (256 * 15 - 9, 256 * 17, 64, 256, 2),   # 255 big tiles
+    (640, 128 * 61, 64, 128, 4),            # 40 tiles on the busiest XCD, as few as any order gives some CU a second one
+    (1150, 128 * 31, 128, 128, 4),          # 36
+])
+def test_bf6_spread_tiles_leave_no_place_empty(M, N, K, tile, group_n):
+    """Problems whose tiles the chip holds at once: equal shares of the XCDs, so one workgroup per XCD at most has no
+    tile (empty places hold a CU's place while it is needed), and every output element against the int8 path."""
+    from dsaquant_amd import _lib
+    from dsaquant_amd.kernels import vdm_w4a4 as v
+
+    rng = np.random.default_rng(M + N + K)
+    qw = rng.integers(-8, 8, (N, K), dtype=np.int8)
+    x = O.synth_linear(M, K, 128, seed=K)[0]
+    _, _, ws, bias = O.synth_linear(1, 64, N, seed=K + 1)
+    print(f"strips M={M} N={N} K={K}", flush=True)
+    old = v.matrix_path()
+    try:
+        out = {}
+        for path in ("bf6", "int8"):
+            v.set_matrix_path(path)
+            out[path] = v.linear_vdm_w4a4(_dev(x), _dev(O.np_pack_wgt_v1(qw)), _dev(O.np_pack_wscales_v1(ws, K)), _dev(bias), clip_ratio=1.0)
+            if path == "bf6":
+                info = _lib.last_gemm_launch()
+                assert (info.tile_m, info.group_n, info.contiguous_runs) == (tile, group_n, int(group_n == 2))
+                if group_n == 2:
+                    assert info.workgroups - -(-M // tile) * -(-N // tile) < 8
+        assert torch.equal(out["bf6"], out["int8"])
+    finally:
+        v.set_matrix_path(old)

@@ -51,8 +51,55 @@ static int check(int tiles_m, int tiles_n, int gn_log2, int mode, bool regroup, 
     return 0;
 }
 
+// The strip order: every tile once, runs of equal length, and no workgroup beyond one per XCD without a tile.
+static int check_strips(int tiles_m, int tiles_n) {
+    Bf6TileMap tm;
+    bf6_tilemap_strips(tm, tiles_m, tiles_n);
+    const int tiles = tiles_m * tiles_n, longest = (tiles + kBf6Xcds - 1) / kBf6Xcds;
+    if (tm.per_log2 != 0 || !tm.contig || tm.total_super != tiles || tm.start[0] != 0 || tm.start[kBf6Xcds] != tiles) return 1;
+    std::vector<int> seen(tiles, 0);
+    int lowest = tiles, highest = 0; /* rows of a strip: they differ by one at most */
+    for (int xcd = 0; xcd < kBf6Xcds; ++xcd) {
+        const int run = tm.start[xcd + 1] - tm.start[xcd];
+        if (run > longest || run < tiles / kBf6Xcds) return 2;
+        for (int seq = 0; seq < longest; ++seq) {
+            const int st = bf6_tilemap_super(tm, xcd, seq);
+            if ((st < 0) != (seq >= run)) return 3;
+            int m = -7, n = -7;
+            if (st < 0) continue;
+            bf6_tilemap_locate_strip(tm, st, m, n);
+            if (m < 0 || m >= tiles_m || n < 0 || n >= tiles_n) return 4;
+            ++seen[m * tiles_n + n];
+        }
+    }
+    for (int v : seen)
+        if (v != 1) return 5;
+    int rows = 0, last_m = -1;
+    for (int st = 0; st < tiles; ++st) {
+        int m, n;
+        bf6_tilemap_locate_strip(tm, st, m, n);
+        if (n != 0) continue;
+        if (m != last_m + 1) return 6; /* column 0 comes in row order */
+        last_m = m;
+        const bool starts = st == 0 || [&] { int pm, pn; bf6_tilemap_locate_strip(tm, st - 1, pm, pn); return pn == tiles_n - 1 && tiles_n > 2; }();
+        if (starts && st != 0) {
+            lowest = rows < lowest ? rows : lowest;
+            highest = rows > highest ? rows : highest;
+            rows = 0;
+        }
+        ++rows;
+    }
+    lowest = rows < lowest ? rows : lowest;
+    highest = rows > highest ? rows : highest;
+    if (tiles_n > 2 && (highest > kBf6StripRows || highest - lowest > 1)) return 7;
+    return 0;
+}
+
 int main() {
     long cases = 0;
+    for (int m = 1; m <= 520; ++m)
+        for (int n = 1; m * n <= 1024; ++n, ++cases)
+            if (int e = check_strips(m, n)) return std::printf("tiles %d x %d in strips: check %d failed\n", m, n, e), 1;
     const int big[][2] = {{296, 60}, {296, 54}, {296, 20}, {107, 56}, {107, 36}, {107, 12}, {128, 35}, {128, 18}, {128, 6}, {2, 40}, {1000, 3}, {3, 1000}, {4096, 1}, {1, 4096}};
     for (int variant = 0; variant < 4; ++variant)
         for (int mode = 0; mode < 3; ++mode) {
