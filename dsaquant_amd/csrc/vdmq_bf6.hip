@@ -927,12 +927,16 @@ int launch_gemm_bf6(const uint8_t *xblocks, const __half *ascale, const uint8_t 
     // running at once.  Measured on 210 shapes (M 1...32768, N 128...15360, K 64...13824): up to there the small tiles take
     // 0.4...0.9 of the time (512 x 5120 -> 10240: 29 -> 25 us, 512 x 1536 -> 3072: 13.5 -> 7.3 us, 5888 x 13824 -> 1408, 506
     // tiles: 97 -> 69 us), beyond, where some CU gets a third one, 0.85...1.4.
-    // Just above one big tile per CU the second round of big ones is nearly empty, and the small ones, a little over two
-    // full rounds of them, win again: us, big / small: 3128 x 1536 -> 4992 (260 big tiles) 27.0 / 22.5, 2700 x 3072 -> 6144
-    // (264) 45.1 / 42.3, 4096 x 1536 -> 4608 (288) 29.8 / 28.0, 9272 x 2048 -> 1920 (296) 32.7 / 30.6; 6712 x 13824 -> 2816
-    // (297) 154 / 158, 5276 x 2048 -> 3968 (336) 32.9 / 35.6.
-    const int64_t big_tiles = ceil_div(M, Bf6Big::BM) * ceil_div(N, Bf6Big::BN);
-    if (ceil_div(M, Bf6Small::BM) * ceil_div(N, Bf6Small::BN) <= kXcds * 32 * 2 || (big_tiles > kXcds * 32 && big_tiles <= kXcds * 36))
+    // Just above one big tile per CU the second round of big ones is nearly empty.  Small ones win there where they fill two
+    // rounds at most (1024 tiles): 0.76...0.99 of the time over 30 shapes with K 512...13824 (5057 x 2560 -> 3200 34.7 / 29.8
+    // us, 17205 x 5120 -> 896 55.4 / 50.4, 4920 x 8960 -> 3328 92.7 / 81.2).  With a few tiles more the third round's cost grows
+    // with K, the big tiles' epilogue, which it replaces, does not: small / big up to 288 big tiles 0.87...1.02 for K <= 1536
+    // (4096 x 1536 -> 4608 26.4 / 25.5 us), 0.95...1.05 for K = 2048...4096, 1.00...1.10 from 5120 on (7302 x 8960 -> 2304 92.6 /
+    // 98.3); the big tiles' epilogue is longer with the gated tail: 0.83...1.00 up to K = 3072, to 1.02 at 4096, to 1.07 at 8960.
+    const int64_t big_tiles = ceil_div(M, Bf6Big::BM) * ceil_div(N, Bf6Big::BN), small_tiles = ceil_div(M, Bf6Small::BM) * ceil_div(N, Bf6Small::BN);
+    const bool has_tail = tail.gate != nullptr || tail.residual != nullptr;
+    const bool above_one_round = big_tiles > kXcds * 32 && big_tiles <= kXcds * 36 && (small_tiles <= kXcds * 32 * 4 || K <= (has_tail ? 3072 : 1536));
+    if (small_tiles <= kXcds * 32 * 2 || above_one_round)
         return launch_bf6_cfg<Bf6Small>(xblocks, ascale, wblocks, wscale, bias, static_cast<__half *>(out), out_dtype == VDMQ_OUT_BF16, acc_out, M,
                                         N, K, ldo, tail, s);
     return launch_bf6_cfg<Bf6Big>(xblocks, ascale, wblocks, wscale, bias, static_cast<__half *>(out), out_dtype == VDMQ_OUT_BF16, acc_out, M, N,

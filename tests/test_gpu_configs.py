@@ -289,3 +289,35 @@ def test_bf6_spread_tiles_leave_no_place_empty(M, N, K, tile, group_n):
         assert torch.equal(out["bf6"], out["int8"])
     finally:
         v.set_matrix_path(old)
+
+
+@pytest.mark.parametrize("M,N,K,gated,tile", [
+    (4096, 4608, 1536, False, 128),   # 288 big tiles, 1152 small ones
+    (4096, 4608, 1600, False, 256),
+    (4096, 4608, 3072, True, 128),
+    (4096, 4608, 3136, True, 256),
+    (4480, 3712, 5120, False, 128),   # 270 big tiles, 1015 small ones: two rounds
+    (7302, 2304, 5120, False, 256),   # 261, 1044
+])
+def test_bf6_tile_size_just_above_one_round_follows_k(M, N, K, gated, tile):
+    """257 ... 288 big tiles: small ones where they fill two rounds at most, or K is short; outputs against the int8 path."""
+    from dsaquant_amd import _lib, fused_ops
+    from dsaquant_amd.kernels import vdm_w4a4 as v
+
+    g = torch.Generator(device="cuda:0").manual_seed(M + K)
+    q = torch.randint(0, 256, (N, K // 2), generator=g, device="cuda:0", dtype=torch.uint8)
+    s = (1e-3 + 9e-3 * torch.rand((N, K // 64), generator=g, device="cuda:0")).half()
+    x = torch.randn((1, M, K), generator=g, device="cuda:0").half()
+    extra = {"residual": torch.randn((1, M, N), generator=g, device="cuda:0").half(), "gate": torch.randn((1, 1, N), generator=g, device="cuda:0").half()} if gated else {}
+    old = v.matrix_path()
+    try:
+        out = {}
+        for path in ("bf6", "int8"):
+            v.set_matrix_path(path)
+            out[path] = fused_ops.linear_fused(x, q, s, None, 0.95, **extra)
+            if path == "bf6":
+                assert _lib.last_gemm_launch().tile_m == tile
+        assert torch.equal(out["bf6"], out["int8"])
+    finally:
+        v.set_matrix_path(old)
+        torch.cuda.empty_cache()
