@@ -35,10 +35,14 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 //   1560 x 1560, 12 heads: 109 / 137 -> 390 / 38      32760 x 32760, 12 heads: 450 / 14640 -> 1060 / 6210
 // Error against 64 bits (2-norm, N(0, 1) operands): 2.73e-4 before, 2.73e-4 now.  The maximum is the exact running one:
 // rescaling only when it has grown by 2^8 is 3...9 % faster, but then the largest probabilities no longer lie just below
-// a power of two, where fp16 is finest, and the error grows by 6 %.  Within 2 %: raised wave priority around the matrix
+// a power of two, where fp16 is finest, and the error grows by 6 %.  The probabilities are held times 2^15: unscaled, those
+// below 2^-14 of the largest are denormal fp16 and below 2^-25 nothing, and tens of thousands of keys there do count; so
+// they are rounded at 2^-11 down to 2^-29 of the largest and gone below 2^-40.  (The power of two goes into the maximum that is
+// subtracted; not for scores beyond 2^20, whose own rounding could then carry a probability past fp16.)  Within 2 %: raised wave priority around the matrix
 // instructions, the two key blocks' instructions interleaved, the next step's loads behind the first product.
 
 constexpr int kHeadDim = 128;
+constexpr float kProbLog2 = 15.0f, kExactShift = 1048576.0f;
 constexpr int kKeys = 64;                       /* keys per step */
 constexpr int kTileBytes = kKeys * kHeadDim * 2; /* one step's K (or V) rows in LDS, 256 bytes each */
 
@@ -118,7 +122,7 @@ __global__ __launch_bounds__(WAVES * 64, 2) void attention_kernel(AttnArgs a) {
     for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int r = 0; r < 16; ++r) o[t][r] = 0.0f;
-    float m_ref = -__builtin_inff(), neg_m = 0.0f, l = 0.0f; /* of the scores times scale_log2 */
+    float m_ref = -__builtin_inff(), shift = 0.0f, l = 0.0f; /* of the scores times scale_log2 */
     const int steps = (a.lk + kKeys - 1) / kKeys;
     const float c = a.scale_log2;
     stage(0, 0);
@@ -156,9 +160,10 @@ __global__ __launch_bounds__(WAVES * 64, 2) void attention_kernel(AttnArgs a) {
         mx = max_halves(mx) * c;
         if (__builtin_amdgcn_ballot_w64(mx > m_ref) != 0) {
             const float m_new = __builtin_fmaxf(m_ref, mx);
-            const float alpha = m_new == m_ref ? 1.0f : __builtin_amdgcn_exp2f(m_ref - m_new);
+            const float shift_new = m_new == -__builtin_inff() ? 0.0f : (__builtin_fabsf(m_new) < kExactShift ? kProbLog2 : 0.0f) - m_new;
+            const float alpha = m_new == m_ref ? 1.0f : m_ref == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(shift_new - shift);
             m_ref = m_new;
-            neg_m = m_new == -__builtin_inff() ? 0.0f : -m_new;
+            shift = shift_new;
             l *= alpha;
 #pragma unroll
             for (int t = 0; t < 4; ++t)
@@ -173,7 +178,7 @@ __global__ __launch_bounds__(WAVES * 64, 2) void attention_kernel(AttnArgs a) {
                 f16x2 p;
 #pragma unroll
                 for (int i = 0; i < 2; ++i)
-                    p[i] = static_cast<_Float16>(__builtin_amdgcn_exp2f(__builtin_fmaf(s[g / 2][(g % 2) * 8 + e + i], c, neg_m)));
+                    p[i] = static_cast<_Float16>(__builtin_amdgcn_exp2f(__builtin_fmaf(s[g / 2][(g % 2) * 8 + e + i], c, shift)));
                 l = __builtin_amdgcn_fdot2(p, f16x2{static_cast<_Float16>(1.0f), static_cast<_Float16>(1.0f)}, l, false);
                 pf[g][e] = p[0];
                 pf[g][e + 1] = p[1];

@@ -320,8 +320,10 @@ int vdmq_pack_weight(const void *w, const void *scale_in, void *qweight_v1, void
                      int64_t K, vdmq_stream_t stream);
 
 /* Mask-free attention between the linears (vdm_attn.py:241-259): out = softmax(scale * q k^T) v per batch element and
- * head, fp16 with fp32 scores, softmax and accumulation.  Head dimension 128 (contiguous); the strides of each operand
- * are given in elements as {row, head, batch}, multiples of 8.  lk >= 1. */
+ * head, fp16 with fp32 scores, exponentials and accumulation.  The probabilities enter both sums, numerator and
+ * denominator, rounded to fp16: to 2^-11 of their value down to 2^-29 of the row's largest, less exactly below, not at all
+ * below 2^-40.  Head dimension 128 (contiguous); the strides of each operand are given in elements as {row, head, batch},
+ * multiples of 8.  lk >= 1. */
 int vdmq_attention_f16(const void *q, const int64_t *q_stride, const void *k, const int64_t *k_stride, const void *v,
                        const int64_t *v_stride, void *out, const int64_t *out_stride, int64_t batch, int64_t heads, int64_t lq, int64_t lk,
                        int64_t head_dim, float scale, vdmq_stream_t stream);

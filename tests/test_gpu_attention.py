@@ -67,6 +67,33 @@ def test_attention_keeps_small_probabilities_large_scores_and_the_tail():
     assert torch.isnan(out[:, 3]).all() and torch.isfinite(out[:, 4:, :, 1:]).all()
 
 
+@pytest.mark.parametrize("exponent", [-20.5, -23.5, -25.5, -28.0])
+def test_attention_keeps_many_tiny_probabilities(exponent):
+    """One key of probability about 1 and 32000 of 2^exponent each: denormal in fp16 or below it, but what v has is theirs."""
+    from dsaquant_amd import fused_ops as f
+
+    q, k = torch.zeros((1, 3, 1, 128), device=DEV).half(), torch.zeros((1, 32001, 1, 128), device=DEV).half()
+    q[..., 0] = 8
+    k[:, 1:, :, 0] = exponent * 128 ** 0.5 / 1.4426950408889634 / 8
+    v = torch.ones_like(k)
+    v[:, 0] = 0
+    want = _reference(q, k, v)[0, 0, 0, 0].item()
+    # the probabilities round alike, by 2^-11 at most, and so does the result (fp16, normal); the sums are fp32
+    assert abs(f.attention(q, k, v)[0, :, 0, 0].double().cpu() - want).max().item() <= 1.05 * 2.0 ** -10 * want
+
+
+def test_attention_with_scores_that_fp32_holds_coarsely():
+    """Scores around 2^20 and 2^25 (times log2 e): a step of fp32 there is up to 4, no probability may leave fp16's range."""
+    from dsaquant_amd import fused_ops as f
+
+    for size in (2048.0, 3000.0, 4096.0, 20000.0):
+        q, k = torch.zeros((1, 33, 1, 128), device=DEV).half(), torch.zeros((1, 70, 1, 128), device=DEV).half()
+        q[..., :4], k[..., :4] = size, size / 2
+        k[:, 37, :, :4] = size
+        v = torch.randn((1, 70, 1, 128), device=DEV).half()
+        assert torch.equal(f.attention(q, k, v), v[:, 37:38].expand(1, 33, 1, 128))
+
+
 def test_attention_refuses_what_it_is_not_for():
     from dsaquant_amd import _lib
     from dsaquant_amd import fused_ops as f
