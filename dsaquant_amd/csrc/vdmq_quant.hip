@@ -943,7 +943,8 @@ int launch_pack_weight(const __half *w, const __half *scale_in, int64_t N, int64
     const int tiles = static_cast<int>(N / kTileRows);
     const int64_t nch = ceil_div(k_padded(K), 512);
     using Kernel = void (*)(const __half *, const __half *, int, int, int, u32x4 *, u32x4 *, __half *, uint32_t *);
-    // (18 chunks are what the 128 registers of a sixteen-wave workgroup hold beside the work, 10 what two of them per CU do)
+    // (18 chunks are what the 128 registers of a sixteen-wave workgroup hold beside the work, 10 -- with four of the 64
+    // registers spilled to 12 bytes of scratch per lane -- what two of them per CU do)
     const Kernel kernel = nch <= 2 ? pack_weight_kernel<2> : nch <= 4 ? pack_weight_kernel<4> : nch <= 6 ? pack_weight_kernel<6> :
                           nch <= 10 ? pack_weight_kernel<10> : nch <= 18 ? pack_weight_kernel<18> : pack_weight_kernel<0>;
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(tiles)), dim3(kTileRows * kWaveSize), 0, s, w, scale_in, tiles, static_cast<int>(K),

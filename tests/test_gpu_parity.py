@@ -683,8 +683,8 @@ def rows_of_blocks(blocks: torch.Tensor, M: int, K: int) -> np.ndarray:
 def test_bf6_quantizers_write_the_oracle_integers(M, K):
     """The quantizers that emit bf6 blocks directly (plain, GELU, LayerNorm): decoded with the format's definition,
     the blocks hold the oracle's integers (plain) / the integers of the int4 quantizer (fused producers), scales equal.
-    Rows longer than 8192 make a workgroup walk several row groups once there are more groups than the chip
-    holds (256 CUs x 1): (4096, 8960) gives every workgroup two, (2100, 13824) a few of them a second, ragged one."""
+    Rows longer than 9216 make a workgroup walk several row groups once there are more groups than the chip
+    holds (256 CUs x 1): (2100, 13824) gives a few of them a second, ragged one; (4096, 8960) are the longest that do not."""
     from dsaquant_amd import fused_ops
 
     v = vk()

@@ -5,7 +5,7 @@ import pytest
 import torch
 
 import oracle as O
-from tests.test_gpu_parity import gpu_gelu_table, rows_of_blocks, special_rows, t16, unpack_native, vk
+from tests.test_gpu_parity import gpu_gelu_table, pack_native, rows_of_blocks, special_rows, t16, unpack_native, vk
 
 pytestmark = pytest.mark.gpu
 
@@ -45,7 +45,7 @@ def test_gelu_table_has_the_order_the_row_maximum_relies_on():
     assert np.isfinite(negative).all() and ((negative.view(np.uint16) & 0x7FFF) < 0x3180).all()
 
 
-@pytest.mark.parametrize("K", [512, 5120, 8192 + 64, 9216, 9216 + 128, 13824, 16384])
+@pytest.mark.parametrize("K", [512, 5120, 7168, 7168 + 64, 8192 + 64, 9216, 9216 + 128, 13824, 16384])
 @pytest.mark.parametrize("clip", [1.0, 0.5, 1e-6])
 def test_gelu_quantizer_row_kinds(K, clip):
     """Rows whose absmax comes from a large positive element, from the negative branch, from a positive element just
@@ -72,6 +72,63 @@ def test_gelu_quantizer_row_kinds(K, clip):
     blocks, sc = v.quantize_activation_bf6(t16(x), clip, act="gelu_tanh")
     assert np.array_equal(sc.cpu().numpy().view(np.uint16), want_s.view(np.uint16))
     assert np.array_equal(rows_of_blocks(blocks, len(x), K), want_q.astype(np.float64))
+
+
+def codes_of_blocks(blocks, rows, K):
+    """The six-bit codes of a bf6 operand, strings in memory order, minus zero as zero (the quantizers keep the sign of what
+    they round to zero, the conversion from native rows has none)."""
+    panels = blocks.view(rows // 8, -1, 384)
+    a, b = panels[..., :256].unflatten(2, (2, 8, 16)), panels[..., 256:].unflatten(2, (2, 8, 8))
+    w = torch.cat([a, b], dim=-1).unflatten(-1, (8, 3)).int()
+    w = w[..., 0] | w[..., 1] << 8 | w[..., 2] << 16
+    codes = torch.stack([w >> 6 * i & 63 for i in range(4)], dim=-1).to(torch.uint8)
+    return torch.where(codes == 32, 0, codes)
+
+
+@pytest.mark.parametrize("act", [None, "gelu_tanh"])
+@pytest.mark.parametrize("M,K", [(25600, 1536), (17408, 2048), (4320, 9216 + 64), (4320, 13824), (4320, 16384)])
+def test_walking_quantizers_over_several_rounds(M, K, act):
+    """Row lengths whose workgroups walk row groups, with more than two groups each: rows of every kind -- the GELU's absmax
+    from the largest element, from the negative branch, NaN, Inf, zeros -- follow one another in a workgroup's sequence,
+    every row against the oracle's integers (brought into blocks by the conversion from native rows)."""
+    v = vk()
+    _, table = gpu_gelu_table()
+    rng = np.random.default_rng(M + K)
+    kinds = rng.standard_normal((61, K)).astype(np.float16)
+    kinds[1::7] = -np.abs(kinds[1::7])                          # the negative branch decides
+    kinds[2::7] = np.minimum(kinds[2::7], np.float16(0.284))
+    kinds[3], kinds[17] = 0, np.float16(6e-8)
+    kinds[4, 3], kinds[18, K - 1], kinds[32, 7], kinds[46, 9] = np.inf, -np.inf, np.nan, 65504
+    kinds[5::7, :: K // 9] *= np.float16(20)
+    x = kinds if act is None else table[kinds.view(np.uint16)]
+    scale = O.np_row_scale(x, 0.95)
+    native = t16(pack_native(O.np_quantize_rows(x, scale), v.k_padded(K)))
+    row = torch.arange(M, device="cuda") * 23 % 61
+    blocks, sc = v.quantize_activation_bf6(t16(kinds)[row], 0.95, act=act)
+    assert torch.equal(sc.view(torch.int16), t16(scale)[row].view(torch.int16))
+    assert torch.equal(codes_of_blocks(blocks, M, K), codes_of_blocks(v.bf6_blocks(native[row], K), M, K))
+
+
+@pytest.mark.parametrize("N,K", [(128, 64), (256, 1088), (128, 5120 + 64), (128, 16384 + 64)])
+def test_row_scale_and_given_scale_entry_points(N, K):
+    """vdmq_row_scale and vdmq_quantize_weight_native of the C interface, rows with NaN / Inf / zeros, given scales of zero,
+    Inf and NaN among ordinary ones."""
+    from dsaquant_amd import _lib
+
+    lib, v = _lib.load(), vk()
+    rng = np.random.default_rng(N + K)
+    w = special_rows((0.05 * rng.standard_normal((N, K))).astype(np.float16))
+    wt, s = t16(w), torch.cuda.current_stream().cuda_stream
+    for clip in (1.0, 0.95, 1e-5):
+        scale = torch.empty(N, dtype=torch.float16, device="cuda")
+        _lib.check(lib.vdmq_row_scale(wt.data_ptr(), N, K, clip, scale.data_ptr(), s))
+        want = O.np_row_scale(w, clip)
+        assert np.array_equal(scale.cpu().numpy().view(np.uint16), want.view(np.uint16))
+    given = np.where(want == 1, want, O.np_row_scale(w, 0.75)).astype(np.float16)
+    given[20:25] = np.array([0.0, -1e-3, np.inf, 6e-8, np.nan], np.float16)
+    native = torch.empty((N, v.k_padded(K) // 2), dtype=torch.uint8, device="cuda")
+    _lib.check(lib.vdmq_quantize_weight_native(wt.data_ptr(), t16(given).data_ptr(), native.data_ptr(), N, K, s))
+    assert np.array_equal(unpack_native(native.cpu().numpy(), K), O.np_quantize_rows(w, given))
 
 
 def _round_fma(a, b, c):
