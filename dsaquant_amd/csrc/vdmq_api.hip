@@ -445,11 +445,10 @@ int vdmq_gemm_w4a4_bf6_acc(const void *xblocks, const void *wblocks, int32_t *ac
 
 int vdmq_bf6_pays(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
-    // Measured, quantizer + GEMM, int8 time / bf6 time on 180 shapes (M 1 ... 32768, N 128 ... 15360).  K >= 1536: 1.01 ...
-    // 1.97 everywhere but one shape at 0.96 (512 x 5120 -> 10240 1.44, 4096 x 1536 -> 4608 1.01, 8192 x 5120 -> 10240
-    // 1.42, 100 x 5120 -> 15360 1.97).  K = 1280: 1.05 ... 1.36 on 12 of 16 shapes, 0.80 ... 0.98 on four.  K = 1024: 11 : 5,
-    // K = 768: 9 : 7 (0.76 ... 1.27); K <= 512: 0.73 ... 1.03 -- the quantizer that writes blocks is the slower one on short
-    // rows and decides such a linear.  M and N no longer matter since the GEMM has a small-tile configuration.
+    // Measured, quantizer + GEMM, int8 time / bf6 time on 156 shapes (M 100 ... 75600, N 1024 ... 8192).  K >= 1280: 1.05 ...
+    // 1.49 (4096 x 1536 -> 4608 1.14, 512 x 5120 -> 4096 1.13, 8192 x 5120 -> 8192 1.43); K = 640 ... 1152: 1.00 ... 1.37; K <= 512:
+    // 0.93 ... 1.21, below 1 on half of them.  The line was drawn with an earlier form of the quantizer that writes blocks,
+    // which lost up to a quarter between 640 and 1280.
     return K >= 1280 ? 1 : 0;
 }
 

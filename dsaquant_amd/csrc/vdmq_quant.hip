@@ -281,9 +281,9 @@ __device__ __forceinline__ void quantize_held_row(const u32x4 (&v)[NCH], int lan
 // block holds q / 16, an E3M2 value for every q of [-8, 8]); its 192 bits are then four 48-bit quarters of four different
 // strings, which are put together in LDS.  (Bringing 32 consecutive k into one lane first, as fp16 through LDS, takes
 // 2.7 times the LDS traffic, an LDS round trip in front of every conversion and 34 KiB of LDS more per workgroup, with
-// which two fit a CU.  Measured, that way / this way, with the reductions below on the VALU: 32760 x 1536 plain 25.5 /
-// 23.1 us, GELU 36 / 30, LayerNorm 42 / 29; 27280 x 3072 LayerNorm 64 / 48; 75637 x 5120 GELU 208 / 171, LayerNorm
-// 243 / 215; the streaming floor at 6.3 TB/s is 22, 37 and 169 us.)
+// which two fit a CU.  Measured, that way / this way, with the reductions below on the VALU: 32760 x 1536 plain 24.2 /
+// 22.8 us, GELU 36 / 30, LayerNorm 41 / 29; 27280 x 3072 LayerNorm 64 / 50; 75637 x 5120 GELU 205 / 169, LayerNorm
+// 239 / 222; the streaming floor at 6.3 TB/s is 22, 37 and 169 us.)
 // The instruction also rounds: E3M2's grid is 1/16 up to 8/16, so round-to-nearest-even of t / 16 onto it is the
 // round-half-even of t the quantizer asks for, ties included (a code's last bit is the integer's).  Only |t| has to
 // stay below 8.5, above -8.5 and t below 7.5; rows whose largest |t| is below 7.5 (a clip ratio above 0.934)
@@ -313,15 +313,17 @@ struct Bf6Scratch { /* LDS of one workgroup: the strings of one group; two copie
 // workgroups share a CU and overlap by themselves (32760 x 8960: 133 walking, 130 not).
 constexpr bool bf6_walks(int nch) { return nch >= 19 || nch <= 4; }
 // Dynamic LDS a launch asks for beside the strings, to keep a third workgroup off the CU: eight-wave workgroups of
-// 10 KiB rows stream best with two of them in flight per CU (75637 x 5120 plain: 163 us with two, 171 with three; the
-// streaming floor is 169 at 6.3 TB/s).  The shorter rows and the fused producers want every wave they can get
-// (27280 x 3072: 37.1 us with three or more, 39.3 with two; 75637 x 5120 with the GELU 171 / 175).
+// 10 KiB rows stream best with two of them in flight per CU once the rows are many (plain, with two / with three, us:
+// 75637 x 5120 162 / 171, x 4096 135 / 141, x 3584 114.5 / 117.4; 32760 x 5120 71 / 73; the streaming floor of the first is 169
+// at 6.3 TB/s).  Not so below: 8192 x 4608 18.6 / 17.9, 8192 x 3136 13.7 / 12.1, 75637 x 3136 106 / 101.  The shorter rows and
+// the fused producers want every wave they can get (27280 x 3072: 37.1 us with three or more, 39.3 with two; 75637 x 5120
+// with the GELU 171 / 175).
 constexpr int bf6_spare_lds(int nch, int act) { return nch > 6 && nch <= 10 && act == VDMQ_ACT_NONE ? 30000 : 0; }
 // Whether a fused activation is evaluated behind the row's absmax (gelu_row_absmax), chunk by chunk during the
 // conversion: with long rows few waves share a SIMD and what they compute between the arrival of a row and its
 // conversion runs with no load in flight.  Measured, in front / behind: 27280 x 14336 268 / 214 us, 75600 x 13824 636 /
 // 548, 32760 x 8960 193 / 152; short rows have the waves to overlap and pay for the second maximum: 75637 x 5120 176 /
-// 180, 27280 x 3072 43 / 45.5.
+// 180, 27280 x 3072 43 / 45.5.  (The chunk counts that rows run on go from 14 to 18: this is K > 7168.)
 constexpr bool bf6_late_act(int nch) { return nch >= 17; }
 struct NoRefill {
     __device__ __forceinline__ void operator()(int) const {}
