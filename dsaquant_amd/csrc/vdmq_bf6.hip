@@ -827,10 +827,11 @@ int launch_bf6_cfg(const uint8_t *xblocks, const __half *ascale, const uint8_t *
     // of four or six rows are up to 1.11 (an XCD's tiles far from square read more operand rows).
     // Kept as they were: problems that give no CU of the busiest XCD a second workgroup (small tiles: and every XCD one
     // super-tile at most), and those where any order gives some CUs a second one and this one not to more than a quarter
-    // (640 x 7808, 5120, 40 tiles on the busiest: 23.0 us, in strips 24.5).
+    // (640 x 7808, 5120, 40 tiles on the busiest: 23.0 us, in strips 24.5; not in the shape of two columns, which leaves
+    // most places empty: 512 x 10240, 5120 24.35, in strips 24.15).
     const int64_t all_tiles = static_cast<int64_t>(tm.tiles_m) * tm.tiles_n;
     const bool at_once = all_tiles <= kXcds * per;
-    const bool few_doubled = all_tiles > kXcds * 32 && best_load <= 40;
+    const bool few_doubled = all_tiles > kXcds * 32 && best_load <= 40 && tm.group_n_log2 == 2;
     const bool spread = at_once ? !few_doubled && (best_load > 32 || (Cfg::kOcc == 2 && tm.total_super > kXcds)) : Cfg::kOcc == 2;
     if (spread && at_once)
         bf6_tilemap_strips(tm, tiles_m, tiles_n);

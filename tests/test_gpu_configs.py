@@ -260,6 +260,7 @@ def test_bf6_tiles_that_run_at_once_are_spread_evenly(M, N, K, tile, group_n, co
     (128 * 11, 128 * 44, 192, 128, 2),
     (70, 128 * 87, 64, 128, 2),             # one tile row
     (128 * 26 - 1, 128 * 11, 64, 128, 2),   # four strips, two of them with a row more
+    (512, 10240, 64, 128, 2),               # 40 on every XCD
     (256 * 15 - 9, 256 * 17, 64, 256, 2),   # 255 big tiles
     (640, 128 * 61, 64, 128, 4),            # 40 tiles on the busiest XCD, as few as any order gives some CU a second one
     (1150, 128 * 31, 128, 128, 4),          # 36
