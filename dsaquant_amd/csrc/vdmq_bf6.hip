@@ -823,9 +823,9 @@ int launch_bf6_cfg(const uint8_t *xblocks, const __half *ascale, const uint8_t *
     // workgroups per XCD took 1.4 times what 64 take.)  M x N, K, us, whole-XCD super-tiles / 4 x 2 super-tiles / strips:
     // 4680 x 1536, 8960 61 / 41 / 42; 4680 x 1536, 1536 17.4 / 12.0 / 11.9; 6000 x 1280, 2048 23.8 / 14.3 / 14.2; 1868 x
     // 4224, 3072 21.3 / 23.8 / 19.0; 867 x 8320, 13824 69 / 85 / 63; 3800 x 4352, 5120 (255 big tiles) 58 / 55 / 38.  On 370
-    // shapes of 20 tiles up 0.88 of whole-XCD super-tiles in the geometric mean, 1.07 at most but for some of 60...120 tiles
-    // at K = 5120 (5632 x 250: 1.10), where eleven tiles' weights no longer stay in an XCD's L2 from one launch to the next
-    // and eight tiles' did; strips of four or six rows are up to 1.11 (an XCD's tiles far from square read more operand rows).
+    // shapes of 20 tiles up 0.88 of whole-XCD super-tiles in the geometric mean, 1.07 at most but for a few of 85...90 tiles at
+    // K = 5120 (250 x 5632 13.5 / 14.9 us, why is not known); strips of four or six rows are up to 1.11 (an XCD's tiles far
+    // from square read more operand rows).
     // Kept as they were: problems that give no CU of the busiest XCD a second workgroup (small tiles: and every XCD one
     // super-tile at most), and those where any order gives some CUs a second one and this one not to more than a quarter
     // (640 x 7808, 5120, 40 tiles on the busiest: 23.0 us, in strips 24.5; not in the shape of two columns, which leaves
