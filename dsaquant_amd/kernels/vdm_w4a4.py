@@ -523,6 +523,7 @@ def pack_weight_with_scale(weight: torch.Tensor, channel_scale: torch.Tensor):
     channel_scales fp16 [N])`` like vdm_w4a4.py:209-214 /
     vdm_w4a4_kernel.cu:697-728.
     """
+    _load_ext()
     weight_h = weight.detach().half().contiguous()
     scale_h = channel_scale.detach().view(-1).half().contiguous().to(weight_h.device)
     _check_device_tensor(weight_h, "weight", torch.float16)
@@ -534,6 +535,7 @@ def pack_weight_with_scale(weight: torch.Tensor, channel_scale: torch.Tensor):
 def quantize_weight_per_channel(weight: torch.Tensor):
     """Derive per-channel scales (absmax/7, clip 1) and pack
     (vdm_w4a4.py:217-219 / vdm_w4a4_kernel.cu:730-763)."""
+    _load_ext()
     weight_h = weight.detach().half().contiguous()
     _check_device_tensor(weight_h, "weight", torch.float16)
     _require(weight_h.dim() == 2, "weight must be [N, K]")
@@ -541,7 +543,7 @@ def quantize_weight_per_channel(weight: torch.Tensor):
 
 
 def _pack_weight(weight_h: torch.Tensor, scale_h: Optional[torch.Tensor]):
-    lib = _load_ext()
+    lib = _lib.load()
     N, K = weight_h.shape
     _require(N % BLOCK_N == 0, f"N must be a multiple of {BLOCK_N}")
     _require(K % WARP_K == 0, f"K must be a multiple of {WARP_K}")

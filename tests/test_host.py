@@ -532,6 +532,25 @@ def test_bf6_tile_order_takes_every_tile_once(tmp_path):
     assert res.returncode == 0 and res.stdout.startswith("ok "), res.stdout
 
 
+@pytest.mark.parametrize("pack", ["quantize_weight_per_channel", "pack_weight_with_scale"])
+def test_packing_asks_for_the_library_first(monkeypatch, pack):
+    """Without the library packing fails with the reason, which load_error() keeps, whatever it was given."""
+    from dsaquant_amd import _lib
+    from dsaquant_amd.kernels import vdm_w4a4 as v
+
+    reason = OSError("no library")
+
+    def missing():
+        raise reason
+
+    monkeypatch.setattr(_lib, "load", missing)
+    monkeypatch.setattr(v, "_LOAD_ERROR", None)
+    args = (torch.zeros(128, 64),) if pack == "quantize_weight_per_channel" else (torch.zeros(128, 64), torch.ones(128))
+    with pytest.raises(OSError, match="no library"):
+        getattr(v, pack)(*args)
+    assert v.load_error() is reason
+
+
 def test_header_is_plain_c_and_a_c_host_links_the_library(tmp_path):
     """include/vdmq.h is what a C or C++ host of the reference's kernels would include: it must compile as C99 with
     every warning an error, and a C program must link libvdmq.so by its declarations alone.  The program calls the
