@@ -27,7 +27,7 @@ class GemmLaunchInfo(ctypes.Structure):
                 ("group_n", ctypes.c_int), ("contiguous_runs", ctypes.c_int), ("workgroups", ctypes.c_int64)]
 
 
-KERNEL_GEMM_W4A4, KERNEL_GEMM_BF6, KERNEL_GEMM_BF6_PERSISTENT = 1, 2, 3
+KERNEL_GEMM_W4A4, KERNEL_GEMM_BF6, KERNEL_GEMM_BF6_PERSISTENT, KERNEL_LINEAR_RESIDENT = 1, 2, 3, 4
 
 # name -> (restype, argtypes); every symbol include/vdmq.h declares
 _i64, _p, _f32, _int = ctypes.c_int64, ctypes.c_void_p, ctypes.c_float, ctypes.c_int
@@ -67,6 +67,10 @@ SIGNATURES = {
     "vdmq_workspace_bytes_bf6": (_i64, [_i64, _i64]),
     "vdmq_bf6_pays": (_int, [_i64, _i64, _i64]),
     "vdmq_linear_w4a4_bf6": (_int, [_p, _i64, _i64, _i64, _f32, _int, _p, _p, _p, _p, _int, _i64, _i64, _p, _i64, _p]),
+    "vdmq_linear_bf6_workspace": (_i64, [_i64, _i64, _i64, _int, _int, _i64, _i64, _int]),
+    "vdmq_linear_bf6": (_int, [_p, _i64, _i64, _i64, _f32, _int, _p, _p, _p, _p, _int, _i64, _i64, _p, _i64, _p]),
+    "vdmq_linear_bf6_ex": (_int, [_p, _i64, _i64, _i64, _f32, _int, _int, _f32, _p, _p, _i64, _i64, _p, _p, _p, _p, _i64, _i64, _p, _i64, _i64, _i64,
+                                  _p, _int, _i64, _i64, _p, _i64, _p]),
     "vdmq_native_to_bf6": (_int, [_p, _i64, _i64, _p, _p]),
     "vdmq_weight_v1_to_bf6": (_int, [_p, _p, _i64, _i64, _p]),
     "vdmq_bf6_to_weight_v1": (_int, [_p, _p, _i64, _i64, _p]),

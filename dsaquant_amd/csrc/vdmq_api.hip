@@ -235,6 +235,21 @@ static int check_split(GemmTail &tail, int64_t N, int64_t split_cols, int64_t pa
     return VDMQ_OK;
 }
 
+// What a GEMM writes and the vectors of its epilogue
+static int check_out(const void *wscale, const void *bias, const void *out, int out_dtype, int64_t N, int64_t ldo, const GemmTail &tail) {
+    VDMQ_TRY(check_ptr(wscale, "wscale"));
+    VDMQ_TRY(check_ptr(out, "out"));
+    if (bias != nullptr) VDMQ_TRY(check_ptr(bias, "bias"));
+    if (out_dtype != VDMQ_OUT_F16 && out_dtype != VDMQ_OUT_BF16) return fail(VDMQ_EINVAL, "unknown out_dtype %d", out_dtype);
+    if (ldo < (tail.split_cols ? tail.split_cols : N) || ldo % 8 != 0 || ldo > kMaxLdo)
+        return fail(VDMQ_ESHAPE, "ldo must be >= the columns of a row, a multiple of 8 and at most %lld (got %lld)", (long long)kMaxLdo, (long long)ldo);
+    if (tail.gate != nullptr || tail.residual != nullptr || tail.split_cols != 0) {
+        if (out_dtype != VDMQ_OUT_F16) return fail(VDMQ_EINVAL, "gate, residual and a split output need an fp16 output");
+        VDMQ_TRY(check_tail(tail, N));
+    }
+    return VDMQ_OK;
+}
+
 static int gemm_checked(const void *qact, const void *ascale, const void *wq, const void *wscale, const void *bias, void *out,
                         int out_dtype, int32_t *acc, int64_t M, int64_t N, int64_t K, int64_t ldo, const GemmTail &tail,
                         vdmq_stream_t stream) {
@@ -246,16 +261,7 @@ static int gemm_checked(const void *qact, const void *ascale, const void *wq, co
     VDMQ_TRY(check_ptr(wq, "wq"));
     if (acc == nullptr) {
         VDMQ_TRY(check_ptr(ascale, "ascale", false));
-        VDMQ_TRY(check_ptr(wscale, "wscale"));
-        VDMQ_TRY(check_ptr(out, "out"));
-        if (bias != nullptr) VDMQ_TRY(check_ptr(bias, "bias"));
-        if (out_dtype != VDMQ_OUT_F16 && out_dtype != VDMQ_OUT_BF16) return fail(VDMQ_EINVAL, "unknown out_dtype %d", out_dtype);
-        if (ldo < (tail.split_cols ? tail.split_cols : N) || ldo % 8 != 0 || ldo > kMaxLdo)
-            return fail(VDMQ_ESHAPE, "ldo must be >= the columns of a row, a multiple of 8 and at most %lld (got %lld)", (long long)kMaxLdo, (long long)ldo);
-        if (tail.gate != nullptr || tail.residual != nullptr || tail.split_cols != 0) {
-            if (out_dtype != VDMQ_OUT_F16) return fail(VDMQ_EINVAL, "gate, residual and a split output need an fp16 output");
-            VDMQ_TRY(check_tail(tail, N));
-        }
+        VDMQ_TRY(check_out(wscale, bias, out, out_dtype, N, ldo, tail));
     } else {
         VDMQ_TRY(check_ptr(acc, "acc"));
     }
@@ -400,16 +406,7 @@ static int gemm_bf6_checked(const void *xblocks, const void *ascale, const void 
     VDMQ_TRY(check_ptr(wblocks, "wblocks"));
     if (acc == nullptr) {
         VDMQ_TRY(check_ptr(ascale, "ascale", false));
-        VDMQ_TRY(check_ptr(wscale, "wscale"));
-        VDMQ_TRY(check_ptr(out, "out"));
-        if (bias != nullptr) VDMQ_TRY(check_ptr(bias, "bias"));
-        if (out_dtype != VDMQ_OUT_F16 && out_dtype != VDMQ_OUT_BF16) return fail(VDMQ_EINVAL, "unknown out_dtype %d", out_dtype);
-        if (ldo < (tail.split_cols ? tail.split_cols : N) || ldo % 8 != 0 || ldo > kMaxLdo)
-            return fail(VDMQ_ESHAPE, "ldo must be >= the columns of a row, a multiple of 8 and at most %lld (got %lld)", (long long)kMaxLdo, (long long)ldo);
-        if (tail.gate != nullptr || tail.residual != nullptr || tail.split_cols != 0) {
-            if (out_dtype != VDMQ_OUT_F16) return fail(VDMQ_EINVAL, "gate, residual and a split output need an fp16 output");
-            VDMQ_TRY(check_tail(tail, N));
-        }
+        VDMQ_TRY(check_out(wscale, bias, out, out_dtype, N, ldo, tail));
     } else {
         VDMQ_TRY(check_ptr(acc, "acc"));
     }
@@ -455,6 +452,94 @@ int vdmq_bf6_pays(int64_t M, int64_t N, int64_t K) {
 int64_t vdmq_workspace_bytes_bf6(int64_t M, int64_t K) {
     if (M < 0 || K <= 0) return 0;
     return (bf6_bytes(M, K) + 255) / 256 * 256 + (M * 2 + 255) / 256 * 256;
+}
+
+// Quantizer and GEMM of the bf6 path for every form of a linear: rows as they are, through an activation or a LayerNorm;
+// output plain, with the gated residual update, or split by columns.  One kernel where the rows' operand fits LDS
+// (vdmq_resident.hip), else the two.
+static int linear_bf6_checked(const ResidentProblem &p, void *workspace, int64_t workspace_bytes, vdmq_stream_t stream) {
+    VDMQ_TRY(check_k(p.K));
+    VDMQ_TRY(check_n(p.N));
+    VDMQ_TRY(check_m(p.M));
+    if (p.M == 0) return VDMQ_OK;
+    if (!resident_takes(p)) {
+        VDMQ_TRY(check_ptr(workspace, "workspace"));
+        if (workspace_bytes < vdmq_workspace_bytes_bf6(p.M, p.K))
+            return fail(VDMQ_ENOSPACE, "workspace has %lld bytes, %lld needed", (long long)workspace_bytes, (long long)vdmq_workspace_bytes_bf6(p.M, p.K));
+        uint8_t *blocks = static_cast<uint8_t *>(workspace);
+        void *scale = blocks + (bf6_bytes(p.M, p.K) + 255) / 256 * 256;
+        if (p.ln_mode != 0)
+            VDMQ_TRY(quantize_act_ln_checked(p.x, p.M, p.K, p.ldx, p.eps, p.ln_mode, p.va, p.vb, p.ldv, p.rows_per_vec, p.clip, 1, blocks, scale, stream));
+        else
+            VDMQ_TRY(quantize_act_checked(p.x, p.M, p.K, p.ldx, p.clip, p.act, 1, blocks, scale, stream));
+        return gemm_bf6_checked(blocks, scale, p.wblocks, p.wscale, p.bias, p.out, p.out_dtype, nullptr, p.M, p.N, p.K, p.ldo, p.tail, stream);
+    }
+    VDMQ_TRY(check_ptr(p.x, "x"));
+    if (p.ldx < p.K || p.ldx % 8 != 0) return fail(VDMQ_ESHAPE, "ldx must be >= K and a multiple of 8 (got %lld)", (long long)p.ldx);
+    ResidentProblem q = p;
+    if (p.ln_mode != 0) VDMQ_TRY(ln_checked(p.x, p.M, p.K, p.ldx, p.ln_mode, p.va, p.vb, p.ldv, q.rows_per_vec));
+    VDMQ_TRY(check_ptr(p.wblocks, "wblocks"));
+    VDMQ_TRY(check_out(p.wscale, p.bias, p.out, p.out_dtype, p.N, p.ldo, p.tail));
+    return launch_linear_resident(q, as_stream(stream));
+}
+
+static ResidentProblem linear_problem(const void *x, int64_t M, int64_t K, int64_t ldx, float clip, int act, const void *wblocks, const void *wscale,
+                                      const void *bias, void *out, int out_dtype, int64_t N, int64_t ldo) {
+    ResidentProblem p = {};
+    p.x = static_cast<const __half *>(x);
+    p.M = M;
+    p.K = K;
+    p.ldx = ldx;
+    p.clip = clip;
+    p.act = act;
+    p.wblocks = static_cast<const uint8_t *>(wblocks);
+    p.wscale = static_cast<const __half *>(wscale);
+    p.bias = static_cast<const __half *>(bias);
+    p.out = out;
+    p.out_dtype = out_dtype;
+    p.N = N;
+    p.ldo = ldo;
+    return p;
+}
+
+int vdmq_linear_bf6(const void *x, int64_t M, int64_t K, int64_t ldx, float clip, int act, const void *wblocks, const void *wscale, const void *bias,
+                    void *out, int out_dtype, int64_t N, int64_t ldo, void *workspace, int64_t workspace_bytes, vdmq_stream_t stream) {
+    return linear_bf6_checked(linear_problem(x, M, K, ldx, clip, act, wblocks, wscale, bias, out, out_dtype, N, ldo), workspace, workspace_bytes, stream);
+}
+
+int vdmq_linear_bf6_ex(const void *x, int64_t M, int64_t K, int64_t ldx, float clip, int act, int ln_mode, float eps, const void *a, const void *b,
+                       int64_t ldv, int64_t rows_per_vec, const void *wblocks, const void *wscale, const void *bias, const void *gate, int64_t ldg,
+                       int64_t rows_per_gate, const void *residual, int64_t ldr, int64_t split_cols, int64_t part_stride, void *out, int out_dtype,
+                       int64_t N, int64_t ldo, void *workspace, int64_t workspace_bytes, vdmq_stream_t stream) {
+    ResidentProblem p = linear_problem(x, M, K, ldx, clip, act, wblocks, wscale, bias, out, out_dtype, N, ldo);
+    p.ln_mode = ln_mode;
+    p.eps = eps;
+    p.va = static_cast<const __half *>(a);
+    p.vb = static_cast<const __half *>(b);
+    p.ldv = ldv;
+    p.rows_per_vec = rows_per_vec;
+    p.tail = make_tail(gate, ldg, rows_per_gate, residual, ldr);
+    if (ln_mode != 0 && act != VDMQ_ACT_NONE) return fail(VDMQ_EINVAL, "an activation cannot be combined with a LayerNorm input");
+    if (split_cols != 0) {
+        if (N <= 0) return check_n(N);
+        VDMQ_TRY(check_split(p.tail, N, split_cols, part_stride));
+        if (gate != nullptr || residual != nullptr) return fail(VDMQ_EINVAL, "a split output takes neither gate nor residual");
+    }
+    return linear_bf6_checked(p, workspace, workspace_bytes, stream);
+}
+
+int64_t vdmq_linear_bf6_workspace(int64_t M, int64_t N, int64_t K, int act, int ln_mode, int64_t rows_per_gate, int64_t ldr, int out_dtype) {
+    if (M <= 0 || N <= 0 || K <= 0) return 0;
+    static const __half some = {};
+    ResidentProblem p = {};
+    p.M = M;
+    p.N = N;
+    p.K = K;
+    p.act = act;
+    p.ln_mode = ln_mode;
+    p.out_dtype = out_dtype;
+    p.tail = make_tail(rows_per_gate > 0 ? &some : nullptr, N, rows_per_gate, ldr > 0 ? &some : nullptr, ldr);
+    return resident_takes(p) ? 0 : vdmq_workspace_bytes_bf6(M, K);
 }
 
 int vdmq_linear_w4a4_bf6(const void *x, int64_t M, int64_t K, int64_t ldx, float clip, int act, const void *wblocks, const void *wscale,

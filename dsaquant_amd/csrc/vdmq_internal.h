@@ -75,6 +75,25 @@ int launch_gemm_bf6(const uint8_t *xblocks, const __half *ascale, const uint8_t 
                     void *out, int out_dtype, int32_t *acc_out, int64_t M, int64_t N, int64_t K, int64_t ldo, const GemmTail &tail,
                     hipStream_t stream);
 
+// quantizer and GEMM in one kernel for short rows (vdmq_resident.hip)
+struct ResidentProblem {
+    const __half *x;
+    int64_t M, K, ldx;
+    float clip;
+    int act, ln_mode; /* ln_mode 0: no LayerNorm */
+    float eps;
+    const __half *va, *vb;
+    int64_t ldv, rows_per_vec;
+    const uint8_t *wblocks;
+    const __half *wscale, *bias;
+    void *out;
+    int out_dtype;
+    int64_t N, ldo;
+    GemmTail tail;
+};
+bool resident_takes(const ResidentProblem &p); /* by its sizes and types alone */
+int launch_linear_resident(const ResidentProblem &p, hipStream_t stream);
+
 // attention between the linears (vdmq_attn.hip); strides in elements: row, head, batch
 struct AttentionArgs {
     const __half *q, *k, *v;

@@ -237,8 +237,12 @@ def linear_fused(
             _k._gemm_dispatch(pre.qact, pre.scales, pre.bf6, weight, b, out, K, gate=g2, rows_per_gate=rows_per_gate, residual=r2)
         elif M:
             bf6 = _k._use_bf6(M, N, K)
-            operand, scales = _k._quantize_for_gemm(x_2d, clip_ratio, act_code, bf6, None if pre is None else pre._args())
-            _k._gemm_dispatch(operand, scales, bf6, weight, b, out, K, gate=g2, rows_per_gate=rows_per_gate, residual=r2)
+            ln_args = None if pre is None else pre._args()
+            if bf6 and K <= 16384 and _k.matrix_path() != "bf6":
+                _k._linear_bf6_ex(x_2d, clip_ratio, act_code, ln_args, weight, b, out, gate=g2, rows_per_gate=rows_per_gate, residual=r2)
+            else:
+                operand, scales = _k._quantize_for_gemm(x_2d, clip_ratio, act_code, bf6, ln_args)
+                _k._gemm_dispatch(operand, scales, bf6, weight, b, out, K, gate=g2, rows_per_gate=rows_per_gate, residual=r2)
     return out.view(*lead, N) if split_cols is None else out.view(N // split_cols, *lead, split_cols)
 
 

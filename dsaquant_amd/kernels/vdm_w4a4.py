@@ -426,9 +426,10 @@ def _native_weights(qweight: torch.Tensor, wscales: torch.Tensor) -> Tuple[torch
 # "int8": v_mfma_i32_32x32x32_i8 on nibbles widened in registers.  "bf6": v_mfma_f32_32x32x64_f8f6f4 on 6-bit
 # floats (twice the rate, no widening work; every int4 value q is held as the E3M2 float q / 16, exactly, and the
 # fp32 accumulation of the products is exact too).
-# Both give bit-identical results.  "auto" asks the library (vdmq_bf6_pays: bf6 from a row length of 1280 on, whatever
-# the other sizes -- its GEMM has a tile configuration for small problems, and only its quantizer is the slower one on
-# short rows).
+# Both give bit-identical results.  "auto" takes bf6 for rows of 640 elements on, whatever the other sizes: up to 1536 the
+# library quantizes and multiplies in one kernel there (vdmq_linear_bf6), beyond them vdmq_bf6_pays holds.  "bf6" always runs
+# the quantizer and the tiled GEMM.
+_BF6_FROM_K = 640
 _MATRIX_PATH = os.environ.get("VDMQ_MATRIX_PATH", "auto")
 
 
@@ -447,9 +448,7 @@ def _use_bf6(M: int, N: int, K: int, out_dtype: torch.dtype = torch.float16, pat
     path = _MATRIX_PATH if path is None else path
     if path == "int8" or M == 0:
         return False
-    if path == "bf6":
-        return True
-    return bool(_lib.load().vdmq_bf6_pays(M, N, K))
+    return path == "bf6" or K >= _BF6_FROM_K
 
 
 def _to_bf6(native: torch.Tensor, rows: int, K: int) -> torch.Tensor:
@@ -512,6 +511,29 @@ def _gemm_dispatch(operand: torch.Tensor, scales: torch.Tensor, bf6: bool, weigh
         return
     _lib.check(lib.vdmq_gemm_w4a4_ex(operand.data_ptr(), scales.data_ptr(), w.data_ptr(), wscale.data_ptr(), bias_p, gate_p, ldg,
                                      rows_per_gate, res_p, ldr, out.data_ptr(), code, M, N, K, out.stride(0), s))
+
+
+def _linear_bf6_ex(x_2d: torch.Tensor, clip_ratio: float, act_code: int, ln_args: Optional[tuple], weight: PreparedWeight,
+                   bias: Optional[torch.Tensor], out: torch.Tensor, gate: Optional[torch.Tensor] = None, rows_per_gate: int = 1,
+                   residual: Optional[torch.Tensor] = None) -> None:
+    """``_quantize_for_gemm`` and ``_gemm_dispatch`` on the bf6 path in one library call, which picks the form (arguments as
+    there).  Must run under ``torch.cuda.device(out.device)``."""
+    lib = _lib.load()
+    M, K = x_2d.shape
+    ln_mode, eps, a, b, ldv, rows_per_vec = (0, 0.0, None, None, 0, 1) if ln_args is None else (ln_args[5], ln_args[4], *ln_args[6:])
+    if out.dim() == 3:
+        _require(gate is None and residual is None and out.dtype == torch.float16, "a split output takes neither gate nor residual and is fp16")
+        N, split_cols, part_stride, ldo = out.shape[0] * out.shape[2], out.shape[2], out.stride(0), out.stride(1)
+    else:
+        N, split_cols, part_stride, ldo = out.shape[1], 0, 0, out.stride(0)
+    gate_p, ldg = (None, 0) if gate is None else (gate.data_ptr(), gate.stride(0))
+    res_p, ldr = (None, 0) if residual is None else (residual.data_ptr(), residual.stride(0))
+    nbytes = lib.vdmq_linear_bf6_workspace(M, N, K, act_code, ln_mode, 0 if gate is None else rows_per_gate, ldr, _lib.VDMQ_OUT_F16)
+    workspace = torch.empty((nbytes,), dtype=torch.uint8, device=out.device) if nbytes else None
+    _lib.check(lib.vdmq_linear_bf6_ex(x_2d.data_ptr(), M, K, x_2d.stride(0), float(clip_ratio), act_code, ln_mode, eps, a, b, ldv, rows_per_vec,
+                                      weight.operand(True).data_ptr(), weight.wscale.data_ptr(), None if bias is None else bias.data_ptr(),
+                                      gate_p, ldg, rows_per_gate, res_p, ldr, split_cols, part_stride, out.data_ptr(), _lib.VDMQ_OUT_F16, N, ldo,
+                                      None if workspace is None else workspace.data_ptr(), nbytes, _stream(out.device)))
 
 
 # -------------------------------------------------------------- public API
@@ -597,12 +619,20 @@ def _linear_2d(x_2d: torch.Tensor, weight: PreparedWeight, bias: Optional[torch.
             # Quantizer and GEMM in one library call with one allocation behind them: a call of this function on a small
             # problem waits for the host, not for the GPU (512 x 1536 -> 3072: two kernels of 11 us, the host took 34 us
             # with two library calls, three allocations and a Stream object for each question after the stream).
-            fn, workspace_bytes = (lib.vdmq_linear_w4a4_bf6, lib.vdmq_workspace_bytes_bf6) if bf6 else (lib.vdmq_linear_w4a4_ex, lib.vdmq_workspace_bytes)
-            workspace = torch.empty((int(workspace_bytes(M, K)),), dtype=torch.uint8, device=dev)
+            out_code = _lib.VDMQ_OUT_F16 if out_dtype == torch.float16 else _lib.VDMQ_OUT_BF16
+            if not bf6:
+                fn, nbytes = lib.vdmq_linear_w4a4_ex, lib.vdmq_workspace_bytes(M, K)
+            elif _MATRIX_PATH == "bf6":
+                fn, nbytes = lib.vdmq_linear_w4a4_bf6, lib.vdmq_workspace_bytes_bf6(M, K)
+            else:
+                fn, nbytes = lib.vdmq_linear_bf6, lib.vdmq_linear_bf6_workspace(M, N, K, act_code, 0, 0, 0, out_code)
+            workspace = torch.empty((nbytes,), dtype=torch.uint8, device=dev) if nbytes else None
             _lib.check(fn(x_2d.data_ptr(), M, K, x_2d.stride(0), float(clip_ratio), act_code, weight.operand(bf6).data_ptr(), weight.wscale.data_ptr(),
-                          None if bias is None else bias.data_ptr(), out.data_ptr(),
-                          _lib.VDMQ_OUT_F16 if out_dtype == torch.float16 else _lib.VDMQ_OUT_BF16, N, N, workspace.data_ptr(), workspace.numel(),
-                          _stream(dev)))
+                          None if bias is None else bias.data_ptr(), out.data_ptr(), out_code, N, N,
+                          None if workspace is None else workspace.data_ptr(), nbytes, _stream(dev)))
+            return out
+        if bf6 and K <= 16384 and _MATRIX_PATH != "bf6":
+            _linear_bf6_ex(x_2d, clip_ratio, act_code, None, weight, bias, out)
             return out
         operand, scales = _quantize_for_gemm(x_2d, clip_ratio, act_code, bf6)
         _gemm_dispatch(operand, scales, bf6, weight, bias, out, K)

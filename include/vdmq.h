@@ -173,6 +173,7 @@ int vdmq_gemm_w4a4_acc(const void *qact, const void *wq, int32_t *acc, int64_t M
 #define VDMQ_KERNEL_GEMM_W4A4 1           /* int8 matrix path */
 #define VDMQ_KERNEL_GEMM_BF6 2            /* bf6 matrix path, one workgroup per tile (256 x 256, or 128 x 128 for small problems) */
 #define VDMQ_KERNEL_GEMM_BF6_PERSISTENT 3 /* bf6 matrix path, one workgroup per CU walking tiles */
+#define VDMQ_KERNEL_LINEAR_RESIDENT 4     /* bf6 matrix path, quantizer and GEMM in one kernel (short rows) */
 typedef struct vdmq_gemm_launch_info {
     int kernel;                 /* VDMQ_KERNEL_* */
     int tile_m, tile_n;         /* output tile of one workgroup: token rows x channels */
@@ -258,6 +259,21 @@ int64_t vdmq_workspace_bytes_bf6(int64_t M, int64_t K);
 int vdmq_linear_w4a4_bf6(const void *x, int64_t M, int64_t K, int64_t ldx, float clip, int act, const void *wblocks, const void *wscale,
                          const void *bias, void *out, int out_dtype, int64_t N, int64_t ldo, void *workspace, int64_t workspace_bytes,
                          vdmq_stream_t stream);
+/* The linear by whichever of the bf6 path's forms is fastest at its sizes: rows of 640 to 1536 elements, as a rule, run in ONE
+ * kernel, which quantizes the rows it works on into LDS (no workspace; `out` must not overlap `x`), all others as
+ * vdmq_linear_w4a4_bf6 does.  The same bits either way.  vdmq_linear_bf6_ex adds what the separate calls offer: ln_mode (0: none)
+ * with the arguments of vdmq_quantize_act_ln, gate and residual of vdmq_gemm_w4a4_ex, split_cols (0: none) and part_stride of
+ * vdmq_gemm_w4a4_split.  vdmq_linear_bf6_workspace: the bytes of workspace such a call needs (0: none); rows_per_gate 0: no
+ * gate, ldr 0: no residual. */
+int64_t vdmq_linear_bf6_workspace(int64_t M, int64_t N, int64_t K, int act, int ln_mode, int64_t rows_per_gate, int64_t ldr, int out_dtype);
+int vdmq_linear_bf6(const void *x, int64_t M, int64_t K, int64_t ldx, float clip, int act, const void *wblocks, const void *wscale,
+                    const void *bias, void *out, int out_dtype, int64_t N, int64_t ldo, void *workspace, int64_t workspace_bytes,
+                    vdmq_stream_t stream);
+int vdmq_linear_bf6_ex(const void *x, int64_t M, int64_t K, int64_t ldx, float clip, int act, int ln_mode, float eps, const void *a,
+                       const void *b, int64_t ldv, int64_t rows_per_vec, const void *wblocks, const void *wscale, const void *bias,
+                       const void *gate, int64_t ldg, int64_t rows_per_gate, const void *residual, int64_t ldr, int64_t split_cols,
+                       int64_t part_stride, void *out, int out_dtype, int64_t N, int64_t ldo, void *workspace, int64_t workspace_bytes,
+                       vdmq_stream_t stream);
 int vdmq_native_to_bf6(const void *native, int64_t rows, int64_t K, void *blocks, vdmq_stream_t stream);
 /* A checkpoint's v1 weight buffer (u8 [N, K/2], weight_quantize_per_channel_kernel's order, vdm_w4a4_kernel.cu:518-551)
  * straight to bf6 blocks: the one relayout a module needs when the bf6 path serves it, made once at load.
