@@ -397,7 +397,7 @@ int vdmq_bf6_to_weight_v1(const void *wblocks, void *qweight_v1, int64_t N, int6
 
 static int gemm_bf6_checked(const void *xblocks, const void *ascale, const void *wblocks, const void *wscale, const void *bias, void *out,
                             int out_dtype, int32_t *acc, int64_t M, int64_t N, int64_t K, int64_t ldo, const GemmTail &tail,
-                            vdmq_stream_t stream) {
+                            vdmq_stream_t stream, bool by_size = false) {
     VDMQ_TRY(check_k(K));
     VDMQ_TRY(check_n(N));
     VDMQ_TRY(check_m(M));
@@ -410,6 +410,9 @@ static int gemm_bf6_checked(const void *xblocks, const void *ascale, const void 
     } else {
         VDMQ_TRY(check_ptr(acc, "acc"));
     }
+    if (by_size && acc == nullptr && ksplit_takes(M, N, K, out_dtype))
+        return launch_gemm_bf6_ksplit(static_cast<const uint8_t *>(xblocks), static_cast<const __half *>(ascale), static_cast<const uint8_t *>(wblocks),
+                                      static_cast<const __half *>(wscale), static_cast<const __half *>(bias), out, M, N, K, ldo, tail, as_stream(stream));
     return launch_gemm_bf6(static_cast<const uint8_t *>(xblocks), static_cast<const __half *>(ascale), static_cast<const uint8_t *>(wblocks),
                            static_cast<const __half *>(wscale), static_cast<const __half *>(bias), out, out_dtype, acc, M, N, K, ldo, tail,
                            as_stream(stream));
@@ -456,7 +459,7 @@ int64_t vdmq_workspace_bytes_bf6(int64_t M, int64_t K) {
 
 // Quantizer and GEMM of the bf6 path for every form of a linear: rows as they are, through an activation or a LayerNorm;
 // output plain, with the gated residual update, or split by columns.  One kernel where the rows' operand fits LDS
-// (vdmq_resident.hip), else the two.
+// (vdmq_resident.hip), else the two, the GEMM by its size (vdmq_bf6_ksplit.hip; the separate entries keep the tiled one).
 static int linear_bf6_checked(const ResidentProblem &p, void *workspace, int64_t workspace_bytes, vdmq_stream_t stream) {
     VDMQ_TRY(check_k(p.K));
     VDMQ_TRY(check_n(p.N));
@@ -472,7 +475,7 @@ static int linear_bf6_checked(const ResidentProblem &p, void *workspace, int64_t
             VDMQ_TRY(quantize_act_ln_checked(p.x, p.M, p.K, p.ldx, p.eps, p.ln_mode, p.va, p.vb, p.ldv, p.rows_per_vec, p.clip, 1, blocks, scale, stream));
         else
             VDMQ_TRY(quantize_act_checked(p.x, p.M, p.K, p.ldx, p.clip, p.act, 1, blocks, scale, stream));
-        return gemm_bf6_checked(blocks, scale, p.wblocks, p.wscale, p.bias, p.out, p.out_dtype, nullptr, p.M, p.N, p.K, p.ldo, p.tail, stream);
+        return gemm_bf6_checked(blocks, scale, p.wblocks, p.wscale, p.bias, p.out, p.out_dtype, nullptr, p.M, p.N, p.K, p.ldo, p.tail, stream, true);
     }
     VDMQ_TRY(check_ptr(p.x, "x"));
     if (p.ldx < p.K || p.ldx % 8 != 0) return fail(VDMQ_ESHAPE, "ldx must be >= K and a multiple of 8 (got %lld)", (long long)p.ldx);

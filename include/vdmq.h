@@ -174,6 +174,7 @@ int vdmq_gemm_w4a4_acc(const void *qact, const void *wq, int32_t *acc, int64_t M
 #define VDMQ_KERNEL_GEMM_BF6 2            /* bf6 matrix path, one workgroup per tile (256 x 256, or 128 x 128 for small problems) */
 #define VDMQ_KERNEL_GEMM_BF6_PERSISTENT 3 /* bf6 matrix path, one workgroup per CU walking tiles */
 #define VDMQ_KERNEL_LINEAR_RESIDENT 4     /* bf6 matrix path, quantizer and GEMM in one kernel (short rows) */
+#define VDMQ_KERNEL_GEMM_BF6_KSPLIT 5     /* bf6 matrix path, K divided among the waves of a workgroup (few tiles, long rows) */
 typedef struct vdmq_gemm_launch_info {
     int kernel;                 /* VDMQ_KERNEL_* */
     int tile_m, tile_n;         /* output tile of one workgroup: token rows x channels */
@@ -261,7 +262,7 @@ int vdmq_linear_w4a4_bf6(const void *x, int64_t M, int64_t K, int64_t ldx, float
                          vdmq_stream_t stream);
 /* The linear by whichever of the bf6 path's forms is fastest at its sizes: rows of 640 to 1536 elements, as a rule, run in ONE
  * kernel, which quantizes the rows it works on into LDS (no workspace; `out` must not overlap `x`), all others as
- * vdmq_linear_w4a4_bf6 does.  The same bits either way.  vdmq_linear_bf6_ex adds what the separate calls offer: ln_mode (0: none)
+ * vdmq_linear_w4a4_bf6 does, with a GEMM of its own for few tiles.  The same bits either way.  vdmq_linear_bf6_ex adds what the separate calls offer: ln_mode (0: none)
  * with the arguments of vdmq_quantize_act_ln, gate and residual of vdmq_gemm_w4a4_ex, split_cols (0: none) and part_stride of
  * vdmq_gemm_w4a4_split.  vdmq_linear_bf6_workspace: the bytes of workspace such a call needs (0: none); rows_per_gate 0: no
  * gate, ldr 0: no residual. */

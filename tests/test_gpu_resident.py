@@ -1,5 +1,6 @@
-"""The one-kernel form of the linear for short rows (vdmq_linear_bf6): the bits of the quantizer and the tiled GEMM in every
-form it takes, at the edges of its row tiles, column strips and K steps, and the forms it leaves to those two."""
+"""The forms of a linear that vdmq_linear_bf6 chooses by size -- one kernel for short rows, K divided among a workgroup's waves for few
+tiles --: the bits of the quantizer and the tiled GEMM in every form they take, at the edges of their tiles, strips and K steps,
+and what they leave to those two."""
 import pytest
 import torch
 
@@ -7,8 +8,9 @@ from tests.test_gpu_parity import vk
 
 pytestmark = pytest.mark.gpu
 
-RESIDENT = 4  # VDMQ_KERNEL_LINEAR_RESIDENT of include/vdmq.h
+RESIDENT, KSPLIT = 4, 5  # VDMQ_KERNEL_* of include/vdmq.h
 F16 = torch.float16
+TILED = (2, 3)
 
 
 @pytest.fixture(scope="module")
@@ -44,7 +46,7 @@ def rows(M, K, seed=0):
     return x
 
 
-def both(f, resident=True):
+def both(f, kernel=RESIDENT):
     """``f()`` by the library's choice and as quantizer and tiled GEMM."""
     from dsaquant_amd import _lib
 
@@ -54,15 +56,16 @@ def both(f, resident=True):
         v.set_matrix_path("auto")
         got = f()
         info = _lib.last_gemm_launch()
-        assert (info.kernel == RESIDENT) == resident, info.kernel
+        assert info.kernel in kernel if isinstance(kernel, tuple) else info.kernel == kernel, info.kernel
         v.set_matrix_path("bf6")
         want = f()
-        assert _lib.last_gemm_launch().kernel != RESIDENT
+        assert _lib.last_gemm_launch().kernel in TILED
     finally:
         v.set_matrix_path(before)
     # NaN rows: the same positions; everything else bit for bit
     assert torch.equal(torch.isnan(got), torch.isnan(want))
-    assert torch.equal(torch.nan_to_num(got).view(torch.int16), torch.nan_to_num(want).view(torch.int16))
+    got, want = (torch.where(torch.isnan(t), torch.zeros_like(t), t) for t in (got, want))
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
     return info
 
 
@@ -92,11 +95,11 @@ def test_gated_residual_and_split(weight, M, N, K):
     both(lambda: F.linear_fused(x, qw, ws, None, 0.95, residual=res))
     both(lambda: F.linear_fused(x, qw, ws, b, 0.95, split_cols=64))
     both(lambda: F.linear_fused(x, qw, ws, b, 0.95, split_cols=N))
-    both(lambda: F.linear_fused(x, qw, ws, b, 0.95, gate=gate), resident=False)
-    both(lambda: F.linear_fused(x, qw, ws, b, 0.95, act="gelu_tanh"), resident=False)
+    both(lambda: F.linear_fused(x, qw, ws, b, 0.95, gate=gate), kernel=TILED + (KSPLIT,))
+    both(lambda: F.linear_fused(x, qw, ws, b, 0.95, act="gelu_tanh"), kernel=TILED + (KSPLIT,))
     if M > 1:
         token_gate = torch.randn(M, N, generator=g, device="cuda").half()
-        both(lambda: F.linear_fused(x, qw, ws, b, 0.95, residual=res, gate=token_gate), resident=False)
+        both(lambda: F.linear_fused(x, qw, ws, b, 0.95, residual=res, gate=token_gate), kernel=TILED + (KSPLIT,))
 
 
 @pytest.mark.parametrize("mode", ["modulate", "affine"])
@@ -111,7 +114,7 @@ def test_layer_norm_in_front(weight, B, L, N, K, mode):
     s, t = ((0.1 * torch.randn(vec, generator=g, device="cuda")).half() for _ in range(2))
     both(lambda: F.linear_ln_vdm_w4a4(F.LnInput(x, s, t, 1e-6, mode), qw, ws, b, 0.95))
     few = x[:, :40].contiguous()
-    both(lambda: F.linear_ln_vdm_w4a4(F.LnInput(few, s, t, 1e-6, mode), qw, ws, b, 0.95), resident=False)
+    both(lambda: F.linear_ln_vdm_w4a4(F.LnInput(few, s, t, 1e-6, mode), qw, ws, b, 0.95), kernel=TILED + (KSPLIT,))
 
 
 def test_strides_workspace_and_refusals_through_the_c_abi(weight):
@@ -169,3 +172,40 @@ def test_replays_from_a_hip_graph(weight):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, step())
+
+
+# K: k-blocks (64 elements, rounded up to an even number) from fewer than the four waves keep in flight to several times as many, each
+# remainder; M, N: one row, the edges of 64 x 64, 128 x 64 and 64 x 128 tiles, the last problems of one tile per CU and the first beyond
+@pytest.mark.parametrize("M,N,K,tile", [(1, 128, 1600, (64, 64)), (63, 256, 1664, (64, 64)), (65, 384, 1792, (64, 64)), (200, 128, 2048, (64, 64)),
+                                        (256, 4096, 2176, (64, 64)), (256, 4096, 13824, (64, 64)), (257, 4096, 4096, (128, 64)),
+                                        (500, 4096, 3328, (128, 64)), (385, 4096, 16384, (128, 64)), (289, 6400, 5120, (64, 128)),
+                                        (512, 4096, 3264, None), (513, 4096, 4096, None)])
+def test_few_tiles(weight, M, N, K, tile):
+    from dsaquant_amd import fused_ops as F
+
+    v = vk()
+    qw, ws, b = weight(N, K)
+    x = rows(M, K, 8)
+    kernel = TILED if tile is None else KSPLIT
+    info = both(lambda: v.linear_vdm_w4a4(x, qw, ws, b, 0.95), kernel)
+    assert tile is None or (info.tile_m, info.tile_n) == tile
+    both(lambda: v.linear_vdm_w4a4(x, qw, ws, None, 1e-3), kernel)
+    both(lambda: v._linear_2d(x, v._prepared_weight(qw, ws), b, 0.95, out_dtype=torch.bfloat16), TILED)
+    g = torch.Generator(device="cuda").manual_seed(11)
+    res = torch.randn(M, N, generator=g, device="cuda").half()
+    gates = [torch.randn(n, N, generator=g, device="cuda").half() for n in {1, M, 2 if M % 2 == 0 else 1}]
+    for gate in gates:
+        both(lambda: F.linear_fused(x, qw, ws, b, 0.95, residual=res, gate=gate), kernel)
+    both(lambda: F.linear_fused(x, qw, ws, None, 0.95, act="gelu_tanh", gate=gates[0]), kernel)
+    both(lambda: F.linear_fused(x, qw, ws, b, 0.95, residual=res), kernel)
+    for split in (64, 128, N):
+        both(lambda: F.linear_fused(x, qw, ws, b, 0.95, split_cols=split), kernel)
+
+
+@pytest.mark.parametrize("K", [640, 704, 768, 896, 1024])
+def test_few_tiles_short_rows(weight, K):
+    """... with fewer k-blocks than twelve or a remainder of each size, where the one-kernel form is not taken."""
+    from dsaquant_amd import fused_ops as F
+
+    qw, ws, b = weight(256, K)
+    both(lambda: F.linear_fused(rows(100, K, 9), qw, ws, b, 0.95, act="gelu_tanh"), KSPLIT)
