@@ -72,9 +72,9 @@ class LnInput:
             raise ValueError(f"unknown LayerNorm mode {mode!r}")
         self.shape = tuple(x.shape)
         K = x.shape[-1]
-        self.x = x.reshape(-1, K).half().contiguous()
+        self.x = _k._half_rows(x, K)
         M = self.x.shape[0]
-        a2, b2 = a.reshape(-1, K).half().contiguous(), b.reshape(-1, K).half().contiguous()
+        a2, b2 = _k._half_rows(a, K), _k._half_rows(b, K)
         if a2.shape != b2.shape:
             raise ValueError("the two LayerNorm vectors must have the same shape")
         nvec = a2.shape[0]
@@ -208,7 +208,7 @@ def linear_fused(
     N = weight.N
     b = bias_half if bias_half is not None else bias
     if b is not None:
-        b = b.half().contiguous().view(-1)
+        b = _k._half_vector(b)
         _k._check_device_tensor(b, "bias", torch.float16)
         _k._require(b.numel() == N, "bias length must equal N")
     g2 = r2 = None
@@ -216,7 +216,7 @@ def linear_fused(
     if gate is not None:
         if gate.shape[-1] != N:
             raise ValueError(f"gate must have {N} channels")
-        g2 = gate.reshape(-1, N).half().contiguous()
+        g2 = _k._half_rows(gate, N)
         _k._check_device_tensor(g2, "gate", torch.float16)
         if g2.shape[0] == 0 or (M and M % g2.shape[0] != 0):
             raise ValueError(f"{g2.shape[0]} gate vectors do not divide {M} rows")
@@ -224,14 +224,14 @@ def linear_fused(
     if residual is not None:
         if tuple(residual.shape) != tuple(lead) + (N,):
             raise ValueError(f"residual must have shape {tuple(lead) + (N,)}, got {tuple(residual.shape)}")
-        r2 = residual.reshape(-1, N).half().contiguous()
+        r2 = _k._half_rows(residual, N)
         _k._check_device_tensor(r2, "residual", torch.float16)
     if split_cols is not None:
         if gate is not None or residual is not None:
             raise ValueError("a split output takes neither gate nor residual")
         if split_cols <= 0 or split_cols % 64 != 0 or N % split_cols != 0:
             raise ValueError(f"split_cols must be a positive multiple of 64 that divides N={N} (got {split_cols})")
-    with torch.cuda.device(dev):
+    with _k._on(dev):
         out = torch.empty((M, N) if split_cols is None else (N // split_cols, M, split_cols), dtype=torch.float16, device=dev)
         if M and isinstance(pre, QuantizedInput):
             _k._gemm_dispatch(pre.qact, pre.scales, pre.bf6, weight, b, out, K, gate=g2, rows_per_gate=rows_per_gate, residual=r2)
