@@ -209,3 +209,24 @@ def test_few_tiles_short_rows(weight, K):
 
     qw, ws, b = weight(256, K)
     both(lambda: F.linear_fused(rows(100, K, 9), qw, ws, b, 0.95, act="gelu_tanh"), KSPLIT)
+
+
+@pytest.mark.parametrize("M,N,K", [(129, 1536, 1536), (2100, 1536, 1472), (200, 512, 4096), (500, 4096, 3328)])
+def test_residual_updated_in_place_through_the_c_abi(weight, M, N, K):
+    """``out`` is the residual: each element is read by the lane that writes it, before."""
+    from dsaquant_amd import _lib, fused_ops as F
+
+    lib, v = _lib.load(), vk()
+    qw, ws, b = weight(N, K)
+    x = rows(M, K, 12).nan_to_num(0.5, 9.0, -9.0)
+    g = torch.Generator(device="cuda").manual_seed(13)
+    out, gate = torch.randn(M, N, generator=g, device="cuda").half(), torch.randn(1, N, generator=g, device="cuda").half()
+    want = F.linear_fused(x, qw, ws, b, 0.95, residual=out, gate=gate)
+    pw = v._prepared_weight(qw, ws)
+    nbytes = lib.vdmq_linear_bf6_workspace(M, N, K, 0, 0, M, N, 0)
+    workspace = torch.empty(max(nbytes, 1), dtype=torch.uint8, device="cuda")
+    _lib.check(lib.vdmq_linear_bf6_ex(x.data_ptr(), M, K, K, 0.95, 0, 0, 0.0, None, None, 0, 1, pw.operand(True).data_ptr(), pw.wscale.data_ptr(),
+                                      b.data_ptr(), gate.data_ptr(), N, M, out.data_ptr(), N, 0, 0, out.data_ptr(), 0, N, N, workspace.data_ptr(),
+                                      nbytes, torch.cuda.current_stream().cuda_stream))
+    assert _lib.last_gemm_launch().kernel in (RESIDENT, KSPLIT)
+    assert torch.equal(out, want)
