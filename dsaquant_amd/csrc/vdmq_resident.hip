@@ -13,7 +13,8 @@
 // the host's), 3613 x 1024 -> 4096 24.6 -> 17.9, 4096 x 1536 -> 4608 31.9 -> 26.2, 32760 x 1536 -> 4608 149 -> 126, -> 1536 with gate
 // and residual 98.5 -> 80.5.  What bounds it: at 32760 x 1536 -> 4608 the matrix cores, busy two thirds of the time at the
 // 1.7 GHz the chip holds under them; taking instructions out of the K step or moving its loads changed nothing there.  At a few
-// thousand rows the quantization, 10 us of 26 at 4096 rows, which is bound by its vector instructions.
+// thousand rows the quantization, repeated in every column group (5 us of 26 at 4096 rows; half the vector instructions in its absmax
+// changed nothing), and the weights' way into the registers for 64 or 32 rows at a time.
 // Why 64 columns and two waves per SIMD: 32 x MI x 64 sums fill half of a wave's registers at MI = 4, and 64 columns are the 128-byte lines
 // that an epilogue needs; weights through LDS would take the room of the rows and a barrier per step, and each weight byte is read once
 // per CU as it is.  Non-temporal stores because the next kernel reads most outputs too late to find them in L2, where
@@ -531,8 +532,9 @@ int launch_pre(const ResidentArgs &args, int pre, bool tail, hipStream_t s) {
 // strips -- takes, at K = 1536, about 2.5 us per 32 rows for the first part (8 with the LayerNorm, which is bound by its
 // instructions) and, for the second, a pass of its eight waves over eight strips 10.6 / 8 / 6 us with 128 / 64 / 32 rows (32 rows load
 // as many weight bytes as 128), half of them (a wave per SIMD) 6.3 / 5 / 4.  Fewer rows suit problems that give the chip's CUs no
-// 128 each; among equals the fewer groups, each of which quantizes the tile again.  On 40 shapes of 34 ... 75600 rows, K 640 ... 1536,
-// the choice is within 10 % of the best one found, within 2 % on three quarters of them.
+// 128 each; among equals the fewer groups, each of which quantizes the tile again.  On 120 shapes of 64 ... 75637 rows, K 640 ...
+// 1536, every candidate timed, the choice takes 1.2 % more than the best one in the geometric mean, 12 % at most.  (Figures fitted to 75 of
+// them: 0.7 and 6 % there, 0.8 and 7 % on the others, but narrow outputs of many rows went to 32 rows at a time.)
 struct ResidentShape {
     int mi, tiles, groups;
     int64_t time; /* estimate at K = 1536, in units of 0.1 us */
