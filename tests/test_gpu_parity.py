@@ -1087,3 +1087,39 @@ def test_reference_written_checkpoint_runs_through_the_kernels(tag):
         bias = None if layer.bias is None else layer.bias.detach().cpu().numpy()
         want = O.np_linear(x, qw, ws, bias, 0.95)[0]
         assert y.dtype == torch.float16 and np.array_equal(y.cpu().numpy().view(np.uint16), want.view(np.uint16))
+
+
+@pytest.mark.parametrize("path", ["auto", "bf6", "int8"])
+@pytest.mark.parametrize("K,N", [(1536, 256), (2048, 256), (640, 128)])
+def test_one_row_of_any_stride(K, N, path):
+    """A single row whose stride is not its length (a slice of wider rows, an expanded vector) runs as its copy does: as the
+    input, the residual, the gate and the LayerNorm's vectors."""
+    from dsaquant_amd import fused_ops as F
+
+    v = vk()
+    g = torch.Generator(device=DEV).manual_seed(K + N)
+    randn = lambda *s: torch.randn(*s, generator=g, device=DEV).half()  # noqa: E731
+    qw, ws, _ = v.pack_weight_with_scale(0.01 * randn(N, K), (0.002 + 0.01 * torch.rand(N, generator=g, device=DEV)).half())
+    b = randn(N)
+
+    def forms(n):
+        return randn(6, n + 4)[2:3, :n], randn(1, n).expand(3, n)[0:1], randn(6, n + 8)[2:3, :n]
+
+    before = v.matrix_path()
+    try:
+        v.set_matrix_path(path)
+        for x, a, s, gate, res in zip(forms(K), forms(K), forms(K), forms(N), forms(N)):
+            assert x.is_contiguous() and x.stride(0) != K and gate.stride(0) != N
+            calls = [lambda x, a, s, gate, res: v.linear_vdm_w4a4(x, qw, ws, b, 0.95),
+                     lambda x, a, s, gate, res: v.linear_vdm_w4a4_prepared(x, v.PreparedWeight([(qw, ws)]), b, 0.95),
+                     lambda x, a, s, gate, res: F.linear_fused(x, qw, ws, b, 0.95, residual=res, gate=gate),
+                     lambda x, a, s, gate, res: F.linear_fused(F.QuantizedInput(x, 0.95), qw, ws, b, 0.95, residual=res, gate=gate),
+                     lambda x, a, s, gate, res: F.linear_ln_vdm_w4a4(F.LnInput(x, a, s, 1e-6, "affine"), qw, ws, b, 0.95),
+                     lambda x, a, s, gate, res: F.LnInput(x, a, s, 1e-6).materialize()]
+            dense = [torch.empty(t.shape, dtype=t.dtype, device=DEV).copy_(t) for t in (x, a, s, gate, res)]
+            assert all(t.stride(0) == t.shape[1] for t in dense)
+            for i, call in enumerate(calls):
+                got, want = call(x, a, s, gate, res), call(*dense)
+                assert torch.equal(got.view(torch.int16), want.view(torch.int16)), i
+    finally:
+        v.set_matrix_path(before)

@@ -532,6 +532,22 @@ def test_bf6_tile_order_takes_every_tile_once(tmp_path):
     assert res.returncode == 0 and res.stdout.startswith("ok "), res.stdout
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_rows_handed_to_the_library_lie_k_apart(dtype):
+    """A single row counts as contiguous whatever its row stride; the kernels' wrapper passes the stride on."""
+    from dsaquant_amd.kernels import vdm_w4a4 as v
+
+    K = 192
+    base = torch.arange(6 * (K + 4)).view(6, K + 4).to(dtype)
+    row, plain = base[3:4, :K], base[:, :K].contiguous()
+    for x in (row, row[0], row[None], row[0].expand(4, K)[1:2], base[:, :K], plain, plain.view(2, 3, K)):
+        got = v._half_rows(x, K)
+        want = x.reshape(-1, K).half().contiguous()
+        assert got.shape == want.shape and got.stride() == want.stride() == (K, 1) and torch.equal(got, want), x.stride()
+    ready = plain.half()
+    assert v._half_rows(ready, K) is ready
+
+
 @pytest.mark.parametrize("pack", ["quantize_weight_per_channel", "pack_weight_with_scale"])
 def test_packing_asks_for_the_library_first(monkeypatch, pack):
     """Without the library packing fails with the reason, which load_error() keeps, whatever it was given."""
