@@ -778,10 +778,16 @@ int launch_bf6_to_weight_v1(const uint8_t *blocks, int64_t N, int64_t K, uint8_t
 
 namespace {
 
+// Order in which the tiles of a problem are taken
+struct Bf6Plan {
+    Bf6TileMap tm;
+    int64_t load;      /* tiles of the XCD that has most, in the order that was chosen by them (0: not counted, below 0: no order) */
+    bool at_once;      /* the chip holds all tiles at once */
+    bool spread;       /* equal runs for the XCDs */
+};
+
 template <class Cfg>
-int launch_bf6_cfg(const uint8_t *xblocks, const __half *ascale, const uint8_t *wblocks, const __half *wscale, const __half *bias,
-                   __half *out, bool out_bf16, int32_t *acc_out, int64_t M, int64_t N, int64_t K, int64_t ldo, const GemmTail &tail,
-                   hipStream_t s) {
+Bf6Plan bf6_plan(int64_t M, int64_t N) {
     const int tiles_m = static_cast<int>(ceil_div(M, Cfg::BM)), tiles_n = static_cast<int>(ceil_div(N, Cfg::BN));
     // Places per super-tile: what an XCD's CUs hold at once.
     constexpr int per_log2 = Cfg::kPerLog2, per = 1 << per_log2;
@@ -838,6 +844,21 @@ int launch_bf6_cfg(const uint8_t *xblocks, const __half *ascale, const uint8_t *
         bf6_tilemap_strips(tm, tiles_m, tiles_n);
     else if (spread) /* (small tiles of more than one round are refilled as they end: 4 x 4, which reads fewer operand rows) */
         bf6_tilemap_shape(tm, tiles_m, tiles_n, 4, 2, true);
+    return {tm, best_load, at_once, spread};
+}
+
+// Rounds of a workgroup per CU position within 15 % of the busiest XCD's tiles / CUs
+bool few_empty_places(int64_t total_super, int64_t busiest) { return ceil_div(total_super, kXcds) * 100 <= ceil_div(busiest, 32) * 115; }
+
+template <class Cfg>
+int launch_bf6_cfg(const uint8_t *xblocks, const __half *ascale, const uint8_t *wblocks, const __half *wscale, const __half *bias,
+                   __half *out, bool out_bf16, int32_t *acc_out, int64_t M, int64_t N, int64_t K, int64_t ldo, const GemmTail &tail,
+                   hipStream_t s) {
+    Bf6Plan plan = bf6_plan<Cfg>(M, N);
+    Bf6TileMap &tm = plan.tm;
+    const int64_t best_load = plan.load, all_tiles = static_cast<int64_t>(tm.tiles_m) * tm.tiles_n;
+    const bool spread = plan.spread;
+    constexpr int per = 1 << Cfg::kPerLog2;
     const int places = 1 << tm.per_log2;
     const int64_t total_super = tm.total_super;
     if (best_load < 0 || total_super * per + kXcds * per > (int64_t(1) << 30))
@@ -884,8 +905,7 @@ int launch_bf6_cfg(const uint8_t *xblocks, const __half *ascale, const uint8_t *
     static int cu_count[kMaxDevices] = {};
     if (cu_count[dev] == 0 && hipDeviceGetAttribute(&cu_count[dev], hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) cu_count[dev] = -1;
     // (its contiguous runs hold equal numbers of super-tiles: a round each, however full)
-    const int64_t rounds_p = ceil_div(total_super, kXcds);
-    const bool persistent = Cfg::kOcc == 1 && !spread && which != 2 && cu_count[dev] == kXcds * per && rounds_p * 100 <= ceil_div(busiest, per) * 115;
+    const bool persistent = Cfg::kOcc == 1 && !spread && which != 2 && cu_count[dev] == kXcds * per && few_empty_places(total_super, busiest);
     if constexpr (Cfg::kOcc == 1) if (persistent) {
         if (contig) bf6_tilemap_runs(tm, false);
         using PKernel = void (*)(const uint8_t *, const uint8_t *, const __half *, const __half *, const __half *, __half *, int, int, int,
@@ -911,34 +931,56 @@ int launch_bf6_cfg(const uint8_t *xblocks, const __half *ascale, const uint8_t *
                        static_cast<int>(M), static_cast<int>(N), static_cast<int>(bf6_kblocks(K)), ldo, tm, tail);
     const int rc = check_launch("gemm_bf6_kernel");
     if (rc == VDMQ_OK)
-        record_gemm_launch({VDMQ_KERNEL_GEMM_BF6, Cfg::BM, Cfg::BN, tm.strips > 0 ? static_cast<int>(ceil_div(tiles_m, tm.strips)) : places >> tm.group_n_log2,
+        record_gemm_launch({VDMQ_KERNEL_GEMM_BF6, Cfg::BM, Cfg::BN, tm.strips > 0 ? static_cast<int>(ceil_div(tm.tiles_m, tm.strips)) : places >> tm.group_n_log2,
                             1 << tm.group_n_log2, tm.contig,
                             static_cast<int64_t>(grid.x)});
     return rc;
 }
 
+// Problems of at most two 128 x 128 tiles per CU -- at most half a 256 x 256 tile, but for the padding of odd edges --
+// take those, two workgroups of four waves per CU: four times as many workgroups for the same K loop, all of them
+// running at once.  Measured on 210 shapes (M 1...32768, N 128...15360, K 64...13824): up to there the small tiles take
+// 0.4...0.9 of the time (512 x 5120 -> 10240: 29 -> 25 us, 512 x 1536 -> 3072: 13.5 -> 7.3 us, 5888 x 13824 -> 1408, 506
+// tiles: 97 -> 69 us), beyond, where some CU gets a third one, 0.85...1.4.
+// Just above one big tile per CU the second round of big ones is nearly empty.  Small ones win there where they fill two
+// rounds at most (1024 tiles): 0.76...0.99 of the time over 30 shapes with K 512...13824 (5057 x 2560 -> 3200 34.7 / 29.8
+// us, 17205 x 5120 -> 896 55.4 / 50.4, 4920 x 8960 -> 3328 92.7 / 81.2).  With a few tiles more the third round's cost grows
+// with K, the big tiles' epilogue, which it replaces, does not: small / big up to 288 big tiles 0.87...1.02 for K <= 1536
+// (4096 x 1536 -> 4608 26.4 / 25.5 us), 0.95...1.05 for K = 2048...4096, 1.00...1.10 from 5120 on (7302 x 8960 -> 2304 92.6 /
+// 98.3); the big tiles' epilogue is longer with the gated tail: 0.83...1.00 up to K = 3072, to 1.02 at 4096, to 1.07 at 8960.
+bool small_tiles_serve(int64_t M, int64_t N, int64_t K, bool has_tail) {
+    const int64_t big_tiles = ceil_div(M, Bf6Big::BM) * ceil_div(N, Bf6Big::BN), small_tiles = ceil_div(M, Bf6Small::BM) * ceil_div(N, Bf6Small::BN);
+    const bool above_one_round = big_tiles > kXcds * 32 && big_tiles <= kXcds * 36 && (small_tiles <= kXcds * 32 * 4 || K <= (has_tail ? 3072 : 1536));
+    return small_tiles <= kXcds * 32 * 2 || above_one_round;
+}
+
 }  // namespace
+
+// Quantizer and tiled GEMM at K = 1280 ... 1536, us: for the rule that sets the one-kernel linear against them (vdmq_resident.hip), as that
+// one's estimate from its sizes alone.  Launches and the quantizer's way through memory, what a CU's tiles take in turn, the output (and
+// residual) bytes.  Fitted to 8300 timings, M to 75600, N to 25600: 0.91 ... 1.08 of what was measured at 90 % of them.
+// Where an XCD's tiles leave partly empty super-tiles, CUs are dealt out by fours: 25, 27 or 30 tiles on its 32 CUs take two
+// rounds (5 x 34 and 3 x 73 tiles 30 us, 5 x 32 and 3 x 64 20).
+double bf6_two_kernels_us(int64_t M, int64_t N, int64_t K, bool has_tail) {
+    const double k = K / 1536.0, x = M * K * 1e-6, out = M * N * 1e-6;
+    auto load_of = [](const Bf6Plan &p) { return p.spread || p.load <= 0 ? ceil_div(static_cast<int64_t>(p.tm.tiles_m) * p.tm.tiles_n, kXcds) : p.load; };
+    if (small_tiles_serve(M, N, K, has_tail)) {
+        const double rounds = ceil_div(load_of(bf6_plan<Bf6Small>(M, N)), 32);
+        return has_tail ? 8.3 + 0.46 * x + 2.8 * rounds * k + 0.69 * out : 7.5 + 0.51 * x + 2.4 * rounds * k + 0.63 * out;
+    }
+    const Bf6Plan p = bf6_plan<Bf6Big>(M, N);
+    const int64_t load = load_of(p);
+    const bool persistent = !p.spread && few_empty_places(p.tm.total_super, load), doubled = p.at_once && !p.spread && load > 24 && load % 4 != 0;
+    const double rounds = persistent ? ceil_div(p.tm.total_super, kXcds) : doubled ? 2 : ceil_div(load, 32);
+    return has_tail ? 6.7 + 0.48 * x + 10.1 * rounds * k + 0.67 * out : 8.6 + 0.45 * x + 7.6 * rounds * k + 0.50 * out;
+}
 
 int launch_gemm_bf6(const uint8_t *xblocks, const __half *ascale, const uint8_t *wblocks, const __half *wscale, const __half *bias,
                     void *out, int out_dtype, int32_t *acc_out, int64_t M, int64_t N, int64_t K, int64_t ldo, const GemmTail &tail,
                     hipStream_t s) {
     if (M == 0 || N == 0) return VDMQ_OK;
     // (both 16-bit output types go through the same staging and stores; the kernels take the pointer as fp16)
-    // Problems of at most two 128 x 128 tiles per CU -- at most half a 256 x 256 tile, but for the padding of odd edges --
-    // take those, two workgroups of four waves per CU: four times as many workgroups for the same K loop, all of them
-    // running at once.  Measured on 210 shapes (M 1...32768, N 128...15360, K 64...13824): up to there the small tiles take
-    // 0.4...0.9 of the time (512 x 5120 -> 10240: 29 -> 25 us, 512 x 1536 -> 3072: 13.5 -> 7.3 us, 5888 x 13824 -> 1408, 506
-    // tiles: 97 -> 69 us), beyond, where some CU gets a third one, 0.85...1.4.
-    // Just above one big tile per CU the second round of big ones is nearly empty.  Small ones win there where they fill two
-    // rounds at most (1024 tiles): 0.76...0.99 of the time over 30 shapes with K 512...13824 (5057 x 2560 -> 3200 34.7 / 29.8
-    // us, 17205 x 5120 -> 896 55.4 / 50.4, 4920 x 8960 -> 3328 92.7 / 81.2).  With a few tiles more the third round's cost grows
-    // with K, the big tiles' epilogue, which it replaces, does not: small / big up to 288 big tiles 0.87...1.02 for K <= 1536
-    // (4096 x 1536 -> 4608 26.4 / 25.5 us), 0.95...1.05 for K = 2048...4096, 1.00...1.10 from 5120 on (7302 x 8960 -> 2304 92.6 /
-    // 98.3); the big tiles' epilogue is longer with the gated tail: 0.83...1.00 up to K = 3072, to 1.02 at 4096, to 1.07 at 8960.
-    const int64_t big_tiles = ceil_div(M, Bf6Big::BM) * ceil_div(N, Bf6Big::BN), small_tiles = ceil_div(M, Bf6Small::BM) * ceil_div(N, Bf6Small::BN);
-    const bool has_tail = tail.gate != nullptr || tail.residual != nullptr;
-    const bool above_one_round = big_tiles > kXcds * 32 && big_tiles <= kXcds * 36 && (small_tiles <= kXcds * 32 * 4 || K <= (has_tail ? 3072 : 1536));
-    if (small_tiles <= kXcds * 32 * 2 || above_one_round)
+    if (small_tiles_serve(M, N, K, tail.gate != nullptr || tail.residual != nullptr))
         return launch_bf6_cfg<Bf6Small>(xblocks, ascale, wblocks, wscale, bias, static_cast<__half *>(out), out_dtype == VDMQ_OUT_BF16, acc_out, M,
                                         N, K, ldo, tail, s);
     return launch_bf6_cfg<Bf6Big>(xblocks, ascale, wblocks, wscale, bias, static_cast<__half *>(out), out_dtype == VDMQ_OUT_BF16, acc_out, M, N,

@@ -75,6 +75,8 @@ int launch_gemm_bf6(const uint8_t *xblocks, const __half *ascale, const uint8_t 
                     void *out, int out_dtype, int32_t *acc_out, int64_t M, int64_t N, int64_t K, int64_t ldo, const GemmTail &tail,
                     hipStream_t stream);
 
+double bf6_two_kernels_us(int64_t M, int64_t N, int64_t K, bool has_tail); /* an estimate, K 1280 ... 1536 */
+
 // problems with few tiles: K divided among a workgroup's waves (vdmq_bf6_ksplit.hip)
 bool ksplit_takes(int64_t M, int64_t N, int64_t K, int out_dtype);
 int launch_gemm_bf6_ksplit(const uint8_t *xblocks, const __half *ascale, const uint8_t *wblocks, const __half *wscale, const __half *bias, void *out, int64_t M,

@@ -537,12 +537,13 @@ int launch_pre(const ResidentArgs &args, int pre, bool tail, hipStream_t s) {
 // them: 0.7 and 6 % there, 0.8 and 7 % on the others, but narrow outputs of many rows went to 32 rows at a time.)
 struct ResidentShape {
     int mi, tiles, groups;
-    int64_t time; /* estimate at K = 1536, in units of 0.1 us */
+    int64_t rounds; /* of units on a CU */
+    int64_t time;   /* estimate at K = 1536, in units of 0.1 us */
 };
 ResidentShape resident_shape(int64_t M, int64_t N, bool ln) {
     constexpr int64_t kCus = 256;
     const int64_t strips = N / kStripCols, quantize = ln ? 80 : 25;
-    ResidentShape best = {0, 0, 0, 0};
+    ResidentShape best = {0, 0, 0, 0, 0};
     const int mis[3] = {4, 2, 1}, full[3] = {106, 80, 60}, part[3] = {63, 50, 40};
     for (int i = 0; i < 3; ++i) {
         const int64_t tiles = ceil_div(M, 32 * mis[i]);
@@ -552,14 +553,33 @@ ResidentShape resident_shape(int64_t M, int64_t N, bool ln) {
             const int64_t per = ceil_div(strips, g), rest = per % kWaves, second = rest - kWaves / 2; /* of the last pass: waves that share a SIMD */
             const int64_t last = rest == 0 ? 0 : part[i] + (second > 0 ? (full[i] - part[i]) * second / (kWaves / 2) : 0);
             const int64_t unit = quantize * mis[i] + per / kWaves * full[i] + last;
-            const int64_t time = ceil_div(tiles * g, kCus) * unit;
-            if (best.mi == 0 || time < best.time) best = {mis[i], static_cast<int>(tiles), static_cast<int>(g), time};
+            const int64_t rounds = ceil_div(tiles * g, kCus), time = rounds * unit;
+            if (best.mi == 0 || time < best.time) best = {mis[i], static_cast<int>(tiles), static_cast<int>(g), rounds, time};
         }
     }
     return best;
 }
 
 }  // namespace
+
+// The one-kernel linear's time at K = 1280 ... 1536, us: quantization and strips of its units as resident_shape counts them, output (and
+// residual), what the XCDs fetch.  A residual that comes from memory -- rows in, residual and output together more than 150 MB --
+// is waited for at every turn of the epilogue.  Fitted to the timings of bf6_two_kernels_us, within 0.91 ... 1.07 at 90 % of them.
+static double resident_us(int64_t M, int64_t N, int64_t K, bool has_tail, const ResidentShape &s) {
+    const double k = K / 1536.0, rows = M * K * 2e-6, w = N * K * 0.75e-6, out = M * N * 1e-6;
+    const double quantize = 2.5 * s.mi * s.rounds, strips = s.time * 0.1 - quantize;
+    const double by_rows = w + rows * (s.groups < kXcds ? s.groups : kXcds), by_weights = rows + w * (s.tiles < kXcds ? s.tiles : kXcds);
+    const double fetch = by_rows < by_weights ? by_rows : by_weights;
+    const double waits = M * (2 * K + 4 * N) > 150000000 ? strips : 0.0;
+    if (!has_tail) {
+        if (s.mi == 1) return 1.77 * quantize + 0.75 * strips * k + 0.83 * out + 0.022 * fetch;
+        if (s.mi == 2) return 1.16 * quantize + 0.50 * strips * k + 0.41 * out + 0.119 * fetch;
+        return 1.32 * quantize + 0.61 * strips * k + 0.26 * out + 0.035 * fetch;
+    }
+    if (s.mi == 1) return 1.50 * quantize + 0.84 * strips * k + 0.99 * out + 0.042 * fetch;
+    if (s.mi == 2) return 1.30 * quantize + 0.39 * strips * k + 0.65 * out + 0.116 * fetch + 0.27 * waits;
+    return 1.30 * quantize + 0.57 * strips * k + 0.48 * out + 0.045 * fetch + 0.47 * waits;
+}
 
 bool resident_takes(const ResidentProblem &p) {
     // Rows of up to 1536 elements fit LDS; shorter ones than 640 are the int8 path's.  In front of it no GELU, in its epilogue
@@ -568,7 +588,18 @@ bool resident_takes(const ResidentProblem &p) {
     const GemmTail &t = p.tail;
     const bool tail = t.residual == nullptr ? t.gate == nullptr : (t.gate == nullptr || t.rows_per_gate >= p.M) && t.ldr <= (1 << 22) && p.ln_mode == 0;
     if (p.K < 640 || p.K > 1536 || p.M > (1 << 24) || p.out_dtype != VDMQ_OUT_F16 || p.act != VDMQ_ACT_NONE || !tail) return false;
-    if (p.ln_mode == 0) return true;
+    if (p.ln_mode == 0) {
+        // Against quantizer and tiled GEMM it takes 0.5 ... 0.95 of the time as a rule, but it loses where their tiles fill the CUs exactly
+        // and its units do not (2459 x 1536 -> 6144 with a residual 33.4 / 26.7 us, 679 x 1472 -> 13056 22.4 / 20.8), and with a residual
+        // from memory in front of a wide output (11450 x 1536 -> 11136 203 / 164): so both are estimated.  Not slower, so not asked:
+        // K < 1280 than the int8 path, which served those (6500 timings, 0.995 at most), N <= 384 (550, 1.03).  Few tiles with K divided
+        // (vdmq_bf6_ksplit.hip): 0.93 of that one's time, 1.11 at most, and a launch less for the host.  Of 22000 timings of K 640 ... 1536
+        // the choice takes over 1.03 of the time of the path that served the size before at 0.9 %, over 1.06 at 0.2 % (always one
+        // kernel: 2.3 and 0.9 %), 1.15 at most.
+        if (p.K < 1280 || p.N <= 384 || ksplit_takes(p.M, p.N, p.K, p.out_dtype) || p.M * p.N > (int64_t(1) << 40)) return true;
+        const ResidentShape shape = resident_shape(p.M, p.N, false);
+        return resident_us(p.M, p.N, p.K, t.residual != nullptr, shape) < bf6_two_kernels_us(p.M, p.N, p.K, t.residual != nullptr);
+    }
     // Behind a LayerNorm only where its instructions, repeated in each column group, cost less than the second launch and the
     // blocks' way through memory: in effect where a row tile is one workgroup's (K = 1536, us, here / as two kernels: 28000 -> 4608 128 /
     // 147, 32760 -> 1536 73 / 85, -> 8960 233 / 289; 4680 -> 4608 47 / 40, 40000 -> 4608 245 / 203).  Two kernels: 29 us for the

@@ -260,12 +260,12 @@ int64_t vdmq_workspace_bytes_bf6(int64_t M, int64_t K);
 int vdmq_linear_w4a4_bf6(const void *x, int64_t M, int64_t K, int64_t ldx, float clip, int act, const void *wblocks, const void *wscale,
                          const void *bias, void *out, int out_dtype, int64_t N, int64_t ldo, void *workspace, int64_t workspace_bytes,
                          vdmq_stream_t stream);
-/* The linear by whichever of the bf6 path's forms is fastest at its sizes: rows of 640 to 1536 elements, as a rule, run in ONE
- * kernel, which quantizes the rows it works on into LDS (no workspace; `out` must not overlap `x`), all others as
- * vdmq_linear_w4a4_bf6 does, with a GEMM of its own for few tiles.  The same bits either way.  vdmq_linear_bf6_ex adds what the separate calls offer: ln_mode (0: none)
- * with the arguments of vdmq_quantize_act_ln, gate and residual of vdmq_gemm_w4a4_ex, split_cols (0: none) and part_stride of
- * vdmq_gemm_w4a4_split.  vdmq_linear_bf6_workspace: the bytes of workspace such a call needs (0: none); rows_per_gate 0: no
- * gate, ldr 0: no residual. */
+/* The linear by the form of the bf6 path that is estimated to be the fastest at its sizes and types: rows of 640 to 1536 elements, as
+ * a rule, run in ONE kernel, which quantizes the rows it works on into LDS (no workspace; `out` must not overlap `x`); all others, and
+ * those sizes whose tiles fill the chip better, run as vdmq_linear_w4a4_bf6 does, with a GEMM of its own for few tiles.  The same bits
+ * either way.  vdmq_linear_bf6_ex adds what the separate calls offer: ln_mode (0: none) with the arguments of vdmq_quantize_act_ln, gate
+ * and residual of vdmq_gemm_w4a4_ex, split_cols (0: none) and part_stride of vdmq_gemm_w4a4_split.  vdmq_linear_bf6_workspace: the bytes of
+ * workspace such a call needs (0: none); rows_per_gate 0: no gate, ldr 0: no residual. */
 int64_t vdmq_linear_bf6_workspace(int64_t M, int64_t N, int64_t K, int act, int ln_mode, int64_t rows_per_gate, int64_t ldr, int out_dtype);
 int vdmq_linear_bf6(const void *x, int64_t M, int64_t K, int64_t ldx, float clip, int act, const void *wblocks, const void *wscale,
                     const void *bias, void *out, int out_dtype, int64_t N, int64_t ldo, void *workspace, int64_t workspace_bytes,

@@ -82,6 +82,19 @@ def test_plain_linear(weight, M, N, tile, K):
     both(lambda: v.linear_vdm_w4a4(x, qw, ws, None, 1e-3 if M % 2 else 1.0))
 
 
+@pytest.mark.parametrize("M,N,K", [(679, 13056, 1472), (720, 10880, 1536)])
+def test_left_to_two_kernels_where_they_are_faster(weight, M, N, K):
+    from dsaquant_amd import fused_ops as F
+
+    v = vk()
+    qw, ws, b = weight(N, K)
+    x = rows(M, K)
+    both(lambda: v.linear_vdm_w4a4(x, qw, ws, b, 0.95), TILED)
+    both(lambda: F.linear_fused(x, qw, ws, b, 0.95, split_cols=64), TILED)
+    res = torch.randn(M, N, device="cuda").half()
+    both(lambda: F.linear_fused(x, qw, ws, b, 0.95, residual=res), TILED if K == 1536 else RESIDENT)
+
+
 @pytest.mark.parametrize("K", [640, 1472, 1536])
 @pytest.mark.parametrize("M,N", [(1, 128), (257, 1536), (1500, 1536), (4100, 1536)])
 def test_gated_residual_and_split(weight, M, N, K):

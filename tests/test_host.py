@@ -515,6 +515,22 @@ def test_library_says_where_the_fp6_path_pays():
     assert not pays(0, 128, 5120) and not pays(-1, 128, 5120)
 
 
+@pytest.mark.parametrize("M,N,K,residual,one", [
+    (679, 13056, 1472, False, False), (720, 10880, 1536, False, False), (590, 13056, 1536, True, False),      # their tiles fill the CUs once
+    (2459, 6144, 1536, True, False), (11450, 11136, 1536, True, False), (35303, 4992, 1536, True, False),     # ... a residual from memory
+    (545, 17536, 1536, False, True), (1043, 8576, 1536, False, True),                                         # ... some CUs twice
+    (512, 3072, 1536, False, True), (4096, 4608, 1536, False, True), (32760, 4608, 1536, False, True), (32760, 1536, 1536, True, True),
+    (4680, 1536, 1536, True, True), (1, 128, 1536, True, True), (33000, 128, 1536, False, True),
+    (679, 13056, 1216, False, True), (3613, 4096, 1024, False, True), (256, 4096, 1600, False, False), (256, 4096, 576, False, False)])
+def test_linear_is_one_kernel_where_that_is_the_faster_form(M, N, K, residual, one):
+    """vdmq_linear_bf6 asks for no workspace where it is one kernel: shapes measured on both sides of the line."""
+    from dsaquant_amd import _lib
+
+    lib = _lib.load()
+    need = lib.vdmq_linear_bf6_workspace(M, N, K, 0, 0, M if residual else 0, N if residual else 0, _lib.VDMQ_OUT_F16)
+    assert need == (0 if one else lib.vdmq_workspace_bytes_bf6(M, K))
+
+
 def test_bf6_tile_order_takes_every_tile_once(tmp_path):
     """The tile order of the bf6 GEMM kernels (regrouped edge super-tiles, round-robin and both kinds of contiguous
     runs) enumerated on the host for every grid up to 72 x 72 tiles and the benchmark shapes: tests/tilemap_check.cpp
