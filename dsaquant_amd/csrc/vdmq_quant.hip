@@ -311,12 +311,16 @@ __device__ __forceinline__ void quantize_held_row_bf6(u32x4 (&v)[NCH], int lane,
 // before it is quantized: the activation kernel between two linears, its write
 // and the quantizer's re-read of its output are saved.
 // FMT: 0 = native row-major int4 (Kp = K padded to the int8 GEMM's K step), 1 = bf6 blocks (Kp = K padded to 128)
+// Registers decide how many workgroups share a CU with short rows: in 64 of them (NCH 1 and 2) four do, in 80 three.  A scalar wave
+// number keeps the row addresses out of them there (32760 rows of 768 / 1024 / 2048 with the GELU 24.2 -> 22.8, 24.9 -> 24.3, 41.1 -> 38.8 us);
+// with longer rows it costs time (3072 with the GELU 49.4 -> 54.1).  (The fused LayerNorm's longest form spills: fewer registers so, 0.95 ...
+// 1.00 of the time for rows of 9216 ... 16384.)
 template <int NCH, bool STREAM_OUT, int ACT, int FMT>
-__global__ __launch_bounds__((FMT == 1 ? kBf6Rows : kRowsPerBlock) * kWaveSize) void quantize_rows_kernel(
+__global__ __launch_bounds__((FMT == 1 ? kBf6Rows : kRowsPerBlock) * kWaveSize, FMT == 1 && NCH <= 2 ? 8 : 1) void quantize_rows_kernel(
     const __half *__restrict__ x, int64_t ldx, int M, int K, int Kp, float clip, uint8_t *__restrict__ qact,
     __half *__restrict__ scale_h, int stream_bf6) {
     constexpr int ROWS = FMT == 1 ? kBf6Rows : kRowsPerBlock;
-    const int lane = threadIdx.x & (kWaveSize - 1), wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & (kWaveSize - 1), wave = FMT == 1 && NCH <= 4 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
     if constexpr (FMT == 1) {
         // The workgroup walks row groups blockIdx.x, blockIdx.x + gridDim.x, ...: with the launcher's grid
         // (what the chip holds at once) the loads of the next group's rows are in flight while this
@@ -394,7 +398,7 @@ __global__ __launch_bounds__((FMT == 1 ? kBf6Rows : kRowsPerBlock) * kWaveSize) 
     const __half *__restrict__ vb, int64_t ldv, int rows_per_vec, float clip, uint8_t *__restrict__ qact,
     __half *__restrict__ scale_h, __half *__restrict__ h_out, int64_t ldh, int stream_bf6) {
     constexpr int ROWS = FMT == 1 ? kBf6Rows : kRowsPerBlock;
-    const int lane = threadIdx.x & (kWaveSize - 1), wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & (kWaveSize - 1), wave = FMT == 1 && NCH > 16 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
     const int64_t row0 = static_cast<int64_t>(blockIdx.x) * ROWS;
     int64_t row = row0 + wave;
     const bool valid = row < M;

@@ -154,15 +154,15 @@ __device__ __forceinline__ u32x4 apply_act(u32x4 v) {
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned int u32x6 __attribute__((ext_vector_type(6)));
 
-// 32 values t, the even ones and the odd ones, as E3M2 floats t / 16: 192 bits.  The instruction writes result registers while it
-// still reads operands, which the compiler does not know: with a result that began at an operand's third register, codes came out
-// wrong.  Safe is a result that begins where the even values do, or before: its i-th register holds codes of values 10 / 3 times i and
-// later.  So all operands but the first six are still wanted behind the conversion, and share no register with the result.
+// 32 values t, the even ones and the odd ones, as E3M2 floats t / 16: 192 bits.  The instruction writes result registers while it still
+// reads operands: with a result that began at an operand's third register, codes came out wrong.  The builtin leaves the compiler free to
+// choose such registers, so this is the instruction itself, with a result that is written before the operands are read for the last time
+// and hence shares no register with them.  (One instruction and no load: nothing in flight, and its operands are results of
+// ordinary fp32 operations, so that no wait is due in front of it or behind.)
 __device__ __forceinline__ u32x6 to_bf6(const f32x16 &even, const f32x16 &odds) {
-    const u32x6 r = __builtin_amdgcn_cvt_scalef32_2xpk16_bf6_f32(even, odds, 16.0f);
+    u32x6 r = {};
 #if defined(__HIP_DEVICE_COMPILE__)
-    asm volatile("" ::"v"(r), "v"(odds), "v"(even[6]), "v"(even[7]), "v"(even[8]), "v"(even[9]), "v"(even[10]), "v"(even[11]), "v"(even[12]),
-                 "v"(even[13]), "v"(even[14]), "v"(even[15]));
+    asm("v_cvt_scalef32_2xpk16_bf6_f32 %0, %1, %2, %3" : "=&v"(r) : "v"(even), "v"(odds), "s"(16.0f));
 #endif
     return r;
 }

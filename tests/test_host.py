@@ -515,6 +515,30 @@ def test_library_says_where_the_fp6_path_pays():
     assert not pays(0, 128, 5120) and not pays(-1, 128, 5120)
 
 
+def test_bf6_conversion_shares_no_register_with_its_operands(tmp_path):
+    """v_cvt_scalef32_2xpk16_bf6_f32 writes result registers while it still reads operands (to_bf6 in vdmq_rowops.h): in the built
+    library no such instruction has a result that overlaps one."""
+    import shutil
+    import subprocess
+
+    from dsaquant_amd import _lib
+
+    objdump = shutil.which("llvm-objdump", path="/opt/rocm/llvm/bin") or shutil.which("llvm-objdump")
+    if objdump is None:
+        pytest.skip("no llvm-objdump")
+    lib = shutil.copy(_lib.LIB_PATH, tmp_path / "libvdmq.so")
+    subprocess.run([objdump, "--offloading", str(lib)], cwd=tmp_path, check=True, stdout=subprocess.DEVNULL)
+    found = 0
+    for code in tmp_path.glob("*gfx950*"):
+        text = subprocess.run([objdump, "-d", str(code)], check=True, stdout=subprocess.PIPE, text=True).stdout
+        for line in re.findall(r"v_cvt_scalef32_2xpk16_bf6_f32 (.*)", text):
+            (r0, r1), *operands = [(int(a), int(b)) for a, b in re.findall(r"v\[(\d+):(\d+)\]", line)]
+            assert (r1 - r0, [b - a for a, b in operands]) == (5, [15, 15]), line
+            assert all(r1 < a or b < r0 for a, b in operands), line
+            found += 1
+    assert found > 0
+
+
 @pytest.mark.parametrize("M,N,K,residual,one", [
     (679, 13056, 1472, False, False), (720, 10880, 1536, False, False), (590, 13056, 1536, True, False),      # their tiles fill the CUs once
     (2459, 6144, 1536, True, False), (11450, 11136, 1536, True, False), (35303, 4992, 1536, True, False),     # ... a residual from memory
