@@ -20,6 +20,7 @@ VDMQ_ACT_NONE = 0
 VDMQ_ACT_GELU_TANH = 1
 VDMQ_LN_MODULATE = 1
 VDMQ_LN_AFFINE = 2
+VDMQ_LINEAR_BF6_MIN_K = 640
 
 class GemmLaunchInfo(ctypes.Structure):
     """vdmq_gemm_launch_info of include/vdmq.h."""

@@ -582,12 +582,12 @@ static double resident_us(int64_t M, int64_t N, int64_t K, bool has_tail, const 
 }
 
 bool resident_takes(const ResidentProblem &p) {
-    // Rows of up to 1536 elements fit LDS; shorter ones than 640 are the int8 path's.  In front of it no GELU, in its epilogue
+    // Rows of up to 1536 elements fit LDS; shorter ones than VDMQ_LINEAR_BF6_MIN_K are the int8 path's.  In front of it no GELU, in its epilogue
     // what the models' blocks ask for (a residual, with one gate vector or none, without a LayerNorm): the rest is left to the quantizers'
     // and the GEMM's kernels.
     const GemmTail &t = p.tail;
     const bool tail = t.residual == nullptr ? t.gate == nullptr : (t.gate == nullptr || t.rows_per_gate >= p.M) && t.ldr <= (1 << 22) && p.ln_mode == 0;
-    if (p.K < 640 || p.K > 1536 || p.M > (1 << 24) || p.out_dtype != VDMQ_OUT_F16 || p.act != VDMQ_ACT_NONE || !tail) return false;
+    if (p.K < VDMQ_LINEAR_BF6_MIN_K || p.K > 1536 || p.M > (1 << 24) || p.out_dtype != VDMQ_OUT_F16 || p.act != VDMQ_ACT_NONE || !tail) return false;
     if (p.ln_mode == 0) {
         // Against quantizer and tiled GEMM it takes 0.5 ... 0.95 of the time as a rule, but it loses where their tiles fill the CUs exactly
         // and its units do not (2459 x 1536 -> 6144 with a residual 33.4 / 26.7 us, 679 x 1472 -> 13056 22.4 / 20.8), and with a residual

@@ -452,10 +452,8 @@ def _native_weights(qweight: torch.Tensor, wscales: torch.Tensor) -> Tuple[torch
 # "int8": v_mfma_i32_32x32x32_i8 on nibbles widened in registers.  "bf6": v_mfma_f32_32x32x64_f8f6f4 on 6-bit
 # floats (twice the rate, no widening work; every int4 value q is held as the E3M2 float q / 16, exactly, and the
 # fp32 accumulation of the products is exact too).
-# Both give bit-identical results.  "auto" takes bf6 for rows of 640 elements on, whatever the other sizes: up to 1536 the
-# library quantizes and multiplies in one kernel there (vdmq_linear_bf6), beyond them vdmq_bf6_pays holds.  "bf6" always runs
-# the quantizer and the tiled GEMM.
-_BF6_FROM_K = 640
+# Both give bit-identical results.  "auto" takes bf6 for rows of VDMQ_LINEAR_BF6_MIN_K elements on, whatever the other sizes, and
+# leaves the form to the library (vdmq_linear_bf6).  "bf6" always runs the quantizer and the tiled GEMM.
 _MATRIX_PATH = os.environ.get("VDMQ_MATRIX_PATH", "auto")
 
 
@@ -474,7 +472,7 @@ def _use_bf6(M: int, N: int, K: int, out_dtype: torch.dtype = torch.float16, pat
     path = _MATRIX_PATH if path is None else path
     if path == "int8" or M == 0:
         return False
-    return path == "bf6" or K >= _BF6_FROM_K
+    return path == "bf6" or K >= _lib.VDMQ_LINEAR_BF6_MIN_K
 
 
 def _to_bf6(native: torch.Tensor, rows: int, K: int) -> torch.Tensor:

@@ -174,7 +174,7 @@ int vdmq_gemm_w4a4_acc(const void *qact, const void *wq, int32_t *acc, int64_t M
 #define VDMQ_KERNEL_GEMM_BF6 2            /* bf6 matrix path, one workgroup per tile (256 x 256, or 128 x 128 for small problems) */
 #define VDMQ_KERNEL_GEMM_BF6_PERSISTENT 3 /* bf6 matrix path, one workgroup per CU walking tiles */
 #define VDMQ_KERNEL_LINEAR_RESIDENT 4     /* bf6 matrix path, quantizer and GEMM in one kernel (short rows) */
-#define VDMQ_KERNEL_GEMM_BF6_KSPLIT 5     /* bf6 matrix path, K divided among the waves of a workgroup (few tiles, long rows) */
+#define VDMQ_KERNEL_GEMM_BF6_KSPLIT 5     /* bf6 matrix path, K divided among the waves of a workgroup (few tiles) */
 typedef struct vdmq_gemm_launch_info {
     int kernel;                 /* VDMQ_KERNEL_* */
     int tile_m, tile_n;         /* output tile of one workgroup: token rows x channels */
@@ -244,11 +244,10 @@ int vdmq_linear_w4a4_noalloc(const void *x, int64_t M, int64_t K, int64_t ldx, f
  * build give results off by a power of two without any error.  They must come from this build's vdmq_quantize_act*_bf6
  * / vdmq_native_to_bf6 / vdmq_weight_v1_to_bf6; what is stored on disk is the v1 layout. */
 int64_t vdmq_bf6_bytes(int64_t rows, int64_t K);
-/* 1 when the bf6 path is the faster one for a linear of this size (quantizer + GEMM, measured on MI355X), 0
- * otherwise.  Its GEMM has 256 x 256 tiles for large problems and 128 x 128 ones for small ones and is the faster
- * GEMM on every shape measured; what decides is the quantizer, which is slower than the int4 one on short rows: the
- * path pays from K = 1280 on, whatever M and N.  A host that keeps both weight forms asks this per call; the results
- * are the same bits either way.  No counterpart in the reference (it has one matrix path). */
+/* 1 when vdmq_linear_w4a4_bf6, or quantizer and GEMM of the bf6 path as separate calls, is the faster choice for a linear of
+ * this size (measured on MI355X), 0 otherwise: from K = 1280 on, whatever M and N.  vdmq_linear_bf6 below pays for shorter rows
+ * too (VDMQ_LINEAR_BF6_MIN_K).  A host that keeps both weight forms asks this per call; the results are the same bits
+ * either way.  No counterpart in the reference (it has one matrix path). */
 int vdmq_bf6_pays(int64_t M, int64_t N, int64_t K);
 int vdmq_quantize_act_bf6(const void *x, int64_t M, int64_t K, int64_t ldx, float clip, int act, void *xblocks, void *scale_h,
                           vdmq_stream_t stream);
@@ -266,6 +265,7 @@ int vdmq_linear_w4a4_bf6(const void *x, int64_t M, int64_t K, int64_t ldx, float
  * either way.  vdmq_linear_bf6_ex adds what the separate calls offer: ln_mode (0: none) with the arguments of vdmq_quantize_act_ln, gate
  * and residual of vdmq_gemm_w4a4_ex, split_cols (0: none) and part_stride of vdmq_gemm_w4a4_split.  vdmq_linear_bf6_workspace: the bytes of
  * workspace such a call needs (0: none); rows_per_gate 0: no gate, ldr 0: no residual. */
+#define VDMQ_LINEAR_BF6_MIN_K 640 /* rows from which on vdmq_linear_bf6 is the faster choice, whatever M and N (shorter ones: vdmq_linear_w4a4) */
 int64_t vdmq_linear_bf6_workspace(int64_t M, int64_t N, int64_t K, int act, int ln_mode, int64_t rows_per_gate, int64_t ldr, int out_dtype);
 int vdmq_linear_bf6(const void *x, int64_t M, int64_t K, int64_t ldx, float clip, int act, const void *wblocks, const void *wscale,
                     const void *bias, void *out, int out_dtype, int64_t N, int64_t ldo, void *workspace, int64_t workspace_bytes,

@@ -60,4 +60,5 @@ def test_documented_bindings_run_and_match_the_oracle():
             torch.cuda.synchronize()
             assert got.shape == (1, M, N) and got.dtype == torch.float16
             assert np.array_equal(got.view(M, N).cpu().numpy().view(np.uint16), want.view(np.uint16)), (name, M, K, N)
-        assert bool(ns["_L"].vdmq_bf6_pays(M, N, K)) == (K >= 1280)
+        one_kernel = K >= _lib.VDMQ_LINEAR_BF6_MIN_K
+        assert _lib.last_gemm_launch().kernel == (_lib.KERNEL_LINEAR_RESIDENT if one_kernel else _lib.KERNEL_GEMM_W4A4)

@@ -24,6 +24,9 @@ def test_library_exports_every_declared_symbol():
     for name in sorted(declared):
         assert hasattr(lib, name), f"libvdmq.so does not export {name}"
     assert declared == set(_lib.SIGNATURES), "ctypes signatures and header disagree"
+    mirrored = {n: int(v) for n, v in re.findall(r"#define (VDMQ_\w+) (\d+)", header) if hasattr(_lib, n)}
+    assert "VDMQ_LINEAR_BF6_MIN_K" in mirrored
+    assert mirrored == {n: getattr(_lib, n) for n in mirrored}, "ctypes constants and header disagree"
     # pure host calls
     assert lib.vdmq_version() == _lib.VDMQ_VERSION == 2
     assert lib.vdmq_arch() == b"gfx950"
