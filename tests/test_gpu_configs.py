@@ -1,4 +1,5 @@
-"""Every linear of the benchmark configurations at its full size, on both matrix paths.
+"""Every linear of the benchmark configurations at its full size, on both matrix paths, and those of short rows by the default
+path, which is one kernel for them.
 
 Config 1 = Wan-2.1 1.3B at 480p x 81 frames (M = 32760), config 2 = Wan-2.2 5B at 704 x 1280 x 121 frames (M = 27280,
 run as the two back-to-back calls of the CFG pair), config 3 = Wan-2.1 14B at 720p (M = 75600; its fused-QKV and
@@ -24,7 +25,7 @@ pytestmark = pytest.mark.gpu
 
 DEV = "cuda:0"
 
-W4, BF6, BF6P = 1, 2, 3  # VDMQ_KERNEL_* of include/vdmq.h
+W4, BF6, BF6P, RESIDENT = 1, 2, 3, 4  # VDMQ_KERNEL_* of include/vdmq.h
 
 # (config, name, M, K, N, calls, {path: (kernel, tile_m, tile_n, group_n, contiguous)})
 CASES = [
@@ -40,6 +41,16 @@ CASES = [
     ("cfg3", "o", 75600, 5120, 5120, 1, {"int8": (W4, 256, 256, 4, 1), "bf6": (BF6P, 256, 256, 4, 0)}),
     ("cfg3", "ffn_up", 75600, 5120, 13824, 1, {"int8": (W4, 256, 256, 4, 1), "bf6": (BF6P, 256, 256, 4, 1)}),
     ("cfg3", "cross_kv", 512, 5120, 10240, 1, {"int8": (W4, 128, 128, 4, 0), "bf6": (BF6, 128, 128, 2, 1)}),
+]
+
+
+# ... and by the default path, where that is a kernel of its own: (config, name, M, K, N, (kernel, tile_m, tile_n, column groups, contiguous))
+DEFAULT_CASES = [
+    ("cfg0", "qkv", 4096, 1536, 4608, (RESIDENT, 64, 64, 4, 1)),
+    ("cfg1", "qkv", 32760, 1536, 4608, (RESIDENT, 128, 64, 1, 1)),
+    ("cfg1", "o", 32760, 1536, 1536, (RESIDENT, 128, 64, 1, 1)),
+    ("cfg1", "ffn_up", 32760, 1536, 8960, (RESIDENT, 128, 64, 1, 1)),
+    ("cfg1", "cross_kv", 512, 1536, 3072, (RESIDENT, 32, 64, 12, 1)),
 ]
 
 
@@ -71,6 +82,15 @@ def _activations(M, K, seed):
 @pytest.mark.parametrize("path", ["int8", "bf6"])
 @pytest.mark.parametrize("cfg,name,M,K,N,calls,expect", CASES, ids=[f"{c[0]}-{c[1]}" for c in CASES])
 def test_full_size_linear(cfg, name, M, K, N, calls, expect, path):
+    _full_size_linear(cfg, name, M, K, N, calls, path, (_expected_bf6_kernel(expect[path][0]),) + expect[path][1:])
+
+
+@pytest.mark.parametrize("cfg,name,M,K,N,expect", DEFAULT_CASES, ids=[f"{c[0]}-{c[1]}" for c in DEFAULT_CASES])
+def test_full_size_linear_by_the_default_path(cfg, name, M, K, N, expect):
+    _full_size_linear(cfg, name, M, K, N, 1, "auto", expect)
+
+
+def _full_size_linear(cfg, name, M, K, N, calls, path, want_choice):
     from dsaquant_amd import _lib
     from dsaquant_amd.kernels import vdm_w4a4 as v
 
@@ -86,7 +106,6 @@ def test_full_size_linear(cfg, name, M, K, N, calls, expect, path):
             y = v.linear_vdm_w4a4(x, qv1, sv1, b, clip_ratio=1.0)
             info = _lib.last_gemm_launch()
             got_choice = (info.kernel, info.tile_m, info.tile_n, info.group_n, info.contiguous_runs)
-            want_choice = (_expected_bf6_kernel(expect[path][0]),) + expect[path][1:]
             assert got_choice == want_choice, f"launcher chose {got_choice}"
             assert y.shape == (M, N) and y.dtype == torch.float16
             rows = np.unique(np.concatenate([np.arange(0, min(M, 40)), np.arange(M // 2, min(M, M // 2 + 24)), np.arange(max(0, M - 40), M)]))

@@ -30,8 +30,7 @@ def weight():
 
 
 def rows(M, K, seed=0):
-    """Rows of every kind: ordinary, zero, tiny, beyond the clamp at small clip ratios, infinite and NaN; none of the special ones
-    comes last, since the kernel reads that one again where it has no row."""
+    """Rows of every kind: ordinary, zero, tiny, beyond the clamp at small clip ratios, infinite and NaN."""
     g = torch.Generator(device="cuda").manual_seed(seed + 7 * M + K)
     x = torch.randn(M, K, generator=g, device="cuda").half()
     x[:, ::97] *= 20
@@ -46,6 +45,21 @@ def rows(M, K, seed=0):
     return x
 
 
+def tiled(f):
+    """``f()`` as quantizer and tiled GEMM."""
+    from dsaquant_amd import _lib
+
+    v = vk()
+    before = v.matrix_path()
+    try:
+        v.set_matrix_path("bf6")
+        want = f()
+        assert _lib.last_gemm_launch().kernel in TILED
+        return want
+    finally:
+        v.set_matrix_path(before)
+
+
 def both(f, kernel=RESIDENT):
     """``f()`` by the library's choice and as quantizer and tiled GEMM."""
     from dsaquant_amd import _lib
@@ -57,11 +71,9 @@ def both(f, kernel=RESIDENT):
         got = f()
         info = _lib.last_gemm_launch()
         assert info.kernel in kernel if isinstance(kernel, tuple) else info.kernel == kernel, info.kernel
-        v.set_matrix_path("bf6")
-        want = f()
-        assert _lib.last_gemm_launch().kernel in TILED
     finally:
         v.set_matrix_path(before)
+    want = tiled(f)
     # NaN rows: the same positions; everything else bit for bit
     assert torch.equal(torch.isnan(got), torch.isnan(want))
     got, want = (torch.where(torch.isnan(t), torch.zeros_like(t), t) for t in (got, want))
@@ -80,6 +92,21 @@ def test_plain_linear(weight, M, N, tile, K):
     info = both(lambda: v.linear_vdm_w4a4(x, qw, ws, b, 0.95))
     assert info.tile_m == tile, info.tile_m
     both(lambda: v.linear_vdm_w4a4(x, qw, ws, None, 1e-3 if M % 2 else 1.0))
+
+
+@pytest.mark.parametrize("value", [0.0, 65504.0, float("inf"), float("nan")])
+@pytest.mark.parametrize("M,N,K", [(33, 4608, 1536), (2500, 4096, 1024), (4097, 4608, 1088), (200, 512, 4096), (500, 4096, 3328)])
+def test_special_rows_at_the_ends_of_tiles(weight, M, N, K, value):
+    """The last row, which the kernels read again where a tile has none, and the ones at tile ends."""
+    v = vk()
+    qw, ws, b = weight(N, K)
+    x = rows(M, K, 20)
+    for at in {31, 63, 127, M - 2, M - 1} & set(range(M)):
+        if value == 0.0:
+            x[at] = 0
+        else:
+            x[at, at % K] = value
+    both(lambda: v.linear_vdm_w4a4(x, qw, ws, b, 0.95), (RESIDENT, KSPLIT))
 
 
 @pytest.mark.parametrize("M,N,K", [(679, 13056, 1472), (720, 10880, 1536)])
@@ -115,8 +142,25 @@ def test_gated_residual_and_split(weight, M, N, K):
         both(lambda: F.linear_fused(x, qw, ws, b, 0.95, residual=res, gate=token_gate), kernel=TILED + (KSPLIT,))
 
 
+# every instantiation the library chooses: 32, 64 and 128 rows to a workgroup, one and two or three chunks of 512, an odd and an even number
+# of K steps each, with the residual and without; a ragged last tile
+@pytest.mark.parametrize("K", [640, 960, 1088, 1472])
+@pytest.mark.parametrize("M,tile", [(257, 32), (4100, 64), (32700, 128)])
+def test_every_tile_with_residual_and_split(weight, M, tile, K):
+    from dsaquant_amd import fused_ops as F
+
+    N = 1536
+    qw, ws, b = weight(N, K)
+    x = rows(M, K, 1)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    res, gate = torch.randn(M, N, generator=g, device="cuda").half(), torch.randn(1, N, generator=g, device="cuda").half()
+    for kw in (dict(), dict(split_cols=N // 3), dict(residual=res), dict(residual=res, gate=gate)):
+        info = both(lambda: F.linear_fused(x, qw, ws, b, 0.95, **kw))
+        assert info.tile_m == tile, (info.tile_m, kw.keys())
+
+
 @pytest.mark.parametrize("mode", ["modulate", "affine"])
-@pytest.mark.parametrize("B,L,N,K", [(1, 32760, 1536, 1536), (1, 31001, 2560, 1472), (2, 16001, 1536, 960), (1, 32700, 1536, 1024)])
+@pytest.mark.parametrize("B,L,N,K", [(1, 32700, 1536, 640), (2, 16001, 1536, 1088), (1, 32760, 1536, 1536), (1, 31001, 2560, 1472), (2, 16001, 1536, 960), (1, 32700, 1536, 1024)])
 def test_layer_norm_in_front(weight, B, L, N, K, mode):
     from dsaquant_amd import fused_ops as F
 
@@ -151,7 +195,7 @@ def test_strides_workspace_and_refusals_through_the_c_abi(weight):
     assert lib.vdmq_linear_bf6_workspace(M, N, K, 0, 0, 0, 0, 0) == 0
     _lib.check(call())
     assert _lib.last_gemm_launch().kernel == RESIDENT
-    want = v.linear_vdm_w4a4(x[:M, :K].contiguous(), qw, ws, b, 0.95)
+    want = tiled(lambda: v.linear_vdm_w4a4(x[:M, :K].contiguous(), qw, ws, b, 0.95))
     assert torch.equal(out[:M, :N], want)
     assert (out[:M, N:] == 3.0).all() and (out[M] == 3.0).all()
     need = lib.vdmq_linear_bf6_workspace(M, N, K, 0, 0, 0, 0, 1)
@@ -184,7 +228,7 @@ def test_replays_from_a_hip_graph(weight):
         x.copy_(torch.randn(1000, K, device="cuda").half() * (turn + 1))
         graph.replay()
         torch.cuda.synchronize()
-        assert torch.equal(out, step())
+        assert torch.equal(out, tiled(step))
 
 
 # K: k-blocks (64 elements, rounded up to an even number) from fewer than the four waves keep in flight to several times as many, each
@@ -234,7 +278,7 @@ def test_residual_updated_in_place_through_the_c_abi(weight, M, N, K):
     x = rows(M, K, 12).nan_to_num(0.5, 9.0, -9.0)
     g = torch.Generator(device="cuda").manual_seed(13)
     out, gate = torch.randn(M, N, generator=g, device="cuda").half(), torch.randn(1, N, generator=g, device="cuda").half()
-    want = F.linear_fused(x, qw, ws, b, 0.95, residual=out, gate=gate)
+    want = tiled(lambda: F.linear_fused(x, qw, ws, b, 0.95, residual=out, gate=gate))
     pw = v._prepared_weight(qw, ws)
     nbytes = lib.vdmq_linear_bf6_workspace(M, N, K, 0, 0, M, N, 0)
     workspace = torch.empty(max(nbytes, 1), dtype=torch.uint8, device="cuda")
@@ -243,3 +287,54 @@ def test_residual_updated_in_place_through_the_c_abi(weight, M, N, K):
                                       nbytes, torch.cuda.current_stream().cuda_stream))
     assert _lib.last_gemm_launch().kernel in (RESIDENT, KSPLIT)
     assert torch.equal(out, want)
+
+
+# resident (32, 64, 128 rows; LayerNorm), K split (64 x 64, 128 x 64)
+@pytest.mark.parametrize("M,N,K,kind", [(257, 1536, 1088, "tail"), (4100, 1536, 960, "tail"), (32700, 1536, 1472, "tail"), (200, 512, 4096, "tail"),
+                                        (500, 4096, 3328, "tail"), (300, 768, 1536, "split"), (4100, 1536, 1024, "split"), (200, 768, 4096, "split"),
+                                        (32700, 1536, 1088, "ln")])
+def test_strides_beyond_the_rows_through_the_c_abi(weight, M, N, K, kind):
+    """Row strides of input, residual, gate, LayerNorm vectors and output beyond their rows, a part stride beyond the part: the
+    bits of the dense call, no byte written outside the rows."""
+    from dsaquant_amd import _lib, fused_ops as F
+
+    lib, v = _lib.load(), vk()
+    qw, ws, b = weight(N, K)
+    g = torch.Generator(device="cuda").manual_seed(17)
+
+    def wide(n, k, pad, fill=7.0):
+        t = torch.full((n + 1, k + pad), fill, device="cuda", dtype=F16)
+        return t, t[:n, :k]
+
+    xw, x = wide(M, K, 72, float("nan"))
+    x.copy_(rows(M, K, 14).nan_to_num(0.5, 9.0, -9.0))
+    split, cols = (N // 3, N // 3) if kind == "split" else (0, N)
+    parts, part_stride = (3, (M + 2) * (cols + 40)) if split else (1, 0)
+    flat = torch.full((parts, M + 2, cols + 40), 3.0, device="cuda", dtype=F16)
+    gate_p, ldg, rpg, res_p, ldr, ln = None, 0, 1, None, 0, (0, 0.0, None, None, 0, 1)
+    kw = dict(split_cols=split) if split else {}
+    if kind == "tail":
+        resw, res = wide(M, N, 56)
+        res.copy_(torch.randn(M, N, generator=g, device="cuda"))
+        gatew, gate = wide(1, N, 24)
+        gate.copy_(torch.randn(1, N, generator=g, device="cuda"))
+        kw = dict(residual=res.contiguous(), gate=gate.clone().view(-1).view(1, N))
+        gate_p, ldg, rpg, res_p, ldr = gatew.data_ptr(), gatew.stride(0), M, resw.data_ptr(), resw.stride(0)
+    dense = x.contiguous()
+    source = dense
+    if kind == "ln":  # one vector for each half of the rows
+        (aw, a), (cw, c) = wide(2, K, 48), wide(2, K, 48)
+        a.copy_(0.1 * torch.randn(2, K, generator=g, device="cuda"))
+        c.copy_(0.1 * torch.randn(2, K, generator=g, device="cuda"))
+        source = F.LnInput(dense.view(2, M // 2, K), a.contiguous(), c.contiguous(), 1e-6)
+        ln = (_lib.VDMQ_LN_MODULATE, 1e-6, aw.data_ptr(), cw.data_ptr(), aw.stride(0), M // 2)
+    want = tiled(lambda: F.linear_fused(source, qw, ws, b, 0.95, **kw)).view(parts, M, cols)
+    pw = v._prepared_weight(qw, ws)
+    nbytes = lib.vdmq_linear_bf6_workspace(M, N, K, 0, ln[0], rpg if gate_p else 0, ldr, 0)
+    workspace = torch.empty(max(nbytes, 1), dtype=torch.uint8, device="cuda")
+    _lib.check(lib.vdmq_linear_bf6_ex(xw.data_ptr(), M, K, xw.stride(0), 0.95, 0, *ln, pw.operand(True).data_ptr(), pw.wscale.data_ptr(), b.data_ptr(),
+                                      gate_p, ldg, rpg, res_p, ldr, split, part_stride, flat.data_ptr(), 0, N, cols + 40, workspace.data_ptr(), nbytes,
+                                      torch.cuda.current_stream().cuda_stream))
+    assert _lib.last_gemm_launch().kernel == (KSPLIT if K > 1536 else RESIDENT)
+    assert torch.equal(flat[:, :M, :cols].contiguous().view(torch.int16), want.contiguous().view(torch.int16))
+    assert (flat[:, :M, cols:] == 3.0).all() and (flat[:, M:] == 3.0).all()
