@@ -24,7 +24,7 @@ timed region.  Prints ONE JSON line.
              a restatement of the reference's CPU-runnable path) on config 0
 
 Beside the headline fields the line carries, all measured in the same run (the figures a reader needs are repeated
-as flat numbers inside the `roofline` object: int8_path_*, quantizer_*, <workload>_gemm_*, <case>_*, config4_*):
+as flat numbers inside the `roofline` object: int8_path_*, quantizer_*, <workload>_gemm_*, *_one_call_*, <case>_*, config4_*):
   int8_path     the same workload with the GEMM forced onto the int8 matrix instructions (gemm_w4a4_kernel), with its
                 own roofline object against the 5.0 POP/s INT8 peak
   workloads     whole-step TOPS of the other block workloads (Wan-2.1 1.3B at 480p, Wan-2.2 5B) on the path the
@@ -32,6 +32,9 @@ as flat numbers inside the `roofline` object: int8_path_*, quantizer_*, <workloa
   cases         single linears: config 0's fused QKV at M = 4096 (the shape the CPU baseline is timed on), the 14B
                 model's cross-attention K/V projection (M = 512 text tokens) and its fused QKV with a ragged last tile
                 (M = 75600 + 37)
+                In both, as in the headline, quantizer and GEMM are separate calls, so that each can be timed; a linear of
+                the package is one call (vdmq_linear_bf6), whose kernel may be another at short rows or few tiles:
+                *_one_call_tops and *_one_call_kernel are the same linears so, in the same run
   config4       the end-to-end Wan-2.1 1.3B DiT harness (30 blocks, 32760 tokens, cond + uncond, 5 steps; bench_dit.py):
                 ms per step and the shares of the W4A4 calls and of attention
   stream_ceiling  what a kernel that only streams sustains with the quantizer's mix of reads and writes over the same
@@ -86,6 +89,8 @@ WORKLOADS = {"wan14b_720p_block": WAN14B_720P, "wan1.3b_480p_block": WAN13B_480P
 CASES = {"cfg0_qkv_m4096": dict(M=4096, linears=[("qkv", 1536, 4608)]),
          "cfg3_cross_kv_m512": dict(M=512, linears=[("cross_kv", 5120, 10240)]),
          "cfg3_qkv_ragged_m75637": dict(M=75637, linears=[("qkv", 5120, 15360)])}
+# VDMQ_KERNEL_* of include/vdmq.h
+KERNEL_NAMES = {1: "gemm_w4a4_kernel", 2: "gemm_bf6_kernel", 3: "gemm_bf6_persistent_kernel", 4: "resident_linear_kernel", 5: "gemm_bf6_ksplit_kernel"}
 SHORT = {"wan1.3b_480p_block": "wan1p3b", "wan5b_704x1280_block": "wan5b", "wan14b_720p_block": "wan14b"}
 
 
@@ -203,7 +208,35 @@ class Workload:
             if events is not None:
                 events[2 * li + 2].record(self.stream)
             if events is not None and "kernel" not in L:
-                L["kernel"] = {1: "gemm_w4a4_kernel", 2: "gemm_bf6_kernel", 3: "gemm_bf6_persistent_kernel"}[_lib.last_gemm_launch().kernel]
+                L["kernel"] = KERNEL_NAMES[_lib.last_gemm_launch().kernel]
+
+    def one_call(self, steps, warmup):
+        """The same linears as the package runs them, one library call each, which picks the form: TOPS over the steps
+        and the kernels' names.  None unless all of them are on the bf6 path."""
+        torch, lib, _lib, M, s = self.torch, self.lib, self._lib, self.M, self.stream.cuda_stream
+        if not all(L["bf6"] for L in self.layers):
+            return None
+        nbytes = max(int(lib.vdmq_linear_bf6_workspace(M, L["N"], L["K"], 0, 0, 0, 0, _lib.VDMQ_OUT_F16)) for L in self.layers)
+        workspace = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=self.dev)
+        kernels = []
+
+        def step():
+            for L in self.layers:
+                _lib.check(lib.vdmq_linear_bf6(L["x"].data_ptr(), M, L["K"], L["K"], 1.0, 0, L["wq"].data_ptr(), L["ws"].data_ptr(), L["bias"].data_ptr(),
+                                               L["out"].data_ptr(), _lib.VDMQ_OUT_F16, L["N"], L["N"], workspace.data_ptr(), nbytes, s))
+                if len(kernels) < len(self.layers):
+                    kernels.append(KERNEL_NAMES[_lib.last_gemm_launch().kernel])
+
+        for _ in range(max(warmup, 1)):
+            step()
+        torch.cuda.synchronize()
+        t0 = time.perf_counter()
+        for _ in range(steps):
+            step()
+        torch.cuda.synchronize()
+        wall = time.perf_counter() - t0
+        return {"tops": round(sum(2.0 * M * L["N"] * L["K"] for L in self.layers) * steps / wall / 1e12, 1),
+                "us": round(wall / steps * 1e6, 2), "kernel": " + ".join(sorted(set(kernels)))}
 
     def measure(self, steps, warmup):
         """W untimed steps, then exactly K timed steps between synchronisations; per-launch times from HIP events
@@ -469,9 +502,10 @@ def main():
         torch.cuda.synchronize()
         del src, dst
 
-    def run(name, path, steps, warmup):
+    def run(name, path, steps, warmup, one_call=False):
         w = Workload(torch, lib, v, name, path, dev)
         r = w.measure(steps, warmup)
+        r["one_call"] = w.one_call(steps, warmup) if one_call and path == "auto" else None
         del w
         torch.cuda.empty_cache()
         return r
@@ -518,31 +552,37 @@ def main():
                          "int8_path_frac": r8["roofline"]["frac"], "int8_path_kernel": r8["roofline"]["kernel"],
                          "int8_path_quantizer_frac": r8["quantizer"]["frac"], "int8_path_step_tops": round(r8["step_tops"], 1)})
 
+        def add_one_call(prefix, res):
+            if res["one_call"] is not None:
+                roof.update({f"{prefix}_one_call_tops": res["one_call"]["tops"], f"{prefix}_one_call_kernel": res["one_call"]["kernel"]})
+
         def workload_section(other):
-            ro = run(other, args.matrix_path, extra_steps, extra_warmup)
+            ro = run(other, args.matrix_path, extra_steps, extra_warmup, one_call=True)
             result.setdefault("workloads", {})[other] = {
                 "M": WORKLOADS[other]["M"], "steps": extra_steps, "warmup": extra_warmup,
                 "step_tops": round(ro["step_tops"], 1), "ms_per_step": round(ro["ms_per_step"], 4),
                 "gemm_tops": ro["roofline"]["achieved"], "gemm_frac": ro["roofline"]["frac"],
                 "gemm_frac_of_int8_peak": ro["roofline"]["frac_of_int8_peak"],
-                "quant_gbs": ro["quantizer"]["achieved"], "quant_gbs_int4_bytes": ro["quantizer"]["achieved_int4_bytes"]}
+                "quant_gbs": ro["quantizer"]["achieved"], "quant_gbs_int4_bytes": ro["quantizer"]["achieved_int4_bytes"], "one_call": ro["one_call"]}
             per_linear[other] = ro["per_linear"]
             k = SHORT[other]
             roof.update({f"{k}_gemm_achieved": ro["roofline"]["achieved"], f"{k}_gemm_frac": ro["roofline"]["frac"],
                          f"{k}_gemm_frac_of_int8_peak": ro["roofline"]["frac_of_int8_peak"], f"{k}_step_tops": round(ro["step_tops"], 1),
                          f"{k}_quantizer_frac_int4_bytes": ro["quantizer"]["frac_int4_bytes"]})
+            add_one_call(k, ro)
 
         def case_section(case, spec):  # single linears: launches of 15 ... 2400 us, so more repetitions for the short ones
             steps_c = 200 if spec["M"] <= 4096 else extra_steps
-            rc = run(case, args.matrix_path, steps_c, 5)
+            rc = run(case, args.matrix_path, steps_c, 5, one_call=True)
             lin = next(iter(rc["per_linear"].values()))
             result.setdefault("cases", {})[case] = {
                 "M": spec["M"], "K": lin["K"], "N": lin["N"], "steps": steps_c, "kernel": lin["kernel"],
                 "gemm_us": round(lin["gemm_ms"] * 1e3, 2), "gemm_tops": lin["gemm_tops"],
                 "quant_us": round(lin["quant_ms"] * 1e3, 2), "quant_gbs_int4_bytes": lin["quant_gbs_int4_bytes"],
-                "linear_tops": round(rc["step_tops"], 1), "linear_us": round(rc["ms_per_step"] * 1e3, 2)}
+                "linear_tops": round(rc["step_tops"], 1), "linear_us": round(rc["ms_per_step"] * 1e3, 2), "one_call": rc["one_call"]}
             roof.update({f"{case}_gemm_achieved": lin["gemm_tops"], f"{case}_gemm_frac": round(lin["gemm_tops"] / rc["roofline"]["peak"], 4),
                          f"{case}_linear_tops": round(rc["step_tops"], 1), f"{case}_kernel": lin["kernel"]})
+            add_one_call(case, rc)
 
         def stream_section():  # the quantizer against a kernel that only streams the same mix of reads and writes over the same volumes
             sc = stream_ceiling(torch, lib, dev, wl["M"], [k for _, k, _ in wl["linears"]], path != "int8")

@@ -126,7 +126,8 @@ def linear_ln_vdm_w4a4(
     bias_half: Optional[torch.Tensor] = None,
 ) -> torch.Tensor:
     """``linear_vdm_w4a4(pre.materialize(), ...)`` without materializing: LayerNorm,
-    modulation and activation quantizer are one kernel, the GEMM the second."""
+    modulation and activation quantizer are one kernel and the GEMM the second, or, for many
+    short rows, all of it is one (``vdmq_linear_bf6_ex``)."""
     return linear_fused(pre, qweight, wscales, bias, clip_ratio, bias_half)
 
 
@@ -166,7 +167,8 @@ def linear_fused(
     gate: Optional[torch.Tensor] = None,
     split_cols: Optional[int] = None,
 ) -> torch.Tensor:
-    """``residual + linear_vdm_w4a4(act(x), ...) * gate`` in two kernels.
+    """``residual + linear_vdm_w4a4(act(x), ...) * gate`` in two kernels, or in one where the
+    rows are short (``vdmq_linear_bf6_ex``).
 
     ``x`` is a tensor (optionally with ``act="gelu_tanh"`` applied to it inside the
     quantizer), an ``LnInput`` or a ``QuantizedInput`` (whose clip ratio must be the
