@@ -595,8 +595,9 @@ bool resident_takes(const ResidentProblem &p) {
         // K < 1280 than the int8 path, which served those (6500 timings, 0.995 at most), N <= 384 (550, 1.03).  Few tiles with K divided
         // (vdmq_bf6_ksplit.hip): 0.93 of that one's time, 1.11 at most, and a launch less for the host.  Of 22000 timings of K 640 ... 1536
         // the choice takes over 1.03 of the time of the path that served the size before at 0.9 %, over 1.06 at 0.2 % (always one
-        // kernel: 2.3 and 0.9 %), 1.15 at most.
-        if (p.K < 1280 || p.N <= 384 || ksplit_takes(p.M, p.N, p.K, p.out_dtype) || p.M * p.N > (int64_t(1) << 40)) return true;
+        // kernel: 2.3 and 0.9 %), 1.15 at most.  Up to 2.5 million outputs the estimates always say one kernel (2.7 million is the least
+        // where they do not), and the call waits for the host, whom they cost 0.3 us each time.
+        if (p.K < 1280 || p.N <= 384 || p.M * p.N <= 2500000 || ksplit_takes(p.M, p.N, p.K, p.out_dtype) || p.M * p.N > (int64_t(1) << 40)) return true;
         const ResidentShape shape = resident_shape(p.M, p.N, false);
         return resident_us(p.M, p.N, p.K, t.residual != nullptr, shape) < bf6_two_kernels_us(p.M, p.N, p.K, t.residual != nullptr);
     }
