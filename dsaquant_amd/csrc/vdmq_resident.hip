@@ -9,16 +9,18 @@
 // instructions.
 //
 // Against quantizer and tiled GEMM it saves a launch and the blocks' way to memory and back, and where tiles of 256 x 256 or 128 x 128
-// leave CUs idle its units need not.  Measured (us, two kernels -> here): 512 x 1536 -> 3072 20.4 -> 15.3 (as a call; what is left is
-// the host's), 3613 x 1024 -> 4096 24.6 -> 17.9, 4096 x 1536 -> 4608 31.9 -> 26.2, 32760 x 1536 -> 4608 149 -> 126, -> 1536 with gate
-// and residual 98.5 -> 80.5.  What bounds it: at 32760 x 1536 -> 4608 the matrix cores, busy two thirds of the time at the
+// leave CUs idle its units need not.  Measured as a call among others, us, two kernels -> here: 512 x 1536 -> 3072 20.7 -> 13.1 (the
+// host's; the kernel takes 9.3), 3613 x 1024 -> 4096 25.3 -> 18.4, 4096 x 1536 -> 4608 32.9 -> 26.5, 32760 x 1536 -> 4608 161 -> 127,
+// -> 1536 with gate and residual 99.5 -> 80.9.  What bounds it: at 32760 x 1536 -> 4608 the matrix cores, busy two thirds of the time at the
 // 1.7 GHz the chip holds under them; taking instructions out of the K step or moving its loads changed nothing there.  At a few
 // thousand rows the quantization, repeated in every column group (5 us of 26 at 4096 rows; half the vector instructions in its absmax
 // changed nothing), and the weights' way into the registers for 64 or 32 rows at a time.
 // Why 64 columns and two waves per SIMD: 32 x MI x 64 sums fill half of a wave's registers at MI = 4, and 64 columns are the 128-byte lines
 // that an epilogue needs; weights through LDS would take the room of the rows and a barrier per step, and each weight byte is read once
 // per CU as it is.  Non-temporal stores because the next kernel reads most outputs too late to find them in L2, where
-// they push out the weights: 32760 x 1536 -> 1536 with gate 97 us with ordinary ones, 72 so.
+// they push out the weights.  Ordinary / non-temporal, us, the kernel back to back on four sets of buffers in turn: 32760 x 1536 ->
+// 4608 170 / 132, -> 8960 309 / 237, -> 1536 66.9 / 57.0 and with gate and residual 83.8 / 80.4 (80.0 / 61.6 on one set), 16000 x 1536 ->
+// 4608 77.0 / 66.5, 3613 x 1024 -> 4096 21.1 / 18.9, 4096 x 1536 -> 4608 27.3 / 26.3, 512 x 1536 -> 3072 9.3 / 9.3.
 #include <type_traits>
 
 #include "vdmq_rowops.h"
@@ -238,6 +240,15 @@ __global__ __launch_bounds__(kWaves * 64, 2) void resident_linear_kernel(const R
         b[ni] = odd_lane ? u32x2{t0, t1} : u32x2{raw.x, raw.y};
         b[2 + ni] = odd_lane ? u32x2{raw.z, raw.w} : u32x2{t0, t1};
     };
+    // The weights, which the next call seldom shares, come from memory: a byte that no XCD has asked for yet takes longer than the two K
+    // steps that it is loaded ahead, and since all workgroups want the same strips at the same time all would wait at every step.  So each
+    // wave asks for 64 lines of 128 bytes at once, all waves together for all of them (as far as that goes), before the rows; from then on
+    // they are in the memory-side cache.  (Every call with weights of its own, us, without / with: 32760 x 1536 -> 4608 157 / 123, -> 8960 289 /
+    // 224, behind a LayerNorm 305 / 235, 32760 x 1024 -> 4096 124 / 98, 4096 x 1536 -> 4608 35.5 / 27.1, 2500 x 640 -> 4096 16.2 / 13.3; always the
+    // same weights 118.6 / 118.8, 215 / 219, 231 / 232, 92 / 87, 26.2 / 25.9, 12.1 / 12.0.)
+    const __amdgpu_buffer_rsrc_t weights = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t *>(args.w), 0, static_cast<int>(min(static_cast<int64_t>(args.N / 32) * rb_bytes, static_cast<int64_t>(0x7FFFFFFF))), 0x00020000);
+    const uint32_t asked = __builtin_amdgcn_raw_buffer_load_b32(weights, ((blockIdx.x * kWaves + wave) * 64 + lane) * 128, 0, 0);
     PartsA a0, a1;
     PartsB b0, b1;
     PartsRaw raw0, raw1;
@@ -295,6 +306,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void resident_linear_kernel(const R
             work_group(va, 0);
         }
     }
+    asm volatile("" ::"v"(asked)); /* (has arrived: the rows were asked for later) */
     __syncthreads();
     // token scales, as they are used for one row-block at a time: fp16, row-blocks 0 and 1 in the lower and upper 32 lanes of the
     // low half, 2 and 3 of the high half (a register instead of four)
