@@ -9,9 +9,9 @@
 // instructions.
 //
 // Against quantizer and tiled GEMM it saves a launch and the blocks' way to memory and back, and where tiles of 256 x 256 or 128 x 128
-// leave CUs idle its units need not.  Measured as a call among others, us, two kernels -> here: 512 x 1536 -> 3072 20.7 -> 13.1 (the
-// host's; the kernel takes 9.3), 3613 x 1024 -> 4096 25.3 -> 18.4, 4096 x 1536 -> 4608 32.9 -> 26.5, 32760 x 1536 -> 4608 161 -> 127,
-// -> 1536 with gate and residual 99.5 -> 80.9.  What bounds it: at 32760 x 1536 -> 4608 the matrix cores, busy two thirds of the time at the
+// leave CUs idle its units need not.  Measured as a call among others, us, two kernels -> here: 512 x 1536 -> 3072 19.9 -> 12.3 (the
+// host's; the kernel takes 10.0), 3613 x 1024 -> 4096 25.1 -> 18.5, 4096 x 1536 -> 4608 32.7 -> 26.4, 32760 x 1536 -> 4608 151 -> 124,
+// -> 1536 with gate and residual 98.7 -> 78.7.  What bounds it: at 32760 x 1536 -> 4608 the matrix cores, busy two thirds of the time at the
 // 1.7 GHz the chip holds under them; taking instructions out of the K step or moving its loads changed nothing there.  At a few
 // thousand rows the quantization, repeated in every column group (5 us of 26 at 4096 rows; half the vector instructions in its absmax
 // changed nothing), and the weights' way into the registers for 64 or 32 rows at a time.
