@@ -575,14 +575,15 @@ ResidentShape resident_shape(int64_t M, int64_t N, bool ln) {
 }  // namespace
 
 // The one-kernel linear's time at K = 1280 ... 1536, us: quantization and strips of its units as resident_shape counts them, output (and
-// residual), what the XCDs fetch.  A residual that comes from memory -- rows in, residual and output together more than 150 MB --
-// is waited for at every turn of the epilogue.  Fitted to the timings of bf6_two_kernels_us, within 0.91 ... 1.07 at 90 % of them.
+// residual), what the XCDs fetch.  A residual that comes from memory -- rows in, residual and output together more than 500 MB; up to
+// 450 MB the terms without it gave 1.04 ... 1.09 of what was measured, beyond 0.78 -- is waited for at every turn of the epilogue.  Fitted to
+// the timings of bf6_two_kernels_us, within 0.91 ... 1.07 at 90 % of them.
 static double resident_us(int64_t M, int64_t N, int64_t K, bool has_tail, const ResidentShape &s) {
     const double k = K / 1536.0, rows = M * K * 2e-6, w = N * K * 0.75e-6, out = M * N * 1e-6;
     const double quantize = 2.5 * s.mi * s.rounds, strips = s.time * 0.1 - quantize;
     const double by_rows = w + rows * (s.groups < kXcds ? s.groups : kXcds), by_weights = rows + w * (s.tiles < kXcds ? s.tiles : kXcds);
     const double fetch = by_rows < by_weights ? by_rows : by_weights;
-    const double waits = M * (2 * K + 4 * N) > 150000000 ? strips : 0.0;
+    const double waits = M * (2 * K + 4 * N) > 500000000 ? strips : 0.0;
     if (!has_tail) {
         if (s.mi == 1) return 1.77 * quantize + 0.75 * strips * k + 0.83 * out + 0.022 * fetch;
         if (s.mi == 2) return 1.16 * quantize + 0.50 * strips * k + 0.41 * out + 0.119 * fetch;
@@ -604,14 +605,18 @@ bool resident_takes(const ResidentProblem &p) {
         // Against quantizer and tiled GEMM it takes 0.5 ... 0.95 of the time as a rule, but it loses where their tiles fill the CUs exactly
         // and its units do not (2459 x 1536 -> 6144 with a residual 33.4 / 26.7 us, 679 x 1472 -> 13056 22.4 / 20.8), and with a residual
         // from memory in front of a wide output (11450 x 1536 -> 11136 203 / 164): so both are estimated.  Not slower, so not asked:
-        // K < 1280 than the int8 path, which served those (6500 timings, 0.995 at most), N <= 384 (550, 1.03).  Few tiles with K divided
-        // (vdmq_bf6_ksplit.hip): 0.93 of that one's time, 1.11 at most, and a launch less for the host.  Of 22000 timings of K 640 ... 1536
-        // the choice takes over 1.03 of the time of the path that served the size before at 0.9 %, over 1.06 at 0.2 % (always one
-        // kernel: 2.3 and 0.9 %), 1.15 at most.  Up to 2.5 million outputs the estimates always say one kernel (2.7 million is the least
-        // where they do not), and the call waits for the host, whom they cost 0.3 us each time.
+        // K < 1280 than the int8 path, which served those (6500 timings, 0.995 at most), N <= 384 (550, 1.03), few tiles with K divided
+        // (vdmq_bf6_ksplit.hip; as calls 0.77 ... 0.83 of that one's time on 320 shapes).  On 2300 shapes of 2.5 ... 400 million outputs, each
+        // timed with one set of buffers and with rows and weights of its own in every call, the choice takes 1.0035 of the faster
+        // form's time in the geometric mean, over 1.06 at 2.3 % (always one kernel 1.0061 and 4.4 %, always two 1.20).
+        // Two kernels are never faster than the host that launches them, 16 us, with gate and residual 20.5 (one: 11.5 and 15.5): without
+        // that 1166 x 1472 -> 3200 with a residual went to two at 20.7 us against 15.5, 230 x 1536 -> 14848 at 17 against 13.4.  Up to 2.5
+        // million outputs the estimates always say one kernel (2.8 million is the least where they do not), and the call waits for the
+        // host, whom they cost 0.2 us each time.
         if (p.K < 1280 || p.N <= 384 || p.M * p.N <= 2500000 || ksplit_takes(p.M, p.N, p.K, p.out_dtype) || p.M * p.N > (int64_t(1) << 40)) return true;
         const ResidentShape shape = resident_shape(p.M, p.N, false);
-        return resident_us(p.M, p.N, p.K, t.residual != nullptr, shape) < bf6_two_kernels_us(p.M, p.N, p.K, t.residual != nullptr);
+        const double two = bf6_two_kernels_us(p.M, p.N, p.K, t.residual != nullptr), host = t.residual != nullptr ? 20.5 : 16.0;
+        return resident_us(p.M, p.N, p.K, t.residual != nullptr, shape) < (two > host ? two : host);
     }
     // Behind a LayerNorm only where its instructions, repeated in each column group, cost less than the second launch and the
     // blocks' way through memory: in effect where a row tile is one workgroup's (K = 1536, us, here / as two kernels: 28000 -> 4608 128 /

@@ -545,7 +545,8 @@ def test_bf6_conversion_shares_no_register_with_its_operands(tmp_path):
 @pytest.mark.parametrize("M,N,K,residual,one", [
     (679, 13056, 1472, False, False), (720, 10880, 1536, False, False), (590, 13056, 1536, True, False),      # their tiles fill the CUs once
     (2459, 6144, 1536, True, False), (11450, 11136, 1536, True, False), (35303, 4992, 1536, True, False),     # ... a residual from memory
-    (83, 32768, 1536, False, False), (76, 32768, 1536, False, True), (97, 28800, 1536, False, False),                     # the fewest outputs so
+    (1166, 3200, 1472, True, True), (4097, 1664, 1280, True, True), (230, 14848, 1536, False, True), (97, 28800, 1536, False, True),  # two wait for the host
+    (324, 21760, 1472, False, False),
     (545, 17536, 1536, False, True), (1043, 8576, 1536, False, True),                                         # ... some CUs twice
     (512, 3072, 1536, False, True), (4096, 4608, 1536, False, True), (32760, 4608, 1536, False, True), (32760, 1536, 1536, True, True),
     (4680, 1536, 1536, True, True), (1, 128, 1536, True, True), (33000, 128, 1536, False, True),
