@@ -240,15 +240,6 @@ __global__ __launch_bounds__(kWaves * 64, 2) void resident_linear_kernel(const R
         b[ni] = odd_lane ? u32x2{t0, t1} : u32x2{raw.x, raw.y};
         b[2 + ni] = odd_lane ? u32x2{raw.z, raw.w} : u32x2{t0, t1};
     };
-    // The weights, which the next call seldom shares, come from memory: a byte that no XCD has asked for yet takes longer than the two K
-    // steps that it is loaded ahead, and since all workgroups want the same strips at the same time all would wait at every step.  So each
-    // wave asks for 64 lines of 128 bytes at once, all waves together for all of them (as far as that goes), before the rows; from then on
-    // they are in the memory-side cache.  (Every call with weights of its own, us, without / with: 32760 x 1536 -> 4608 157 / 123, -> 8960 289 /
-    // 224, behind a LayerNorm 305 / 235, 32760 x 1024 -> 4096 124 / 98, 4096 x 1536 -> 4608 35.5 / 27.1, 2500 x 640 -> 4096 16.2 / 13.3; always the
-    // same weights 118.6 / 118.8, 215 / 219, 231 / 232, 92 / 87, 26.2 / 25.9, 12.1 / 12.0.)
-    const __amdgpu_buffer_rsrc_t weights = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint8_t *>(args.w), 0, static_cast<int>(min(static_cast<int64_t>(args.N / 32) * rb_bytes, static_cast<int64_t>(0x7FFFFFFF))), 0x00020000);
-    const uint32_t asked = __builtin_amdgcn_raw_buffer_load_b32(weights, ((blockIdx.x * kWaves + wave) * 64 + lane) * 128, 0, 0);
     PartsA a0, a1;
     PartsB b0, b1;
     PartsRaw raw0, raw1;
@@ -265,6 +256,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void resident_linear_kernel(const R
         a1[ni] = load16(lane_a, ni); /* (the rest: see step) */
     }
 
+    uint32_t asked;
     // ---- the token rows: 4 * MI per wave, four at a time, the next four on their way
     {
         const int row0 = wave * 4 * MI, rb = row0 / 32;
@@ -294,6 +286,16 @@ __global__ __launch_bounds__(kWaves * 64, 2) void resident_linear_kernel(const R
             quantize_four_rows<MI, NCH>(v, lane, rb, r % 32, kblocks, args.clip, lds, stage);
         };
         load_group(va, 0);
+        // The weights, which the next call seldom shares, come from memory: a byte that no XCD has asked for yet takes longer than the two K
+        // steps that it is loaded ahead, and since all workgroups want the same strips at the same time all would wait at every step.
+        // So each wave asks for 64 lines of 128 bytes at once, all waves together for all of them (as far as that goes), behind its
+        // first rows, which so need not wait for them; from then on they are in the memory-side cache.  (Every call with weights of
+        // its own, us, without / with: 32760 x 1536 -> 4608 157 / 123, -> 8960 289 / 224, behind a LayerNorm 305 / 235, 32760 x 1024 ->
+        // 4096 124 / 98, 4096 x 1536 -> 4608 35.5 / 27.1, 2500 x 640 -> 4096 16.2 / 13.4; always the same weights 118.6 / 118.8, 215 / 219,
+        // 231 / 232, 92 / 87, 26.2 / 25.9, 12.0 / 12.0.)
+        const __amdgpu_buffer_rsrc_t weights = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<uint8_t *>(args.w), 0, static_cast<int>(min(static_cast<int64_t>(args.N / 32) * rb_bytes, static_cast<int64_t>(0x7FFFFFFF))), 0x00020000);
+        asked = __builtin_amdgcn_raw_buffer_load_b32(weights, ((blockIdx.x * kWaves + wave) * 64 + lane) * 128, 0, 0);
         if constexpr (MI > 1) {
 #pragma unroll 1
             for (int g = 0; g < MI; g += 2) {
