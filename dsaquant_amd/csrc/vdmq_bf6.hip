@@ -832,14 +832,19 @@ Bf6Plan bf6_plan(int64_t M, int64_t N) {
     // shapes of 20 tiles up 0.88 of whole-XCD super-tiles in the geometric mean, 1.07 at most but for a few of 85...90 tiles at
     // K = 5120 (250 x 5632 13.5 / 14.9 us, why is not known); strips of four or six rows are up to 1.11 (an XCD's tiles far
     // from square read more operand rows).
-    // Kept as they were: problems that give no CU of the busiest XCD a second workgroup (small tiles: and every XCD one
-    // super-tile at most), and those where any order gives some CUs a second one and this one not to more than a quarter
-    // (640 x 7808, 5120, 40 tiles on the busiest: 23.0 us, in strips 24.5; not in the shape of two columns, which leaves
-    // most places empty: 512 x 10240, 5120 24.35, in strips 24.15).
+    // Kept as they were: problems that give every XCD one super-tile at most and no CU of the busiest a second workgroup, and
+    // those where any order gives some CUs a second one and this one not to more than a quarter (640 x 7808, 5120, 40 tiles on
+    // the busiest: 23.0 us, in strips 24.5; not in the shape of two columns, which leaves most places empty: 512 x 10240, 5120
+    // 24.35, in strips 24.15).
     const int64_t all_tiles = static_cast<int64_t>(tm.tiles_m) * tm.tiles_n;
     const bool at_once = all_tiles <= kXcds * per;
     const bool few_doubled = all_tiles > kXcds * 32 && best_load <= 40 && tm.group_n_log2 == 2;
-    const bool spread = at_once ? !few_doubled && (best_load > 32 || (Cfg::kOcc == 2 && tm.total_super > kXcds)) : Cfg::kOcc == 2;
+    // More super-tiles than XCDs are partly empty ones here, and big tiles, a CU each, do not bear that: an XCD deals its workgroups to its
+    // four shader engines in turn, those without a tile too, so that one engine can get more tiles than its eight CUs while others
+    // idle (5 x 39 tiles as super-tiles of 16 x 2, ten full places each: 9, 9, 6 and 6), two rounds.  As super-tiles / in strips, us: 1049 x
+    // 9856, K 6400 69.8 / 42.3; 1280 x 11264, K 6400 72.8 / 46.0; 1280 x 8704, K 1536 26.8 / 16.7; 21785 x 512, K 13184 125 / 74.  Of 250
+    // problems of 6 ... 17 million outputs 39 change their order: 0.58 ... 0.94 of the time.
+    const bool spread = at_once ? !few_doubled && (best_load > 32 || tm.total_super > kXcds) : Cfg::kOcc == 2;
     if (spread && at_once)
         bf6_tilemap_strips(tm, tiles_m, tiles_n);
     else if (spread) /* (small tiles of more than one round are refilled as they end: 4 x 4, which reads fewer operand rows) */
@@ -959,8 +964,6 @@ bool small_tiles_serve(int64_t M, int64_t N, int64_t K, bool has_tail) {
 // Quantizer and tiled GEMM at K = 1280 ... 1536, us: for the rule that sets the one-kernel linear against them (vdmq_resident.hip), as that
 // one's estimate from its sizes alone.  Launches and the quantizer's way through memory, what a CU's tiles take in turn, the output (and
 // residual) bytes.  Fitted to 8300 timings, M to 75600, N to 25600: 0.91 ... 1.08 of what was measured at 90 % of them.
-// Where an XCD's tiles leave partly empty super-tiles, CUs are dealt out by fours: 25, 27 or 30 tiles on its 32 CUs take two
-// rounds (5 x 34 and 3 x 73 tiles 30 us, 5 x 32 and 3 x 64 20).
 double bf6_two_kernels_us(int64_t M, int64_t N, int64_t K, bool has_tail) {
     const double k = K / 1536.0, x = M * K * 1e-6, out = M * N * 1e-6;
     auto load_of = [](const Bf6Plan &p) { return p.spread || p.load <= 0 ? ceil_div(static_cast<int64_t>(p.tm.tiles_m) * p.tm.tiles_n, kXcds) : p.load; };
@@ -970,8 +973,8 @@ double bf6_two_kernels_us(int64_t M, int64_t N, int64_t K, bool has_tail) {
     }
     const Bf6Plan p = bf6_plan<Bf6Big>(M, N);
     const int64_t load = load_of(p);
-    const bool persistent = !p.spread && few_empty_places(p.tm.total_super, load), doubled = p.at_once && !p.spread && load > 24 && load % 4 != 0;
-    const double rounds = persistent ? ceil_div(p.tm.total_super, kXcds) : doubled ? 2 : ceil_div(load, 32);
+    const bool persistent = !p.spread && few_empty_places(p.tm.total_super, load);
+    const double rounds = persistent ? ceil_div(p.tm.total_super, kXcds) : ceil_div(load, 32);
     return has_tail ? 6.7 + 0.48 * x + 10.1 * rounds * k + 0.67 * out : 8.6 + 0.45 * x + 7.6 * rounds * k + 0.50 * out;
 }
 

@@ -283,6 +283,8 @@ def test_bf6_tiles_that_run_at_once_are_spread_evenly(M, N, K, tile, group_n, co
     (256 * 15 - 9, 256 * 17, 64, 256, 2),   # 255 big tiles
     (640, 128 * 61, 64, 128, 4),            # 40 tiles on the busiest XCD, as few as any order gives some CU a second one
     (1150, 128 * 31, 128, 128, 4),          # 36
+    (1049, 128 * 77, 64, 256, 2),           # 5 x 39 big tiles: three partly empty super-tiles on some XCDs
+    (21785, 512, 128, 256, 2),              # 86 x 2
 ])
 def test_bf6_spread_tiles_leave_no_place_empty(M, N, K, tile, group_n):
     """Problems whose tiles the chip holds at once: equal shares of the XCDs, so one workgroup per XCD at most has no
