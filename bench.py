@@ -90,7 +90,7 @@ CASES = {"cfg0_qkv_m4096": dict(M=4096, linears=[("qkv", 1536, 4608)]),
          "cfg3_cross_kv_m512": dict(M=512, linears=[("cross_kv", 5120, 10240)]),
          "cfg3_qkv_ragged_m75637": dict(M=75637, linears=[("qkv", 5120, 15360)])}
 # VDMQ_KERNEL_* of include/vdmq.h
-KERNEL_NAMES = {1: "gemm_w4a4_kernel", 2: "gemm_bf6_kernel", 3: "gemm_bf6_persistent_kernel", 4: "resident_linear_kernel", 5: "gemm_bf6_ksplit_kernel"}
+KERNEL_NAMES = {1: "gemm_w4a4_kernel", 2: "gemm_bf6_kernel", 3: "gemm_bf6_persistent_kernel", 4: "resident_linear_kernel", 5: "gemm_bf6_ksplit_kernel", 6: "gemm_bf6_pair_kernel"}
 SHORT = {"wan1.3b_480p_block": "wan1p3b", "wan5b_704x1280_block": "wan5b", "wan14b_720p_block": "wan14b"}
 
 

@@ -28,7 +28,7 @@ class GemmLaunchInfo(ctypes.Structure):
                 ("group_n", ctypes.c_int), ("contiguous_runs", ctypes.c_int), ("workgroups", ctypes.c_int64)]
 
 
-KERNEL_GEMM_W4A4, KERNEL_GEMM_BF6, KERNEL_GEMM_BF6_PERSISTENT, KERNEL_LINEAR_RESIDENT, KERNEL_GEMM_BF6_KSPLIT = 1, 2, 3, 4, 5
+KERNEL_GEMM_W4A4, KERNEL_GEMM_BF6, KERNEL_GEMM_BF6_PERSISTENT, KERNEL_LINEAR_RESIDENT, KERNEL_GEMM_BF6_KSPLIT, KERNEL_GEMM_BF6_PAIR = 1, 2, 3, 4, 5, 6
 
 # name -> (restype, argtypes); every symbol include/vdmq.h declares
 _i64, _p, _f32, _int = ctypes.c_int64, ctypes.c_void_p, ctypes.c_float, ctypes.c_int

@@ -413,6 +413,9 @@ static int gemm_bf6_checked(const void *xblocks, const void *ascale, const void 
     if (by_size && acc == nullptr && ksplit_takes(M, N, K, out_dtype))
         return launch_gemm_bf6_ksplit(static_cast<const uint8_t *>(xblocks), static_cast<const __half *>(ascale), static_cast<const uint8_t *>(wblocks),
                                       static_cast<const __half *>(wscale), static_cast<const __half *>(bias), out, M, N, K, ldo, tail, as_stream(stream));
+    if (by_size && acc == nullptr && pair_takes(M, N, K, out_dtype, tail))
+        return launch_gemm_bf6_pair(static_cast<const uint8_t *>(xblocks), static_cast<const __half *>(ascale), static_cast<const uint8_t *>(wblocks),
+                                    static_cast<const __half *>(wscale), static_cast<const __half *>(bias), out, M, N, K, ldo, tail, as_stream(stream));
     return launch_gemm_bf6(static_cast<const uint8_t *>(xblocks), static_cast<const __half *>(ascale), static_cast<const uint8_t *>(wblocks),
                            static_cast<const __half *>(wscale), static_cast<const __half *>(bias), out, out_dtype, acc, M, N, K, ldo, tail,
                            as_stream(stream));
@@ -459,7 +462,7 @@ int64_t vdmq_workspace_bytes_bf6(int64_t M, int64_t K) {
 
 // Quantizer and GEMM of the bf6 path for every form of a linear: rows as they are, through an activation or a LayerNorm;
 // output plain, with the gated residual update, or split by columns.  One kernel where the rows' operand fits LDS
-// (vdmq_resident.hip), else the two, the GEMM by its size (vdmq_bf6_ksplit.hip; the separate entries keep the tiled one).
+// (vdmq_resident.hip), else the two, the GEMM by its size (vdmq_bf6_ksplit.hip, vdmq_bf6_pair.hip; the separate entries keep the tiled one).
 static int linear_bf6_checked(const ResidentProblem &p, void *workspace, int64_t workspace_bytes, vdmq_stream_t stream) {
     VDMQ_TRY(check_k(p.K));
     VDMQ_TRY(check_n(p.N));

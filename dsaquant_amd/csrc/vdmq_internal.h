@@ -82,6 +82,11 @@ bool ksplit_takes(int64_t M, int64_t N, int64_t K, int out_dtype);
 int launch_gemm_bf6_ksplit(const uint8_t *xblocks, const __half *ascale, const uint8_t *wblocks, const __half *wscale, const __half *bias, void *out, int64_t M,
                            int64_t N, int64_t K, int64_t ldo, const GemmTail &tail, hipStream_t stream);
 
+// problems between few tiles and many (vdmq_bf6_pair.hip)
+bool pair_takes(int64_t M, int64_t N, int64_t K, int out_dtype, const GemmTail &tail);
+int launch_gemm_bf6_pair(const uint8_t *xblocks, const __half *ascale, const uint8_t *wblocks, const __half *wscale, const __half *bias, void *out, int64_t M,
+                         int64_t N, int64_t K, int64_t ldo, const GemmTail &tail, hipStream_t s);
+
 // quantizer and GEMM in one kernel for short rows (vdmq_resident.hip)
 struct ResidentProblem {
     const __half *x;

@@ -175,6 +175,7 @@ int vdmq_gemm_w4a4_acc(const void *qact, const void *wq, int32_t *acc, int64_t M
 #define VDMQ_KERNEL_GEMM_BF6_PERSISTENT 3 /* bf6 matrix path, one workgroup per CU walking tiles */
 #define VDMQ_KERNEL_LINEAR_RESIDENT 4     /* bf6 matrix path, quantizer and GEMM in one kernel (short rows) */
 #define VDMQ_KERNEL_GEMM_BF6_KSPLIT 5     /* bf6 matrix path, K divided among the waves of a workgroup (few tiles) */
+#define VDMQ_KERNEL_GEMM_BF6_PAIR 6       /* bf6 matrix path, K divided between two groups of waves (a tile per CU) */
 typedef struct vdmq_gemm_launch_info {
     int kernel;                 /* VDMQ_KERNEL_* */
     int tile_m, tile_n;         /* output tile of one workgroup: token rows x channels */

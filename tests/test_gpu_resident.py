@@ -1,5 +1,6 @@
 """The forms of a linear that vdmq_linear_bf6 chooses by size -- one kernel for short rows, K divided among a workgroup's waves for few
-tiles --: the bits of the quantizer and the tiled GEMM in every form they take, at the edges of their tiles, strips and K steps,
+tiles, between two groups of them for a tile per CU --: the bits of the quantizer and the tiled GEMM in every form they take, at the
+edges of their tiles, strips and K steps,
 and what they leave to those two."""
 import pytest
 import torch
@@ -8,7 +9,7 @@ from tests.test_gpu_parity import vk
 
 pytestmark = pytest.mark.gpu
 
-RESIDENT, KSPLIT = 4, 5  # VDMQ_KERNEL_* of include/vdmq.h
+RESIDENT, KSPLIT, PAIR = 4, 5, 6  # VDMQ_KERNEL_* of include/vdmq.h
 F16 = torch.float16
 TILED = (2, 3)
 
@@ -268,7 +269,33 @@ def test_few_tiles_short_rows(weight, K):
     both(lambda: F.linear_fused(rows(100, K, 9), qw, ws, b, 0.95, act="gelu_tanh"), KSPLIT)
 
 
-@pytest.mark.parametrize("M,N,K", [(129, 1536, 1536), (2100, 1536, 1472), (200, 512, 4096), (500, 4096, 3328)])
+# each tile, the last rows and columns of a ragged one, an odd and an even number of 128 k steps with and without a half one, the
+# first K each is taken at, and problems next to the rule's lines
+@pytest.mark.parametrize("M,N,K,tile", [(1021, 4224, 1984, (128, 160)), (257, 13568, 2112, (128, 160)), (2151, 2432, 3328, (128, 192)),
+                                        (11473, 512, 3392, (192, 128)), (4680, 1536, 7424, (192, 160)), (2881, 2944, 2624, (192, 192)),
+                                        (5579, 1536, 11072, (192, 192)), (1021, 4224, 1920, None), (1024, 4096, 4096, None), (2880, 2944, 2560, None)])
+def test_between_few_tiles_and_many(weight, M, N, K, tile):
+    from dsaquant_amd import fused_ops as F
+
+    v = vk()
+    qw, ws, b = weight(N, K)
+    x = rows(M, K, 21)
+    kernel = TILED if tile is None else PAIR
+    info = both(lambda: v.linear_vdm_w4a4(x, qw, ws, b, 0.95), kernel)
+    assert tile is None or (info.tile_m, info.tile_n) == tile
+    both(lambda: F.linear_fused(x, qw, ws, None, 1e-3, split_cols=64), kernel)
+    both(lambda: v._linear_2d(x, v._prepared_weight(qw, ws), b, 0.95, out_dtype=torch.bfloat16), TILED)
+    if tile is not None:
+        g = torch.Generator(device="cuda").manual_seed(11)
+        res = torch.randn(M, N, generator=g, device="cuda").half()
+        for n in {1, M, 2 if M % 2 == 0 else 1}:
+            gate = torch.randn(n, N, generator=g, device="cuda").half()
+            both(lambda: F.linear_fused(x, qw, ws, b, 0.95, residual=res, gate=gate), PAIR)
+        both(lambda: F.linear_fused(x, qw, ws, b, 0.95, residual=res), PAIR)
+        both(lambda: F.linear_fused(x, qw, ws, None, 0.95, act="gelu_tanh", gate=gate), PAIR)
+
+
+@pytest.mark.parametrize("M,N,K", [(129, 1536, 1536), (2100, 1536, 1472), (200, 512, 4096), (500, 4096, 3328), (1021, 4224, 1984)])
 def test_residual_updated_in_place_through_the_c_abi(weight, M, N, K):
     """``out`` is the residual: each element is read by the lane that writes it, before."""
     from dsaquant_amd import _lib, fused_ops as F
@@ -285,14 +312,14 @@ def test_residual_updated_in_place_through_the_c_abi(weight, M, N, K):
     _lib.check(lib.vdmq_linear_bf6_ex(x.data_ptr(), M, K, K, 0.95, 0, 0, 0.0, None, None, 0, 1, pw.operand(True).data_ptr(), pw.wscale.data_ptr(),
                                       b.data_ptr(), gate.data_ptr(), N, M, out.data_ptr(), N, 0, 0, out.data_ptr(), 0, N, N, workspace.data_ptr(),
                                       nbytes, torch.cuda.current_stream().cuda_stream))
-    assert _lib.last_gemm_launch().kernel in (RESIDENT, KSPLIT)
+    assert _lib.last_gemm_launch().kernel in (RESIDENT, KSPLIT, PAIR)
     assert torch.equal(out, want)
 
 
 # resident (32, 64, 128 rows; LayerNorm), K split (64 x 64, 128 x 64)
 @pytest.mark.parametrize("M,N,K,kind", [(257, 1536, 1088, "tail"), (4100, 1536, 960, "tail"), (32700, 1536, 1472, "tail"), (200, 512, 4096, "tail"),
                                         (500, 4096, 3328, "tail"), (300, 768, 1536, "split"), (4100, 1536, 1024, "split"), (200, 768, 4096, "split"),
-                                        (32700, 1536, 1088, "ln")])
+                                        (32700, 1536, 1088, "ln"), (1021, 4224, 1984, "tail"), (1021, 4224, 2112, "split")])
 def test_strides_beyond_the_rows_through_the_c_abi(weight, M, N, K, kind):
     """Row strides of input, residual, gate, LayerNorm vectors and output beyond their rows, a part stride beyond the part: the
     bits of the dense call, no byte written outside the rows."""
@@ -335,6 +362,6 @@ def test_strides_beyond_the_rows_through_the_c_abi(weight, M, N, K, kind):
     _lib.check(lib.vdmq_linear_bf6_ex(xw.data_ptr(), M, K, xw.stride(0), 0.95, 0, *ln, pw.operand(True).data_ptr(), pw.wscale.data_ptr(), b.data_ptr(),
                                       gate_p, ldg, rpg, res_p, ldr, split, part_stride, flat.data_ptr(), 0, N, cols + 40, workspace.data_ptr(), nbytes,
                                       torch.cuda.current_stream().cuda_stream))
-    assert _lib.last_gemm_launch().kernel == (KSPLIT if K > 1536 else RESIDENT)
+    assert _lib.last_gemm_launch().kernel == (PAIR if N == 4224 else KSPLIT if K > 1536 else RESIDENT)
     assert torch.equal(flat[:, :M, :cols].contiguous().view(torch.int16), want.contiguous().view(torch.int16))
     assert (flat[:, :M, cols:] == 3.0).all() and (flat[:, M:] == 3.0).all()
