@@ -12,6 +12,7 @@ LIB_PATH = _PKG / "libvdmq.so"
 CSRC = _PKG / "csrc"
 
 _LIB: Optional[ctypes.CDLL] = None
+host = None  # the extension module _vdmq_host, once load() has run
 
 VDMQ_VERSION = 2  # include/vdmq.h; also the version of the bf6 block format
 VDMQ_OUT_F16 = 0
@@ -106,13 +107,15 @@ def build(verbose: bool = False) -> Path:
 
 def load() -> ctypes.CDLL:
     """Load the built library; raises if it is missing (no fallback exists)."""
-    global _LIB
+    global _LIB, host
     if _LIB is not None:
         return _LIB
     if not LIB_PATH.exists():
         raise FileNotFoundError(
             f"{LIB_PATH} is missing: build it with `python -c 'import __graft_entry__ as g; g.build()'` "
             f"or `make -C {CSRC}`")
+    import torch  # noqa: F401  (the extension module below needs its libraries, and the HIP runtime that serves both is the one loaded first)
+
     lib = ctypes.CDLL(str(LIB_PATH))
     for name, (restype, argtypes) in SIGNATURES.items():
         fn = getattr(lib, name)
@@ -120,6 +123,11 @@ def load() -> ctypes.CDLL:
         fn.argtypes = argtypes
     if lib.vdmq_version() != VDMQ_VERSION:
         raise RuntimeError(f"{LIB_PATH} has interface version {lib.vdmq_version()}, this package expects {VDMQ_VERSION}: rebuild it (make -C {CSRC})")
+    # (the host side of the package's own calls: vdmq_host.cpp, built with the library)
+    from . import _vdmq_host
+
+    _vdmq_host.init(*(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in ("vdmq_linear_bf6_ex", "vdmq_linear_bf6_workspace", "vdmq_pack_weight")))
+    host = _vdmq_host
     _LIB = lib
     return lib
 

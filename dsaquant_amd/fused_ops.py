@@ -72,17 +72,28 @@ class LnInput:
             raise ValueError(f"unknown LayerNorm mode {mode!r}")
         self.shape = tuple(x.shape)
         K = x.shape[-1]
-        self.x = _k._half_rows(x, K)
-        M = self.x.shape[0]
-        a2, b2 = _k._half_rows(a, K), _k._half_rows(b, K)
-        if a2.shape != b2.shape:
-            raise ValueError("the two LayerNorm vectors must have the same shape")
-        nvec = a2.shape[0]
+        self._rows = None
+        if all(t.dtype is torch.float16 and t.is_contiguous() for t in (x, a, b)) and a.shape == b.shape and K > 0 and a.dim() and a.shape[-1] == K:
+            M, nvec = x.numel() // K, a.numel() // K
+        else:
+            self._rows = tuple(_k._half_rows(t, K) for t in (x, a, b))
+            if self._rows[1].shape != self._rows[2].shape:
+                raise ValueError("the two LayerNorm vectors must have the same shape")
+            M, nvec = self._rows[0].shape[0], self._rows[1].shape[0]
         if nvec == 0 or M % nvec != 0:
             raise ValueError(f"{nvec} vectors do not divide {M} rows")
-        self.a, self.b, self.rows_per_vec = a2, b2, M // nvec
+        self._given = x, a, b
+        self.rows_per_vec = M // nvec
         self.eps, self.mode = float(eps), mode
         self.code = _lib.VDMQ_LN_MODULATE if mode == "modulate" else _lib.VDMQ_LN_AFFINE
+
+    def _two_d(self, i: int) -> torch.Tensor:
+        # rows of K, made when they are asked for: a call that takes the tensors as they were given (3 us less on the host) never does
+        if self._rows is None:
+            self._rows = tuple(_k._half_rows(t, self.shape[-1]) for t in self._given)
+        return self._rows[i]
+
+    x, a, b = (property(lambda self, i=i: self._two_d(i)) for i in range(3))
 
     def _args(self):
         M, K = self.x.shape
@@ -180,6 +191,10 @@ def linear_fused(
     fused projection.  ``split_cols``: the output columns as N / split_cols contiguous tensors, stacked in front
     (``[N / split_cols, ..., split_cols]``; without gate and residual).  Returns a new tensor; nothing is updated in place."""
     _k._load_ext()  # raises when the library is missing
+    if not isinstance(x, QuantizedInput) and (act is None or act == "gelu_tanh") and (split_cols is None or split_cols):
+        out = _native_fused(x, qweight, wscales, bias_half if bias_half is not None else bias, clip_ratio, act, residual, gate, split_cols or 0)
+        if out is not None:
+            return out
     if isinstance(x, LnInput):
         if act is not None:
             raise ValueError("an activation cannot be combined with a LayerNorm input")
@@ -246,6 +261,21 @@ def linear_fused(
                 operand, scales = _k._quantize_for_gemm(x_2d, clip_ratio, act_code, bf6, ln_args)
                 _k._gemm_dispatch(operand, scales, bf6, weight, b, out, K, gate=g2, rows_per_gate=rows_per_gate, residual=r2)
     return out.view(*lead, N) if split_cols is None else out.view(N // split_cols, *lead, split_cols)
+
+
+def _native_fused(x, qweight, wscales, bias, clip_ratio, act, residual, gate, split_cols):
+    prepared = type(qweight) is _k.PreparedWeight
+    if not prepared and (isinstance(qweight, _k.PreparedWeight) or wscales is None):
+        return None
+    if type(x) is LnInput:
+        if act is not None:
+            return None
+        rows, a, b = x._given if x._rows is None else x._rows
+        return _k._native_linear(rows, qweight, None if prepared else wscales, bias, clip_ratio, shape=None if x._rows is None else x.shape,
+                                 ln=(x.code, x.eps, a, b, x.rows_per_vec),
+                                 residual=residual, gate=gate, split_cols=split_cols)
+    return _k._native_linear(x, qweight, None if prepared else wscales, bias, clip_ratio, act=_lib.VDMQ_ACT_NONE if act is None else _lib.VDMQ_ACT_GELU_TANH,
+                             residual=residual, gate=gate, split_cols=split_cols)
 
 
 def qkv_projections_ln(attn, pre: LnInput):

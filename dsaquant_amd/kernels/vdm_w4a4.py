@@ -316,8 +316,9 @@ class PreparedWeight:
             if getattr(self, other) is not None and not self._used[other]:
                 setattr(self, other, None)  # made ahead for a call pattern that did not come
                 self._ready.pop(other, None)
-        self._order_behind("wscale")
-        self._order_behind(form)
+        if self._ready:
+            self._order_behind("wscale")
+            self._order_behind(form)
         return getattr(self, form)
 
     def extra_bytes(self) -> int:
@@ -396,6 +397,28 @@ def _prepared_weight(qweight: torch.Tensor, wscales: torch.Tensor) -> PreparedWe
             qweight.__dict__["_vdmq_contiguous"] = kept
         qweight, wscales = kept[2], kept[3]
     return _prepared([(qweight, wscales)])
+
+
+def _operands(qweight, wscales: Optional[torch.Tensor], device_index: int):
+    """``(bf6 blocks, channel scales, N, stream)`` of a packed weight (``wscales`` None: of a PreparedWeight) for a call on the
+    current stream; None where the device is not the current one."""
+    if torch._C._cuda_getDevice() != device_index:
+        return None
+    weight = qweight if wscales is None else _prepared([(qweight, wscales)])
+    return weight.operand(True), weight.wscale, weight.N, torch._C._cuda_getCurrentRawStream(device_index)
+
+
+def _native_linear(x: torch.Tensor, qweight, wscales: Optional[torch.Tensor], bias: Optional[torch.Tensor], clip_ratio: float, *, shape=None,
+                   check=(None, None), act: int = 0, ln=(0, 0.0, None, None, 1), residual=None, gate=None, split_cols: int = 0, views: int = 0):
+    """The whole call in the extension module (vdmq_host.cpp) where its operands are plain and the bf6 path is the library's choice; None: they
+    are not, and nothing has been done.  ``qweight`` may be a PreparedWeight, without ``wscales``."""
+    if _MATRIX_PATH != "auto":
+        return None
+    out = _lib.host.linear(_operands, x, shape, qweight, wscales, check[0], check[1], bias, clip_ratio, act, ln[0], ln[1], ln[2], ln[3], ln[4], residual,
+                           gate, split_cols, views)
+    if type(out) is int:
+        _lib.check(out)
+    return out
 
 
 def prepare_weight(qweight: torch.Tensor, wscales: torch.Tensor, tokens: Optional[int] = None, path: Optional[str] = None) -> PreparedWeight:
@@ -570,6 +593,10 @@ def pack_weight_with_scale(weight: torch.Tensor, channel_scale: torch.Tensor):
     vdm_w4a4_kernel.cu:697-728.
     """
     _load_ext()
+    if channel_scale.dtype is torch.float16 and channel_scale.is_contiguous():
+        out = _native_pack(weight, channel_scale.detach().view(-1))
+        if out is not None:
+            return out
     weight_h = weight.detach().half().contiguous()
     scale_h = channel_scale.detach().view(-1).half().contiguous().to(weight_h.device)
     _check_device_tensor(weight_h, "weight", torch.float16)
@@ -582,10 +609,24 @@ def quantize_weight_per_channel(weight: torch.Tensor):
     """Derive per-channel scales (absmax/7, clip 1) and pack
     (vdm_w4a4.py:217-219 / vdm_w4a4_kernel.cu:730-763)."""
     _load_ext()
+    out = _native_pack(weight, None)
+    if out is not None:
+        return out
     weight_h = weight.detach().half().contiguous()
     _check_device_tensor(weight_h, "weight", torch.float16)
     _require(weight_h.dim() == 2, "weight must be [N, K]")
     return _pack_weight(weight_h, None)
+
+
+def _native_pack(weight: torch.Tensor, channel_scale: Optional[torch.Tensor]):
+    # (for the int8 path's rows the pass writes that path's form too)
+    if _MATRIX_PATH == "int8":
+        return None
+    index = torch._C._cuda_getDevice()
+    out = _lib.host.pack(weight, channel_scale, index, torch._C._cuda_getCurrentRawStream(index))
+    if type(out) is int:
+        _lib.check(out)
+    return out
 
 
 def _pack_weight(weight_h: torch.Tensor, scale_h: Optional[torch.Tensor]):
@@ -677,6 +718,9 @@ def linear_vdm_w4a4(
     against the packed weights, per-token x per-channel scale and fp16 bias.
     Signature and semantics of vdm_w4a4.py:222-244; the output is always fp16."""
     _load_ext()
+    out = _native_linear(x, qweight, wscales, bias_half if bias_half is not None else bias, clip_ratio)
+    if out is not None:
+        return out
     x_2d, orig_shape = _as_2d_half_contiguous(x)
     _check_linear_shapes(x_2d, qweight, wscales)
     _require(x_2d.is_cuda, "input must be a CUDA tensor")
@@ -691,6 +735,10 @@ def linear_vdm_w4a4_prepared(x: torch.Tensor, weight: PreparedWeight, bias_half:
     contiguous tensors, returned stacked as ``[N / split_cols, ..., split_cols]`` -- the bits of
     ``out.split(split_cols, -1)``, without the strided views (the GEMM epilogue writes them in place)."""
     _load_ext()
+    if type(weight) is PreparedWeight and (split_cols is None or split_cols):
+        out = _native_linear(x, weight, None, bias_half, clip_ratio, split_cols=split_cols or 0)
+        if out is not None:
+            return out
     x_2d, orig_shape = _as_2d_half_contiguous(x)
     if weight.K != x_2d.shape[1]:
         raise ValueError("qweight shape must be [N, K/2]")
@@ -840,6 +888,13 @@ def linear_vdm_w4a4_qkv(
     self-contained, so the concatenation's operand is the parts' operands one after the other) and that is kept.
     ``contiguous_outputs`` (not in the reference): q, k and v are written by the GEMM epilogue as three contiguous
     tensors instead of strided views of one -- the same bits."""
+    if w_qkv_packed is not None and w_qkv_scale is not None and (qkv_bias_half is not None or (q_bias is None and k_bias is None and v_bias is None)):
+        _load_ext()
+        n = q_weight_packed.shape[0]
+        out = _native_linear(x, w_qkv_packed, w_qkv_scale, qkv_bias_half, clip_ratio, check=(q_weight_packed, q_weight_scale),
+                             split_cols=n if contiguous_outputs else 0, views=0 if contiguous_outputs else n)
+        if out is not None:
+            return out.unbind(0) if contiguous_outputs else out
     if w_qkv_packed is None or w_qkv_scale is None:
         weight = _prepared([(q_weight_packed.contiguous(), q_weight_scale.contiguous()), (k_weight_packed.contiguous(), k_weight_scale.contiguous()),
                             (v_weight_packed.contiguous(), v_weight_scale.contiguous())])
