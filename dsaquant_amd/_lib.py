@@ -81,6 +81,9 @@ SIGNATURES = {
     "vdmq_gemm_w4a4_bf6_acc": (_int, [_p, _p, _p, _i64, _i64, _i64, _p]),
     "vdmq_attention_f16": (_int, [_p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _f32, _p]),
     "vdmq_rms_norm_rope_f16": (_int, [_p, _i64, _p, _p, _p, _i64, _p, _p, _i64, _i64, _f32, _p, _i64, _i64, _p]),
+    "vdmq_row_squares_f32": (_int, [_p, _i64, _p, _p, _i64, _p, _i64, _i64, _p]),
+    "vdmq_scale_rows": (_int, [_p, _i64, _p, _p, _p, _p, _i64, _p, _p, _p, _int, _i64, _i64, _p]),
+    "vdmq_modulate_rows_f16": (_int, [_p, _p, _p, _p, _i64, _i64, _p]),
     "vdmq_rope_table": (_int, [_p, _i64, _i64, _i64, _i64, _p]),
     "vdmq_timestep_embedding_f16": (_int, [_p, _p, _i64, _i64, _p]),
     "vdmq_copy_u128": (_int, [_p, _p, _i64, _p]),

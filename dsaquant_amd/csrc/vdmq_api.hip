@@ -727,6 +727,57 @@ int vdmq_rms_norm_rope_f16(const void *x0, int64_t ldx0, const void *w0, void *o
                             table != nullptr ? positions : 1, as_stream(stream));
 }
 
+static int rows_checked(const void *const *x, const int64_t *ldx, void *const *out, int matrices, int64_t rows, int64_t K) {
+    VDMQ_TRY(check_m(rows));
+    if (K <= 0 || K % 8 != 0 || K > kMaxDim) return fail(VDMQ_ESHAPE, "K must be a positive multiple of 8 (got %lld)", (long long)K);
+    for (int i = 0; i < matrices && rows > 0; ++i) {
+        VDMQ_TRY(check_ptr(x[i], "x"));
+        VDMQ_TRY(check_ptr(out[i], "out"));
+        if (ldx[i] < K || ldx[i] % 8 != 0) return fail(VDMQ_ESHAPE, "ldx must be >= K and a multiple of 8 (got %lld)", (long long)ldx[i]);
+    }
+    return VDMQ_OK;
+}
+
+int vdmq_row_squares_f32(const void *x0, int64_t ldx0, void *out0, const void *x1, int64_t ldx1, void *out1, int64_t rows, int64_t K, vdmq_stream_t stream) {
+    const void *x[2] = {x0, x1};
+    void *out[2] = {out0, out1};
+    const int64_t ldx[2] = {ldx0, ldx1};
+    const int matrices = x1 != nullptr ? 2 : 1;
+    VDMQ_TRY(rows_checked(x, ldx, out, matrices, rows, K));
+    if (rows == 0) return VDMQ_OK;
+    const __half *xs[2] = {static_cast<const __half *>(x0), static_cast<const __half *>(x1)};
+    float *outs[2] = {static_cast<float *>(out0), static_cast<float *>(out1)};
+    return launch_row_squares(xs, ldx, outs, matrices, rows, K, as_stream(stream));
+}
+
+int vdmq_scale_rows(const void *x0, int64_t ldx0, const void *r0, const void *w0, void *out0, const void *x1, int64_t ldx1, const void *r1, const void *w1,
+                    void *out1, int out_f32, int64_t rows, int64_t K, vdmq_stream_t stream) {
+    const void *x[2] = {x0, x1}, *r[2] = {r0, r1}, *w[2] = {w0, w1};
+    void *out[2] = {out0, out1};
+    const int64_t ldx[2] = {ldx0, ldx1};
+    const int matrices = x1 != nullptr ? 2 : 1;
+    VDMQ_TRY(rows_checked(x, ldx, out, matrices, rows, K));
+    if (rows == 0) return VDMQ_OK;
+    for (int i = 0; i < matrices; ++i) {
+        VDMQ_TRY(check_ptr(w[i], "w"));
+        VDMQ_TRY(check_ptr(r[i], "r", false));
+    }
+    const __half *xs[2] = {static_cast<const __half *>(x0), static_cast<const __half *>(x1)}, *ws[2] = {static_cast<const __half *>(w0), static_cast<const __half *>(w1)};
+    const float *rs[2] = {static_cast<const float *>(r0), static_cast<const float *>(r1)};
+    return launch_scale_rows(xs, ldx, rs, ws, out, out_f32 != 0, matrices, rows, K, as_stream(stream));
+}
+
+int vdmq_modulate_rows_f16(const void *y, const void *a, const void *b, void *out, int64_t rows, int64_t K, vdmq_stream_t stream) {
+    void *outs[1] = {out};
+    const int64_t ldy[1] = {K};
+    VDMQ_TRY(rows_checked(&y, ldy, outs, 1, rows, K));
+    if (rows == 0) return VDMQ_OK;
+    VDMQ_TRY(check_ptr(a, "a"));
+    VDMQ_TRY(check_ptr(b, "b"));
+    return launch_modulate_rows(static_cast<const float *>(y), static_cast<const __half *>(a), static_cast<const __half *>(b), static_cast<__half *>(out), rows, K,
+                                as_stream(stream));
+}
+
 int vdmq_rope_table(void *table, int64_t head_dim, int64_t f, int64_t h, int64_t w, vdmq_stream_t stream) {
     if (head_dim <= 0 || head_dim > 4096 || f < 0 || h < 0 || w < 0 || f > kMaxDim || h > kMaxDim || w > kMaxDim)
         return fail(VDMQ_ESHAPE, "head_dim, f, h or w out of range");

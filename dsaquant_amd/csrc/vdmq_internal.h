@@ -118,6 +118,11 @@ int launch_attention(const AttentionArgs &args, hipStream_t stream);
 // table == nullptr: no rotation
 int launch_norm_rope(const __half *const *x, const int64_t *ldx, const __half *const *w, __half *const *out, int matrices, int64_t rows, int64_t K,
                      float eps, const float *table, int64_t head_dim, int64_t positions, hipStream_t stream);
+// the parts of an RMS-norm around its row means; a modulation behind an fp32 LayerNorm
+int launch_row_squares(const __half *const *x, const int64_t *ldx, float *const *out, int matrices, int64_t rows, int64_t K, hipStream_t s);
+int launch_scale_rows(const __half *const *x, const int64_t *ldx, const float *const *r, const __half *const *w, void *const *out, bool out_f32, int matrices,
+                      int64_t rows, int64_t K, hipStream_t s);
+int launch_modulate_rows(const float *y, const __half *a, const __half *b, __half *out, int64_t rows, int64_t K, hipStream_t s);
 int launch_rope_table(float *table, int64_t head_dim, int64_t f, int64_t h, int64_t w, hipStream_t stream);
 int launch_timestep_embedding(const double *t, __half *out, int64_t batch, int64_t half, hipStream_t stream);
 

@@ -611,8 +611,9 @@ bool resident_takes(const ResidentProblem &p) {
         // (vdmq_bf6_ksplit.hip; as calls 0.77 ... 0.83 of that one's time on 320 shapes).  On 2300 shapes of 2.5 ... 400 million outputs, each
         // timed with one set of buffers and with rows and weights of its own in every call, the choice takes 1.0035 of the faster
         // form's time in the geometric mean, over 1.06 at 2.3 % (always one kernel 1.0061 and 4.4 %, always two 1.20).
-        // Two kernels are never faster than the host that launches them, 16 us, with gate and residual 20.5 (one: 11.5 and 15.5): without
-        // that 1166 x 1472 -> 3200 with a residual went to two at 20.7 us against 15.5, 230 x 1536 -> 14848 at 17 against 13.4.  Up to 2.5
+        // Two kernels count as never faster than 16 us, with gate and residual 20.5, which the host took for them when the line was drawn.  It
+        // takes 11.5 now (one: 8.2), and the two forms are within 8 % of each other where that matters: 1166 x 1472 -> 3200 with a
+        // residual 15.5 us as one kernel and 14.5 as two, 230 x 1536 -> 14848 with it 13.6 and 13.5, without 13.4 and 12.6.  Up to 2.5
         // million outputs the estimates always say one kernel (2.8 million is the least where they do not), and the call waits for the
         // host, whom they cost 0.2 us each time.
         if (p.K < 1280 || p.N <= 384 || p.M * p.N <= 2500000 || ksplit_takes(p.M, p.N, p.K, p.out_dtype) || p.M * p.N > (int64_t(1) << 40)) return true;

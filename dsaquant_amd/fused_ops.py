@@ -368,6 +368,43 @@ def rms_norm_rope(xs, weights, eps: float, freqs: Optional[torch.Tensor], heads:
     return outs
 
 
+def rms_norm_exact(xs, weights, eps: float, floats: bool = False):
+    """The RMS-norm of one or two [B, L, K] fp16 tensors with the bits of ``(xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) +
+    eps)).half() * weight``, xf = x.float(): the row means stay torch's, whose order of summation they have, and the passes
+    around them are two kernels.  ``floats``: the same values as fp32, what a rotary embedding converts them to."""
+    lib = _k._load_ext()
+    B, L, K = xs[0].shape
+    dev = xs[0].device
+    with _k._on(dev):
+        stream, two = _k._stream(dev), len(xs) == 2
+        squares = [torch.empty((B, L, K), dtype=torch.float32, device=dev) for _ in xs]
+        args = [a for x, s in zip(xs, squares) for a in (x.data_ptr(), x.stride(1), s.data_ptr())]
+        _lib.check(lib.vdmq_row_squares_f32(*args, *(() if two else (None, 0, None)), B * L, K, stream))
+        r = [torch.rsqrt(s.mean(dim=-1, keepdim=True) + eps) for s in squares]
+        outs = squares if floats else [torch.empty((B, L, K), dtype=torch.float16, device=dev) for _ in xs]  # (the squares have been read)
+        args = [a for x, t, w, o in zip(xs, r, weights, outs) for a in (x.data_ptr(), x.stride(1), t.data_ptr(), w.data_ptr(), o.data_ptr())]
+        _lib.check(lib.vdmq_scale_rows(*args, *(() if two else (None, 0, None, None, None)), int(floats), B * L, K, stream))
+    return outs
+
+
+def modulate_supported(y: torch.Tensor, a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Whether ``modulate`` takes these operands."""
+    grad = torch.is_grad_enabled()
+    return (y.is_cuda and y.dtype == torch.float32 and y.is_contiguous() and y.dim() == 3 and y.shape[2] % 8 == 0 and y.numel() > 0 and y.data_ptr() % 16 == 0
+            and not (grad and y.requires_grad)
+            and all(t.dtype == torch.float16 and t.device == y.device and t.numel() == y.shape[2] and t.is_contiguous() and t.data_ptr() % 16 == 0
+                    and not (grad and t.requires_grad) for t in (a, b)))
+
+
+def modulate(y: torch.Tensor, a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
+    """``y.half() * (1 + a) + b`` for an fp32 [B, L, K] and one fp16 vector of K each, the same bits in one pass."""
+    lib = _k._load_ext()
+    with _k._on(y.device):
+        out = torch.empty(y.shape, dtype=torch.float16, device=y.device)
+        _lib.check(lib.vdmq_modulate_rows_f16(y.data_ptr(), a.data_ptr(), b.data_ptr(), out.data_ptr(), y.shape[0] * y.shape[1], y.shape[2], _k._stream(y.device)))
+    return out
+
+
 def rope_table(head_dim: int, f: int, h: int, w: int, device) -> torch.Tensor:
     """The complex64 [f * h * w, 1, head_dim / 2] table of rotations, computed on the GPU in double precision."""
     lib = _k._load_ext()

@@ -106,10 +106,11 @@ def timestep_embedding(freq_dim: int, timestep: torch.Tensor) -> torch.Tensor:
     return torch.cat([torch.cos(ang), torch.sin(ang)], dim=1)
 
 
-def apply_rope(x: torch.Tensor, freqs: torch.Tensor) -> torch.Tensor:
-    """x [B, L, H, D]; consecutive channel pairs are rotated (fp32 complex arithmetic)."""
+def apply_rope(x: torch.Tensor, freqs: torch.Tensor, dtype: Optional[torch.dtype] = None) -> torch.Tensor:
+    """x [B, L, H, D]; consecutive channel pairs are rotated (fp32 complex arithmetic).  ``dtype``: what x's values are of, where
+    x is a conversion of them to fp32."""
     xc = torch.view_as_complex(x.float().reshape(*x.shape[:-1], -1, 2))
-    return torch.view_as_real(xc * freqs).flatten(3).to(x.dtype)
+    return torch.view_as_real(xc * freqs).flatten(3).to(dtype or x.dtype)
 
 
 class SharedContext:
@@ -239,11 +240,13 @@ class Attention(nn.Module):
             if context is None and self._kernel_norm((q, k), (self.norm_q, self.norm_k), freqs):
                 q, k = fused_ops.rms_norm_rope((q, k), (self.norm_q.weight, self.norm_k.weight), self.norm_q.eps, freqs, self.heads)
                 freqs = None  # (the rotation is in it)
+            elif context is None and self._exact_norm((q, k), (self.norm_q, self.norm_k)):
+                q, k = fused_ops.rms_norm_exact((q, k), (self.norm_q.weight, self.norm_k.weight), self.norm_q.eps, floats=freqs is not None)
             else:
                 q, k = self._normed(q, self.norm_q), self._normed(k, self.norm_k)
         q, k, v = (t.unflatten(2, (self.heads, -1)) for t in (q, k, v))
         if freqs is not None:
-            q, k = apply_rope(q, freqs), apply_rope(k, freqs)
+            q, k = apply_rope(q, freqs, v.dtype), apply_rope(k, freqs, v.dtype)
         if timers is not None:
             timers.start("attention")
         if self._on_kernels() and fused_ops.attention_supported(q, k, v):
@@ -255,8 +258,18 @@ class Attention(nn.Module):
             timers.stop("attention")
         return _project_and_update(self.to_out[0], o, None, residual, gate)
 
+    def _projected_on_kernels(self) -> bool:
+        return all(getattr(layer, "use_vdm_kernel", False) for layer in (self.to_q, self.to_k, self.to_v))
+
     def _on_kernels(self) -> bool:
-        return self.fuse_attention and all(getattr(layer, "use_vdm_kernel", False) for layer in (self.to_q, self.to_k, self.to_v))
+        return self.fuse_attention and self._projected_on_kernels()
+
+    # the norm's passes around its row means on the library's kernels: the tensor operations' bits, so nothing asks for it
+    def _exact_norm(self, tensors, norms) -> bool:
+        from . import fused_ops
+
+        return (self._projected_on_kernels() and all(_is_plain_norm(n) and n.eps == norms[0].eps for n in norms)
+                and fused_ops.rms_norm_rope_supported(tensors, [n.weight for n in norms], None, self.heads))
 
     def _kernel_norm(self, tensors, norms, freqs) -> bool:
         from . import fused_ops
@@ -269,6 +282,8 @@ class Attention(nn.Module):
 
         if self._kernel_norm((x,), (norm,), None):
             return fused_ops.rms_norm_rope((x,), (norm.weight,), norm.eps, None, self.heads)[0]
+        if self._exact_norm((x,), (norm,)):
+            return fused_ops.rms_norm_exact((x,), (norm.weight,), norm.eps)[0]
         return norm(x)
 
 
@@ -383,6 +398,16 @@ class WanDiT(nn.Module):
     # The last LayerNorm and its modulation in one kernel, the one of the blocks' ``fuse_ln`` (last bits as there).
     fuse_head = False
 
+    def _head_norm(self, x, scale, shift):
+        if self._kernel_mode() and _plain_fp16(x):
+            from . import fused_ops
+
+            y = F.layer_norm(x.float(), (x.shape[-1],), None, None, self.args.eps)
+            if fused_ops.modulate_supported(y, scale, shift):  # (the same bits as below, in one pass over y instead of three)
+                return fused_ops.modulate(y, scale, shift)
+            return y.to(x.dtype) * (1 + scale) + shift
+        return fp32_layer_norm(x, None, None, self.args.eps) * (1 + scale) + shift
+
     # The blocks run on the W4A4 kernels: the tables in front of them may be made on the GPU by the library, the same values.
     def _kernel_mode(self) -> bool:
         return len(self.blocks) > 0 and getattr(self.blocks[0].ffn.up, "use_vdm_kernel", False)
@@ -425,7 +450,7 @@ class WanDiT(nn.Module):
 
             x = LnInput(x, scale, shift, a.eps, "modulate").materialize()
         else:
-            x = fp32_layer_norm(x, None, None, a.eps) * (1 + scale.unsqueeze(1)) + shift.unsqueeze(1)
+            x = self._head_norm(x, scale.unsqueeze(1), shift.unsqueeze(1))
         return self.unpatchify(self.proj_out(x), f, h, w)
 
 

@@ -354,7 +354,20 @@ int vdmq_rms_norm_rope_f16(const void *x0, int64_t ldx0, const void *w0, void *o
                            void *out1, int64_t rows, int64_t K, float eps, const void *table, int64_t head_dim, int64_t positions,
                            vdmq_stream_t stream);
 
-/* That table for an f x h x w grid of positions, computed in double (modules/embedding.py:114-157):
+/* The parts of an RMS-norm around its row means, for a host that takes those itself: vdmq_row_squares_f32 writes the fp32
+ * squares of fp16 rows (exact), vdmq_scale_rows writes y = fp16(fp16(x * r) * w), r fp32 [rows], w fp16 [K], as fp16 or, with
+ * out_f32, as floats of the same values; every operation rounded once, as the tensor operations are (modules/
+ * attention.py:149-163).  One or two matrices of the same size (x1 NULL: one) in one launch; outputs are contiguous. */
+int vdmq_row_squares_f32(const void *x0, int64_t ldx0, void *out0, const void *x1, int64_t ldx1, void *out1, int64_t rows, int64_t K,
+                         vdmq_stream_t stream);
+int vdmq_scale_rows(const void *x0, int64_t ldx0, const void *r0, const void *w0, void *out0, const void *x1, int64_t ldx1, const void *r1,
+                    const void *w1, void *out1, int out_f32, int64_t rows, int64_t K, vdmq_stream_t stream);
+
+/* out = fp16(fp16(fp16(y) * (1 + a)) + b), each operation rounded once, for fp32 rows y (contiguous, K % 8 == 0) and one fp16 vector
+ * a and b [K] for all rows: a modulation behind an fp32 LayerNorm (modules/dit_block.py:100). */
+int vdmq_modulate_rows_f16(const void *y, const void *a, const void *b, void *out, int64_t rows, int64_t K, vdmq_stream_t stream);
+
+/* The table of rotations for an f x h x w grid of positions, computed in double (modules/embedding.py:114-157):
  * [f * h * w][(head_dim - 2 * (head_dim / 3)) / 2 + 2 * (head_dim / 3 / 2)] (cos, sin) pairs. */
 int vdmq_rope_table(void *table, int64_t head_dim, int64_t f, int64_t h, int64_t w, vdmq_stream_t stream);
 

@@ -299,3 +299,70 @@ def test_harness_calls_norms_that_carry_hooks(hook):
         if handle is not None:
             handle.remove()
     assert attn.norm_k in seen
+
+
+def _same_bits(a, b):
+    assert a.shape == b.shape and a.dtype == b.dtype and a.is_contiguous() == b.is_contiguous()
+    assert torch.equal(torch.isnan(a), torch.isnan(b))
+    zero = torch.zeros((), dtype=a.dtype, device=a.device)
+    ints = torch.int16 if a.dtype == torch.float16 else torch.int32
+    assert torch.equal(torch.where(torch.isnan(a), zero, a).view(ints), torch.where(torch.isnan(b), zero, b).view(ints))
+
+
+# one piece of eight, rows that fill no workgroup, more rows than one; row strides beyond the row
+@pytest.mark.parametrize("B,L,K,pad", [(1, 1, 8, 0), (1, 7, 1536, 0), (2, 33, 5120, 0), (1, 513, 4104, 64), (1, 4680, 1536, 3072)])
+def test_norm_around_its_means_has_the_bits_of_the_tensor_operations(B, L, K, pad):
+    from dsaquant_amd import fused_ops as f
+    from dsaquant_amd import wan_harness as W
+
+    g = torch.Generator(device=DEV).manual_seed(B + L + K)
+    xs = [torch.randn((B, L, K + pad), generator=g, device=DEV).half()[..., :K] for _ in range(2)]
+    for x in xs:  # subnormals, zeros, an overflowing square's row, infinities, a NaN
+        x[:, ::5] *= 1e-6
+        x[0, 0, :4] = torch.tensor([0.0, -0.0, 6e-8, 65504.0], device=DEV).half()
+        if L > 6:
+            x[0, 2] = 65504.0
+            x[0, 3, 1], x[0, 4, 2], x[0, 5] = float("inf"), float("nan"), 0.0
+    norms = [W.RMSNormAcrossHeads(K, 1e-6).half().to(DEV) for _ in xs]
+    with torch.no_grad():
+        for n in norms:
+            n.weight.copy_(torch.randn(K, generator=g, device=DEV))
+            n.weight[:2] = torch.tensor([6e-8, 0.0], device=DEV)
+        assert f.rms_norm_rope_supported(xs, [n.weight for n in norms], None, 1)
+        want = [n(x) for n, x in zip(norms, xs)]
+        weights = [n.weight for n in norms]
+        for got, w in zip(f.rms_norm_exact(xs, weights, 1e-6), want):
+            _same_bits(got, w)
+        for got, w in zip(f.rms_norm_exact(xs, weights, 1e-6, floats=True), want):
+            _same_bits(got, w.float())
+        _same_bits(f.rms_norm_exact(xs[1:], weights[1:], 1e-6)[0], want[1])
+        a, b = (torch.randn((1, 1, K), generator=g, device=DEV).half() for _ in range(2))
+        y = torch.randn((B, L, K), generator=g, device=DEV) * 10
+        y[0, 0, :3] = torch.tensor([1e6, float("nan"), 1e-7], device=DEV)
+        assert f.modulate_supported(y, a, b) and not f.modulate_supported(y.half(), a, b)
+        _same_bits(f.modulate(y, a, b), y.half() * (1 + a) + b)
+
+
+@pytest.mark.parametrize("frames,h,w", [(1, 6, 10), (2, 10, 14), (3, 34, 50)])
+def test_harness_forward_keeps_its_bits_on_the_norm_kernels(monkeypatch, frames, h, w):
+    from dataclasses import replace
+
+    from dsaquant_amd import fused_ops
+    from dsaquant_amd import wan_harness as W
+
+    args = replace(W.WAN21_1P3B, num_layers=2, num_heads=2, ffn_dim=512, text_dim=128)
+    model = W.build_quantized(args, DEV, seed=12)
+    g = torch.Generator(device=DEV).manual_seed(13)
+    latent = torch.randn((1, 16, frames, h, w), generator=g, device=DEV).half()
+    ctx, t = torch.randn((1, 77, args.text_dim), generator=g, device=DEV).half(), torch.tensor([500.0], device=DEV)
+    calls = []
+    for name in ("rms_norm_exact", "modulate"):
+        kernel = getattr(fused_ops, name)
+        monkeypatch.setattr(fused_ops, name, lambda *a, kernel=kernel, name=name, **k: (calls.append(name), kernel(*a, **k))[1])
+    with torch.no_grad():
+        got = model(latent, t, ctx)
+        assert calls == ["rms_norm_exact"] * 6 + ["modulate"]  # per block: q and k, then q, then k of the context
+        monkeypatch.setattr(fused_ops, "rms_norm_rope_supported", lambda *a: False)
+        monkeypatch.setattr(fused_ops, "modulate_supported", lambda *a: False)
+        want = model(latent, t, ctx)
+    assert len(calls) == 7 and torch.equal(got, want)
