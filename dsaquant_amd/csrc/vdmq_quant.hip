@@ -484,27 +484,33 @@ __global__ __launch_bounds__(256) void quantize_given_scale_kernel(const __half 
 }
 
 // Weights [N, K] into the checkpoint's v1 buffers (pack_weight_with_scale, quantize_weight_per_channel) in one pass: a
-// workgroup owns one 16-row tile of the v1 order (vdmq_layout.hip), a wave per row, the row in registers (NCH chunks of
-// 512; 0: rows too long for that are read twice, the second time mostly from the caches).  The scale is the given one
-// or absmax / 7; 2048 k at a time the rows' words meet in LDS and leave as the tile's 512-byte runs.  `native`
-// (optional) takes the row-major int4 form as well.  HBM-bound: 2.5 bytes per weight.  As four kernels -- row scale,
-// quantize, relayout, scale replication: two reads of the weights and two more of the nibbles -- a 13824 x 5120 weight
-// took 84 us; here 37 (29 at the 6.3 TB/s of the copy kernel).
-constexpr int kTileRows = 16, kPackWords = 256 /* words of a row per 2048 k */, kPackRowWords = kPackWords + 4 /* bank spread */;
+// workgroup owns a quarter of a 16-row tile of the v1 order (vdmq_layout.hip), rows 2p, 2p + 1, 2p + 8 and 2p + 9, whose words
+// share the order's 16-byte pieces; a wave per row, the row in registers (NCH chunks of 512; 0: rows too long for that are
+// read twice, the second time mostly from the caches).  The scale is the given one or absmax / 7; 2048 k at a time the
+// rows' words meet in LDS and leave as 128-byte runs.  `native` (optional) takes the row-major int4 form as well.
+// Bound by memory, 2.5 bytes per weight, where loads and conversions overlap: the rows of a workgroup arrive together and are
+// then converted together, so the fewer rows it has, the earlier the first is at work while the next load.  us for a whole tile /
+// half / a quarter / an eighth of one per workgroup (16, 8, 4, 2 waves; sixteen leave long rows half the registers, too): 13824 x 5120
+// 38.0 / 34.1 / 32.6 / 33.7, 5120 x 13824 61.7 / 49.0 / 36.7 / 37.6, 3072 x 14336 51 / 32.4 / 24.1 / 24.5, 13824 x 13824 159 / 119 / 90 / 93,
+// 1536 x 1536 5.2 / 4.6 / 4.6 / 4.6 (6.3 TB/s: 28, 28, 18, 76 and 1).
+constexpr int kTileRows = 16, kPackRows = 4, kPackParts = kTileRows / kPackRows, kPackWords = 256 /* words of a row per 2048 k */, kPackRowWords = kPackWords + 4 /* bank spread */;
+// waves a SIMD holds, which is what bounds the registers: the row's 4 * NCH and some 40 more
+constexpr int pack_waves(int nch) { return nch <= 6 ? 8 : nch <= 10 ? 6 : nch <= 18 ? 4 : nch <= 28 ? 3 : 2; }
 
 template <int NCH>
-__global__ __launch_bounds__(kTileRows * kWaveSize, NCH <= 10 ? 8 : 4) void pack_weight_kernel(const __half *__restrict__ w, const __half *__restrict__ scale_in,
-                                                                            int tiles, int K, int Kp, u32x4 *__restrict__ q_v1,
-                                                                            u32x4 *__restrict__ scales_v1, __half *__restrict__ scale_out,
+__global__ __launch_bounds__(kPackRows * kWaveSize, pack_waves(NCH)) void pack_weight_kernel(const __half *__restrict__ w, const __half *__restrict__ scale_in,
+                                                                            int units, int K, int Kp, u32x4 *__restrict__ q_v1,
+                                                                            u32x2 *__restrict__ scales_v1, __half *__restrict__ scale_out,
                                                                             uint32_t *__restrict__ native) {
-    __shared__ __attribute__((aligned(16))) uint32_t words[2][kTileRows][kPackRowWords];
-    __shared__ unsigned short scales[kTileRows];
-    // the eight tiles of a 128-row block interleave in memory: they go to one XCD, one after the other, whose L2 joins
+    __shared__ __attribute__((aligned(16))) uint32_t words[2][kPackRows][kPackRowWords];
+    __shared__ unsigned short scales[kPackRows];
+    // the 32 quarters of a 128-row block interleave in memory: they go to one XCD, one after the other, whose L2 joins
     // their runs (blocks are dealt to the XCDs in turn)
-    int tile = blockIdx.x;
-    if ((tile | 63) < tiles) tile = (tile & ~63) | (tile & 7) << 3 | (tile >> 3 & 7);
+    int unit = blockIdx.x;
+    if ((unit | 255) < units) unit = (unit & ~255) | (unit & 7) << 5 | (unit >> 3 & 31);
+    const int tile = unit / kPackParts, part = unit % kPackParts;
     const int lane = threadIdx.x & (kWaveSize - 1), wave = threadIdx.x >> 6;
-    const int64_t row = static_cast<int64_t>(tile) * kTileRows + wave;
+    const int64_t row = static_cast<int64_t>(tile) * kTileRows + 2 * part + (wave & 1) + 8 * (wave >> 1);
     const u32x4 *src = reinterpret_cast<const u32x4 *>(w + row * K);
     auto load = [&](int c) { return c * 512 + lane * 8 < K ? __builtin_nontemporal_load(src + c * 64 + lane) : u32x4{0u, 0u, 0u, 0u}; };
     u32x4 v[NCH > 0 ? NCH : 1];
@@ -544,7 +550,7 @@ __global__ __launch_bounds__(kTileRows * kWaveSize, NCH <= 10 ? 8 : 4) void pack
 
     const int KG = K / 64;
     const int64_t tile_base = static_cast<int64_t>(tile >> 3) * KG * 8 + (tile & 7); /* in 512-byte runs: + 8 per 64 k */
-    const int g8 = threadIdx.x & 31, row_lo = g8 >> 2, t4 = g8 & 3;
+    const int piece = threadIdx.x & 7, row_lo = piece >> 2, t4 = piece & 3, k64 = threadIdx.x >> 3;
     auto group = [&](int g, auto &&chunk) __attribute__((always_inline)) {
         const int copy = g & 1;
 #pragma unroll
@@ -556,10 +562,10 @@ __global__ __launch_bounds__(kTileRows * kWaveSize, NCH <= 10 ? 8 : 4) void pack
             if (native != nullptr && k0 < Kp) native[row * (Kp / 8) + k0 / 8] = word;
         }
         __syncthreads(); /* one per group: the copy written next was read before the barrier in front of this one */
-        const int bk = 32 * g + (threadIdx.x >> 5);
+        const int bk = 32 * g + k64;
         if (bk < KG) {
-            const uint32_t *lo = words[copy][row_lo] + (threadIdx.x >> 5) * 8 + t4, *hi = lo + 8 * kPackRowWords;
-            q_v1[(tile_base + 8ll * bk) * 32 + g8] = u32x4{lo[0], lo[4], hi[0], hi[4]};
+            const uint32_t *lo = words[copy][row_lo] + k64 * 8 + t4, *hi = lo + 2 * kPackRowWords;
+            q_v1[(tile_base + 8ll * bk) * 32 + 8 * part + piece] = u32x4{lo[0], lo[4], hi[0], hi[4]};
         }
     };
     if constexpr (NCH > 0) {
@@ -568,16 +574,10 @@ __global__ __launch_bounds__(kTileRows * kWaveSize, NCH <= 10 ? 8 : 4) void pack
     } else {
         for (int g = 0; g < (chunks + 3) / 4; ++g) group(g, load);
     }
-    // the tile's sixteen scales per 64 k, 32 bytes in the order of pack_wscales: row r at 4 * (r % 8 / 2) + 2 * (r / 8) + r % 2
-    for (int i = threadIdx.x; i < 2 * KG; i += kTileRows * kWaveSize) {
-        uint32_t o[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int r = (e & 1) * 8 + 2 * (e >> 1) + 4 * (i & 1);
-            o[e] = scales[r] | static_cast<uint32_t>(scales[r + 1]) << 16;
-        }
-        scales_v1[(static_cast<int64_t>(tile >> 3) * KG + (i >> 1)) * 16 + (tile & 7) * 2 + (i & 1)] = u32x4{o[0], o[1], o[2], o[3]};
-    }
+    // the tile's sixteen scales per 64 k, 32 bytes in the order of pack_wscales: row r at 4 * (r % 8 / 2) + 2 * (r / 8) + r % 2; this
+    // quarter's four are adjacent
+    const u32x2 four = {scales[0] | static_cast<uint32_t>(scales[1]) << 16, scales[2] | static_cast<uint32_t>(scales[3]) << 16};
+    for (int i = threadIdx.x; i < KG; i += kPackRows * kWaveSize) scales_v1[(static_cast<int64_t>(tile >> 3) * KG + i) * 32 + (tile & 7) * 4 + part] = four;
 }
 
 constexpr int64_t kStreamOutBytes = int64_t(224) << 20; /* outputs larger than this bypass the caches */
@@ -736,15 +736,17 @@ int launch_row_scale(const __half *x, int64_t rows, int64_t K, float clip, __hal
 int launch_pack_weight(const __half *w, const __half *scale_in, int64_t N, int64_t K, uint8_t *q_v1, __half *scales_v1, __half *scale_out,
                        uint8_t *native, hipStream_t s) {
     if (N == 0) return VDMQ_OK;
-    const int tiles = static_cast<int>(N / kTileRows);
     const int64_t nch = ceil_div(k_padded(K), 512);
-    using Kernel = void (*)(const __half *, const __half *, int, int, int, u32x4 *, u32x4 *, __half *, uint32_t *);
-    // (18 chunks are what the 128 registers of a sixteen-wave workgroup hold beside the work, 10 -- with four of the 64
-    // registers spilled to 12 bytes of scratch per lane -- what two of them per CU do)
-    const Kernel kernel = nch <= 2 ? pack_weight_kernel<2> : nch <= 4 ? pack_weight_kernel<4> : nch <= 6 ? pack_weight_kernel<6> :
-                          nch <= 10 ? pack_weight_kernel<10> : nch <= 18 ? pack_weight_kernel<18> : pack_weight_kernel<0>;
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(tiles)), dim3(kTileRows * kWaveSize), 0, s, w, scale_in, tiles, static_cast<int>(K),
-                       static_cast<int>(k_padded(K)), reinterpret_cast<u32x4 *>(q_v1), reinterpret_cast<u32x4 *>(scales_v1), scale_out,
+    using Kernel = void (*)(const __half *, const __half *, int, int, int, u32x4 *, u32x2 *, __half *, uint32_t *);
+    // (a chunk that a row does not have is still loaded, converted and staged as zeros: 4608 x 4096 on 10 chunks 13.3 us, on 8
+    // 12.3; 2048 x 16384 read twice 43, on 32 20.9)
+    const Kernel kernel = nch <= 2 ? pack_weight_kernel<2> : nch <= 3 ? pack_weight_kernel<3> : nch <= 4 ? pack_weight_kernel<4> :
+                          nch <= 6 ? pack_weight_kernel<6> : nch <= 8 ? pack_weight_kernel<8> : nch <= 10 ? pack_weight_kernel<10> :
+                          nch <= 14 ? pack_weight_kernel<14> : nch <= 18 ? pack_weight_kernel<18> : nch <= 24 ? pack_weight_kernel<24> :
+                          nch <= 28 ? pack_weight_kernel<28> : nch <= 32 ? pack_weight_kernel<32> : pack_weight_kernel<0>;
+    const int units = static_cast<int>(N / kPackRows);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(units)), dim3(kPackRows * kWaveSize), 0, s, w, scale_in, units, static_cast<int>(K),
+                       static_cast<int>(k_padded(K)), reinterpret_cast<u32x4 *>(q_v1), reinterpret_cast<u32x2 *>(scales_v1), scale_out,
                        reinterpret_cast<uint32_t *>(native));
     return check_launch("pack_weight_kernel");
 }

@@ -190,7 +190,9 @@ def test_layer_norm_sums_in_its_defined_order(K, mode):
     assert np.array_equal(rows_of_blocks(blocks, len(x), K), want_q.astype(np.float64))
 
 
-@pytest.mark.parametrize("N,K", [(128, 64), (128, 1088), (1152, 448), (640, 2112), (256, 5120 + 64), (128, 9216), (128, 9216 + 64), (1024 + 128, 13824)])
+@pytest.mark.parametrize("N,K", [(128, 64), (128, 1088), (1152, 448), (640, 2112), (256, 5120 + 64), (128, 9216), (128, 9216 + 64), (1024 + 128, 13824),
+                                 (128, 1536), (128, 1600), (128, 4096), (128, 4160), (128, 7168), (128, 7232), (128, 12288), (128, 12352),
+                                 (128, 14336), (128, 14400), (2048, 16384), (128, 16448)])
 def test_pack_weight_edges(N, K):
     """One-pass weight packing: row tiles beyond and within a full group of eight 128-row blocks, rows on both sides of
     every register form and the two-pass one, rows with NaN / Inf, zero rows and scales of zero, negative and Inf; the
