@@ -146,14 +146,21 @@ __device__ __forceinline__ void quantize_held_row(const u32x4 (&v)[NCH], int lan
 // stay below 8.5, above -8.5 and t below 7.5; rows whose largest |t| is below 7.5 (a clip ratio above 0.934)
 // skip the clamp, all others (NaN, Inf, a scale of zero, a small clip ratio) take it.  Rows of the last row-block beyond
 // M stay unwritten (the GEMM never stores them); K is padded to 128 with zeros.
-constexpr int kBf6Rows = 8;          /* rows (= waves) per workgroup of the bf6 quantizers */
+constexpr int kPanelRows = 8;        /* rows of a panel of the bf6 blocks */
 constexpr int kStringsPerGroup = 64; /* 2048 k = 64 strings of 32 k per row and group */
 constexpr int kStringBytes = 24;
 // 16 bytes of padding per row: sixteen lanes that read 8 bytes each of eight rows and two strings meet 32 banks
 constexpr int kStringRowBytes = kStringsPerGroup * kStringBytes + 16;
 
+// A workgroup owns ROWS rows, one per wave: a panel or half of one (bf6_split says which).  The halves of a panel go to one
+// XCD, one after the other, whose L2 joins their runs (blocks are dealt to the XCDs in turn): the b-th of `groups` groups of rows.
+template <int ROWS>
+__device__ __forceinline__ int bf6_group(int b, int groups) {
+    return ROWS == kPanelRows || (b | 15) >= groups ? b : (b & ~15) | (b & 7) << 1 | (b >> 3 & 1);
+}
+template <int ROWS>
 struct Bf6Scratch { /* LDS of one workgroup: the strings of one group; two copies in turn: one barrier per group is enough */
-    uint8_t strings[2][kBf6Rows][kStringRowBytes];
+    uint8_t strings[2][ROWS][kStringRowBytes];
 };
 
 // `valid`: the wave's row exists (a workgroup's waves all run this function -- it synchronises them --
@@ -183,10 +190,10 @@ constexpr bool bf6_late_act(int nch) { return nch >= 17; }
 struct NoRefill {
     __device__ __forceinline__ void operator()(int) const {}
 };
-template <int NCH, int ACT, class Refill>
+template <int NCH, int ACT, int ROWS, class Refill>
 __device__ __forceinline__ void quantize_held_row_bf6(u32x4 (&v)[NCH], int lane, int wave, int64_t row0, bool valid, int M, int Kb,
                                                       float clip, uint8_t *__restrict__ blocks, __half *__restrict__ scale_h,
-                                                      bool stream_out, Bf6Scratch &lds, int &phase, Refill &&refill) {
+                                                      bool stream_out, Bf6Scratch<ROWS> &lds, int &phase, Refill &&refill) {
     // `late`: the activation is evaluated chunk by chunk below, in front of the conversion (see gelu_row_absmax)
     uint32_t m16 = 0;
     const bool late = ACT == VDMQ_ACT_GELU_TANH && gelu_row_absmax<NCH>(v, m16);
@@ -227,7 +234,7 @@ __device__ __forceinline__ void quantize_held_row_bf6(u32x4 (&v)[NCH], int lane,
     const uint32_t string0 = (lane >> 2) * kStringBytes + (lane & 3) * 6, off32 = string0 + (odd ? 2 : 0), off16 = string0 + (odd ? 0 : 4);
     // the thread's share of the cooperative store: string t / 8 of row t % 8 -- eight consecutive
     // threads write the eight rows' parts of one string slot, 128 (and 64) contiguous bytes
-    const int t = wave * kWaveSize + lane, srow = t % kBf6Rows, sidx = t / kBf6Rows;
+    const int t = wave * kWaveSize + lane, srow = t % ROWS, sidx = t / ROWS;
     const int64_t grow = row0 + srow;
     constexpr int NG = (NCH + 3) / 4;
 #pragma unroll
@@ -315,21 +322,20 @@ __device__ __forceinline__ void quantize_held_row_bf6(u32x4 (&v)[NCH], int lane,
 // number keeps the row addresses out of them there (32760 rows of 768 / 1024 / 2048 with the GELU 24.2 -> 22.8, 24.9 -> 24.3, 41.1 -> 38.8 us);
 // with longer rows it costs time (3072 with the GELU 49.4 -> 54.1).  (The fused LayerNorm's longest form spills: fewer registers so, 0.95 ...
 // 1.00 of the time for rows of 9216 ... 16384.)
-template <int NCH, bool STREAM_OUT, int ACT, int FMT>
-__global__ __launch_bounds__((FMT == 1 ? kBf6Rows : kRowsPerBlock) * kWaveSize, FMT == 1 && NCH <= 2 ? 8 : 1) void quantize_rows_kernel(
+template <int NCH, bool STREAM_OUT, int ACT, int FMT, int ROWS>
+__global__ __launch_bounds__(ROWS * kWaveSize, FMT == 1 && NCH <= 2 ? 8 : FMT == 1 ? 2 : 1) void quantize_rows_kernel(
     const __half *__restrict__ x, int64_t ldx, int M, int K, int Kp, float clip, uint8_t *__restrict__ qact,
-    __half *__restrict__ scale_h, int stream_bf6) {
-    constexpr int ROWS = FMT == 1 ? kBf6Rows : kRowsPerBlock;
+    __half *__restrict__ scale_h, int stream_out_bf6) {
     const int lane = threadIdx.x & (kWaveSize - 1), wave = FMT == 1 && NCH <= 4 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
     if constexpr (FMT == 1) {
         // The workgroup walks row groups blockIdx.x, blockIdx.x + gridDim.x, ...: with the launcher's grid
         // (what the chip holds at once) the loads of the next group's rows are in flight while this
         // group's rows are converted -- a long row leaves room for one workgroup per CU only, whose load and
         // convert phases would otherwise alternate.
-        __shared__ __attribute__((aligned(16))) Bf6Scratch scratch;
+        __shared__ __attribute__((aligned(16))) Bf6Scratch<ROWS> scratch;
         const int groups = (M + ROWS - 1) / ROWS;
         auto row_ptr = [&](int group) {
-            const int64_t r = static_cast<int64_t>(group) * ROWS + wave;
+            const int64_t r = static_cast<int64_t>(bf6_group<ROWS>(group, groups)) * ROWS + wave;
             return reinterpret_cast<const u32x4 *>(x + (r < M ? r : M - 1) * ldx); /* waves past M stay, on a copy of the last row */
         };
         auto load = [&](const u32x4 *src, int c) {
@@ -343,13 +349,13 @@ __global__ __launch_bounds__((FMT == 1 ? kBf6Rows : kRowsPerBlock) * kWaveSize, 
         for (; group < groups; group += gridDim.x) {
             const bool more = bf6_walks(NCH) && group + static_cast<int>(gridDim.x) < groups;
             const u32x4 *next = row_ptr(more ? group + gridDim.x : group);
-            const int64_t row0 = static_cast<int64_t>(group) * ROWS;
+            const int64_t row0 = static_cast<int64_t>(bf6_group<ROWS>(group, groups)) * ROWS;
             if (ACT != VDMQ_ACT_NONE && !bf6_late_act(NCH)) {
 #pragma unroll
                 for (int c = 0; c < NCH; ++c)
                     if (c * 512 + lane * 8 < K) v[c] = apply_act<ACT>(v[c]);
             }
-            quantize_held_row_bf6<NCH, bf6_late_act(NCH) ? ACT : VDMQ_ACT_NONE>(v, lane, wave, row0, row0 + wave < M, M, Kp, clip, qact, scale_h, stream_bf6 != 0, scratch, phase,
+            quantize_held_row_bf6<NCH, bf6_late_act(NCH) ? ACT : VDMQ_ACT_NONE, ROWS>(v, lane, wave, row0, row0 + wave < M, M, Kp, clip, qact, scale_h, stream_out_bf6 != 0, scratch, phase,
                                             [&](int c) {
                                                 if constexpr (bf6_walks(NCH))
                                                     if (more) v[c] = load(next, c);
@@ -391,15 +397,19 @@ constexpr int ln_full_chunks(int nch) {
 //                     fp32 with one rounding (FP32LayerNorm with elementwise_affine, norm2)
 // Row m takes vector row m / rows_per_vec of a and b (stride ldv elements): one
 // vector per batch element, or one per token.  EMIT_H writes h itself instead of
-// quantizing it (the same arithmetic: the checker's view of h).
+// quantizing it (the same arithmetic: the tests' view of h).
+// Bound by vector instructions and the reductions between them, so the bf6 form has four rows per workgroup, half a panel, whose halves L2
+// joins (so no streamed stores): one workgroup's reductions run under another's loads and conversions.  us, eight rows (streamed beyond 128 MiB)
+// / four: 512 x 5120 8.1 / 6.8, 4680 x 1536 8.5 / 7.9, 27280 x 3072 54 / 48, 32760 x 4096 92 / 77, 60000 x 5120 181 / 165, 20000 x 13824 222 / 207; 6000
+// rows of up to 3072 1.00; with the GEMM behind it 60000 x 3072 -> 3072 399 / 372, 75600 x 5120 -> 13824 2433 / 2392.
 template <int NCH, int LNMODE, bool EMIT_H, int FMT>
-__global__ __launch_bounds__((FMT == 1 ? kBf6Rows : kRowsPerBlock) * kWaveSize) void ln_quantize_rows_kernel(
+__global__ __launch_bounds__(kRowsPerBlock * kWaveSize, FMT == 1 ? 2 : 1) void ln_quantize_rows_kernel(
     const __half *__restrict__ x, int64_t ldx, int M, int K, int Kp, float eps, const __half *__restrict__ va,
     const __half *__restrict__ vb, int64_t ldv, int rows_per_vec, float clip, uint8_t *__restrict__ qact,
-    __half *__restrict__ scale_h, __half *__restrict__ h_out, int64_t ldh, int stream_bf6) {
-    constexpr int ROWS = FMT == 1 ? kBf6Rows : kRowsPerBlock;
+    __half *__restrict__ scale_h, __half *__restrict__ h_out, int64_t ldh) {
+    constexpr int ROWS = kRowsPerBlock;
     const int lane = threadIdx.x & (kWaveSize - 1), wave = FMT == 1 && NCH > 16 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
-    const int64_t row0 = static_cast<int64_t>(blockIdx.x) * ROWS;
+    const int64_t row0 = static_cast<int64_t>(FMT == 1 ? bf6_group<ROWS>(blockIdx.x, (M + ROWS - 1) / ROWS) : blockIdx.x) * ROWS;
     int64_t row = row0 + wave;
     const bool valid = row < M;
     if (!valid) {
@@ -425,9 +435,9 @@ __global__ __launch_bounds__((FMT == 1 ? kBf6Rows : kRowsPerBlock) * kWaveSize) 
         return;
     }
     if (FMT == 1) {
-        __shared__ __attribute__((aligned(16))) Bf6Scratch scratch;
+        __shared__ __attribute__((aligned(16))) Bf6Scratch<ROWS> scratch;
         int phase = 0;
-        quantize_held_row_bf6<NCH, VDMQ_ACT_NONE>(v, lane, wave, row0, valid, M, Kp, clip, qact, scale_h, stream_bf6 != 0, scratch, phase, NoRefill{});
+        quantize_held_row_bf6<NCH, VDMQ_ACT_NONE, ROWS>(v, lane, wave, row0, valid, M, Kp, clip, qact, scale_h, false, scratch, phase, NoRefill{});
     } else {
         quantize_held_row<NCH, false>(v, lane, row, Kp, clip, qact, scale_h);
     }
@@ -584,9 +594,8 @@ constexpr int64_t kStreamOutBytes = int64_t(224) << 20; /* outputs larger than t
 // The same for the bf6 blocks, judged by the quantizer and the GEMM that reads its output together: streamed stores
 // cost the GEMM the part of its operand that plain stores leave in the Infinity Cache (38 MB and 63 MB of blocks:
 // the pair 3 % and 2 % slower), and spare it the wait for the dirty lines of a large one (220 MB, 290 MB, 780 MB:
-// the pair 3 %, 0.7 % and 0.7 % faster).
-constexpr int64_t kStreamOutBytesBf6 = int64_t(128) << 20;
-int stream_bf6(int64_t M, int64_t K) { return bf6_bytes(M, K) > kStreamOutBytesBf6 ? 1 : 0; }
+// the pair 3 %, 0.7 % and 0.7 % faster).  For workgroups of a whole panel; halves of one never stream (bf6_split).
+constexpr int64_t kStreamOutBytesBf6 = int64_t(128) << 20, kInfinityCacheBytes = int64_t(256) << 20;
 
 // Workgroups of `kernel` the current device runs at once (CUs x workgroups per CU), or -1.  The answer is
 // kept per device in `cache` (one array per kernel, zero-initialised): the occupancy query costs tens of
@@ -606,25 +615,55 @@ int64_t resident_workgroups(const void *kernel, int threads, int (&cache)[kMaxDe
     return cache[dev];
 }
 
+// Rows per workgroup of the bf6 quantizer, and whether it streams its output.  The rows of a workgroup arrive together and are then
+// reduced and converted together: with four the next workgroup's loads run under that, few rows spread over twice as many CUs, and many leave a
+// smaller last wave of workgroups.  Against that stand half-panel runs of 64 and 32 bytes, which plain stores join in L2 and streamed ones do
+// not (75600 x 5120 streamed: 162 / 220 us with eight / four).  What computes more gains more.  us, eight / four:
+//   plain            512 x 5120 5.8 / 5.0   1000 x 13824 12.0 / 10.4   2500 x 8960 15.3 / 13.7   12000 x 8960 50.3 / 48.4
+//                    12000 x 3072 18.1 / 18.8   32760 x 1536 23.4 / 24.1
+//   GELU             512 x 5120 8.3 / 6.3   2500 x 10240 31.9 / 25.1   4680 x 8960 36.0 / 31.0   32760 x 1536 34.4 / 32
+//                    streamed / plain stores: 32760 x 8960 151 / 142, with its GEMM 384 / 366; 60000 x 7168 197 / 218, 32760 x 13824 240 / 272
+// Rows that are only quantized keep eight where there are many short ones.  With the activation evaluated late (bf6_late_act) four and plain stores
+// still win while the output stays in the memory-side cache.
+struct Bf6Split {
+    int rows, stream_out;
+};
+template <int NCH, int ACT>
+Bf6Split bf6_split(int64_t M, int64_t K) {
+    const int64_t bytes = bf6_bytes(M, K);
+    const bool large = bytes > kStreamOutBytesBf6;
+    const bool four = ACT == VDMQ_ACT_NONE ? !large && (M <= 5120 || K > 3584)
+                                           : !large || (bf6_late_act(NCH) && K <= 9216 && bytes <= kInfinityCacheBytes);
+    return four ? Bf6Split{kPanelRows / 2, 0} : Bf6Split{kPanelRows, large ? 1 : 0};
+}
+
+template <int NCH, int ACT, int ROWS>
+int launch_reg_bf6(const __half *x, int64_t M, int64_t K, int64_t ldx, float clip, uint8_t *qact, __half *scale_h, int stream_out, hipStream_t s) {
+    const int64_t groups = ceil_div(M, ROWS);
+    static int cache[kMaxDevices];
+    const int64_t resident = !bf6_walks(NCH) ? groups
+                                             : resident_workgroups(reinterpret_cast<const void *>(&quantize_rows_kernel<NCH, false, ACT, 1, ROWS>),
+                                                                   ROWS * kWaveSize, cache);
+    if (resident <= 0) return fail(VDMQ_ELAUNCH, "quantize_rows_kernel: the occupancy query for the current device failed");
+    hipLaunchKernelGGL((quantize_rows_kernel<NCH, false, ACT, 1, ROWS>), dim3(static_cast<unsigned>(groups < resident ? groups : resident)),
+                       dim3(ROWS * kWaveSize), ROWS == kPanelRows ? bf6_spare_lds(NCH, ACT) : 0, s, x, ldx, static_cast<int>(M),
+                       static_cast<int>(K), static_cast<int>(bf6_kblocks(K) * 64), clip, qact, scale_h, stream_out);
+    return check_launch("quantize_rows_kernel");
+}
+
 template <int NCH, int ACT>
 int launch_reg(const __half *x, int64_t M, int64_t K, int64_t ldx, float clip, int fmt, uint8_t *qact, __half *scale_h, hipStream_t s) {
-    const dim3 grid(static_cast<unsigned>(ceil_div(M, kRowsPerBlock))), block(kRowsPerBlock * kWaveSize);
     if (fmt == 1) {
-        const int64_t groups = ceil_div(M, kBf6Rows);
-        static int cache[kMaxDevices];
-        const int64_t resident = !bf6_walks(NCH) ? groups
-                                 : resident_workgroups(reinterpret_cast<const void *>(&quantize_rows_kernel<NCH, false, ACT, 1>),
-                                                       kBf6Rows * kWaveSize, cache);
-        if (resident <= 0) return fail(VDMQ_ELAUNCH, "quantize_rows_kernel: the occupancy query for the current device failed");
-        hipLaunchKernelGGL((quantize_rows_kernel<NCH, false, ACT, 1>), dim3(static_cast<unsigned>(!bf6_walks(NCH) || groups < resident ? groups : resident)),
-                           dim3(kBf6Rows * kWaveSize), bf6_spare_lds(NCH, ACT), s, x, ldx, static_cast<int>(M), static_cast<int>(K),
-                           static_cast<int>(bf6_kblocks(K) * 64), clip, qact, scale_h, stream_bf6(M, K));
+        const Bf6Split split = bf6_split<NCH, ACT>(M, K);
+        return split.rows == kPanelRows ? launch_reg_bf6<NCH, ACT, kPanelRows>(x, M, K, ldx, clip, qact, scale_h, split.stream_out, s)
+                                        : launch_reg_bf6<NCH, ACT, kPanelRows / 2>(x, M, K, ldx, clip, qact, scale_h, split.stream_out, s);
     }
-    else if (M * (k_padded(K) / 2) > kStreamOutBytes)
-        hipLaunchKernelGGL((quantize_rows_kernel<NCH, true, ACT, 0>), grid, block, 0, s, x, ldx, static_cast<int>(M), static_cast<int>(K),
+    const dim3 grid(static_cast<unsigned>(ceil_div(M, kRowsPerBlock))), block(kRowsPerBlock * kWaveSize);
+    if (M * (k_padded(K) / 2) > kStreamOutBytes)
+        hipLaunchKernelGGL((quantize_rows_kernel<NCH, true, ACT, 0, kRowsPerBlock>), grid, block, 0, s, x, ldx, static_cast<int>(M), static_cast<int>(K),
                            static_cast<int>(k_padded(K)), clip, qact, scale_h, 0);
     else
-        hipLaunchKernelGGL((quantize_rows_kernel<NCH, false, ACT, 0>), grid, block, 0, s, x, ldx, static_cast<int>(M), static_cast<int>(K),
+        hipLaunchKernelGGL((quantize_rows_kernel<NCH, false, ACT, 0, kRowsPerBlock>), grid, block, 0, s, x, ldx, static_cast<int>(M), static_cast<int>(K),
                            static_cast<int>(k_padded(K)), clip, qact, scale_h, 0);
     return check_launch("quantize_rows_kernel");
 }
@@ -664,15 +703,13 @@ int launch_ln_reg(const __half *x, int64_t M, int64_t K, int64_t ldx, float eps,
     const dim3 grid(static_cast<unsigned>(ceil_div(M, kRowsPerBlock))), block(kRowsPerBlock * kWaveSize);
     if (h_out != nullptr)
         hipLaunchKernelGGL((ln_quantize_rows_kernel<NCH, LNMODE, true, 0>), grid, block, 0, s, x, ldx, static_cast<int>(M), static_cast<int>(K),
-                           static_cast<int>(k_padded(K)), eps, va, vb, ldv, static_cast<int>(rows_per_vec), clip, qact, scale_h, h_out, ldh, 0);
-    else if (fmt == 1)
-        hipLaunchKernelGGL((ln_quantize_rows_kernel<NCH, LNMODE, false, 1>), dim3(static_cast<unsigned>(ceil_div(M, kBf6Rows))),
-                           dim3(kBf6Rows * kWaveSize), 0, s, x, ldx, static_cast<int>(M), static_cast<int>(K),
-                           static_cast<int>(bf6_kblocks(K) * 64), eps, va, vb, ldv, static_cast<int>(rows_per_vec), clip, qact, scale_h, h_out, ldh,
-                           stream_bf6(M, K));
+                           static_cast<int>(k_padded(K)), eps, va, vb, ldv, static_cast<int>(rows_per_vec), clip, qact, scale_h, h_out, ldh);
+    else if (fmt == 1) /* (four rows per workgroup, half a panel, and plain stores at any size: see ln_quantize_rows_kernel) */
+        hipLaunchKernelGGL((ln_quantize_rows_kernel<NCH, LNMODE, false, 1>), grid, block, 0, s, x, ldx, static_cast<int>(M), static_cast<int>(K),
+                           static_cast<int>(bf6_kblocks(K) * 64), eps, va, vb, ldv, static_cast<int>(rows_per_vec), clip, qact, scale_h, h_out, ldh);
     else
         hipLaunchKernelGGL((ln_quantize_rows_kernel<NCH, LNMODE, false, 0>), grid, block, 0, s, x, ldx, static_cast<int>(M), static_cast<int>(K),
-                           static_cast<int>(k_padded(K)), eps, va, vb, ldv, static_cast<int>(rows_per_vec), clip, qact, scale_h, h_out, ldh, 0);
+                           static_cast<int>(k_padded(K)), eps, va, vb, ldv, static_cast<int>(rows_per_vec), clip, qact, scale_h, h_out, ldh);
     return check_launch("ln_quantize_rows_kernel");
 }
 

@@ -85,6 +85,39 @@ def codes_of_blocks(blocks, rows, K):
     return torch.where(codes == 32, 0, codes)
 
 
+@pytest.mark.parametrize("M,K,producer", [(5121, 1536, None), (5121, 3584, None), (5123, 3648, None), (12999, 13824, None), (20001, 9216, None),
+                                          (5121, 1536, "gelu_tanh"), (20001, 9216, "gelu_tanh"), (20001, 9280, "gelu_tanh"), (40005, 8960, "gelu_tanh"),
+                                          (13, 1536, "modulate"), (35005, 5120, "modulate")])
+def test_whole_and_half_panel_workgroups(M, K, producer):
+    """A workgroup takes a panel of eight rows or half of one, by the number of rows, their length, the producer in front and the
+    size of the output: on both sides of those lines the rows' codes and scales are those of the same rows in slices of 2048, which
+    workgroups of four always serve (and which the other tests compare with the oracle)."""
+    from dsaquant_amd import fused_ops
+
+    v = vk()
+    g = torch.Generator("cuda").manual_seed(M)
+    x = torch.randn(M, K, generator=g, device="cuda").half()
+    vectors = [0.1 * torch.randn(1, K, generator=g, device="cuda").half() for _ in range(2)]
+
+    def quantize(rows):
+        if producer == "modulate":
+            return fused_ops.LnInput(rows, *vectors, 1e-6, producer).quantize(0.95, bf6=True)
+        return v.quantize_activation_bf6(rows, 0.95, act=producer)
+
+    def by_row(blocks, rows):
+        panels = blocks.view(-(-rows // 32) * 4, -1, 384)
+        planes = [panels[..., :256].unflatten(2, (2, 8, 16)), panels[..., 256:].unflatten(2, (2, 8, 8))]
+        return [p.movedim(3, 1).flatten(0, 1)[:rows] for p in planes]
+
+    blocks, scales = quantize(x)
+    whole = by_row(blocks, M)
+    for r in range(0, M, 2048):
+        rows = x[r:r + 2048]
+        part, part_scales = quantize(rows)
+        assert torch.equal(scales[r:r + 2048], part_scales)
+        assert all(torch.equal(w[r:r + 2048], p) for w, p in zip(whole, by_row(part, len(rows))))
+
+
 @pytest.mark.parametrize("act", [None, "gelu_tanh"])
 @pytest.mark.parametrize("M,K", [(25600, 1536), (17408, 2048), (4320, 9216 + 64), (4320, 13824), (4320, 16384)])
 def test_walking_quantizers_over_several_rounds(M, K, act):
