@@ -152,11 +152,13 @@ constexpr int kStringBytes = 24;
 // 16 bytes of padding per row: sixteen lanes that read 8 bytes each of eight rows and two strings meet 32 banks
 constexpr int kStringRowBytes = kStringsPerGroup * kStringBytes + 16;
 
-// A workgroup owns ROWS rows, one per wave: a panel or half of one (bf6_split says which).  The halves of a panel go to one
-// XCD, one after the other, whose L2 joins their runs (blocks are dealt to the XCDs in turn): the b-th of `groups` groups of rows.
+// A workgroup owns ROWS rows: a panel or half of one, a wave per row (bf6_split says which), or a quarter, four waves per row (rows_in_parts).
+// The parts of a panel go to one XCD, one after the other, whose L2 joins their runs (blocks are dealt to the XCDs in turn): the b-th of `groups`
+// groups of rows.
 template <int ROWS>
 __device__ __forceinline__ int bf6_group(int b, int groups) {
-    return ROWS == kPanelRows || (b | 15) >= groups ? b : (b & ~15) | (b & 7) << 1 | (b >> 3 & 1);
+    constexpr int P = kPanelRows / ROWS;
+    return P == 1 || (b | (8 * P - 1)) >= groups ? b : (b & ~(8 * P - 1)) | (b & 7) * P | (b >> 3 & (P - 1));
 }
 template <int ROWS>
 struct Bf6Scratch { /* LDS of one workgroup: the strings of one group; two copies in turn: one barrier per group is enough */
@@ -164,7 +166,8 @@ struct Bf6Scratch { /* LDS of one workgroup: the strings of one group; two copie
 };
 
 // `valid`: the wave's row exists (a workgroup's waves all run this function -- it synchronises them --
-// the ones past M on a copy of the last row, storing nothing).  `refill(c)` runs once chunk c of the
+// the ones past M on a copy of the last row, storing nothing).  PARTS > 1: the row is shared by PARTS waves, `part` is this one's (its chunks and its
+// staging copies are its own) and `part_max` takes their maxima.  `refill(c)` runs once chunk c of the
 // row has been converted and its registers are free: a workgroup that walks several
 // row groups loads the next row's chunk there, so those loads overlap the rest of this row's
 // conversion.  `phase` counts the groups this workgroup has staged (it picks the staging copy).
@@ -187,13 +190,18 @@ constexpr int bf6_spare_lds(int nch, int act) { return nch > 6 && nch <= 10 && a
 // 548, 32760 x 8960 193 / 152; short rows have the waves to overlap and pay for the second maximum: 75637 x 5120 176 /
 // 180, 27280 x 3072 43 / 45.5.  (The chunk counts that rows run on go from 14 to 18: this is K > 7168.)
 constexpr bool bf6_late_act(int nch) { return nch >= 17; }
+struct Bf6PartMax {
+    float mx;
+    int finite;
+};
 struct NoRefill {
     __device__ __forceinline__ void operator()(int) const {}
 };
-template <int NCH, int ACT, int ROWS, class Refill>
+template <int NCH, int ACT, int ROWS, int PARTS, class Refill>
 __device__ __forceinline__ void quantize_held_row_bf6(u32x4 (&v)[NCH], int lane, int wave, int64_t row0, bool valid, int M, int Kb,
                                                       float clip, uint8_t *__restrict__ blocks, __half *__restrict__ scale_h,
-                                                      bool stream_out, Bf6Scratch<ROWS> &lds, int &phase, Refill &&refill) {
+                                                      bool stream_out, Bf6Scratch<ROWS> &lds, int &phase, Refill &&refill, int part = 0,
+                                                      Bf6PartMax *part_max = nullptr) {
     // `late`: the activation is evaluated chunk by chunk below, in front of the conversion (see gelu_row_absmax)
     uint32_t m16 = 0;
     const bool late = ACT == VDMQ_ACT_GELU_TANH && gelu_row_absmax<NCH>(v, m16);
@@ -207,13 +215,23 @@ __device__ __forceinline__ void quantize_held_row_bf6(u32x4 (&v)[NCH], int lane,
         m16 = (m2 & 0xFFFFu) > (m2 >> 16) ? (m2 & 0xFFFFu) : (m2 >> 16);
         m16 = wave_max(m16);
     }
-    const bool finite = m16 < 0x7C00u;
+    bool finite = m16 < 0x7C00u;
     float mx = half_bits_to_float(m16);
     if (!finite) {
         mx = 0.0f;
 #pragma unroll
         for (int c = 0; c < NCH; ++c) mx = absmax_exact(v[c], mx);
         mx = wave_max(mx);
+    }
+    if constexpr (PARTS > 1) { /* the row's other parts */
+        if (lane == 0) part_max[part * ROWS + wave] = {mx, finite ? 1 : 0};
+        __syncthreads();
+#pragma unroll
+        for (int p = 0; p < PARTS; ++p) {
+            const Bf6PartMax other = part_max[p * ROWS + wave];
+            mx = __builtin_fmaxf(mx, other.mx);
+            finite = finite && other.finite != 0;
+        }
     }
     const __half sh = scale_from_absmax(mx, clip);
     const bool fast = __builtin_amdgcn_readfirstlane(finite && scale_is_ordinary(sh) ? 1 : 0) != 0;
@@ -225,7 +243,7 @@ __device__ __forceinline__ void quantize_held_row_bf6(u32x4 (&v)[NCH], int lane,
     // (of a finite row the largest |x| gives the largest |t|: the products round monotonically.  The same in every lane: a
     // scalar branch)
     const bool clamp_u = __builtin_amdgcn_readfirstlane(fast && mx * rscale < 7.5f ? 0 : 1) != 0;
-    if (lane == 0 && valid) scale_h[row0 + wave] = sh;
+    if (lane == 0 && valid && (PARTS == 1 || part == 0)) scale_h[row0 + wave] = sh;
 
     const int kblocks = Kb / 64;
     // the lane's quarter of a string: string lane / 4 of each chunk's sixteen, bytes 6p ... 6p + 5, p = lane % 4.  Those
@@ -288,8 +306,8 @@ __device__ __forceinline__ void quantize_held_row_bf6(u32x4 (&v)[NCH], int lane,
             }
         }
         __syncthreads(); /* also orders this group's writes after every thread's reads of the group before last */
-        const int k0 = 2048 * g + 32 * sidx;
-        if (k0 < Kb && grow < M) {
+        const int k0 = part * (NCH * 512) + 2048 * g + 32 * sidx;
+        if (k0 < Kb && grow < M && (PARTS == 1 || 2048 * g + 32 * sidx < NCH * 512)) {
             const int kb = k0 >> 6, h = (k0 >> 5) & 1;
             const u32x2 *string = reinterpret_cast<const u32x2 *>(lds.strings[copy][srow] + sidx * kStringBytes);
             const u32x2 s0 = string[0], s1 = string[1], part_b = string[2];
@@ -355,7 +373,7 @@ __global__ __launch_bounds__(ROWS * kWaveSize, FMT == 1 && NCH <= 2 ? 8 : FMT ==
                 for (int c = 0; c < NCH; ++c)
                     if (c * 512 + lane * 8 < K) v[c] = apply_act<ACT>(v[c]);
             }
-            quantize_held_row_bf6<NCH, bf6_late_act(NCH) ? ACT : VDMQ_ACT_NONE, ROWS>(v, lane, wave, row0, row0 + wave < M, M, Kp, clip, qact, scale_h, stream_out_bf6 != 0, scratch, phase,
+            quantize_held_row_bf6<NCH, bf6_late_act(NCH) ? ACT : VDMQ_ACT_NONE, ROWS, 1>(v, lane, wave, row0, row0 + wave < M, M, Kp, clip, qact, scale_h, stream_out_bf6 != 0, scratch, phase,
                                             [&](int c) {
                                                 if constexpr (bf6_walks(NCH))
                                                     if (more) v[c] = load(next, c);
@@ -374,6 +392,29 @@ __global__ __launch_bounds__(ROWS * kWaveSize, FMT == 1 && NCH <= 2 ? 8 : FMT ==
         }
         quantize_held_row<NCH, STREAM_OUT>(v, lane, row, Kp, clip, qact, scale_h);
     }
+}
+
+// The same for few rows, which a wave each would leave to a part of the chip, one long chain of loads, maximum and conversions per row: PARTS waves
+// share a row, NCH chunks each, and exchange their maxima once.  Bound by that chain (512 x 5120: 4.4 us for 9 MB); no walking, and the
+// activation goes in front, its absmax is the part's own.
+template <int NCH, int ACT, int ROWS, int PARTS>
+__global__ __launch_bounds__(ROWS * PARTS * kWaveSize) void quantize_row_parts_kernel(const __half *__restrict__ x, int64_t ldx, int M, int K, int Kp, float clip,
+                                                                                      uint8_t *__restrict__ blocks, __half *__restrict__ scale_h) {
+    __shared__ __attribute__((aligned(16))) Bf6Scratch<ROWS> scratch[PARTS];
+    __shared__ Bf6PartMax part_max[PARTS * ROWS];
+    const int lane = threadIdx.x & (kWaveSize - 1), w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wave = w % ROWS, part = w / ROWS;
+    const int64_t row0 = static_cast<int64_t>(bf6_group<ROWS>(blockIdx.x, (M + ROWS - 1) / ROWS)) * ROWS, row = row0 + wave;
+    const u32x4 *src = reinterpret_cast<const u32x4 *>(x + (row < M ? row : M - 1) * ldx) + part * (NCH * 64);
+    u32x4 v[NCH];
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) v[c] = (part * NCH + c) * 512 + lane * 8 < K ? __builtin_nontemporal_load(src + c * 64 + lane) : u32x4{0u, 0u, 0u, 0u};
+    if (ACT != VDMQ_ACT_NONE) {
+#pragma unroll
+        for (int c = 0; c < NCH; ++c) v[c] = apply_act<ACT>(v[c]);
+    }
+    int phase = 0;
+    quantize_held_row_bf6<NCH, VDMQ_ACT_NONE, ROWS, PARTS>(v, lane, wave, row0, row < M, M, Kp, clip, blocks, scale_h, false, scratch[part], phase, NoRefill{},
+                                                           part, part_max);
 }
 
 // Chunk counts the fused LayerNorm kernel is instantiated for (launch_ln_impl picks the first that covers the row):
@@ -437,7 +478,7 @@ __global__ __launch_bounds__(kRowsPerBlock * kWaveSize, FMT == 1 ? 2 : 1) void l
     if (FMT == 1) {
         __shared__ __attribute__((aligned(16))) Bf6Scratch<ROWS> scratch;
         int phase = 0;
-        quantize_held_row_bf6<NCH, VDMQ_ACT_NONE, ROWS>(v, lane, wave, row0, valid, M, Kp, clip, qact, scale_h, false, scratch, phase, NoRefill{});
+        quantize_held_row_bf6<NCH, VDMQ_ACT_NONE, ROWS, 1>(v, lane, wave, row0, valid, M, Kp, clip, qact, scale_h, false, scratch, phase, NoRefill{});
     } else {
         quantize_held_row<NCH, false>(v, lane, row, Kp, clip, qact, scale_h);
     }
@@ -668,10 +709,31 @@ int launch_reg(const __half *x, int64_t M, int64_t K, int64_t ldx, float clip, i
     return check_launch("quantize_rows_kernel");
 }
 
+// Whether rows go to four waves each (quantize_row_parts_kernel): while a wave per row leaves CUs idle or with one workgroup.  us, a wave per row /
+// four: 64 x 2048 2.7 / 2.6, 512 x 5120 5.0 / 4.4, 512 x 13824 8.0 / 6.5, 1200 x 5120 6.6 / 6.3, 1200 x 13824 13.2 / 11.0; with the GELU 512 x 2048
+// 3.8 / 3.5, 512 x 5120 6.3 / 5.3, 800 x 5120 6.6 / 6.8, 512 x 13824 13.2 / 8.5, 1200 x 13824 21.0 / 16.8.  Beyond: 1200 x 2048 3.8 / 4.3, 3000 x 5120
+// 9.4 / 11.4, 2000 x 13824 15.8 / 16.5.
+constexpr int kPartRows = 2, kParts = 4;
+bool rows_in_parts(int64_t M, int64_t K) { return K > 1536 && M <= (K > 2560 ? 1536 : 512); }
+
+template <int ACT>
+int launch_row_parts(const __half *x, int64_t M, int64_t K, int64_t ldx, float clip, uint8_t *qact, __half *scale_h, hipStream_t s) {
+    const int64_t nch = ceil_div(k_padded(K), 512 * kParts);
+    using Kernel = void (*)(const __half *, int64_t, int, int, int, float, uint8_t *, __half *);
+    const Kernel kernel = nch <= 1 ? quantize_row_parts_kernel<1, ACT, kPartRows, kParts> : nch <= 2 ? quantize_row_parts_kernel<2, ACT, kPartRows, kParts> :
+                          nch <= 3 ? quantize_row_parts_kernel<3, ACT, kPartRows, kParts> : nch <= 4 ? quantize_row_parts_kernel<4, ACT, kPartRows, kParts> :
+                          nch <= 5 ? quantize_row_parts_kernel<5, ACT, kPartRows, kParts> : nch <= 6 ? quantize_row_parts_kernel<6, ACT, kPartRows, kParts> :
+                          nch <= 7 ? quantize_row_parts_kernel<7, ACT, kPartRows, kParts> : quantize_row_parts_kernel<8, ACT, kPartRows, kParts>;
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(ceil_div(M, kPartRows))), dim3(kPartRows * kParts * kWaveSize), 0, s, x, ldx,
+                       static_cast<int>(M), static_cast<int>(K), static_cast<int>(bf6_kblocks(K) * 64), clip, qact, scale_h);
+    return check_launch("quantize_row_parts_kernel");
+}
+
 template <int ACT>
 int launch_quantize_act_impl(const __half *x, int64_t M, int64_t K, int64_t ldx, float clip, int fmt, uint8_t *qact, __half *scale_h,
                              hipStream_t s) {
     const int64_t nch = ceil_div(k_padded(K), 512);
+    if (fmt == 1 && nch <= 8 * kParts && rows_in_parts(M, K)) return launch_row_parts<ACT>(x, M, K, ldx, clip, qact, scale_h, s);
 #define VDMQ_CASE(n) \
     if (nch <= n) return launch_reg<n, ACT>(x, M, K, ldx, clip, fmt, qact, scale_h, s)
     // Rows are held in registers, so the chunk count is a template parameter; a row runs on the first count that

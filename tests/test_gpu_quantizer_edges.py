@@ -85,13 +85,20 @@ def codes_of_blocks(blocks, rows, K):
     return torch.where(codes == 32, 0, codes)
 
 
+def by_row(blocks, rows):
+    """The two planes of a bf6 operand's first rows, [row, k-block, half, byte] each."""
+    panels = blocks.view(-(-rows // 32) * 4, -1, 384)
+    planes = [panels[..., :256].unflatten(2, (2, 8, 16)), panels[..., 256:].unflatten(2, (2, 8, 8))]
+    return [p.movedim(3, 1).flatten(0, 1)[:rows] for p in planes]
+
+
 @pytest.mark.parametrize("M,K,producer", [(5121, 1536, None), (5121, 3584, None), (5123, 3648, None), (12999, 13824, None), (20001, 9216, None),
                                           (5121, 1536, "gelu_tanh"), (20001, 9216, "gelu_tanh"), (20001, 9280, "gelu_tanh"), (40005, 8960, "gelu_tanh"),
                                           (13, 1536, "modulate"), (35005, 5120, "modulate")])
 def test_whole_and_half_panel_workgroups(M, K, producer):
     """A workgroup takes a panel of eight rows or half of one, by the number of rows, their length, the producer in front and the
     size of the output: on both sides of those lines the rows' codes and scales are those of the same rows in slices of 2048, which
-    workgroups of four always serve (and which the other tests compare with the oracle)."""
+    workgroups of four or fewer rows serve (and which the other tests compare with the oracle)."""
     from dsaquant_amd import fused_ops
 
     v = vk()
@@ -104,11 +111,6 @@ def test_whole_and_half_panel_workgroups(M, K, producer):
             return fused_ops.LnInput(rows, *vectors, 1e-6, producer).quantize(0.95, bf6=True)
         return v.quantize_activation_bf6(rows, 0.95, act=producer)
 
-    def by_row(blocks, rows):
-        panels = blocks.view(-(-rows // 32) * 4, -1, 384)
-        planes = [panels[..., :256].unflatten(2, (2, 8, 16)), panels[..., 256:].unflatten(2, (2, 8, 8))]
-        return [p.movedim(3, 1).flatten(0, 1)[:rows] for p in planes]
-
     blocks, scales = quantize(x)
     whole = by_row(blocks, M)
     for r in range(0, M, 2048):
@@ -116,6 +118,26 @@ def test_whole_and_half_panel_workgroups(M, K, producer):
         part, part_scales = quantize(rows)
         assert torch.equal(scales[r:r + 2048], part_scales)
         assert all(torch.equal(w[r:r + 2048], p) for w, p in zip(whole, by_row(part, len(rows))))
+
+
+@pytest.mark.parametrize("act", [None, "gelu_tanh"])
+@pytest.mark.parametrize("K", [1600, 2560, 2624, 4096, 4160, 6208, 7168, 8256, 9216, 12288, 13824, 14400, 16384])
+def test_rows_shared_by_four_waves(K, act):
+    """Few rows go to four waves each: the codes and scales are those of the same rows among many, which have a wave each, with rows of
+    every kind (the largest element and NaN or Inf in any part, zeros, the GELU's negative branch) and numbers of rows around the line."""
+    v = vk()
+    g = torch.Generator("cuda").manual_seed(K)
+    x = torch.randn(1600, K, generator=g, device="cuda").half()
+    x[torch.arange(1600), torch.arange(1600) * 131 % K] *= 20
+    x[1::11] = -x[1::11].abs()
+    x[2::97] = 0
+    x[3::101, K - 1], x[5::103, K // 2], x[7::107, 3], x[8::109, K // 4] = float("inf"), float("nan"), float("-inf"), 65504
+    many, many_scales = v.quantize_activation_bf6(x, 0.95, act=act)
+    want = by_row(many, 1600)
+    for rows in (1, 2, 31, 513, 1536) if K > 2560 else (1, 2, 31, 511, 512):
+        blocks, scales = v.quantize_activation_bf6(x[:rows], 0.95, act=act)
+        assert torch.equal(scales.view(torch.int16), many_scales[:rows].view(torch.int16))
+        assert all(torch.equal(w[:rows], p) for w, p in zip(want, by_row(blocks, rows)))
 
 
 @pytest.mark.parametrize("act", [None, "gelu_tanh"])
