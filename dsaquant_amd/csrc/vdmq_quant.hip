@@ -439,16 +439,17 @@ constexpr int ln_full_chunks(int nch) {
 // Row m takes vector row m / rows_per_vec of a and b (stride ldv elements): one
 // vector per batch element, or one per token.  EMIT_H writes h itself instead of
 // quantizing it (the same arithmetic: the tests' view of h).
-// Bound by vector instructions and the reductions between them, so the bf6 form has four rows per workgroup, half a panel, whose halves L2
+// Bound by vector instructions and the reductions between them, so the bf6 form has ROWS = 4 per workgroup, half a panel, whose halves L2
 // joins (so no streamed stores): one workgroup's reductions run under another's loads and conversions.  us, eight rows (streamed beyond 128 MiB)
 // / four: 512 x 5120 8.1 / 6.8, 4680 x 1536 8.5 / 7.9, 27280 x 3072 54 / 48, 32760 x 4096 92 / 77, 60000 x 5120 181 / 165, 20000 x 13824 222 / 207; 6000
 // rows of up to 3072 1.00; with the GEMM behind it 60000 x 3072 -> 3072 399 / 372, 75600 x 5120 -> 13824 2433 / 2392.
-template <int NCH, int LNMODE, bool EMIT_H, int FMT>
-__global__ __launch_bounds__(kRowsPerBlock * kWaveSize, FMT == 1 ? 2 : 1) void ln_quantize_rows_kernel(
+// Up to 512 rows a workgroup has two, so that they spread over the CUs, us, two / four: 512 x 1536 3.64 / 3.71, 512 x 5120 6.3 / 6.7, 512 x 8960 11.6 /
+// 12.5; more rows than that are a second workgroup on some CUs (1000 x 5120 8.4 / 7.6).
+template <int NCH, int LNMODE, bool EMIT_H, int FMT, int ROWS>
+__global__ __launch_bounds__(ROWS * kWaveSize, FMT == 1 ? 2 : 1) void ln_quantize_rows_kernel(
     const __half *__restrict__ x, int64_t ldx, int M, int K, int Kp, float eps, const __half *__restrict__ va,
     const __half *__restrict__ vb, int64_t ldv, int rows_per_vec, float clip, uint8_t *__restrict__ qact,
     __half *__restrict__ scale_h, __half *__restrict__ h_out, int64_t ldh) {
-    constexpr int ROWS = kRowsPerBlock;
     const int lane = threadIdx.x & (kWaveSize - 1), wave = FMT == 1 && NCH > 16 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
     const int64_t row0 = static_cast<int64_t>(FMT == 1 ? bf6_group<ROWS>(blockIdx.x, (M + ROWS - 1) / ROWS) : blockIdx.x) * ROWS;
     int64_t row = row0 + wave;
@@ -759,18 +760,28 @@ int launch_quantize_act_impl(const __half *x, int64_t M, int64_t K, int64_t ldx,
     return check_launch("quantize_rows_anyk_kernel");
 }
 
+constexpr int64_t kLnFewRows = 512; /* two rows per workgroup up to here: a workgroup per CU (see ln_quantize_rows_kernel) */
+
 template <int NCH, int LNMODE>
 int launch_ln_reg(const __half *x, int64_t M, int64_t K, int64_t ldx, float eps, const __half *va, const __half *vb, int64_t ldv,
                   int64_t rows_per_vec, float clip, int fmt, uint8_t *qact, __half *scale_h, __half *h_out, int64_t ldh, hipStream_t s) {
     const dim3 grid(static_cast<unsigned>(ceil_div(M, kRowsPerBlock))), block(kRowsPerBlock * kWaveSize);
     if (h_out != nullptr)
-        hipLaunchKernelGGL((ln_quantize_rows_kernel<NCH, LNMODE, true, 0>), grid, block, 0, s, x, ldx, static_cast<int>(M), static_cast<int>(K),
+        hipLaunchKernelGGL((ln_quantize_rows_kernel<NCH, LNMODE, true, 0, kRowsPerBlock>), grid, block, 0, s, x, ldx, static_cast<int>(M), static_cast<int>(K),
                            static_cast<int>(k_padded(K)), eps, va, vb, ldv, static_cast<int>(rows_per_vec), clip, qact, scale_h, h_out, ldh);
-    else if (fmt == 1) /* (four rows per workgroup, half a panel, and plain stores at any size: see ln_quantize_rows_kernel) */
-        hipLaunchKernelGGL((ln_quantize_rows_kernel<NCH, LNMODE, false, 1>), grid, block, 0, s, x, ldx, static_cast<int>(M), static_cast<int>(K),
-                           static_cast<int>(bf6_kblocks(K) * 64), eps, va, vb, ldv, static_cast<int>(rows_per_vec), clip, qact, scale_h, h_out, ldh);
+    else if (fmt == 1) { /* (plain stores at any size: see ln_quantize_rows_kernel) */
+        auto launch = [&](auto kernel, int rows) {
+            hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(ceil_div(M, rows))), dim3(rows * kWaveSize), 0, s, x, ldx, static_cast<int>(M),
+                               static_cast<int>(K), static_cast<int>(bf6_kblocks(K) * 64), eps, va, vb, ldv, static_cast<int>(rows_per_vec), clip, qact,
+                               scale_h, h_out, ldh);
+        };
+        if (M <= kLnFewRows)
+            launch(ln_quantize_rows_kernel<NCH, LNMODE, false, 1, 2>, 2);
+        else
+            launch(ln_quantize_rows_kernel<NCH, LNMODE, false, 1, kPanelRows / 2>, kPanelRows / 2);
+    }
     else
-        hipLaunchKernelGGL((ln_quantize_rows_kernel<NCH, LNMODE, false, 0>), grid, block, 0, s, x, ldx, static_cast<int>(M), static_cast<int>(K),
+        hipLaunchKernelGGL((ln_quantize_rows_kernel<NCH, LNMODE, false, 0, kRowsPerBlock>), grid, block, 0, s, x, ldx, static_cast<int>(M), static_cast<int>(K),
                            static_cast<int>(k_padded(K)), eps, va, vb, ldv, static_cast<int>(rows_per_vec), clip, qact, scale_h, h_out, ldh);
     return check_launch("ln_quantize_rows_kernel");
 }

@@ -94,7 +94,8 @@ def by_row(blocks, rows):
 
 @pytest.mark.parametrize("M,K,producer", [(5121, 1536, None), (5121, 3584, None), (5123, 3648, None), (12999, 13824, None), (20001, 9216, None),
                                           (5121, 1536, "gelu_tanh"), (20001, 9216, "gelu_tanh"), (20001, 9280, "gelu_tanh"), (40005, 8960, "gelu_tanh"),
-                                          (13, 1536, "modulate"), (35005, 5120, "modulate")])
+                                          (13, 1536, "modulate"), (2347, 1536, "modulate"), (2347, 8960, "modulate"),
+                                          (35005, 5120, "modulate")])
 def test_whole_and_half_panel_workgroups(M, K, producer):
     """A workgroup takes a panel of eight rows or half of one, by the number of rows, their length, the producer in front and the
     size of the output: on both sides of those lines the rows' codes and scales are those of the same rows in slices of 2048, which
