@@ -250,8 +250,8 @@ __device__ __forceinline__ void quantize_held_row_bf6(u32x4 (&v)[NCH], int lane,
     // are a word and a half word, the word first for even p and last for odd p (so that it is aligned).
     const bool odd = (lane & 1) != 0;
     const uint32_t string0 = (lane >> 2) * kStringBytes + (lane & 3) * 6, off32 = string0 + (odd ? 2 : 0), off16 = string0 + (odd ? 0 : 4);
-    // the thread's share of the cooperative store: string t / 8 of row t % 8 -- eight consecutive
-    // threads write the eight rows' parts of one string slot, 128 (and 64) contiguous bytes
+    // the thread's share of the cooperative store: string t / ROWS of row t % ROWS -- ROWS consecutive threads write
+    // the rows' parts of one string slot, contiguous bytes: 128 (and 64) of a whole panel
     const int t = wave * kWaveSize + lane, srow = t % ROWS, sidx = t / ROWS;
     const int64_t grow = row0 + srow;
     constexpr int NG = (NCH + 3) / 4;
@@ -286,7 +286,7 @@ __device__ __forceinline__ void quantize_held_row_bf6(u32x4 (&v)[NCH], int lane,
         for (int cc = 0; cc < 4; ++cc)
             if (4 * g + cc < NCH) refill(4 * g + cc);
         // per-lane stores would scatter pieces over 64 cache lines per instruction (measured: 2x slower than the
-        // HBM-bound int4 quantizer): collect the workgroup's strings in LDS -- its eight rows are one panel, whose
+        // HBM-bound int4 quantizer): collect the workgroup's strings in LDS -- its rows are a panel or part of one, whose
         // 128-byte and 64-byte runs of one k-block are adjacent in memory
         const int copy = phase & 1;
         ++phase;
