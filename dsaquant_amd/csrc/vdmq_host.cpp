@@ -60,18 +60,20 @@ bool packed_pair(PyObject *qweight, PyObject *wscales, c10::Device device, int64
     return N > 0;
 }
 
-// linear(prepare, x, shape, qweight, wscales, check_q, check_s, bias, clip, act, ln_mode, eps, a, b, rows_per_vec, residual, gate, split_cols,
-//        views)
+// linear(prepare, x, shape, qweight, wscales, prepared_k, check_q, check_s, bias, clip, act, ln_mode, eps, a, b, rows_per_vec, residual, gate,
+//        split_cols, views)
 //
 // `shape`: what x stands for, a tuple, or None where that is its own shape.
-// `prepare(qweight, wscales, device index)` gives (blocks, scales, N, stream), or None where the device is not the current one; `wscales` None:
-// qweight is a prepared weight, of which N comes back too.  check_q, check_s: a packed pair whose shapes the call checks besides, or None.
+// `prepare(qweight, wscales, device index)` gives (blocks, scales, N, stream), or None where the device is not the current one.
+// prepared_k: None, or qweight is a prepared weight of rows of that many elements (without `wscales`), of which N comes back too.  The row
+// length of x is what the library multiplies by: a weight of another is read beyond its end.
+// check_q, check_s: a packed pair whose shapes the call checks besides, or None.
 // Returns the output [..., N], with split_cols [N / split_cols, ..., split_cols], with views the tuple of its parts of that many
 // columns; None: not served; an int: the library's error code.
 PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     HANDLE_TH_ERRORS
-    if (nargs != 19) {
-        PyErr_SetString(PyExc_TypeError, "linear takes 19 arguments");
+    if (nargs != 20) {
+        PyErr_SetString(PyExc_TypeError, "linear takes 20 arguments");
         return nullptr;
     }
     PyObject *const prepare = args[0];
@@ -94,21 +96,25 @@ PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     }
     if (M <= 0 || K % 64 != 0 || K < VDMQ_LINEAR_BF6_MIN_K || K > kMaxK) Py_RETURN_NONE;
     int64_t N = 0, checked = 0;
-    const bool packed = args[4] != Py_None;
+    const bool packed = args[5] == Py_None;
     if (packed && !packed_pair(args[3], args[4], device, K, N)) Py_RETURN_NONE;
-    if (args[5] != Py_None && !packed_pair(args[5], args[6], device, K, checked)) Py_RETURN_NONE;
-    const double clip = PyFloat_AsDouble(args[8]), eps = PyFloat_AsDouble(args[11]);
-    const long act = PyLong_AsLong(args[9]), ln_mode = PyLong_AsLong(args[10]);
-    const int64_t rows_per_vec = PyLong_AsLongLong(args[14]), split_cols = PyLong_AsLongLong(args[17]), views = PyLong_AsLongLong(args[18]);
+    if (!packed && PyLong_AsLongLong(args[5]) != K) {
+        PyErr_Clear();
+        Py_RETURN_NONE;
+    }
+    if (args[6] != Py_None && !packed_pair(args[6], args[7], device, K, checked)) Py_RETURN_NONE;
+    const double clip = PyFloat_AsDouble(args[9]), eps = PyFloat_AsDouble(args[12]);
+    const long act = PyLong_AsLong(args[10]), ln_mode = PyLong_AsLong(args[11]);
+    const int64_t rows_per_vec = PyLong_AsLongLong(args[15]), split_cols = PyLong_AsLongLong(args[18]), views = PyLong_AsLongLong(args[19]);
     if (PyErr_Occurred()) { /* (the general code says what is wrong with it) */
         PyErr_Clear();
         Py_RETURN_NONE;
     }
     const at::Tensor *bias = nullptr, *a = nullptr, *b = nullptr, *residual = nullptr, *gate = nullptr;
-    if (args[7] != Py_None && ((bias = plain_half(args[7], device)) == nullptr || bias->dim() != 1)) Py_RETURN_NONE;
-    if (ln_mode != 0 && ((a = plain_half(args[12], device)) == nullptr || (b = plain_half(args[13], device)) == nullptr)) Py_RETURN_NONE;
-    if (args[15] != Py_None && (residual = plain_half(args[15], device)) == nullptr) Py_RETURN_NONE;
-    if (args[16] != Py_None && ((gate = plain_half(args[16], device)) == nullptr || gate->dim() < 1 || gate->numel() == 0)) Py_RETURN_NONE;
+    if (args[8] != Py_None && ((bias = plain_half(args[8], device)) == nullptr || bias->dim() != 1)) Py_RETURN_NONE;
+    if (ln_mode != 0 && ((a = plain_half(args[13], device)) == nullptr || (b = plain_half(args[14], device)) == nullptr)) Py_RETURN_NONE;
+    if (args[16] != Py_None && (residual = plain_half(args[16], device)) == nullptr) Py_RETURN_NONE;
+    if (args[17] != Py_None && ((gate = plain_half(args[17], device)) == nullptr || gate->dim() < 1 || gate->numel() == 0)) Py_RETURN_NONE;
     // what is left to check depends on the outputs, whose number a prepared weight knows
     auto fits = [&](int64_t n) {
         if (n <= 0 || (bias != nullptr && bias->numel() != n)) return false;

@@ -414,7 +414,8 @@ def _native_linear(x: torch.Tensor, qweight, wscales: Optional[torch.Tensor], bi
     are not, and nothing has been done.  ``qweight`` may be a PreparedWeight, without ``wscales``."""
     if _MATRIX_PATH != "auto":
         return None
-    out = _lib.host.linear(_operands, x, shape, qweight, wscales, check[0], check[1], bias, clip_ratio, act, ln[0], ln[1], ln[2], ln[3], ln[4], residual,
+    k = qweight.K if wscales is None else None
+    out = _lib.host.linear(_operands, x, shape, qweight, wscales, k, check[0], check[1], bias, clip_ratio, act, ln[0], ln[1], ln[2], ln[3], ln[4], residual,
                            gate, split_cols, views)
     if type(out) is int:
         _lib.check(out)

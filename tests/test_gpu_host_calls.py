@@ -144,6 +144,40 @@ def test_calls_left_to_the_general_code(operands):
         assert Seen.calls > 0
 
 
+@pytest.mark.parametrize("other", [K - 64, K + 64])
+def test_rows_of_another_length_than_a_prepared_weights(operands, other):
+    """Shorter rows would multiply by the wrong weights, longer ones read behind the last: refused, with the general code's error,
+    before the weight's form is asked for."""
+    from types import SimpleNamespace
+
+    from dsaquant_amd import fused_ops as F
+    from dsaquant_amd.fused_qkv import get_qkv_projections
+
+    v, o = vk(), operands
+    qw, ws = o["qw"].clone(), o["ws"].clone()
+    x, a = torch.ones((2, 33, other), device="cuda").half(), torch.ones((2, 1, other), device="cuda").half()
+    pw = v._prepared_weight(qw, ws)
+    for call in (lambda: v.linear_vdm_w4a4_prepared(x, pw, o["b"], 0.95), lambda: v.linear_vdm_w4a4_prepared(x, pw, o["b"], 0.95, split_cols=128),
+                 lambda: F.linear_fused(x, pw, None, o["b"], 0.95), lambda: F.linear_fused(x, pw, None, o["b"], 0.95, act="gelu_tanh"),
+                 lambda: F.linear_fused(x, pw, None, o["b"], 0.95, residual=o["res"], gate=o["gate"]), lambda: F.linear_fused(x, pw, None, split_cols=128),
+                 lambda: F.linear_fused(F.LnInput(x, a, a, 1e-6), pw, None, o["b"], 0.95),
+                 lambda: F.linear_fused(F.LnInput(x.float(), a, a, 1e-6, "affine"), pw, None, o["b"], 0.95)):
+        assert same(call, False) == (ValueError, "qweight shape must be [N, K/2]")
+    assert pw.bf6 is None
+    layer = lambda: SimpleNamespace(vdm_weight_packed=qw.clone(), vdm_weight_scale_packed=ws.clone(), _bias_half=None, kernel_clip_ratio=0.95)  # noqa: E731
+    for contiguous in (False, True):
+        for cross in (None, 128):
+            attn = SimpleNamespace(to_q=lambda t: t, to_k=layer(), to_v=layer(), cross_attention_dim_head=cross, use_fused_qkv_kernel=True,
+                                   qkv_kernel_backend="vdm", qkv_contiguous_outputs=contiguous)
+            if cross is None:
+                attn.to_q = layer()
+                calls = [lambda: get_qkv_projections(attn, x, None), lambda: F.qkv_projections_ln(attn, F.LnInput(x, a, a, 1e-6))]
+            else:
+                calls = [lambda: get_qkv_projections(attn, x, x), lambda: F.kv_projections(attn, x)]
+            for call in calls:
+                assert same(call, False) == (ValueError, "qweight shape must be [N, K/2]")
+
+
 def test_on_the_current_stream_and_in_a_graph(operands):
     v, o = vk(), operands
     x = o["x"].clone()
