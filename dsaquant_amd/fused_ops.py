@@ -264,17 +264,14 @@ def linear_fused(
 
 
 def _native_fused(x, qweight, wscales, bias, clip_ratio, act, residual, gate, split_cols):
-    prepared = type(qweight) is _k.PreparedWeight
-    if not prepared and (isinstance(qweight, _k.PreparedWeight) or wscales is None):
-        return None
+    weight = qweight if type(qweight) is _k.PreparedWeight else (qweight, wscales)
     if type(x) is LnInput:
         if act is not None:
             return None
         rows, a, b = x._given if x._rows is None else x._rows
-        return _k._native_linear(rows, qweight, None if prepared else wscales, bias, clip_ratio, shape=None if x._rows is None else x.shape,
-                                 ln=(x.code, x.eps, a, b, x.rows_per_vec),
+        return _k._native_linear(rows, weight, bias, clip_ratio, shape=None if x._rows is None else x.shape, ln=(x.code, x.eps, a, b, x.rows_per_vec),
                                  residual=residual, gate=gate, split_cols=split_cols)
-    return _k._native_linear(x, qweight, None if prepared else wscales, bias, clip_ratio, act=_lib.VDMQ_ACT_NONE if act is None else _lib.VDMQ_ACT_GELU_TANH,
+    return _k._native_linear(x, weight, bias, clip_ratio, act=_lib.VDMQ_ACT_NONE if act is None else _lib.VDMQ_ACT_GELU_TANH,
                              residual=residual, gate=gate, split_cols=split_cols)
 
 

@@ -408,13 +408,13 @@ def _operands(qweight, wscales: Optional[torch.Tensor], device_index: int):
     return weight.operand(True), weight.wscale, weight.N, torch._C._cuda_getCurrentRawStream(device_index)
 
 
-def _native_linear(x: torch.Tensor, qweight, wscales: Optional[torch.Tensor], bias: Optional[torch.Tensor], clip_ratio: float, *, shape=None,
-                   check=(None, None), act: int = 0, ln=(0, 0.0, None, None, 1), residual=None, gate=None, split_cols: int = 0, views: int = 0):
+def _native_linear(x: torch.Tensor, weight, bias: Optional[torch.Tensor], clip_ratio: float, *, shape=None, check=(None, None),
+                   act: int = 0, ln=(0, 0.0, None, None, 1), residual=None, gate=None, split_cols: int = 0, views: int = 0):
     """The whole call in the extension module (vdmq_host.cpp) where its operands are plain and the bf6 path is the library's choice; None: they
-    are not, and nothing has been done.  ``qweight`` may be a PreparedWeight, without ``wscales``."""
+    are not, and nothing has been done.  ``weight``: ``(qweight, wscales)`` as the caller was given them, or a PreparedWeight."""
     if _MATRIX_PATH != "auto":
         return None
-    k = qweight.K if wscales is None else None
+    qweight, wscales, k = (*weight, None) if type(weight) is tuple else (weight, None, weight.K)
     out = _lib.host.linear(_operands, x, shape, qweight, wscales, k, check[0], check[1], bias, clip_ratio, act, ln[0], ln[1], ln[2], ln[3], ln[4], residual,
                            gate, split_cols, views)
     if type(out) is int:
@@ -719,7 +719,7 @@ def linear_vdm_w4a4(
     against the packed weights, per-token x per-channel scale and fp16 bias.
     Signature and semantics of vdm_w4a4.py:222-244; the output is always fp16."""
     _load_ext()
-    out = _native_linear(x, qweight, wscales, bias_half if bias_half is not None else bias, clip_ratio)
+    out = _native_linear(x, (qweight, wscales), bias_half if bias_half is not None else bias, clip_ratio)
     if out is not None:
         return out
     x_2d, orig_shape = _as_2d_half_contiguous(x)
@@ -737,7 +737,7 @@ def linear_vdm_w4a4_prepared(x: torch.Tensor, weight: PreparedWeight, bias_half:
     ``out.split(split_cols, -1)``, without the strided views (the GEMM epilogue writes them in place)."""
     _load_ext()
     if type(weight) is PreparedWeight and (split_cols is None or split_cols):
-        out = _native_linear(x, weight, None, bias_half, clip_ratio, split_cols=split_cols or 0)
+        out = _native_linear(x, weight, bias_half, clip_ratio, split_cols=split_cols or 0)
         if out is not None:
             return out
     x_2d, orig_shape = _as_2d_half_contiguous(x)
@@ -892,7 +892,7 @@ def linear_vdm_w4a4_qkv(
     if w_qkv_packed is not None and w_qkv_scale is not None and (qkv_bias_half is not None or (q_bias is None and k_bias is None and v_bias is None)):
         _load_ext()
         n = q_weight_packed.shape[0]
-        out = _native_linear(x, w_qkv_packed, w_qkv_scale, qkv_bias_half, clip_ratio, check=(q_weight_packed, q_weight_scale),
+        out = _native_linear(x, (w_qkv_packed, w_qkv_scale), qkv_bias_half, clip_ratio, check=(q_weight_packed, q_weight_scale),
                              split_cols=n if contiguous_outputs else 0, views=0 if contiguous_outputs else n)
         if out is not None:
             return out.unbind(0) if contiguous_outputs else out

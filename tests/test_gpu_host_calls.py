@@ -119,6 +119,10 @@ def test_calls_left_to_the_general_code(operands):
                 lambda: F.LnInput(x, o["a"], o["shift"][:1], 1e-6), lambda: F.LnInput(x, o["a"][..., :64], o["shift"][..., :64], 1e-6),
                 lambda: torch.func.vmap(lambda t: v.linear_vdm_w4a4(t, qw, ws, b, 0.95))(x)):
         assert isinstance(same(bad, False), tuple)
+    pw = v._prepared_weight(qw, ws)  # the packed entries take packed weights only, with their scales
+    for refused in (lambda: v.linear_vdm_w4a4(x, pw, None, b, 0.95), lambda: v.linear_vdm_w4a4(x, qw, None, b, 0.95),
+                    lambda: F.linear_fused(x, qw, None, b, 0.95), lambda: v.linear_vdm_w4a4(x, pw, ws, b, 0.95)):
+        assert same(refused, False)[0] is AttributeError
     for path in ("int8", "bf6"):
         before = v.matrix_path()
         try:
