@@ -60,13 +60,14 @@ bool packed_pair(PyObject *qweight, PyObject *wscales, c10::Device device, int64
     return N > 0;
 }
 
-// linear(prepare, x, shape, qweight, wscales, prepared_k, check_q, check_s, bias, clip, act, ln_mode, eps, a, b, rows_per_vec, residual, gate,
+// linear(prepare, x, shape, qweight, wscales, prepared, check_q, check_s, bias, clip, act, ln_mode, eps, a, b, rows_per_vec, residual, gate,
 //        split_cols, views)
 //
 // `shape`: what x stands for, a tuple, or None where that is its own shape.
-// `prepare(qweight, wscales, device index)` gives (blocks, scales, N, stream), or None where the device is not the current one.
-// prepared_k: None, or qweight is a prepared weight of rows of that many elements (without `wscales`), of which N comes back too.  The row
-// length of x is what the library multiplies by: a weight of another is read beyond its end.
+// `prepare(qweight, wscales, device index)` gives (blocks, scales, stream), or None where the device is not the current one.  It may make the
+// weight's form, so everything else is checked in front of it.
+// `prepared`: None, or qweight is a prepared weight (without `wscales`) and this its (N, K).  The row length of x is what the library multiplies
+// by: a weight of another is read beyond its end.
 // check_q, check_s: a packed pair whose shapes the call checks besides, or None.
 // Returns the output [..., N], with split_cols [N / split_cols, ..., split_cols], with views the tuple of its parts of that many
 // columns; None: not served; an int: the library's error code.
@@ -97,10 +98,13 @@ PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     if (M <= 0 || K % 64 != 0 || K < VDMQ_LINEAR_BF6_MIN_K || K > kMaxK) Py_RETURN_NONE;
     int64_t N = 0, checked = 0;
     const bool packed = args[5] == Py_None;
-    if (packed && !packed_pair(args[3], args[4], device, K, N)) Py_RETURN_NONE;
-    if (!packed && PyLong_AsLongLong(args[5]) != K) {
-        PyErr_Clear();
-        Py_RETURN_NONE;
+    if (packed) {
+        if (!packed_pair(args[3], args[4], device, K, N)) Py_RETURN_NONE;
+    } else {
+        long long n = 0, k = 0;
+        if (!PyArg_ParseTuple(args[5], "LL", &n, &k)) return nullptr;
+        if (k != K || n <= 0) Py_RETURN_NONE;
+        N = n;
     }
     if (args[6] != Py_None && !packed_pair(args[6], args[7], device, K, checked)) Py_RETURN_NONE;
     const double clip = PyFloat_AsDouble(args[9]), eps = PyFloat_AsDouble(args[12]);
@@ -115,19 +119,15 @@ PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     if (ln_mode != 0 && ((a = plain_half(args[13], device)) == nullptr || (b = plain_half(args[14], device)) == nullptr)) Py_RETURN_NONE;
     if (args[16] != Py_None && (residual = plain_half(args[16], device)) == nullptr) Py_RETURN_NONE;
     if (args[17] != Py_None && ((gate = plain_half(args[17], device)) == nullptr || gate->dim() < 1 || gate->numel() == 0)) Py_RETURN_NONE;
-    // what is left to check depends on the outputs, whose number a prepared weight knows
-    auto fits = [&](int64_t n) {
-        if (n <= 0 || (bias != nullptr && bias->numel() != n)) return false;
-        if (gate != nullptr && (gate->size(-1) != n || M % (gate->numel() / n) != 0)) return false;
-        if (residual != nullptr) {
-            if (residual->dim() != static_cast<int64_t>(lead.size()) + 1 || residual->size(-1) != n) return false;
-            for (size_t i = 0; i < lead.size(); ++i)
-                if (residual->size(static_cast<int64_t>(i)) != lead[i]) return false;
-        }
-        if (split_cols != 0 && (split_cols < 0 || split_cols % 64 != 0 || n % split_cols != 0 || residual != nullptr || gate != nullptr)) return false;
-        return views >= 0 && (views == 0 || n % views == 0);
-    };
-    if (packed && !fits(N)) Py_RETURN_NONE;
+    if (bias != nullptr && bias->numel() != N) Py_RETURN_NONE;
+    if (gate != nullptr && (gate->size(-1) != N || M % (gate->numel() / N) != 0)) Py_RETURN_NONE;
+    if (residual != nullptr) {
+        if (residual->dim() != static_cast<int64_t>(lead.size()) + 1 || residual->size(-1) != N) Py_RETURN_NONE;
+        for (size_t i = 0; i < lead.size(); ++i)
+            if (residual->size(static_cast<int64_t>(i)) != lead[i]) Py_RETURN_NONE;
+    }
+    if (split_cols != 0 && (split_cols < 0 || split_cols % 64 != 0 || N % split_cols != 0 || residual != nullptr || gate != nullptr)) Py_RETURN_NONE;
+    if (views < 0 || (views != 0 && N % views != 0)) Py_RETURN_NONE;
     PyObject *const index = PyLong_FromLong(device.index());
     if (index == nullptr) return nullptr;
     PyObject *const question[3] = {args[3], args[4], index};
@@ -136,15 +136,8 @@ PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     if (!prepared) return nullptr;
     if (prepared.get() == Py_None) Py_RETURN_NONE;
     PyObject *blocks_obj, *wscale_obj;
-    long long n = 0;
     unsigned long long stream = 0;
-    if (!PyArg_ParseTuple(prepared.get(), "OOLK", &blocks_obj, &wscale_obj, &n, &stream)) return nullptr;
-    if (!packed) {
-        const at::Tensor *w = plain(blocks_obj);
-        if (w == nullptr || w->device() != device || !fits(n)) Py_RETURN_NONE;
-        N = n;
-    }
-    if (!THPVariable_Check(blocks_obj) || !THPVariable_Check(wscale_obj) || n != N) Py_RETURN_NONE;
+    if (!PyArg_ParseTuple(prepared.get(), "O!O!K", THPVariableClass, &blocks_obj, THPVariableClass, &wscale_obj, &stream)) return nullptr;
     const at::Tensor &blocks = THPVariable_Unpack(blocks_obj), &wscale = THPVariable_Unpack(wscale_obj);
 
     c10::SmallVector<int64_t, 8> shape;

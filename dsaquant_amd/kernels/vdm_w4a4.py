@@ -400,12 +400,12 @@ def _prepared_weight(qweight: torch.Tensor, wscales: torch.Tensor) -> PreparedWe
 
 
 def _operands(qweight, wscales: Optional[torch.Tensor], device_index: int):
-    """``(bf6 blocks, channel scales, N, stream)`` of a packed weight (``wscales`` None: of a PreparedWeight) for a call on the
-    current stream; None where the device is not the current one."""
-    if torch._C._cuda_getDevice() != device_index:
+    """``(bf6 blocks, channel scales, stream)`` of a packed weight (``wscales`` None: of a PreparedWeight) for a call on the
+    current stream; None where the device is not the current one or not the weight's."""
+    if torch._C._cuda_getDevice() != device_index or (wscales is None and qweight.device.index != device_index):
         return None
     weight = qweight if wscales is None else _prepared([(qweight, wscales)])
-    return weight.operand(True), weight.wscale, weight.N, torch._C._cuda_getCurrentRawStream(device_index)
+    return weight.operand(True), weight.wscale, torch._C._cuda_getCurrentRawStream(device_index)
 
 
 def _native_linear(x: torch.Tensor, weight, bias: Optional[torch.Tensor], clip_ratio: float, *, shape=None, check=(None, None),
@@ -414,8 +414,8 @@ def _native_linear(x: torch.Tensor, weight, bias: Optional[torch.Tensor], clip_r
     are not, and nothing has been done.  ``weight``: ``(qweight, wscales)`` as the caller was given them, or a PreparedWeight."""
     if _MATRIX_PATH != "auto":
         return None
-    qweight, wscales, k = (*weight, None) if type(weight) is tuple else (weight, None, weight.K)
-    out = _lib.host.linear(_operands, x, shape, qweight, wscales, k, check[0], check[1], bias, clip_ratio, act, ln[0], ln[1], ln[2], ln[3], ln[4], residual,
+    qweight, wscales, sizes = (*weight, None) if type(weight) is tuple else (weight, None, (weight.N, weight.K))
+    out = _lib.host.linear(_operands, x, shape, qweight, wscales, sizes, check[0], check[1], bias, clip_ratio, act, ln[0], ln[1], ln[2], ln[3], ln[4], residual,
                            gate, split_cols, views)
     if type(out) is int:
         _lib.check(out)

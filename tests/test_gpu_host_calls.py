@@ -182,6 +182,26 @@ def test_rows_of_another_length_than_a_prepared_weights(operands, other):
                 assert same(call, False) == (ValueError, "qweight shape must be [N, K/2]")
 
 
+def test_refused_calls_leave_a_prepared_weight_as_it_was(operands):
+    """A call that is refused for another operand has made no form of the weight and dropped none that was made ahead."""
+    from dsaquant_amd import fused_ops as F
+
+    v, o = vk(), operands
+    x, b = o["x"], o["b"]
+    qw, ws = o["qw"].clone(), o["ws"].clone()
+    pw = v._prepared_weight(qw, ws)
+    native = pw.operand(False, eager=True)
+    for refused in (lambda: v.linear_vdm_w4a4_prepared(x, pw, b[:128], 0.95), lambda: v.linear_vdm_w4a4_prepared(x, pw, b, 0.95, split_cols=96),
+                    lambda: F.linear_fused(x, pw, None, b, 0.95, gate=o["gate"][..., :128]), lambda: F.linear_fused(x[:, :32], pw, None, b, 0.95, gate=o["res"][0, :3]),
+                    lambda: F.linear_fused(x, pw, None, b, 0.95, residual=o["res"][:1]), lambda: F.linear_fused(x, pw, None, b[:128], 0.95),
+                    lambda: F.linear_fused(x, pw, None, b, 0.95, gate=o["gate"], split_cols=128), lambda: v.linear_vdm_w4a4(x, qw, ws, b[:128], 0.95),
+                    lambda: v.linear_vdm_w4a4(x, qw, ws, b, "much")):
+        assert isinstance(same(refused, False), tuple)
+        assert pw.native is native and pw.bf6 is None
+    same(lambda: v.linear_vdm_w4a4_prepared(x, pw, b, 0.95), True)
+    assert pw.native is None and pw.bf6 is not None
+
+
 def test_on_the_current_stream_and_in_a_graph(operands):
     v, o = vk(), operands
     x = o["x"].clone()
