@@ -2,8 +2,11 @@
 from __future__ import annotations
 
 import ctypes
+import importlib
 import os
 import subprocess
+import sys
+import warnings
 from pathlib import Path
 from typing import Optional
 
@@ -12,7 +15,7 @@ LIB_PATH = _PKG / "libvdmq.so"
 CSRC = _PKG / "csrc"
 
 _LIB: Optional[ctypes.CDLL] = None
-host = None  # the extension module _vdmq_host, once load() has run
+host = None  # the extension module _vdmq_host, once load() has run; None where it cannot be used: the general code serves every call
 
 VDMQ_VERSION = 2  # include/vdmq.h; also the version of the bf6 block format
 VDMQ_OUT_F16 = 0
@@ -22,6 +25,8 @@ VDMQ_ACT_GELU_TANH = 1
 VDMQ_LN_MODULATE = 1
 VDMQ_LN_AFFINE = 2
 VDMQ_LINEAR_BF6_MIN_K = 640
+HOST_INTERFACE = 1  # the arguments of _vdmq_host's functions (kInterface in vdmq_host.cpp)
+
 
 class GemmLaunchInfo(ctypes.Structure):
     """vdmq_gemm_launch_info of include/vdmq.h."""
@@ -98,8 +103,8 @@ class VdmqError(RuntimeError):
 
 
 def build(verbose: bool = False) -> Path:
-    """Compile libvdmq.so for gfx950 with hipcc (``make -C dsaquant_amd/csrc``)."""
-    cmd = ["make", "-C", str(CSRC), "-j", str(min(8, os.cpu_count() or 1)), "-B"]
+    """Compile libvdmq.so for gfx950 with hipcc, and the extension module for this interpreter (``make -C dsaquant_amd/csrc``)."""
+    cmd = ["make", "-C", str(CSRC), "-j", str(min(8, os.cpu_count() or 1)), "-B", f"PYTHON={sys.executable}"]
     res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if verbose or res.returncode != 0:
         print(res.stdout)
@@ -126,13 +131,25 @@ def load() -> ctypes.CDLL:
         fn.argtypes = argtypes
     if lib.vdmq_version() != VDMQ_VERSION:
         raise RuntimeError(f"{LIB_PATH} has interface version {lib.vdmq_version()}, this package expects {VDMQ_VERSION}: rebuild it (make -C {CSRC})")
-    # (the host side of the package's own calls: vdmq_host.cpp, built with the library)
-    from . import _vdmq_host
-
-    _vdmq_host.init(*(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in ("vdmq_linear_bf6_ex", "vdmq_linear_bf6_workspace", "vdmq_pack_weight")))
-    host = _vdmq_host
+    host = _load_host(lib, torch.__version__)
     _LIB = lib
     return lib
+
+
+def _load_host(lib: ctypes.CDLL, torch_version: str):
+    """The host side of the package's own calls (vdmq_host.cpp, built with the library); None, with a warning, where there is none
+    for this interpreter, torch and package: its calls then run through ctypes, with the same results and 4 ... 12 us more each."""
+    try:
+        module = importlib.import_module("._vdmq_host", __package__)
+        built = getattr(module, "interface", None), getattr(module, "torch_version", None)
+        reason = None if built == (HOST_INTERFACE, torch_version.split("+")[0]) else f"it is of interface {built[0]} and torch {built[1]}"
+    except ImportError as exc:
+        reason = str(exc)
+    if reason is not None:
+        warnings.warn(f"the extension module _vdmq_host cannot be used ({reason}): build it with `make -C {CSRC} PYTHON={sys.executable}`", RuntimeWarning, 3)
+        return None
+    module.init(*(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in ("vdmq_linear_bf6_ex", "vdmq_linear_bf6_workspace", "vdmq_pack_weight")))
+    return module
 
 
 def last_gemm_launch() -> GemmLaunchInfo:

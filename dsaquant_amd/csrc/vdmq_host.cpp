@@ -15,6 +15,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/object_ptr.h>
 #include <torch/csrc/utils/pybind.h>
+#include <torch/version.h>
 
 #include "vdmq.h"
 
@@ -24,6 +25,7 @@ decltype(&vdmq_linear_bf6_ex) linear_bf6_ex;
 decltype(&vdmq_linear_bf6_workspace) linear_bf6_workspace;
 decltype(&vdmq_pack_weight) pack_weight;
 
+constexpr int kInterface = 1; /* of the functions below; the package compares it with its own */
 constexpr int64_t kMaxK = 16384; /* what the quantizers that write bf6 blocks take */
 
 // Nothing intercepts operations: no __torch_function__ mode, no __torch_dispatch__ mode, no functorch transform.
@@ -223,4 +225,11 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_vdmq_host", nullptr, -1, methods,
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__vdmq_host(void) { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__vdmq_host(void) {
+    PyObject *const m = PyModule_Create(&module);
+    if (m != nullptr && (PyModule_AddIntConstant(m, "interface", kInterface) != 0 || PyModule_AddStringConstant(m, "torch_version", TORCH_VERSION) != 0)) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
+}

@@ -412,7 +412,7 @@ def _native_linear(x: torch.Tensor, weight, bias: Optional[torch.Tensor], clip_r
                    act: int = 0, ln=(0, 0.0, None, None, 1), residual=None, gate=None, split_cols: int = 0, views: int = 0):
     """The whole call in the extension module (vdmq_host.cpp) where its operands are plain and the bf6 path is the library's choice; None: they
     are not, and nothing has been done.  ``weight``: ``(qweight, wscales)`` as the caller was given them, or a PreparedWeight."""
-    if _MATRIX_PATH != "auto":
+    if _MATRIX_PATH != "auto" or _lib.host is None:
         return None
     qweight, wscales, sizes = (*weight, None) if type(weight) is tuple else (weight, None, (weight.N, weight.K))
     out = _lib.host.linear(_operands, x, shape, qweight, wscales, sizes, check[0], check[1], bias, clip_ratio, act, ln[0], ln[1], ln[2], ln[3], ln[4], residual,
@@ -621,7 +621,7 @@ def quantize_weight_per_channel(weight: torch.Tensor):
 
 def _native_pack(weight: torch.Tensor, channel_scale: Optional[torch.Tensor]):
     # (for the int8 path's rows the pass writes that path's form too)
-    if _MATRIX_PATH == "int8":
+    if _MATRIX_PATH == "int8" or _lib.host is None:
         return None
     index = torch._C._cuda_getDevice()
     out = _lib.host.pack(weight, channel_scale, index, torch._C._cuda_getCurrentRawStream(index))

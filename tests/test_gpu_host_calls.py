@@ -202,6 +202,23 @@ def test_refused_calls_leave_a_prepared_weight_as_it_was(operands):
     assert pw.native is None and pw.bf6 is not None
 
 
+def test_calls_without_the_extension_module(operands, monkeypatch):
+    from dsaquant_amd import _lib, fused_ops as F
+
+    v, o = vk(), operands
+    x, qw, ws, b = o["x"], o["qw"], o["ws"], o["b"]
+    parts = [t for pair in zip(qw.chunk(3), ws.chunk(3)) for t in pair]
+    calls = (lambda: v.linear_vdm_w4a4(x, qw, ws, b, 0.95), lambda: v.linear_vdm_w4a4_prepared(x, v._prepared_weight(qw, ws), b, 0.95, split_cols=128),
+             lambda: torch.cat(v.linear_vdm_w4a4_qkv(x, *parts, clip_ratio=0.95, w_qkv_packed=qw, w_qkv_scale=ws, qkv_bias_half=b)),
+             lambda: F.linear_fused(x, qw, ws, b, 0.95, act="gelu_tanh", residual=o["res"], gate=o["gate"]),
+             lambda: F.linear_ln_vdm_w4a4(F.LnInput(x, o["a"], o["shift"], 1e-6), qw, ws, b, 0.95),
+             lambda: v.quantize_weight_per_channel(o["w"])[0], lambda: v.pack_weight_with_scale(o["w"], o["s"])[1])
+    want = [c() for c in calls]
+    monkeypatch.setattr(_lib, "host", None)
+    for c, w in zip(calls, want):
+        assert torch.equal(c().view(torch.uint8), w.view(torch.uint8))
+
+
 def test_on_the_current_stream_and_in_a_graph(operands):
     v, o = vk(), operands
     x = o["x"].clone()

@@ -612,6 +612,35 @@ def test_packing_asks_for_the_library_first(monkeypatch, pack):
     assert v.load_error() is reason
 
 
+def test_extension_module_is_built_for_this_interpreter_and_torch():
+    import sysconfig
+
+    from dsaquant_amd import _lib
+
+    _lib.load()
+    assert _lib.host is not None and _lib.host.interface == _lib.HOST_INTERFACE
+    assert _lib.host.__file__.endswith("_vdmq_host" + sysconfig.get_config_var("EXT_SUFFIX"))
+
+
+@pytest.mark.parametrize("found", [None, dict(interface=0, torch_version=torch.__version__.split("+")[0]), dict(interface=1, torch_version="1.0.0"), {}])
+def test_library_loads_without_the_extension_module(monkeypatch, found):
+    """Not built, or built for another package or torch: the library serves every call all the same, and a warning says why."""
+    import sys
+    from types import SimpleNamespace
+
+    from dsaquant_amd import _lib
+
+    def init(*_):
+        raise AssertionError("a module of another interface was called")
+
+    monkeypatch.setattr(_lib, "_LIB", None)
+    monkeypatch.setattr(_lib, "host", None)
+    monkeypatch.setitem(sys.modules, "dsaquant_amd._vdmq_host", None if found is None else SimpleNamespace(init=init, **found))
+    with pytest.warns(RuntimeWarning, match="_vdmq_host"):
+        lib = _lib.load()
+    assert lib.vdmq_version() == _lib.VDMQ_VERSION and _lib.load() is lib and _lib.host is None
+
+
 def test_header_is_plain_c_and_a_c_host_links_the_library(tmp_path):
     """include/vdmq.h is what a C or C++ host of the reference's kernels would include: it must compile as C99 with
     every warning an error, and a C program must link libvdmq.so by its declarations alone.  The program calls the
