@@ -25,7 +25,7 @@ VDMQ_ACT_GELU_TANH = 1
 VDMQ_LN_MODULATE = 1
 VDMQ_LN_AFFINE = 2
 VDMQ_LINEAR_BF6_MIN_K = 640
-HOST_INTERFACE = 1  # the arguments of _vdmq_host's functions (kInterface in vdmq_host.cpp)
+HOST_INTERFACE = 2  # the arguments of _vdmq_host's functions (kInterface in vdmq_host.cpp)
 
 
 class GemmLaunchInfo(ctypes.Structure):

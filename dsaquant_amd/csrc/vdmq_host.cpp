@@ -25,7 +25,7 @@ decltype(&vdmq_linear_bf6_ex) linear_bf6_ex;
 decltype(&vdmq_linear_bf6_workspace) linear_bf6_workspace;
 decltype(&vdmq_pack_weight) pack_weight;
 
-constexpr int kInterface = 1; /* of the functions below; the package compares it with its own */
+constexpr int kInterface = 2; /* of the functions below; the package compares it with its own */
 constexpr int64_t kMaxK = 16384; /* what the quantizers that write bf6 blocks take */
 
 // Nothing intercepts operations: no __torch_function__ mode, no __torch_dispatch__ mode, no functorch transform.
@@ -208,6 +208,19 @@ PyObject *pack(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     END_HANDLE_TH_ERRORS
 }
 
+// plain(tensors...): whether tensor operations on them can be replaced by a kernel without anybody noticing: torch's own class over ordinary device
+// memory, nothing that intercepts operations, and no tangent of forward-mode differentiation on any of them.
+PyObject *plain_tensors(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    if (!plain_calls()) Py_RETURN_FALSE;
+    for (Py_ssize_t i = 0; i < nargs; ++i) {
+        const at::Tensor *const t = plain(args[i]);
+        if (t == nullptr || t->_fw_grad(0).defined()) Py_RETURN_FALSE;
+    }
+    Py_RETURN_TRUE;
+    END_HANDLE_TH_ERRORS
+}
+
 PyObject *init(PyObject *, PyObject *args) {
     unsigned long long linear_at, workspace_at, pack_at;
     if (!PyArg_ParseTuple(args, "KKK", &linear_at, &workspace_at, &pack_at)) return nullptr;
@@ -219,6 +232,7 @@ PyObject *init(PyObject *, PyObject *args) {
 
 PyMethodDef methods[] = {{"init", init, METH_VARARGS, "addresses of vdmq_linear_bf6_ex, vdmq_linear_bf6_workspace and vdmq_pack_weight"},
                          {"linear", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(linear)), METH_FASTCALL, "a linear on plain operands, or None"},
+                         {"plain", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(plain_tensors)), METH_FASTCALL, "whether a kernel may stand in for operations on these tensors"},
                          {"pack", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(pack)), METH_FASTCALL, "a weight's packed buffers, or None"},
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_vdmq_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

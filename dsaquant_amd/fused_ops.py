@@ -384,10 +384,21 @@ def rms_norm_exact(xs, weights, eps: float, floats: bool = False):
     return outs
 
 
+def _unseen(*tensors: torch.Tensor) -> bool:
+    # Whether nobody sees a difference between tensor operations on these and a kernel with their bits: no mode, transform, trace or
+    # tangent.  Without the extension module, which knows (a linear in front has loaded it): not.
+    return _lib.host is not None and not torch.compiler.is_compiling() and _lib.host.plain(*tensors)
+
+
+def rms_norm_exact_supported(xs, weights, heads: int) -> bool:
+    """Whether ``rms_norm_exact`` may stand in for the tensor operations on these operands."""
+    return _unseen(*xs, *weights) and rms_norm_rope_supported(xs, weights, None, heads)
+
+
 def modulate_supported(y: torch.Tensor, a: torch.Tensor, b: torch.Tensor) -> bool:
-    """Whether ``modulate`` takes these operands."""
+    """Whether ``modulate`` may stand in for the tensor operations on these operands."""
     grad = torch.is_grad_enabled()
-    return (y.is_cuda and y.dtype == torch.float32 and y.is_contiguous() and y.dim() == 3 and y.shape[2] % 8 == 0 and y.numel() > 0 and y.data_ptr() % 16 == 0
+    return (_unseen(y, a, b) and y.is_cuda and y.dtype == torch.float32 and y.is_contiguous() and y.dim() == 3 and y.shape[2] % 8 == 0 and y.numel() > 0 and y.data_ptr() % 16 == 0
             and not (grad and y.requires_grad)
             and all(t.dtype == torch.float16 and t.device == y.device and t.numel() == y.shape[2] and t.is_contiguous() and t.data_ptr() % 16 == 0
                     and not (grad and t.requires_grad) for t in (a, b)))

@@ -269,7 +269,7 @@ class Attention(nn.Module):
         from . import fused_ops
 
         return (self._projected_on_kernels() and all(_is_plain_norm(n) and n.eps == norms[0].eps for n in norms)
-                and fused_ops.rms_norm_rope_supported(tensors, [n.weight for n in norms], None, self.heads))
+                and fused_ops.rms_norm_exact_supported(tensors, [n.weight for n in norms], self.heads))
 
     def _kernel_norm(self, tensors, norms, freqs) -> bool:
         from . import fused_ops

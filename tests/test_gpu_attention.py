@@ -343,6 +343,92 @@ def test_norm_around_its_means_has_the_bits_of_the_tensor_operations(B, L, K, pa
         _same_bits(f.modulate(y, a, b), y.half() * (1 + a) + b)
 
 
+def _small_model():
+    from dataclasses import replace
+
+    from dsaquant_amd import wan_harness as W
+
+    args = replace(W.WAN21_1P3B, num_layers=1, num_heads=2, ffn_dim=512, text_dim=128)
+    return W.build_quantized(args, DEV, seed=12), args
+
+
+@pytest.mark.parametrize("kind", ["function", "dispatch"])
+def test_operation_modes_see_the_norms_and_the_modulation(monkeypatch, kind):
+    """What no switch turns on is not there for who watches the tensor operations: every one of the norms and the head's reaches a mode."""
+    from collections import Counter
+
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from dsaquant_amd import fused_ops
+
+    model, args = _small_model()
+    g = torch.Generator(device=DEV).manual_seed(13)
+    latent = torch.randn((1, 16, 1, 6, 10), generator=g, device=DEV).half()
+    ctx, t = torch.randn((1, 77, args.text_dim), generator=g, device=DEV).half(), torch.tensor([500.0], device=DEV)
+
+    class Functions(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen[getattr(func, "__name__", str(func))] += 1
+            return func(*args, **(kwargs or {}))
+
+    class Dispatched(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen[str(func)] += 1
+            return func(*args, **(kwargs or {}))
+
+    def under_mode():
+        with (Functions if kind == "function" else Dispatched)():
+            return model(latent, t, ctx)
+
+    with torch.no_grad():
+        want = model(latent, t, ctx)
+        seen = Counter()
+        got, first = under_mode(), seen
+        monkeypatch.setattr(fused_ops, "rms_norm_exact_supported", lambda *a: False)
+        monkeypatch.setattr(fused_ops, "modulate_supported", lambda *a: False)
+        seen = Counter()
+        under_mode()
+    assert torch.equal(got, want)
+    for name in ("rsqrt", "pow", "mean") if kind == "function" else ("aten.rsqrt.default", "aten.pow.Tensor_Scalar", "aten.mean.dim", "aten.mul.Tensor", "aten.add.Tensor"):
+        assert first[name] == seen[name] > 0
+
+
+def test_tangents_pass_the_norms_and_the_head():
+    """Forward-mode differentiation through the residual stream does not end, unnoticed, at a norm or at the head."""
+    import torch.autograd.forward_ad as fwad
+
+    model, args = _small_model()
+    attn = model.blocks[0].attn1
+    g = torch.Generator(device=DEV).manual_seed(14)
+    rnd = lambda *shape: torch.randn(*shape, generator=g, device=DEV).half()  # noqa: E731
+    x, t, scale, shift = rnd(1, 40, args.dim), rnd(1, 40, args.dim), rnd(1, 1, args.dim), rnd(1, 1, args.dim)
+    with torch.no_grad():
+        attn.to_q(x)  # (loads the library)
+        plain = attn._normed(x, attn.norm_q), model._head_norm(x, scale, shift)
+        with fwad.dual_level():
+            dual = fwad.make_dual(x, t)
+            for out, want in zip((attn._normed(dual, attn.norm_q), model._head_norm(dual, scale, shift)), plain):
+                primal, tangent = fwad.unpack_dual(out)
+                assert tangent is not None and torch.isfinite(tangent).all() and torch.equal(primal, want)
+            out = model._head_norm(x, scale, fwad.make_dual(shift, scale))
+            assert fwad.unpack_dual(out).tangent is not None
+
+
+def test_norm_kernels_leave_subclasses_alone():
+    from dsaquant_amd import fused_ops as f
+
+    class Sub(torch.Tensor):
+        pass
+
+    model, args = _small_model()
+    x = torch.ones((1, 8, args.dim), device=DEV).half()
+    w = [torch.ones(args.dim, device=DEV).half()]
+    model.blocks[0].attn1.to_q(x)
+    assert f.rms_norm_exact_supported([x], w, 2) and not f.rms_norm_exact_supported([x.as_subclass(Sub)], w, 2)
+    assert isinstance(model._head_norm(x.as_subclass(Sub), x[:, :1], x[:, :1]), Sub)
+
+
 @pytest.mark.parametrize("frames,h,w", [(1, 6, 10), (2, 10, 14), (3, 34, 50)])
 def test_harness_forward_keeps_its_bits_on_the_norm_kernels(monkeypatch, frames, h, w):
     from dataclasses import replace

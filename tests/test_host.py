@@ -622,7 +622,7 @@ def test_extension_module_is_built_for_this_interpreter_and_torch():
     assert _lib.host.__file__.endswith("_vdmq_host" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 
-@pytest.mark.parametrize("found", [None, dict(interface=0, torch_version=torch.__version__.split("+")[0]), dict(interface=1, torch_version="1.0.0"), {}])
+@pytest.mark.parametrize("found", [None, dict(interface=0, torch_version=torch.__version__.split("+")[0]), dict(interface=2, torch_version="1.0.0"), {}])
 def test_library_loads_without_the_extension_module(monkeypatch, found):
     """Not built, or built for another package or torch: the library serves every call all the same, and a warning says why."""
     import sys
