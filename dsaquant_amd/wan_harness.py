@@ -217,6 +217,7 @@ class Attention(nn.Module):
         then runs in the output projection's GEMM epilogue if that projection is in kernel mode)."""
         from . import fused_ops
 
+        rotated = None  # the type of q's and k's values where they come as floats of them
         if context is not None and (self.cache_cross_kv or isinstance(context, SharedContext)):
             tq = self.to_q
             if isinstance(x, fused_ops.LnInput):
@@ -241,12 +242,13 @@ class Attention(nn.Module):
                 q, k = fused_ops.rms_norm_rope((q, k), (self.norm_q.weight, self.norm_k.weight), self.norm_q.eps, freqs, self.heads)
                 freqs = None  # (the rotation is in it)
             elif context is None and self._exact_norm((q, k), (self.norm_q, self.norm_k)):
+                rotated = q.dtype
                 q, k = fused_ops.rms_norm_exact((q, k), (self.norm_q.weight, self.norm_k.weight), self.norm_q.eps, floats=freqs is not None)
             else:
                 q, k = self._normed(q, self.norm_q), self._normed(k, self.norm_k)
         q, k, v = (t.unflatten(2, (self.heads, -1)) for t in (q, k, v))
         if freqs is not None:
-            q, k = apply_rope(q, freqs, v.dtype), apply_rope(k, freqs, v.dtype)
+            q, k = apply_rope(q, freqs, rotated), apply_rope(k, freqs, rotated)
         if timers is not None:
             timers.start("attention")
         if self._on_kernels() and fused_ops.attention_supported(q, k, v):

@@ -197,6 +197,20 @@ def test_attention_module_against_written_out_sequence():
         assert torch.allclose(att(x, ctx, None), written_out(x, ctx, None), atol=1e-5, rtol=1e-5)
 
 
+def test_rotation_keeps_the_type_of_the_rows_it_rotates():
+    """q and k leave the rotary embedding in their own type: norms that widen them meet v in the attention as they would without it."""
+    torch.manual_seed(5)
+    att = W.Attention(256, 2, 1e-6, cross=False).half()
+    att.norm_q.float()
+    att.norm_k.float()
+    x, freqs = torch.randn(1, 4, 256).half(), W.rope_frequencies(128, 1, 2, 2, "cpu")
+    with torch.no_grad():
+        assert att.norm_q(att.to_q(x)).dtype == torch.float32
+        for f in (None, freqs):
+            with pytest.raises(RuntimeError, match="same dtype"):
+                att(x, None, f)
+
+
 def _meta_packed_checkpoint(model):
     """A packed checkpoint of meta tensors with the shapes the loader expects."""
     from dsaquant_amd.checkpoints import packed_checkpoint as pc
