@@ -93,7 +93,12 @@ class LnInput:
             self._rows = tuple(_k._half_rows(t, self.shape[-1]) for t in self._given)
         return self._rows[i]
 
-    x, a, b = (property(lambda self, i=i: self._two_d(i)) for i in range(3))
+    def _replace(self, i: int, rows: torch.Tensor) -> None:
+        kept = [self._two_d(j) for j in range(3)]
+        kept[i] = rows
+        self._rows = tuple(kept)
+
+    x, a, b = (property(lambda self, i=i: self._two_d(i), lambda self, rows, i=i: self._replace(i, rows)) for i in range(3))
 
     def _args(self):
         M, K = self.x.shape

@@ -82,6 +82,10 @@ def test_served_calls(operands):
     for a, s in ((o["a"], o["shift"]), (o["a"][0, 0], o["shift"][0, 0])):
         same(lambda: F.linear_ln_vdm_w4a4(F.LnInput(x, a, s, 1e-6), qw, ws, b, 0.95), True)
     same(lambda: F.linear_fused(F.LnInput(x.float(), o["a"], o["shift"], 1e-6, "affine"), qw, ws, b, 0.95, residual=o["res"]), True)
+    pre = F.LnInput(x, o["a"], o["a"], 1e-6)
+    pre.b = o["shift"].view(2, K)
+    same(lambda: F.linear_ln_vdm_w4a4(pre, qw, ws, b, 0.95), True)
+    assert torch.equal(F.linear_ln_vdm_w4a4(pre, qw, ws, b, 0.95), F.linear_ln_vdm_w4a4(F.LnInput(x, o["a"], o["shift"], 1e-6), qw, ws, b, 0.95))
     same(lambda: v.quantize_weight_per_channel(o["w"]), True)
     same(lambda: v.pack_weight_with_scale(o["w"], o["s"].view(-1, 1)), True)
     with torch.inference_mode():

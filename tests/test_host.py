@@ -612,6 +612,23 @@ def test_packing_asks_for_the_library_first(monkeypatch, pack):
     assert v.load_error() is reason
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_layer_norm_input_takes_other_rows_and_vectors(dtype):
+    """x, a and b of a LayerNorm input are attributes: read as rows of K fp16 values, and assignable."""
+    from dsaquant_amd.fused_ops import LnInput
+
+    x, a, b = torch.randn(2, 3, 128).to(dtype), torch.randn(2, 1, 128).to(dtype), torch.randn(2, 1, 128).to(dtype)
+    pre = LnInput(x, a, b, 1e-6)
+    for name, given in (("x", x), ("a", a), ("b", b)):
+        other = torch.randn(given.numel() // 128, 128).half()
+        setattr(pre, name, other)
+        assert getattr(pre, name) is other
+    assert pre._args()[:4] == (pre.x.data_ptr(), 6, 128, 128) and pre._args()[6:] == (pre.a.data_ptr(), pre.b.data_ptr(), 128, 3)
+    pre = LnInput(x, a, b, 1e-6)
+    pre.b = other
+    assert torch.equal(pre.x, x.half().view(6, 128)) and torch.equal(pre.a, a.half().view(2, 128)) and pre.b is other
+
+
 def test_extension_module_is_built_for_this_interpreter_and_torch():
     import sysconfig
 
