@@ -668,6 +668,8 @@ def _linear_2d(x_2d: torch.Tensor, weight: PreparedWeight, bias: Optional[torch.
     M, K = x_2d.shape
     N = weight.N
     dev = x_2d.device
+    if weight.K != K:  # (a cached concatenation need not be of the projections an entry has looked at)
+        raise ValueError("qweight shape must be [N, K/2]")
     _require(weight.device == dev, "weights and input must be on the same device")
     if bias is not None:
         _check_device_tensor(bias, "bias", torch.float16)

@@ -184,6 +184,12 @@ def test_rows_of_another_length_than_a_prepared_weights(operands, other):
                 calls = [lambda: get_qkv_projections(attn, x, x), lambda: F.kv_projections(attn, x)]
             for call in calls:
                 assert same(call, False) == (ValueError, "qweight shape must be [N, K/2]")
+    # a cached concatenation of another row length than the projections it is said to be of
+    g = torch.Generator(device="cuda").manual_seed(5)
+    part = v.pack_weight_with_scale(torch.randn((128, other), generator=g, device="cuda").half(), torch.ones(128, device="cuda").half())[:2]
+    for contiguous in (False, True):
+        assert same(lambda: v.linear_vdm_w4a4_qkv(x, *part, *part, *part, clip_ratio=0.95, w_qkv_packed=qw, w_qkv_scale=ws, contiguous_outputs=contiguous),
+                    False) == (ValueError, "qweight shape must be [N, K/2]")
 
 
 def test_refused_calls_leave_a_prepared_weight_as_it_was(operands):

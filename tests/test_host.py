@@ -593,6 +593,18 @@ def test_rows_handed_to_the_library_lie_k_apart(dtype):
     assert v._half_rows(ready, K) is ready
 
 
+@pytest.mark.parametrize("K", [640, 768])
+def test_rows_and_weight_of_different_length_never_reach_the_library(K):
+    """Whatever an entry has checked, the rows' length is compared with that of the very weight that is multiplied by."""
+    from types import SimpleNamespace
+
+    from dsaquant_amd.kernels import vdm_w4a4 as v
+
+    weight = SimpleNamespace(K=704, N=128, device=torch.device("cpu"))
+    with pytest.raises(ValueError, match=r"qweight shape must be \[N, K/2\]"):
+        v._linear_2d(torch.zeros(4, K).half(), weight, None, 1.0)
+
+
 @pytest.mark.parametrize("pack", ["quantize_weight_per_channel", "pack_weight_with_scale"])
 def test_packing_asks_for_the_library_first(monkeypatch, pack):
     """Without the library packing fails with the reason, which load_error() keeps, whatever it was given."""
