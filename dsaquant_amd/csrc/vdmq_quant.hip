@@ -665,7 +665,11 @@ int64_t resident_workgroups(const void *kernel, int threads, int (&cache)[kMaxDe
 //                    12000 x 3072 18.1 / 18.8   32760 x 1536 23.4 / 24.1
 //   GELU             512 x 5120 8.3 / 6.3   2500 x 10240 31.9 / 25.1   4680 x 8960 36.0 / 31.0   32760 x 1536 34.4 / 32
 //                    streamed / plain stores: 32760 x 8960 151 / 142, with its GEMM 384 / 366; 60000 x 7168 197 / 218, 32760 x 13824 240 / 272
-// Rows that are only quantized keep eight where there are many short ones.  With the activation evaluated late (bf6_late_act) four and plain stores
+// Rows that are only quantized keep eight where there are many short ones, and where long ones (a CU holds one workgroup of eight or two of
+// four, the chip 2048 rows) fill more than half of the last round: then four have only the shorter runs.  After one round, us, eight / four: 3328 x
+// 8960 17.1 / 18.3, 4096 x 8960 19.1 / 20.6, 3840 x 7168 15.5 / 16.1, 4096 x 13824 30.6 / 31.4 (2304 x 8960 15.4 / 13.8, 4608 x 13824 37.2 / 33.8); after
+// two 5376 x 13824 39.4 / 41.9, 6144 x 8960 29.7 / 31.5, 6144 x 5632 18.9 / 19.5; after three 7168 x 13824 53.3 / 55.8, 7424 x 12288 47.7 / 50.0, 8192 x 16384 77.1 / 79.0, but 7936 x 8960 37.8 / 37.2.
+// Beyond 10240 elements and four rounds eight in any case: 11776 x 13824 84.5 / 87.7, 9216 x 16384 87.5 / 90.4.  With the activation evaluated late (bf6_late_act) four and plain stores
 // still win while the output stays in the memory-side cache.
 struct Bf6Split {
     int rows, stream_out;
@@ -674,7 +678,9 @@ template <int NCH, int ACT>
 Bf6Split bf6_split(int64_t M, int64_t K) {
     const int64_t bytes = bf6_bytes(M, K);
     const bool large = bytes > kStreamOutBytesBf6;
-    const bool four = ACT == VDMQ_ACT_NONE ? !large && (M <= 5120 || K > 3584)
+    const bool full_round = M > 2048 && M <= (K > 10240 ? 8192 : 7680) && (M - 1) % 2048 >= (M > 6144 ? 896 : 1024) && K > (M > 5120 && M <= 6144 ? 5120 : 6144);
+    const bool many_long = M > 8704 && K > 10240;
+    const bool four = ACT == VDMQ_ACT_NONE ? !large && (M <= 5120 || K > 3584) && !full_round && !many_long
                                            : !large || (bf6_late_act(NCH) && K <= 9216 && bytes <= kInfinityCacheBytes);
     return four ? Bf6Split{kPanelRows / 2, 0} : Bf6Split{kPanelRows, large ? 1 : 0};
 }

@@ -93,6 +93,7 @@ def by_row(blocks, rows):
 
 
 @pytest.mark.parametrize("M,K,producer", [(5121, 1536, None), (5121, 3584, None), (5123, 3648, None), (12999, 13824, None), (20001, 9216, None),
+                                          (3073, 6208, None), (4096, 13824, None), (5633, 5184, None), (7041, 8960, None), (7681, 8960, None), (8192, 10304, None), (8705, 10304, None),
                                           (5121, 1536, "gelu_tanh"), (20001, 9216, "gelu_tanh"), (20001, 9280, "gelu_tanh"), (40005, 8960, "gelu_tanh"),
                                           (13, 1536, "modulate"), (2347, 1536, "modulate"), (2347, 8960, "modulate"),
                                           (35005, 5120, "modulate")])
