@@ -43,12 +43,13 @@ struct Pair {
     static constexpr int kSets = SETS_;
     static constexpr int MB = MB_, NB = NB_, BM = 32 * MB, BN = 32 * NB, OB = MB / 2; /* OB: token blocks a wave keeps */
     static constexpr int kUnit = (2 * MB + 2 * NB) * kFrag;                            /* bytes of 128 k of the tile's operands */
-    static constexpr int kLdsMax = 160 * 1024, S = (kLdsMax - 2048) / kUnit < 6 ? (kLdsMax - 2048) / kUnit : 6;
+    static constexpr int kLdsMax = 160 * 1024, S = (kLdsMax - 2048) / kUnit; /* units the ring holds */
+    static constexpr int kMinUnits = S + 1; /* the K loop fills the ring in front and refills it at least once */
     static constexpr int kLoadsAll = kUnit / 1024, kLoads = (kLoadsAll + kWaves - 1) / kWaves;
     static constexpr int kArea = OB * NB * 1024, kStageRow = NB * 32 + 16;
     static constexpr int kSideBytes = (BM + 2 * BN) * 2; /* fp16 token scales, channel scales and bias */
     static constexpr int kSideAt = S * kUnit > kWaves * kArea ? S * kUnit : kWaves * kArea, kLds = kSideAt + kSideBytes;
-    static_assert(MB % 2 == 0 && kUnit % 1024 == 0 && S >= 3 && kLds <= kLdsMax, "the ring, the sums and the side vectors fit LDS");
+    static_assert(MB % 2 == 0 && kUnit % 1024 == 0 && S >= 4 && S <= 5 && kLds <= kLdsMax, "the ring, the sums and the side vectors fit LDS");
     static_assert(OB * 16 * kStageRow <= kArea, "a wave's outputs are staged where it received its sums");
     static_assert(kLoads * (S - 2) < 64, "vmcnt is a 6-bit counter");
 };
@@ -99,9 +100,8 @@ struct PairKLoop {
         constexpr int lgkm = READ ? 0 : 15;
         const int n = units - 2 - at.p;
         if (STEADY || n >= S - 2) __builtin_amdgcn_s_waitcnt(waitcnt_imm((S - 2) * L, lgkm));
-        else if (S >= 6 && n == 3) __builtin_amdgcn_s_waitcnt(waitcnt_imm(3 * L, lgkm));
-        else if (S >= 5 && n == 2) __builtin_amdgcn_s_waitcnt(waitcnt_imm(2 * L, lgkm));
-        else if (S >= 4 && n == 1) __builtin_amdgcn_s_waitcnt(waitcnt_imm(L, lgkm));
+        else if (S == 5 && n == 2) __builtin_amdgcn_s_waitcnt(waitcnt_imm(2 * L, lgkm));
+        else if (n == 1) __builtin_amdgcn_s_waitcnt(waitcnt_imm(L, lgkm));
         else __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, lgkm));
         lds_barrier();
         advance(at);
@@ -162,16 +162,12 @@ struct PairKLoop {
     __device__ __forceinline__ void run(Acc &acc, int group, Hook &&first_read) const {
 #pragma unroll
         for (int u = 0; u < S; ++u)
-            if (u < units) {
 #pragma unroll
-                for (int i = 0; i < L; ++i) load_one(i, u, u * Cfg::kUnit);
-            }
-        if (units >= S) __builtin_amdgcn_s_waitcnt(waitcnt_imm((S - 1) * L, 15));
-        else __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 15));
+            for (int i = 0; i < L; ++i) load_one(i, u, u * Cfg::kUnit);
+        __builtin_amdgcn_s_waitcnt(waitcnt_imm((S - 1) * L, 15));
         lds_barrier();
         Place at = {0, 0, kRing - Cfg::kUnit};
         if (group == 1) end_phase<L, false, false>(at);
-        if (group >= units) return first_read(); /* a single unit, the other group's */
         WFrags wf;
         XFrags x0;
         v8i w0;
@@ -351,6 +347,7 @@ int launch_cfg(PairArgs &args, hipStream_t s) {
     using Kernel = void (*)(const PairArgs);
     const Kernel kernels[2] = {gemm_bf6_pair_kernel<Cfg, false>, gemm_bf6_pair_kernel<Cfg, true>};
     const bool has_tail = args.tail.gate != nullptr || args.tail.residual != nullptr;
+    if (args.kblocks / 2 < Cfg::kMinUnits) return fail(VDMQ_ESHAPE, "gemm_bf6_pair_kernel needs K >= %d", 128 * Cfg::kMinUnits - 127);
     args.tiles_m = static_cast<int>(ceil_div(args.M, Cfg::BM));
     args.tiles_n = static_cast<int>(ceil_div(args.N, Cfg::BN));
     const int tiles = args.tiles_m * args.tiles_n, per_xcd = static_cast<int>(ceil_div(tiles, kXcds));
