@@ -94,32 +94,47 @@ def by_row(blocks, rows):
 
 @pytest.mark.parametrize("M,K,producer", [(5121, 1536, None), (5121, 3584, None), (5123, 3648, None), (12999, 13824, None), (20001, 9216, None),
                                           (3073, 6208, None), (4096, 13824, None), (5633, 5184, None), (7041, 8960, None), (7681, 8960, None), (8192, 10304, None), (8705, 10304, None),
-                                          (5121, 1536, "gelu_tanh"), (20001, 9216, "gelu_tanh"), (20001, 9280, "gelu_tanh"), (40005, 8960, "gelu_tanh"),
-                                          (13, 1536, "modulate"), (2347, 1536, "modulate"), (2347, 8960, "modulate"),
-                                          (35005, 5120, "modulate")])
+                                          (5121, 1536, "gelu_tanh"), (20001, 9216, "gelu_tanh"), (20001, 9280, "gelu_tanh"), (40005, 8960, "gelu_tanh")])
 def test_whole_and_half_panel_workgroups(M, K, producer):
     """A workgroup takes a panel of eight rows or half of one, by the number of rows, their length, the producer in front and the
     size of the output: on both sides of those lines the rows' codes and scales are those of the same rows in slices of 2048, which
     workgroups of four or fewer rows serve (and which the other tests compare with the oracle)."""
-    from dsaquant_amd import fused_ops
-
     v = vk()
     g = torch.Generator("cuda").manual_seed(M)
     x = torch.randn(M, K, generator=g, device="cuda").half()
-    vectors = [0.1 * torch.randn(1, K, generator=g, device="cuda").half() for _ in range(2)]
-
-    def quantize(rows):
-        if producer == "modulate":
-            return fused_ops.LnInput(rows, *vectors, 1e-6, producer).quantize(0.95, bf6=True)
-        return v.quantize_activation_bf6(rows, 0.95, act=producer)
-
-    blocks, scales = quantize(x)
+    blocks, scales = v.quantize_activation_bf6(x, 0.95, act=producer)
     whole = by_row(blocks, M)
     for r in range(0, M, 2048):
         rows = x[r:r + 2048]
-        part, part_scales = quantize(rows)
+        part, part_scales = v.quantize_activation_bf6(rows, 0.95, act=producer)
         assert torch.equal(scales[r:r + 2048], part_scales)
         assert all(torch.equal(w[r:r + 2048], p) for w, p in zip(whole, by_row(part, len(rows))))
+
+
+@pytest.mark.parametrize("mode", ["modulate", "affine"])
+@pytest.mark.parametrize("M,K", [(517, 64), (517, 1536), (517, 1600), (517, 3072), (517, 5120), (517, 8960), (517, 13824), (517, 16384), (2347, 1536),
+                                 (2347, 8960), (35005, 5120)])
+def test_layer_norm_with_two_and_four_rows_per_workgroup(M, K, mode):
+    """Behind a LayerNorm up to 512 rows go by twos and more by fours (the last group of either not full): the first and the last rows
+    of a call have the codes and scales that they have in calls of their own, of either kind."""
+    from dsaquant_amd import fused_ops
+
+    g = torch.Generator("cuda").manual_seed(K)
+    x = torch.randn(M, K, generator=g, device="cuda").half()
+    x[3::41] = 0
+    x[5, K - 1], x[8, 3], x[511, 0] = float("inf"), float("nan"), 65504
+    vectors = [0.1 * torch.randn(M, K, generator=g, device="cuda").half() for _ in range(2)]
+
+    def quantize(rows):
+        return fused_ops.LnInput(x[rows], *(t[rows] for t in vectors), 1e-6, mode).quantize(0.95, bf6=True)
+
+    blocks, scales = quantize(slice(M))
+    by_fours = by_row(blocks, M)
+    for n in (1, 2, 13, 511, 512, 513):
+        for rows in (slice(n), slice(M - n, M)):
+            part, part_scales = quantize(rows)
+            assert torch.equal(scales[rows].view(torch.int16), part_scales.view(torch.int16))
+            assert all(torch.equal(w[rows], p) for w, p in zip(by_fours, by_row(part, n)))
 
 
 @pytest.mark.parametrize("act", [None, "gelu_tanh"])
