@@ -40,14 +40,6 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 #define VDMQ_GLOBAL_PTR(p) ((const __attribute__((address_space(1))) void *)(p))
 #define VDMQ_LDS_PTR(p) ((__attribute__((address_space(3))) void *)(p))
 
-[[maybe_unused]] constexpr int waitcnt_imm(int vm, int lgkm) { return (vm & 15) | ((vm >> 4) << 14) | (7 << 4) | ((lgkm & 15) << 8); }
-
-[[maybe_unused]] __device__ __forceinline__ void lds_barrier() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
-
 constexpr int kBlkBytes = 1536;                 /* 32 rows x 64 k */
 [[maybe_unused]] constexpr int kBlkPlaneB = 1024;                /* offset of the 8-byte plane */
 constexpr int KS = 128;                         /* K step: two k-blocks per stage */

@@ -55,16 +55,6 @@ struct Pair {
 };
 
 #if defined(__HIP_DEVICE_COMPILE__)
-constexpr int waitcnt_imm(int vm, int lgkm) { return (vm & 15) | ((vm >> 4) << 14) | (7 << 4) | ((lgkm & 15) << 8); }
-
-__device__ __forceinline__ void lds_barrier() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
-#endif
-
-#if defined(__HIP_DEVICE_COMPILE__)
 // The K loop.  A phase is the time between two barriers.  Unit u (128 k) belongs to group u % 2, whose waves read it from LDS in phase u, while
 // they finish their previous unit, and work on it in phases u + 1 and u + 2: in every phase one group is in its first half and
 // the other, which reads, in its second.  The loads of phase p fill the slot that unit p - 1 has left.

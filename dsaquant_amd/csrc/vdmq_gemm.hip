@@ -45,16 +45,6 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 #define VDMQ_GLOBAL_PTR(p) ((const __attribute__((address_space(1))) void *)(p))
 #define VDMQ_LDS_PTR(p) ((__attribute__((address_space(3))) void *)(p))
 
-
-// s_waitcnt immediate for gfx9: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt[15:14]
-[[maybe_unused]] constexpr int waitcnt_imm(int vm, int lgkm) { return (vm & 15) | ((vm >> 4) << 14) | (7 << 4) | ((lgkm & 15) << 8); }
-
-[[maybe_unused]] __device__ __forceinline__ void lds_barrier() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
-
 [[maybe_unused]] __device__ __forceinline__ v4i widen(uint32_t p0, uint32_t p1) {
     v4i r;
     r[0] = static_cast<int>((p0 << 4) & 0xF0F0F0F0u);

@@ -15,6 +15,16 @@ constexpr int kKStep = 256;
 
 constexpr int kWaveSize = 64;
 
+// s_waitcnt immediate for gfx9: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt[15:14]
+constexpr int waitcnt_imm(int vm, int lgkm) { return (vm & 15) | ((vm >> 4) << 14) | (7 << 4) | ((lgkm & 15) << 8); }
+
+// A barrier that waits for nothing by itself: the caller waits for what the other waves are to see
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
 int fail(int code, const char *fmt, ...) __attribute__((format(printf, 2, 3)));
 int check_launch(const char *what);
 void record_gemm_launch(const vdmq_gemm_launch_info &info); /* what vdmq_last_gemm_launch reports */
