@@ -2,11 +2,13 @@
 // five sizes that gives the chip's 256 CUs at most one each, and two groups of four waves that take the tile's K in turns.
 //
 // 257 ... 512 tiles of 128 x 128 (vdmq_bf6.hip) are two on some CUs, which take two tiles' time however few they are, and just above
-// that 256 x 256 tiles leave half the CUs idle.  What bounds a tile's K loop is LDS, 128 bytes per clock: operands in, and out again once for
-// each wave that wants them.  With K divided between two groups a wave owns a quarter of the tile and four waves instead of eight read a
-// unit of 128 k: a 128 x 160 tile takes 630 cycles per unit, 83 KB through LDS (a 128 x 128 one of four waves 620 of 74 KB).  Eight waves
-// because four fetch only 30 ... 47 bytes per clock from L2, eight 60.  The sums of the two groups meet in LDS at the end (integers: exact
-// in any order), 1.3 us with the conversion.  GEMM alone, us, tiled / here: 512 x 10240, K 5120 25.6 / 21.4; 1021 x 4224, K 7680 36.3 /
+// that 256 x 256 tiles leave half the CUs idle.  A tile's operands go through LDS, in once and out again once for each wave that wants them.
+// With K divided between two groups a wave owns a quarter of the tile and four waves instead of eight read a unit of 128 k; eight waves
+// because four fetch only 30 ... 47 bytes per clock from L2, eight 60.  Cycles per unit by the counters (K = 7680 ... 15360), in brackets those in
+// which the matrix pipes work: 128 x 160 562 (320), 128 x 192 624 (384), 192 x 160 819 (480), 192 x 192 927 (576); the tiled kernel's 128 x
+// 128 with four waves 590 (256).  No pipe is full: of the 562 LDS works 216 for 55 KB of fragments, without a bank conflict, and 28 KB come in,
+// 49 bytes per clock.  The sums of the two groups meet in LDS at the end (integers: exact in any order); with launch, first loads and
+// stores what is not K loop takes 7.5 us of a 128 x 160 tile, 10 of a 192 x 192 one.  GEMM alone, us, tiled / here: 512 x 10240, K 5120 25.6 / 21.4; 1021 x 4224, K 7680 36.3 /
 // 27.0; 3589 x 1152, K 10432 48.9 / 33.4; 4355 x 1408, K 8640 42.4 / 35.6; 5579 x 1536, K 11072 81.7 / 56.5.
 #include <type_traits>
 

@@ -718,8 +718,9 @@ int launch_reg(const __half *x, int64_t M, int64_t K, int64_t ldx, float clip, i
 
 // Whether rows go to four waves each (quantize_row_parts_kernel): while a wave per row leaves CUs idle or with one workgroup.  us, a wave per row /
 // four: 64 x 2048 2.7 / 2.6, 512 x 5120 5.0 / 4.4, 512 x 13824 8.0 / 6.5, 1200 x 5120 6.6 / 6.3, 1200 x 13824 13.2 / 11.0; with the GELU 512 x 2048
-// 3.8 / 3.5, 512 x 5120 6.3 / 5.3, 800 x 5120 6.6 / 6.8, 512 x 13824 13.2 / 8.5, 1200 x 13824 21.0 / 16.8.  Beyond: 1200 x 2048 3.8 / 4.3, 3000 x 5120
-// 9.4 / 11.4, 2000 x 13824 15.8 / 16.5.
+// 3.8 / 3.5, 512 x 5120 6.3 / 5.3, 512 x 13824 13.2 / 8.5, 1200 x 13824 21.0 / 16.8.  Beyond: 1200 x 2048 3.8 / 4.3, 3000 x 5120
+// 9.4 / 11.4, 2000 x 13824 15.8 / 16.5.  One line for both producers, although the GELU's shortest rows are the same either way around 800 (x 5120
+// 6.6 / 6.8; a wave per row by eights, as such calls ran before, 8.7).
 constexpr int kPartRows = 2, kParts = 4;
 bool rows_in_parts(int64_t M, int64_t K) { return K > 1536 && M <= (K > 2560 ? 1536 : 512); }
 

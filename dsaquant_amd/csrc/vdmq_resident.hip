@@ -612,8 +612,10 @@ bool resident_takes(const ResidentProblem &p) {
         // timed with one set of buffers and with rows and weights of its own in every call, the choice takes 1.0035 of the faster
         // form's time in the geometric mean, over 1.06 at 2.3 % (always one kernel 1.0061 and 4.4 %, always two 1.20).
         // Two kernels count as never faster than 16 us, with gate and residual 20.5, which the host took for them when the line was drawn.  It
-        // takes 11.5 now (one: 8.2), and the two forms are within 8 % of each other where that matters: 1166 x 1472 -> 3200 with a
-        // residual 15.5 us as one kernel and 14.5 as two, 230 x 1536 -> 14848 with it 13.6 and 13.5, without 13.4 and 12.6.  Up to 2.5
+        // takes 11.5 now (one: 8.2), but the line stays: with 11.5 and 12 in its place 12 of 4000 problems of up to 40 million outputs
+        // would be two kernels, and as one they take 0.87 ... 1.09 of that time on the GPU, 0.98 in the mean (1166 x 1472 -> 3200 with a residual 13.8 us as
+        // one, 15.1 as two; the choice knowingly loses 205 x 1280 -> 30336, 16.3 and 15.0, and 230 x 1536 -> 14848, 13.9 and 12.9).  The tiled GEMM
+        // stands for two kernels here, also where K = 1536 with a residual would be the pair kernel's (vdmq_bf6_pair.hip).  Up to 2.5
         // million outputs the estimates always say one kernel (2.8 million is the least where they do not), and the call waits for the
         // host, whom they cost 0.2 us each time.
         if (p.K < 1280 || p.N <= 384 || p.M * p.N <= 2500000 || ksplit_takes(p.M, p.N, p.K, p.out_dtype) || p.M * p.N > (int64_t(1) << 40)) return true;
